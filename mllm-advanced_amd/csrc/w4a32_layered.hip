@@ -647,7 +647,7 @@ int head_row(const Run& r, int cur, int pending, int row, int M, float* logits) 
 
 int pick_token(const Run& r, int64_t* token_out, int* pos_to_advance) {
   return from_hip(w4::launch_argmax_parts(r.f32(r.g.amax_v), reinterpret_cast<const int*>(r.ws + r.g.amax_i),
-                                          w4::row_linear_partials(w4::kRowNorm, r.c->vocab), token_out, pos_to_advance, r.s));
+                                          w4::row_linear_partials(r.c->vocab), token_out, pos_to_advance, r.s));
 }
 
 int check_call(const w4a32_layered_config* c, const w4a32_layered_weights* w, const void* st, const void* ws) {

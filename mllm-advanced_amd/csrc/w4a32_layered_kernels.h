@@ -106,7 +106,7 @@ struct RowPrologue {
 // y[n] = sum_k row[k] W[n][k], f32 output; W T [N][Kp]; optionally one (max, first column) pair per wavefront
 hipError_t launch_row_linear(int kind, int dtype, const RowPrologue& pro, const void* w, int N, int Kp, float* y,
                              float* amax_val, int* amax_idx, hipStream_t s);
-int row_linear_partials(int kind, int N);  // wavefronts of that launch (<= 4096)
+int row_linear_partials(int N);  // wavefronts of that launch (<= 4096)
 bool row_linear_fits(int Kp);
 
 // bf16 product; parts > 1: C [parts][M][ldc] f32 partial products

@@ -125,11 +125,20 @@ __global__ __launch_bounds__(kRowThreads) void row_linear_kernel(const RowProlog
   }
 }
 
-// rows of W a wavefront takes at a time. A merged attention row is expensive to produce: fewer workgroups.
-int rows_per_group(int kind, int N) { return N >= 4096 ? 4 : N >= 2048 || kind == kRowMerge ? 2 : 1; }
-int row_grid(int kind, int N) {
-  const int R = rows_per_group(kind, N), groups = (N + R - 1) / R;
-  return std::min((groups + kRowWaves - 1) / kRowWaves, 512);
+// Rows of W a wavefront takes at a time, and workgroups. One row, so that the rows come out even over the wavefronts that fit at
+// once (norm: 85 registers, two workgroups per CU, 512 in all). bf16 [8960][1536] behind a norm: 8.6 us = 3.2 TB/s; four rows
+// at a time took 11.0 us: 280 workgroups of which only one fits a CU, so that 24 ran behind the others. [6144][1536]: 7.9 -> 6.8
+// us, [4632][1536]: 7.3 -> 6.7. Two rows
+//  - between 2048 and 4096 of them, where they make one workgroup per CU and single ones one and a half ([2560][2560] behind a
+//    gate: 6.8 us against 7.5 with one, [3584][3584]: 9.3 against 9.9, merged 11.3 against 15.6; [2048][2048]: 5.0 against 4.7);
+//  - from 12288 on, where the imbalance is small and half the reductions and reads of the row are saved ([18944][3584]: 26.8 us
+//    against 27.5, with four rows 28.8).
+// A large head is faster with one workgroup per CU, whose prologues are then half as many ([151936][1536]: 77.2 us = 6.0 TB/s
+// against 79.6, with four rows 81.7; [100000][2048]: 70.8 against 73.8, but [65536][1024]: 28.9 against 25.2).
+int rows_per_group(int N) { return N >= 12288 || (N > 2048 && N <= 4096) ? 2 : 1; }
+int row_grid(int N) {
+  const int R = rows_per_group(N), groups = (N + R - 1) / R;
+  return std::min((groups + kRowWaves - 1) / kRowWaves, N >= 98304 ? 256 : 512);
 }
 
 template <typename WT, int kKind, int R, int U>
@@ -141,21 +150,25 @@ hipError_t launch_row_r(const RowPrologue& p, const void* w, int N, int Kp, floa
   if (lds > 159 * 1024) return hipErrorInvalidValue;
   if (lds > 60 * 1024)
     if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), 159 * 1024); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3(row_grid(kKind, N)), dim3(kRowThreads), lds, s, p, static_cast<const WT*>(w), N, Kp, y, av,
+  hipLaunchKernelGGL(kern, dim3(row_grid(N)), dim3(kRowThreads), lds, s, p, static_cast<const WT*>(w), N, Kp, y, av,
                      ai);
   return hipGetLastError();
 }
 
+// A short row is requested whole; of a longer one, six kilobytes at a time (bf16 [1536][8960] behind PolyNorm: 9.2 us, with nine
+// 9.7, with three 9.4; f32 [1024][4096]: 7.5 us for four, eight or sixteen).
 template <typename WT, int kKind>
 hipError_t launch_row_k(const RowPrologue& p, const void* w, int N, int Kp, float* y, float* av, int* ai,
                         hipStream_t s) {
-  switch (rows_per_group(kKind, N)) {
-    case 4: return launch_row_r<WT, kKind, 4, 3>(p, w, N, Kp, y, av, ai, s);
-    case 2: return launch_row_r<WT, kKind, 2, 3>(p, w, N, Kp, y, av, ai, s);
-    default:
-      if (Kp > 6 * 512) return launch_row_r<WT, kKind, 1, 9>(p, w, N, Kp, y, av, ai, s);
-      return launch_row_r<WT, kKind, 1, 3>(p, w, N, Kp, y, av, ai, s);
-  }
+  constexpr int kStep = 64 * Raw<WT>::kE;
+  const int steps = (Kp + kStep - 1) / kStep;
+  if (rows_per_group(N) == 2)
+    return steps <= 3 ? launch_row_r<WT, kKind, 2, 3>(p, w, N, Kp, y, av, ai, s)
+                      : launch_row_r<WT, kKind, 2, 4>(p, w, N, Kp, y, av, ai, s);
+  if (steps <= 3) return launch_row_r<WT, kKind, 1, 3>(p, w, N, Kp, y, av, ai, s);
+  if (steps == 4) return launch_row_r<WT, kKind, 1, 4>(p, w, N, Kp, y, av, ai, s);
+  if (steps == 7 || steps == 8) return launch_row_r<WT, kKind, 1, 8>(p, w, N, Kp, y, av, ai, s);
+  return launch_row_r<WT, kKind, 1, 6>(p, w, N, Kp, y, av, ai, s);
 }
 
 template <typename WT>
@@ -191,7 +204,7 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
   return launch_tile<128, 128, 2, 2>(pa, pb, c, M, N, K, ldc, c_bf16, parts, s);
 }
 
-int row_linear_partials(int kind, int N) { return row_grid(kind, N) * kRowWaves; }
+int row_linear_partials(int N) { return row_grid(N) * kRowWaves; }
 // (the slices' weights of a merged attention row lie behind the row)
 bool row_linear_fits(int Kp) { return sizeof(float) * (size_t)Kp <= 140 * 1024; }
 

@@ -386,41 +386,30 @@ __device__ __forceinline__ void row_prologue(const RowPrologue& p, int Kp, float
   }
 }
 
-// eight consecutive weights as they come from memory
+// sixteen bytes of weights as they come from memory: kE consecutive elements. (A native vector: as HIP's float4, arrays of these
+// that are passed to a lambda go to scratch memory. A decode Linear of [4096][1024] in f32 took 26.8 us with that.)
 template <typename WT>
-struct Raw;
-template <>
-struct Raw<__bf16> {
-  uint4 v;
-  __device__ __forceinline__ void load(const __bf16* p) { v = *reinterpret_cast<const uint4*>(p); }
+struct Raw {
+  static constexpr int kE = 16 / (int)sizeof(WT);
+  u32x4 v;
+  __device__ __forceinline__ void load(const WT* p) { v = *reinterpret_cast<const u32x4*>(p); }
   __device__ __forceinline__ float get(int e) const {
-    const uint32_t w = e < 2 ? v.x : e < 4 ? v.y : e < 6 ? v.z : v.w;
-    return __uint_as_float(e & 1 ? w & 0xFFFF0000u : w << 16);
-  }
-};
-template <>
-struct Raw<float> {
-  float4 a, b;
-  __device__ __forceinline__ void load(const float* p) {
-    a = load4(p);
-    b = load4(p + 4);
-  }
-  __device__ __forceinline__ float get(int e) const {
-    const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    return f[e];
+    if constexpr (sizeof(WT) == 2) return __uint_as_float(e & 1 ? v[e / 2] & 0xFFFF0000u : v[e / 2] << 16);
+    else return __uint_as_float(v[e]);
   }
 };
 
-// R rows of weights at a time per wavefront, lane l multiplies k = 512 i + 8 l .. + 7; U steps of i are in flight while the
-// previous U are multiplied. ptr(g, r, k): where row r of group g has its elements k .. k + 7 (k a multiple of 8 below Kp).
+// R rows of weights at a time per wavefront, lane l multiplies k = kE (64 i + l) .. + kE - 1; U steps of i are in flight while
+// the previous U are multiplied. ptr(g, r, k): where row r of group g has its elements k .. (k a multiple of kE below Kp).
 template <typename WT, int R, int U, typename Ptr>
 __device__ __forceinline__ void fetch_rows(Raw<WT> (&raw)[R][U], int g, int bt, int Kp, Ptr ptr) {
   const int lane = threadIdx.x & 63;
+  constexpr int kE = Raw<WT>::kE;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = 512 * (bt * U + u) + 8 * lane;
+      const int k = kE * (64 * (bt * U + u) + lane);
       raw[r][u].load(ptr(g, r, k < Kp ? k : 0));
     }
 }
@@ -431,7 +420,8 @@ template <typename WT, int R, int U, typename Ptr, typename Emit>
 __device__ __forceinline__ void stream_rows(Raw<WT> (&cur)[R][U], int gw, int nw, int groups, int Kp, const float* s_x,
                                             Ptr ptr, Emit emit) {
   const int lane = threadIdx.x & 63;
-  const int steps = (Kp + 511) / 512, batches = (steps + U - 1) / U;
+  constexpr int kE = Raw<WT>::kE;
+  const int steps = (Kp + 64 * kE - 1) / (64 * kE), batches = (steps + U - 1) / U;
   for (int g = gw; g < groups; g += nw) {
     float acc[R];
 #pragma unroll
@@ -450,14 +440,15 @@ __device__ __forceinline__ void stream_rows(Raw<WT> (&cur)[R][U], int gw, int nw
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int k = 512 * (bt * U + u) + 8 * lane;
+        const int k = kE * (64 * (bt * U + u) + lane);
         if (k < Kp) {
-          const float4 x0 = load4(s_x + k), x1 = load4(s_x + k + 4);
-          const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+          f32x4 xs[kE / 4];
+#pragma unroll
+          for (int i = 0; i < kE / 4; ++i) xs[i] = load_row4(s_x + k + 4 * i);
 #pragma unroll
           for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[r] = __fmaf_rn(cur[r][u].get(e), xs[e], acc[r]);
+            for (int e = 0; e < kE; ++e) acc[r] = __fmaf_rn(cur[r][u].get(e), xs[e / 4][e % 4], acc[r]);
         }
       }
 #pragma unroll
