@@ -114,20 +114,23 @@ __device__ __forceinline__ void wave_layer_norm(const float* __restrict__ x, con
 constexpr int kNcWaves = 8;
 
 // A workgroup normalises the rows t0 - (TAPS - 1) .. t0 + TR - 1 into LDS, a wavefront per row (rows before the portion
-// come from the ring), and convolves its TR rows from there.
+// come from the ring), and convolves its TR rows from there. The first one also leaves the portion's tail in the ring, which no
+// other may then read: a portion that has rows in front of it goes in blocks of at least TAPS - 1 rows (kRowsAndTail), or, where
+// so many do not fit the LDS, in two launches.
+enum NormConvPhase { kRowsAndTail, kRowsOnly, kTailOnly };
 template <int TAPS, typename YT>
 __global__ __launch_bounds__(64 * kNcWaves) void norm_conv_kernel(
     const float* __restrict__ x, const float* __restrict__ parts, int n_parts, float* __restrict__ x_out,
     const float* __restrict__ norm_w, NormSpec spec, const float* __restrict__ conv, float* __restrict__ ring, int M, int H,
-    int ld, int pos0, int TR, YT* __restrict__ y) {
+    int ld, int pos0, int TR, YT* __restrict__ y, NormConvPhase phase) {
   extern __shared__ __align__(16) float s_h[];  // [halo + TR][ld]
   constexpr int halo = TAPS > 0 ? TAPS - 1 : 0, kRing = TAPS > 0 ? TAPS : 1;
-  const int t0 = blockIdx.x * TR, rows = min(TR, M - t0);
+  const int t0 = blockIdx.x * TR, rows = phase == kTailOnly ? 0 : min(TR, M - t0);
   const int wave = threadIdx.x >> 6;
   float4 w[kRing];  // this thread's first columns of the convolution, requested early
 #pragma unroll
   for (int j = 0; j < TAPS; ++j) w[j] = load4(conv + (size_t)j * ld + min(4 * (int)threadIdx.x, ld - 4));
-  for (int r = wave; r < halo + rows; r += kNcWaves) {
+  for (int r = wave; r < halo + rows && rows > 0; r += kNcWaves) {
     const int t = t0 - halo + r;
     float* dst = s_h + (size_t)r * ld;
     if (t >= 0) {
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(64 * kNcWaves) void norm_conv_kernel(
     }
   }
   __syncthreads();
-  for (int c = 4 * threadIdx.x; c < ld; c += 256 * kNcWaves) {
+  for (int c = 4 * threadIdx.x; c < ld && rows > 0; c += 256 * kNcWaves) {
     float4 win[kRing];  // win[j]: h of the position j before the current one
     if (c >= 256 * kNcWaves) {
 #pragma unroll
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(64 * kNcWaves) void norm_conv_kernel(
       store4(y + (size_t)(t0 + r) * ld + c, v);
     }
   }
-  if (blockIdx.x != 0 || TAPS < 2) return;
+  if (blockIdx.x != 0 || TAPS < 2 || phase == kRowsOnly) return;
   // the tail for the next portion: this workgroup has read the ring, nobody else does
   __syncthreads();
   for (int t = max(0, M - halo) + wave; t < M; t += kNcWaves) {
@@ -364,14 +367,22 @@ template <int TAPS, typename YT>
 static hipError_t norm_conv_t(const float* x, const float* parts, int n_parts, float* x_out, const float* norm_w,
                               const NormSpec& spec, const float* conv, float* ring, int M, int H, int ld, int pos0, YT* y,
                               hipStream_t s) {
-  const int TR = norm_conv_rows(M, ld, TAPS);
+  int TR = norm_conv_rows(M, ld, TAPS);
+  bool split = false;
+  if (constexpr int halo = TAPS > 0 ? TAPS - 1 : 0; pos0 > 0 && TR < halo && TR < M) {
+    if (norm_conv_lds(ld, TAPS, halo) <= 160 * 1024) TR = halo;
+    else split = true;
+  }
   const size_t lds = norm_conv_lds(ld, TAPS, TR);
   auto kern = norm_conv_kernel<TAPS, YT>;
   static LdsLimitOnce raised;
   if (lds > 64 * 1024)
     if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), 160 * 1024); e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((M + TR - 1) / TR), dim3(64 * kNcWaves), lds, s, x, parts, n_parts, x_out, norm_w, spec,
-                     conv, ring, M, H, ld, pos0, TR, y);
+                     conv, ring, M, H, ld, pos0, TR, y, split ? kRowsOnly : kRowsAndTail);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || !split) return e;
+  hipLaunchKernelGGL(kern, dim3(1), dim3(64 * kNcWaves), lds, s, x, parts, n_parts, nullptr, norm_w, spec, conv, ring, M, H, ld,
+                     pos0, TR, y, kTailOnly);
   return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
 """GPU: the layered decoder's kernels at the sizes where a variant or a split of the work changes, against the float64 oracle or
 a float64 product."""
+import numpy as np
 import pytest
 
 import layered_models as lm
@@ -26,3 +27,32 @@ def test_decode_linear_splits(width, vocab, ff, dtype):
     ref = lo.forward(cfg, w, tokens)
     for i, t in enumerate(tokens):
         assert lm.errors(dec.forward(state, [t], i), ref[i:i + 1]).max() < TOL[dtype], i
+
+
+@pytest.mark.parametrize("H,taps,first,rest", [
+    (64, 8, 3, 45),      # more workgroups than one would read the ring if each took a single row
+    (1600, 4, 2, 40),
+    (330, 4, 1, 3),
+    (5100, 8, 9, 20),    # seven rows of halo and seven more do not fit the LDS: rows and tail in two launches
+    (5100, 8, 4, 3),     # ... with a tail that keeps older rows
+])
+def test_norm_conv_leaves_its_tail_when_nobody_reads_the_ring(pkg, H, taps, first, rest):
+    import torch
+
+    rng = np.random.default_rng(H + taps)
+    T, ld = first + rest + 5, (H + 63) // 64 * 64
+    x, w, cw = rng.standard_normal((T, H)), rng.standard_normal(H), rng.standard_normal((H, taps)) * 0.5
+    h = lo.layer_norm(x, w, 1e-5)
+    ref = h + lo.causal_conv(h, cw)
+
+    def dev(a):
+        out = torch.zeros(a.shape[:-1] + (ld,), device="cuda")
+        out[..., :H] = torch.tensor(a)
+        return out
+    for _ in range(20):
+        ring, at = torch.full((taps, ld), float("nan"), device="cuda"), 0
+        for n in (first, rest, 5):
+            y, _ = pkg.op_layernorm_conv(dev(x[at:at + n]), dev(w), 1e-5, dev(cw.T), ring, H, at)
+            # f32 sums of up to 5100 terms of size 1: a few 1e-6 of the largest value
+            assert np.abs(y.double().cpu().numpy()[:, :H] - ref[at:at + n]).max() < 5e-6 * np.abs(ref).max(), (at, n)
+            at += n
