@@ -35,9 +35,6 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 #define W4_LAUNCH(expr) W4_TRY(from_hip(expr))
 
 constexpr int kArgmaxParts = 4096;
-constexpr size_t kSplitFloats = (size_t)768 * 128 * 128;  // what a product split over k leaves at most (fewer than
-                                                          // 768 tiles of 128 x 128, or 1536 of 64 x 64)
-
 struct LayerGeom {
   int rows;         // rows of in_proj
   int conv_rows;    // ... of which pass the short convolution
@@ -176,7 +173,7 @@ Geom geometry(const w4a32_layered_config* c) {
     return at;
   };
   int raw = 0, cx = 0, q = 0, mix = 0, ff = 0, z = 0, ofl = 0, mlfl = 0, cq = 0, qa = 0, head_out = 0, experts = 0;
-  size_t rec = 0, expand = 0, moe = 0, parts = g.Hp * Mb;
+  size_t rec = 0, expand = 0, moe = 0, parts = 2 * g.Hp * Mb;
   g.runs = layer_runs(c);
   auto rot_table = [&](int dims, double base) {
     if (dims == 0) return -1;
@@ -299,7 +296,7 @@ Geom geometry(const w4a32_layered_config* c) {
   g.cx = take(sizeof(float) * Mb * cx);
   g.q = take((size_t)g.elem * Mb * q);
   g.mix = take((size_t)g.elem * Mb * mix);
-  g.parts = take(sizeof(float) * std::max(parts, kSplitFloats));
+  g.parts = take(sizeof(float) * std::max(parts, w4::kSplitFloats));
   g.ff = take((size_t)g.elem * Mb * ff);
   g.z = take(sizeof(float) * std::max(ff, z));
   g.o = take(sizeof(float) * ofl);

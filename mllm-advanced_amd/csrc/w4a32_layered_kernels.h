@@ -112,7 +112,9 @@ bool row_linear_fits(int Kp);
 // bf16 product; parts > 1: C [parts][M][ldc] f32 partial products
 hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int N, int K, int ldc, bool c_bf16,
                               int parts, hipStream_t s);
-int matmul_bf16_parts(int M, int N, int K);  // parts worth using for few tiles
+// Parts worth using: 1, or as many as fit max(kSplitFloats, 2 M N) floats.
+int matmul_bf16_parts(int M, int N, int K);
+constexpr size_t kSplitFloats = (size_t)768 * 128 * 128;
 
 // ---- rows of a prefill ----
 hipError_t launch_embed_rows(int dtype, const int64_t* ids, const void* table, int M, int H, int ld, int vocab,

@@ -1,12 +1,14 @@
 // Linears with bf16 (or f32) weights for the layered decoder.
 //
-//   matmul_bf16_kernel   C = A B^T, bf16 operands, f32 accumulation (v_mfma_f32_32x32x16_bf16), for prefill rows.
+//   matmul_bf16_kernel   C = A B^T, bf16 operands, f32 accumulation (v_mfma_f32_32x32x16_bf16), for prefill rows: tiles from
+//                        64 x 64 to 256 x 256, the k range dealt to several workgroups where the caller adds the parts up.
 //   row_linear_kernel    one decode row through [N][K] weights, read once, with the operator that produces the row
 //                        in front (residual add + norm + input convolution, merge of the attention's key slices,
 //                        per-head norm and gate, PolyNorm, none): HBM-bound, N * K * sizeof(weight) bytes.
 //
 // The tile of C a workgroup owns and the rows a decode Linear multiplies are in w4a32_mfma_tile.h and w4a32_row_prologue.h.
 #include <algorithm>
+#include <cmath>
 
 #include "w4a32_layered.h"
 #include "w4a32_layered_kernels.h"
@@ -17,11 +19,11 @@ namespace w4 {
 
 namespace {
 
-template <int BM, int BN, int WM, int WN, typename CT>
+template <int BM, int BN, int WM, int WN, int D, typename CT>
 __global__ __launch_bounds__(64 * WM * WN) void matmul_bf16_kernel(const __bf16* __restrict__ a,
                                                                    const __bf16* __restrict__ b, CT* __restrict__ c,
                                                                    int M, int N, int K, int ldc, int mt, int nt) {
-  using Tile = MfmaTile<__bf16, BM, BN, WM, WN>;
+  using Tile = MfmaTile<__bf16, BM, BN, WM, WN, D>;
   constexpr int FM = Tile::FM, FN = Tile::FN, kBK = Tile::kBK;
   extern __shared__ __align__(16) uint8_t smem[];
 
@@ -35,54 +37,102 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_bf16_kernel(const __bf16*
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
 
-  const __bf16* ga[Tile::LA];
-  const __bf16* gb[Tile::LB];
+  unsigned oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
-  for (int i = 0; i < Tile::LA; ++i) ga[i] = a + (size_t)min(m0 + Tile::row(i), M - 1) * K + Tile::k();
+  for (int i = 0; i < Tile::LA; ++i) oa[i] = 2u * Tile::row(i) * K + Tile::column();
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) gb[i] = b + (size_t)min(n0 + Tile::row(i), N - 1) * K + Tile::k();
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = 2u * Tile::row(i) * K + Tile::column();
+  const int ma = min(M - m0, BM), nb = min(N - n0, BN);
   f32x16 acc[FM][FN];
-  Tile::run(smem, ga, gb, kb, ke, acc);
+  Tile::run(smem, rows_buffer(a + (size_t)m0 * K, (size_t)2 * ma * K), oa,
+            rows_buffer(b + (size_t)n0 * K, (size_t)2 * nb * K), ob, kb, ke, acc);
 
-  c += (size_t)blockIdx.y * M * ldc;
+  // rows past the last one lie past the buffer's end, columns are sent there: what is stored there is dropped
+  c += (size_t)blockIdx.y * M * ldc + (size_t)m0 * ldc;
+  const __amdgpu_buffer_rsrc_t out = rows_buffer(c, sizeof(CT) * ma * ldc);
+  const unsigned step = (unsigned)sizeof(CT) * ldc;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int col = n0 + wn + 32 * j + (lane & 31);
+      unsigned off = col < N ? (unsigned)sizeof(CT) * ((wm + 32 * i + 4 * (lane >> 5)) * ldc + col) : 0xF0000000u;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        if (row < M && col < N) c[(size_t)row * ldc + col] = (CT)acc[i][j][v];
+        float x = acc[i][j][v];
+        asm volatile("" : "+v"(x), "+v"(off));  // or all offsets, and a copy of acc as integers, are made first, and spilled
+        if constexpr (sizeof(CT) == 4) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), out, off, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (CT)x), out, off, 0, 0);
+        off += v % 4 == 3 ? 5 * step : step;
       }
     }
 }
 
-template <int BM, int BN, int WM, int WN>
-hipError_t launch_tile(const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, bool c_bf16, int parts,
-                       hipStream_t s) {
+template <int BM, int BN, int WM, int WN, int D, typename CT>
+hipError_t launch_tile_t(const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
   const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
-  const dim3 grid(mt * nt, parts), block(64 * WM * WN);  // parts <= K / kBK: no share is empty
-  constexpr size_t lds = MfmaTile<__bf16, BM, BN, WM, WN>::kLds;
-  if (c_bf16) {
-    auto kern = matmul_bf16_kernel<BM, BN, WM, WN, __bf16>;
-    static LdsLimitOnce raised;
-    if (lds > 64 * 1024)
-      if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, grid, block, lds, s, a, b, static_cast<__bf16*>(c), M, N, K, ldc, mt, nt);
-  } else {
-    auto kern = matmul_bf16_kernel<BM, BN, WM, WN, float>;
-    static LdsLimitOnce raised;
-    if (lds > 64 * 1024)
-      if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, grid, block, lds, s, a, b, static_cast<float*>(c), M, N, K, ldc, mt, nt);
-  }
+  constexpr size_t lds = MfmaTile<__bf16, BM, BN, WM, WN, D>::kLds;
+  auto kern = matmul_bf16_kernel<BM, BN, WM, WN, D, CT>;
+  static LdsLimitOnce raised;
+  if (lds > 64 * 1024)
+    if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
+  // parts <= K / kBK: no share is empty
+  hipLaunchKernelGGL(kern, dim3(mt * nt, parts), dim3(64 * WM * WN), lds, s, a, b, static_cast<CT*>(c), M, N, K, ldc, mt, nt);
   return hipGetLastError();
 }
 
-// 128 x 128 tiles where they fill the CUs (dealt over k when the caller takes partial products), else 64 x 64
-long tiles_of(int M, int N, int t) { return (long)((M + t - 1) / t) * ((N + t - 1) / t); }
-bool small_tiles(int M, int N, int parts) { return tiles_of(M, N, 128) < (parts > 1 ? 96 : 192); }
+// The shapes, and what they cost. A CU that is alone takes tile_us per 64 k of a tile; with all of them busy the chip's clock
+// drops and it delivers `tflops`. (Fitted to 16 sizes from [40][1536] x [8960][1536] to [2048][3584] x [14336][3584], within
+// 15 %.)
+struct Shape {
+  int bm, bn;
+  double tile_us, tflops;
+};
+constexpr Shape kShapes[] = {
+    {256, 256, 1.13, 1270}, {256, 128, 0.70, 1060}, {128, 128, 0.46, 950}, {64, 128, 0.36, 660}, {64, 64, 0.25, 490}};
+constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
+
+// us: rounds of the CUs, and the results' way to memory (and, as partial products, back)
+double shape_us(const Shape& t, int M, int N, int K, int parts, int c_bytes) {
+  const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
+  const double k_tiles = (double)K / 64 / parts, flops = 2.0 * t.bm * t.bn * 64 * k_tiles;
+  auto round_us = [&](long n) { return std::max(t.tile_us * k_tiles, n * flops / (t.tflops * 1e6)); };
+  const double out = (double)M * N * c_bytes * (2 * parts - 1) / 5e6;
+  return 2.5 + tiles / 256 * round_us(256) + (tiles % 256 ? round_us(tiles % 256) : 0.0) + out;
+}
+
+struct Plan {
+  int shape, parts;
+};
+
+// The cheapest shape; with most_parts > 1 also the number of partial products (1, 2, 4, 8) that go with it.
+Plan best_plan(int M, int N, int K, int parts, int most_parts, int c_bytes) {
+  Plan best{0, parts};
+  double least = INFINITY;
+  for (int p = parts; p <= most_parts; p *= 2) {
+    if (p > parts && K / p < 512) break;
+    for (int i = 0; i < kShapeCount; ++i) {
+      const double us = shape_us(kShapes[i], M, N, K, p, c_bytes);
+      if (us < least) {
+        least = us;
+        best = {i, p};
+      }
+    }
+  }
+  return best;
+}
+
+template <typename CT>
+hipError_t launch_shape(int shape, const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, int parts,
+                        hipStream_t s) {
+  switch (shape) {
+    case 0: return launch_tile_t<256, 256, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 1: return launch_tile_t<256, 128, 4, 2, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 2: return launch_tile_t<128, 128, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 3: return launch_tile_t<64, 128, 2, 4, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
+    default: return launch_tile_t<64, 64, 2, 2, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
+  }
+}
 
 // ---------------------------------------------------------------------------------------------
 template <typename WT, int kKind, int R, int U>
@@ -188,11 +238,9 @@ hipError_t launch_row_t(int kind, const RowPrologue& p, const void* w, int N, in
 }  // namespace
 
 int matmul_bf16_parts(int M, int N, int K) {
-  const bool small = small_tiles(M, N, 2);
-  const long tiles = tiles_of(M, N, small ? 64 : 128), enough = small ? 768 : 384;
-  int parts = 1;
-  while (parts < 8 && tiles * parts < enough && K / (2 * parts) >= 512) parts *= 2;
-  return parts;
+  int most = 8;  // two always fit what the caller has for them
+  while (most > 2 && (size_t)most * M * N > kSplitFloats) most /= 2;
+  return best_plan(M, N, K, 1, most, 4).parts;
 }
 
 hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int N, int K, int ldc, bool c_bf16,
@@ -200,8 +248,9 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
   if (K % kPad != 0 || parts < 1 || parts > K / kPad || (parts > 1 && c_bf16)) return hipErrorInvalidValue;
   const __bf16* pa = static_cast<const __bf16*>(a);
   const __bf16* pb = static_cast<const __bf16*>(b);
-  if (small_tiles(M, N, parts)) return launch_tile<64, 64, 2, 2>(pa, pb, c, M, N, K, ldc, c_bf16, parts, s);
-  return launch_tile<128, 128, 2, 2>(pa, pb, c, M, N, K, ldc, c_bf16, parts, s);
+  const int shape = best_plan(M, N, K, parts, parts, c_bf16 ? 2 : 4).shape;
+  return c_bf16 ? launch_shape<__bf16>(shape, pa, pb, c, M, N, K, ldc, parts, s)
+                : launch_shape<float>(shape, pa, pb, c, M, N, K, ldc, parts, s);
 }
 
 int row_linear_partials(int N) { return row_grid(N) * kRowWaves; }

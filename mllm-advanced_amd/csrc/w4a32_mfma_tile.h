@@ -1,11 +1,21 @@
 // The tile of C = A B^T that one workgroup computes: WM x WN wavefronts, each with FM x FN accumulators of 32 x 32. bf16
-// operands on v_mfma_f32_32x32x16_bf16, f32 operands on v_mfma_f32_32x32x2_f32. The caller says where the rows lie (a row per
-// pointer, so they may be gathered) and what becomes of the accumulators: lane l of a 32 x 32 block holds column l % 32 and,
-// in register v, row 8 (v / 4) + 4 (l / 32) + v % 4.
+// operands on v_mfma_f32_32x32x16_bf16, f32 operands on v_mfma_f32_32x32x2_f32. The caller says where the rows lie (a buffer and
+// a byte offset per row, so they may be gathered; what lies past the buffer's end reads as zeros) and what becomes of the
+// accumulators: lane l of a 32 x 32 block holds column l % 32 and, in register v, row 8 (v / 4) + 4 (l / 32) + v % 4. Every shape
+// adds the products of an output in the same order.
 //
-// bf16: tiles of 64 k are brought in through registers (requested one or two tiles ahead) and double-buffered in LDS as rows of
-// 64 + 8 elements: the 144-byte stride puts 16 consecutive rows' 16-byte operands on all 64 banks once. f32 (the
-// exact format, not tuned): tiles of 16 k, rows of 16 + 1 floats.
+// bf16: tiles of 64 k, brought in through registers (D tiles requested ahead) and double-buffered in LDS as rows of 64 + 8
+// elements: the 144-byte stride puts 16 consecutive rows' 16-byte operands on all 64 banks once. What bounds a shape: a
+// wavefront reads FM + FN kilobytes of LDS for FM x FN products of 32 clocks on its SIMD, all four SIMDs share 128 bytes a
+// clock, and the tile's own writes come on top. 128 x 128 on four wavefronts needs 768 LDS clocks for 512 clocks of products,
+// 256 x 128 on eight 1152 for 1024, 256 x 256 on eight 2048 for 2048 with two wavefronts to a SIMD that fill each other's gaps.
+// The order inside a tile is written out and fenced, as the compiler otherwise moves all LDS reads in front of the products:
+// behind each product come the next step's fragments, in the first two steps the next tile's way from registers to LDS, in the
+// last two the request for a tile D further on. The one barrier per tile stands in front of the last step's products, whose
+// fragments are in registers by then, so that the next tile's first fragments are on their way under them.
+// [2048][3584] x [14336][3584]: 128 x 128 on four wavefronts without this order 272 us (775 TFLOP/s), with it 235; 256 x 128
+// 213, 256 x 256 185 us (1140 TFLOP/s, and at 1.3 GHz the clock is what the chip sustains under it).
+// f32 (the exact format, not tuned): tiles of 16 k, rows of 16 + 1 floats.
 #pragma once
 
 #include "w4a32_layered_kernels.h"
@@ -19,42 +29,65 @@ __device__ __forceinline__ int xcd_tile(int block, int tiles) {
   return x * per + min(x, rem) + i;
 }
 
-template <typename T, int BM, int BN, int WM, int WN>
+// `bytes` at base as a buffer; loads past its end give zeros. base and bytes are the same in all lanes.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* base, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(unsigned)bytes, 0x00020000);
+}
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned lane_off, unsigned off) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int D>
 struct MfmaTile;
 
-template <int BM, int BN, int WM, int WN>
-struct MfmaTile<__bf16, BM, BN, WM, WN> {
+template <int BM, int BN, int WM, int WN, int D>
+struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
   static constexpr int kThreads = 64 * WM * WN;
-  static constexpr int FM = BM / WM / 32, FN = BN / WN / 32;           // 32 x 32 blocks of a wavefront
+  static constexpr int FM = BM / WM / 32, FN = BN / WN / 32;            // 32 x 32 blocks of a wavefront
   static constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads;  // 16-byte pieces a thread brings per tile
-  static constexpr int kBK = 64, kLd = kBK + 8;                         // k per LDS tile; LDS row, elements
+  static constexpr int kBK = 64, kLd = kBK + 8, kSteps = kBK / 16;      // k per LDS tile; LDS row, elements
   static constexpr size_t kLds = 2 * (BM + BN) * kLd * sizeof(__bf16);
-  // the row of A (B) that this thread's piece i is from, and the piece's first k
+  // the row of A (B) that this thread's piece i is from, and the piece's first byte in it
   static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x + kThreads * i) >> 3; }
-  static __device__ __forceinline__ int k() { return 8 * (threadIdx.x & 7); }
+  static __device__ __forceinline__ unsigned column() { return 16 * (threadIdx.x & 7); }
 
-  // acc = rows of A times rows of B over k in [kb, ke), a range of whole tiles that is not empty
-  static __device__ __forceinline__ void run(uint8_t* smem, const __bf16* const (&ga)[LA], const __bf16* const (&gb)[LB],
-                                             int kb, int ke, f32x16 (&acc)[FM][FN]) {
-    __bf16* s_a = reinterpret_cast<__bf16*>(smem);                 // [2][BM][kLd]
-    __bf16* s_b = s_a + 2 * BM * kLd;                              // [2][BN][kLd]
+  // acc = rows of A times rows of B over k in [kb, ke), a range of whole tiles that is not empty; oa, ob: where the pieces'
+  // rows start, with column() added
+  static __device__ __forceinline__ void run(uint8_t* smem, __amdgpu_buffer_rsrc_t a, const unsigned (&oa)[LA],
+                                             __amdgpu_buffer_rsrc_t b, const unsigned (&ob)[LB], int kb, int ke,
+                                             f32x16 (&acc)[FM][FN]) {
+    __bf16* s_a = reinterpret_cast<__bf16*>(smem);  // [2][BM][kLd]
+    __bf16* s_b = s_a + 2 * BM * kLd;               // [2][BN][kLd]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-    // two register sets: two tiles in flight
-    u32x4 ra0[LA], rb0[LB], ra1[LA], rb1[LB];
-    auto fetch = [&](int k, u32x4 (&ra)[LA], u32x4 (&rb)[LB]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const u32x4*>(ga[i] + k);
-#pragma unroll
-      for (int i = 0; i < LB; ++i) rb[i] = *reinterpret_cast<const u32x4*>(gb[i] + k);
-    };
+    constexpr int kPieces = LA + LB, kFrags = FM + FN, kProducts = FM * FN;
+    u32x4 ra[D][LA], rb[D][LB];
+    bf16x8 fa[2][FM], fb[2][FN];
     __bf16* const sa_w = s_a + (tid >> 3) * kLd + 8 * (tid & 7);
     __bf16* const sb_w = s_b + (tid >> 3) * kLd + 8 * (tid & 7);
-    auto stash = [&](int buf, const u32x4 (&ra)[LA], const u32x4 (&rb)[LB]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) *reinterpret_cast<u32x4*>(sa_w + (buf * BM + kThreads / 8 * i) * kLd) = ra[i];
-#pragma unroll
-      for (int i = 0; i < LB; ++i) *reinterpret_cast<u32x4*>(sb_w + (buf * BN + kThreads / 8 * i) * kLd) = rb[i];
+    const __bf16* const sa_r = s_a + (wm + (lane & 31)) * kLd + 8 * (lane >> 5);
+    const __bf16* const sb_r = s_b + (wn + (lane & 31)) * kLd + 8 * (lane >> 5);
+    auto fetch = [&](int set, int p, int k) __attribute__((always_inline)) {
+      if (p < LA) ra[set][p < LA ? p : 0] = load16(a, oa[p < LA ? p : 0], 2 * k);
+      else rb[set][p < LA ? 0 : p - LA] = load16(b, ob[p < LA ? 0 : p - LA], 2 * k);
+    };
+    auto stash = [&](int set, int p, int buf) __attribute__((always_inline)) {
+      if (p < LA) *reinterpret_cast<u32x4*>(sa_w + (buf * BM + kThreads / 8 * p) * kLd) = ra[set][p < LA ? p : 0];
+      else *reinterpret_cast<u32x4*>(sb_w + (buf * BN + kThreads / 8 * (p - LA)) * kLd) = rb[set][p < LA ? 0 : p - LA];
+    };
+    // fragment r of step ks, in the order of their first use: b0, a0, b1, a1, ..
+    auto frag = [&](int r, int set, int buf, int ks) __attribute__((always_inline)) {
+      constexpr int kPairs = 2 * (FM < FN ? FM : FN);
+      const bool of_b = r < kPairs ? (r & 1) == 0 : FN > FM;
+      const int i = r < kPairs ? r / 2 : r - kPairs / 2;
+      if (of_b) fb[set][i] = *reinterpret_cast<const bf16x8*>(sb_r + (buf * BN + 32 * i) * kLd + 16 * ks);
+      else fa[set][i] = *reinterpret_cast<const bf16x8*>(sa_r + (buf * BM + 32 * i) * kLd + 16 * ks);
+    };
+    // every wavefront's LDS traffic so far is done (loads from memory stay on their way)
+    auto barrier = [] __attribute__((always_inline)) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
     };
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -63,59 +96,74 @@ struct MfmaTile<__bf16, BM, BN, WM, WN> {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-    auto products = [&](int buf) __attribute__((always_inline)) {
-      const __bf16* pa = s_a + (size_t)buf * BM * kLd + (wm + (lane & 31)) * kLd + 8 * (lane >> 5);
-      const __bf16* pb = s_b + (size_t)buf * BN * kLd + (wn + (lane & 31)) * kLd + 8 * (lane >> 5);
+    const int last = ke - kBK;  // a tile past the end is fetched as the last one again and not used
 #pragma unroll
-      for (int ks = 0; ks < kBK / 16; ++ks) {
-        bf16x8 fa[FM], fb[FN];
+    for (int d = 0; d < D; ++d)
 #pragma unroll
-        for (int i = 0; i < FM; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(pa + 32 * i * kLd + 16 * ks);
+      for (int p = 0; p < kPieces; ++p) fetch(d, p, min(kb + d * kBK, last));
 #pragma unroll
-        for (int j = 0; j < FN; ++j) fb[j] = *reinterpret_cast<const bf16x8*>(pb + 32 * j * kLd + 16 * ks);
+    for (int p = 0; p < kPieces; ++p) stash(0, p, 0);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+    for (int p = 0; p < kPieces; ++p) fetch(0, p, min(kb + D * kBK, last));
+    barrier();
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    for (int r = 0; r < kFrags; ++r) frag(r, 0, 0, 0);
+
+    // Tile u (of a turn) out of buffer u % 2; the tile behind it goes from register set (u + 1) % D to the other buffer, and the
+    // set takes the tile at k.
+    auto tile = [&](int u, int k) __attribute__((always_inline)) {
+      const int buf = u & 1, set = (u + 1) % D;
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) {
+        if (ks == kSteps - 1) barrier();
+#pragma unroll
+        for (int m = 0; m < kProducts; ++m) {
+          const int i = m / FN, j = m % FN;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks & 1][i], fb[ks & 1][j], acc[i][j], 0, 0, 0);
+          // the fragments are spread over three quarters of the products
+          constexpr int kSlots = kProducts < 4 ? 1 : kProducts * 3 / 4;
+#pragma unroll
+          for (int r = 0; r < kFrags; ++r)
+            if (r * kSlots / kFrags == m) {
+              if (ks + 1 < kSteps) frag(r, (ks + 1) & 1, buf, ks + 1);
+              else frag(r, 0, buf ^ 1, 0);
+            }
+#pragma unroll
+          for (int p = 0; p < kPieces; ++p)
+            if (p * 2 * kProducts / kPieces == (ks & 1) * kProducts + m) {
+              if (ks < 2) stash(set, p, buf ^ 1);
+              else fetch(set, p, k);
+            }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     };
-
-    // Tile i is stashed from register set i & 1 into LDS buffer i & 1; while it is multiplied, tiles i + 1 and i + 2
-    // are on their way.
-    const int last = ke - kBK;  // a tile past the end is fetched as the last one again and not used
-    fetch(kb, ra0, rb0);
-    fetch(min(kb + kBK, last), ra1, rb1);
-    stash(0, ra0, rb0);
-    fetch(min(kb + 2 * kBK, last), ra0, rb0);
-    __syncthreads();
-    for (int k = kb; k < ke; k += 2 * kBK) {
-      // even tile: LDS buffer 0; the next one sits in register set 1
-      stash(1, ra1, rb1);
-      fetch(min(k + 3 * kBK, last), ra1, rb1);
-      products(0);
-      __syncthreads();
-      if (k + kBK >= ke) break;
-      stash(0, ra0, rb0);
-      fetch(min(k + 4 * kBK, last), ra0, rb0);
-      products(1);
-      __syncthreads();
+    constexpr int kTurn = D < 2 ? 2 : D;
+    static_assert(kTurn % 2 == 0, "buffers and register sets come round together");
+    int k = kb;
+    for (; k + (kTurn - 1) * kBK < ke; k += kTurn * kBK) {
+#pragma unroll
+      for (int u = 0; u < kTurn; ++u) tile(u, min(k + (u + 1 + D) * kBK, last));
     }
+#pragma unroll
+    for (int u = 0; u < kTurn - 1; ++u)  // (not by leaving the loop: its accumulators would be copied)
+      if (k + u * kBK < ke) tile(u, last);
   }
 };
 
-template <int BM, int BN, int WM, int WN>
-struct MfmaTile<float, BM, BN, WM, WN> {
+template <int BM, int BN, int WM, int WN, int D>
+struct MfmaTile<float, BM, BN, WM, WN, D> {
   static constexpr int kThreads = 64 * WM * WN;
   static constexpr int FM = BM / WM / 32, FN = BN / WN / 32;
   static constexpr int LA = BM * 4 / kThreads, LB = BN * 4 / kThreads;
   static constexpr int kBK = 16, kLd = kBK + 1;
   static constexpr size_t kLds = (BM + BN) * kLd * sizeof(float);
   static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x + kThreads * i) >> 2; }
-  static __device__ __forceinline__ int k() { return 4 * (threadIdx.x & 3); }
+  static __device__ __forceinline__ unsigned column() { return 16 * (threadIdx.x & 3); }
 
-  static __device__ __forceinline__ void run(uint8_t* smem, const float* const (&ga)[LA], const float* const (&gb)[LB],
-                                             int kb, int ke, f32x16 (&acc)[FM][FN]) {
+  static __device__ __forceinline__ void run(uint8_t* smem, __amdgpu_buffer_rsrc_t a, const unsigned (&oa)[LA],
+                                             __amdgpu_buffer_rsrc_t b, const unsigned (&ob)[LB], int kb, int ke,
+                                             f32x16 (&acc)[FM][FN]) {
     float* s_a = reinterpret_cast<float*>(smem);
     float* s_b = s_a + BM * kLd;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -129,18 +177,18 @@ struct MfmaTile<float, BM, BN, WM, WN> {
     for (int k0 = kb; k0 < ke; k0 += kBK) {
       f32x4 ra[LA], rb[LB];
 #pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const f32x4*>(ga[i] + k0);
+      for (int i = 0; i < LA; ++i) ra[i] = __builtin_bit_cast(f32x4, load16(a, oa[i], 4 * k0));
 #pragma unroll
-      for (int i = 0; i < LB; ++i) rb[i] = *reinterpret_cast<const f32x4*>(gb[i] + k0);
+      for (int i = 0; i < LB; ++i) rb[i] = __builtin_bit_cast(f32x4, load16(b, ob[i], 4 * k0));
       __syncthreads();  // the previous tile's reads are done
 #pragma unroll
       for (int i = 0; i < LA; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s_a[row(i) * kLd + k() + e] = ra[i][e];
+        for (int e = 0; e < 4; ++e) s_a[row(i) * kLd + 4 * (threadIdx.x & 3) + e] = ra[i][e];
 #pragma unroll
       for (int i = 0; i < LB; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s_b[row(i) * kLd + k() + e] = rb[i][e];
+        for (int e = 0; e < 4; ++e) s_b[row(i) * kLd + 4 * (threadIdx.x & 3) + e] = rb[i][e];
       __syncthreads();
 #pragma unroll
       for (int kk = 0; kk < kBK; kk += 2) {

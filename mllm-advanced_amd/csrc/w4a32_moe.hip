@@ -22,9 +22,14 @@ constexpr int kMaxParts = kMoeLogitParts;
 constexpr int kLogitRegs = W4A32_LAYERED_MAX_EXPERTS / 64;
 static_assert(W4A32_LAYERED_MAX_TOP <= 64, "a lane per chosen expert");
 
+// T: what the result is rounded to. For bf16 the hardware's exponential and reciprocal (1 ulp of f32 each) do: in the epilogue of
+// a grouped product the correctly rounded ones took as long as a fifth of its products.
+template <typename T>
 __device__ __forceinline__ float clamped_glu(float g, float u, float limit) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
+  if constexpr (sizeof(T) == 2)
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kGluAlpha * 1.44269504f * g)) * (u + 1.0f);
   return g * sigmoid_f(kGluAlpha * g) * (u + 1.0f);
 }
 
@@ -98,9 +103,10 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
   }
 }
 
+// A tile of an expert: all of them say the same, so that a workgroup needs one of them only, whichever of them it takes.
 struct MoeTile {
-  int expert, row0, rows;  // rows of the sorted list
-  int first, tiles;        // the expert's first tile and how many it has
+  int expert, row0, rows;  // the expert's rows of the sorted list
+  int first, tiles;        // its first tile and how many it has
   int pad[3];
 };
 
@@ -169,95 +175,119 @@ __global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __res
     if (ids[i] == e) order[at++] = i;
   const int count = total, mt = (count + bm - 1) / bm;
   for (int t = tid; t < mt; t += kPlanThreads)
-    tiles[first + t] = MoeTile{e, offset + t * bm, min(bm, count - t * bm), first, mt, {0, 0, 0}};
+    tiles[first + t] = MoeTile{e, offset, count, first, mt, {0, 0, 0}};
   if (e == experts - 1 && tid == 0) *n_tiles = first + mt;
 }
 static_assert(kPlanThreads >= W4A32_LAYERED_MAX_EXPERTS, "a thread per expert");
 
 // The tile of a workgroup: an expert's tiles are numbered rows fastest, experts one after the other; consecutive numbers on one
-// XCD. Returns false past the last one.
-__device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, const int* __restrict__ n_tiles, int nt,
+// XCD. `row0` and `rows` become the tile's. Returns false past the last one.
+__device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, const int* __restrict__ n_tiles, int bm, int nt,
                                          MoeTile* tile, int* n) {
   const int total = *n_tiles * nt;
   if ((int)blockIdx.x >= total) return false;
   const int t = xcd_tile(blockIdx.x, total);
-  const MoeTile any = tiles[t / nt];  // a tile of the expert
-  if (any.tiles <= 0) return false;
-  const int local = t - any.first * nt;
-  *tile = tiles[any.first + local % any.tiles];
-  *n = local / any.tiles;
+  *tile = tiles[t / nt];
+  if (tile->tiles <= 0) return false;
+  const int local = t - tile->first * nt, at = local % tile->tiles * bm;
+  *n = local / tile->tiles;
+  tile->row0 += at;
+  tile->rows = min(bm, tile->rows - at);
   return true;
 }
 
-// act [sorted pair][Fp] = glu(h gate^T, h up^T)
-template <typename T, int BM>
-__global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ h, const T* __restrict__ w,
-                                                          T* __restrict__ act, const int* __restrict__ order,
-                                                          const MoeTile* __restrict__ tiles, const int* __restrict__ n_tiles,
-                                                          int top, int Hp, int Fp, float limit) {
-  using Tile = MfmaTile<T, BM, 128, 2, 2>;
+// act [sorted pair][Fp] = glu(h gate^T, h up^T). A wavefront's column blocks are gate and up of the same 32 columns, in turn.
+template <typename T, int BM, int BN, int WM, int WN, int D>
+__global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __restrict__ h, const T* __restrict__ w,
+                                                                   T* __restrict__ act, const int* __restrict__ order,
+                                                                   const MoeTile* __restrict__ tiles,
+                                                                   const int* __restrict__ n_tiles, int M, int top, int Hp,
+                                                                   int Fp, float limit) {
+  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
+  static_assert(Tile::FN % 2 == 0, "gate and up in one wavefront");
   extern __shared__ __align__(16) uint8_t smem[];
   MoeTile tile;
   int n;
   const int N = 2 * Fp;
-  if (!moe_tile(tiles, n_tiles, (N + 127) / 128, &tile, &n)) return;
-  const int n0 = 128 * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const T* we = w + (size_t)tile.expert * N * Hp;
-  const T* ga[Tile::LA];
-  const T* gb[Tile::LB];
+  if (!moe_tile(tiles, n_tiles, BM, (N + BN - 1) / BN, &tile, &n)) return;
+  const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  unsigned oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
   for (int i = 0; i < Tile::LA; ++i)
-    ga[i] = h + (size_t)(order[tile.row0 + min(Tile::row(i), tile.rows - 1)] / top) * Hp + Tile::k();
+    oa[i] = (unsigned)sizeof(T) * (order[tile.row0 + min(Tile::row(i), tile.rows - 1)] / top) * Hp + Tile::column();
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) gb[i] = we + (size_t)min(n0 + Tile::row(i), N - 1) * Hp + Tile::k();
-  f32x16 acc[Tile::FM][2];
-  Tile::run(smem, ga, gb, 0, Hp, acc);
-  const int col = (n0 + 64 * (wave & 1)) / 2 + (lane & 31);
-  if (col >= Fp) return;
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * Hp + Tile::column();
+  f32x16 acc[Tile::FM][Tile::FN];
+  Tile::run(smem, rows_buffer(h, sizeof(T) * M * Hp), oa,
+            rows_buffer(w + ((size_t)tile.expert * N + n0) * Hp, sizeof(T) * min(BN, N - n0) * Hp), ob, 0, Hp, acc);
+  const __amdgpu_buffer_rsrc_t out = rows_buffer(act + (size_t)tile.row0 * Fp, sizeof(T) * tile.rows * Fp);
 #pragma unroll
-  for (int i = 0; i < Tile::FM; ++i)
+  for (int j = 0; j < Tile::FN; j += 2) {
+    const int col = (n0 + BN / WN * (wave % WN) + 32 * j) / 2 + (lane & 31);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int r = (wave >> 1) * (BM / 2) + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-      if (r < tile.rows) act[(size_t)(tile.row0 + r) * Fp + col] = (T)clamped_glu(acc[i][0][v], acc[i][1][v], limit);
+    for (int i = 0; i < Tile::FM; ++i) {
+      const int r = BM / WM * (wave / WN) + 32 * i + 4 * (lane >> 5);
+      unsigned off = col < Fp ? (unsigned)sizeof(T) * (r * Fp + col) : 0xF0000000u;  // past the end: not stored
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float g = acc[i][j][v], u = acc[i][j + 1][v];
+        asm volatile("" : "+v"(g), "+v"(u), "+v"(off));  // one after the other, or all of it is in registers at once
+        const T y = (T)clamped_glu<T>(g, u, limit);
+        if constexpr (sizeof(T) == 2) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, y), out, off, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), out, off, 0, 0);
+        off += (unsigned)sizeof(T) * (v % 4 == 3 ? 5 : 1) * Fp;
+      }
     }
+  }
 }
 
-// parts [slot][token][Hp] = weight * act down^T
-template <typename T, int BM>
-__global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ act, const T* __restrict__ w,
-                                                       float* __restrict__ parts, const int* __restrict__ order,
-                                                       const float* __restrict__ wts, const MoeTile* __restrict__ tiles,
-                                                       const int* __restrict__ n_tiles, int top, int M, int Hp, int Fp) {
-  using Tile = MfmaTile<T, BM, 128, 2, 2>;
+// parts [slot][token][Hp] = weight * act down^T; a slot has rows_all tokens
+template <typename T, int BM, int BN, int WM, int WN, int D>
+__global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restrict__ act, const T* __restrict__ w,
+                                                                float* __restrict__ parts, const int* __restrict__ order,
+                                                                const float* __restrict__ wts,
+                                                                const MoeTile* __restrict__ tiles,
+                                                                const int* __restrict__ n_tiles, int top, int rows_all, int Hp,
+                                                                int Fp) {
+  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
   extern __shared__ __align__(16) uint8_t smem[];
   MoeTile tile;
   int n;
-  if (!moe_tile(tiles, n_tiles, (Hp + 127) / 128, &tile, &n)) return;
-  const int n0 = 128 * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const T* we = w + (size_t)tile.expert * Hp * Fp;
-  const T* ga[Tile::LA];
-  const T* gb[Tile::LB];
+  if (!moe_tile(tiles, n_tiles, BM, (Hp + BN - 1) / BN, &tile, &n)) return;
+  const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // a row's place and weight, asked for now and handed round through LDS behind the products
+  static_assert(BM <= Tile::kThreads, "a thread per row");
+  const int own = order[tile.row0 + min((int)threadIdx.x, tile.rows - 1)];
+  unsigned oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
-  for (int i = 0; i < Tile::LA; ++i)
-    ga[i] = act + (size_t)(tile.row0 + min(Tile::row(i), tile.rows - 1)) * Fp + Tile::k();
+  for (int i = 0; i < Tile::LA; ++i) oa[i] = (unsigned)sizeof(T) * Tile::row(i) * Fp + Tile::column();
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) gb[i] = we + (size_t)min(n0 + Tile::row(i), Hp - 1) * Fp + Tile::k();
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * Fp + Tile::column();
   f32x16 acc[Tile::FM][Tile::FN];
-  Tile::run(smem, ga, gb, 0, Fp, acc);
+  Tile::run(smem, rows_buffer(act + (size_t)tile.row0 * Fp, sizeof(T) * tile.rows * Fp), oa,
+            rows_buffer(w + ((size_t)tile.expert * Hp + n0) * Fp, sizeof(T) * min(BN, Hp - n0) * Fp), ob, 0, Fp, acc);
+  const float weight = wts[own];
+  __syncthreads();
+  float* s_w = reinterpret_cast<float*>(smem);            // [BM]
+  int* s_row = reinterpret_cast<int*>(smem) + BM;         // [BM], row of parts
+  if (threadIdx.x < BM) {
+    const int m = own / top;
+    s_w[threadIdx.x] = weight;
+    s_row[threadIdx.x] = (own - m * top) * rows_all + m;
+  }
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < Tile::FM; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int r = (wave >> 1) * (BM / 2) + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      const int r = BM / WM * (wave / WN) + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
       if (r >= tile.rows) continue;
-      const int pair = order[tile.row0 + r], m = pair / top;
-      const float a = wts[pair];
-      float* dst = parts + ((size_t)(pair - m * top) * M + m) * Hp;
+      const float a = s_w[r];
+      float* dst = parts + (size_t)s_row[r] * Hp;
 #pragma unroll
-      for (int c = 0; c < Tile::FN; ++c) {
-        const int col = n0 + 64 * (wave & 1) + 32 * c + (lane & 31);
-        if (col < Hp) dst[col] = a * acc[i][c][v];
+      for (int j = 0; j < Tile::FN; ++j) {
+        const int col = n0 + BN / WN * (wave % WN) + 32 * j + (lane & 31);
+        if (col < Hp) dst[col] = a * acc[i][j][v];
       }
     }
 }
@@ -300,7 +330,7 @@ __global__ __launch_bounds__(kRowThreads) void moe_row_gate_up_kernel(const RowP
     const float a = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), slot));
 #pragma unroll
     for (int i = 0; i < P; ++i)
-      if (lane == 0) z[(size_t)g * P + i] = a * clamped_glu(t[2 * i], t[2 * i + 1], limit);
+      if (lane == 0) z[(size_t)g * P + i] = a * clamped_glu<float>(t[2 * i], t[2 * i + 1], limit);
   });
 }
 
@@ -342,7 +372,10 @@ struct Scratch {
   size_t ids, wts, order, tiles, n_tiles, act, bytes;
   int max_tiles;
 };
-int tile_rows(int M, int experts, int top) { return (long)M * top >= 96L * experts ? 128 : 64; }
+int tile_rows(int dtype, int M, int experts, int top) {
+  const long per = (long)M * top / experts;  // rows an expert has on average
+  return per >= 768 && dtype == W4A32_LAYERED_BF16 ? 256 : per >= 96 ? 128 : 64;
+}
 Scratch scratch_of(int dtype, int M, int experts, int top, int Fp) {
   const size_t n = (size_t)M * top, elem = dtype == W4A32_LAYERED_BF16 ? 2 : 4;
   Scratch c;
@@ -363,46 +396,85 @@ Scratch scratch_of(int dtype, int M, int experts, int top, int Fp) {
   return c;
 }
 
-template <typename T, int BM>
-hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down, int M, float* parts, uint8_t* ws,
-                   const Scratch& c, hipStream_t s) {
+// Up, Down: the two products' tiles, of equal height
+template <typename Up, typename Down, typename T>
+hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down, int M, int rows_all, float* parts,
+                   uint8_t* ws, const Scratch& c, hipStream_t s) {
+  static_assert(Up::kRows == Down::kRows, "one list of tiles");
   int* order = reinterpret_cast<int*>(ws + c.order);
   MoeTile* tiles = reinterpret_cast<MoeTile*>(ws + c.tiles);
   int* n_tiles = reinterpret_cast<int*>(ws + c.n_tiles);
   T* act = reinterpret_cast<T*>(ws + c.act);
-  const int most = (int)(((size_t)M * g.top + BM - 1) / BM) + g.experts;  // workgroups past the last tile return
-  constexpr size_t lds = MfmaTile<T, BM, 128, 2, 2>::kLds;
-  auto up = moe_gate_up_kernel<T, BM>;
-  auto dn = moe_down_kernel<T, BM>;
+  const int most = (int)(((size_t)M * g.top + Up::kRows - 1) / Up::kRows) + g.experts;  // workgroups past the last tile return
+  auto up = moe_gate_up_kernel<T, Up::kRows, Up::kCols, Up::kWM, Up::kWN, Up::kDepth>;
+  auto dn = moe_down_kernel<T, Down::kRows, Down::kCols, Down::kWM, Down::kWN, Down::kDepth>;
   static LdsLimitOnce raised_up, raised_dn;
-  if (lds > 64 * 1024) {
-    if (hipError_t e = raised_up.raise(reinterpret_cast<const void*>(up), lds); e != hipSuccess) return e;
-    if (hipError_t e = raised_dn.raise(reinterpret_cast<const void*>(dn), lds); e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(up, dim3((unsigned)most * ((2 * g.Fp + 127) / 128)), dim3(256), lds, s, h, gate_up, act, order, tiles,
-                     n_tiles, g.top, g.Hp, g.Fp, g.limit);
+  if (Up::kLds > 64 * 1024)
+    if (hipError_t e = raised_up.raise(reinterpret_cast<const void*>(up), Up::kLds); e != hipSuccess) return e;
+  if (Down::kLds > 64 * 1024)
+    if (hipError_t e = raised_dn.raise(reinterpret_cast<const void*>(dn), Down::kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(up, dim3((unsigned)most * ((2 * g.Fp + Up::kCols - 1) / Up::kCols)), dim3(64 * Up::kWM * Up::kWN), Up::kLds,
+                     s, h, gate_up, act, order, tiles, n_tiles, M, g.top, g.Hp, g.Fp, g.limit);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  hipLaunchKernelGGL(dn, dim3((unsigned)most * ((g.Hp + 127) / 128)), dim3(256), lds, s, act, down, parts, order,
-                     reinterpret_cast<const float*>(ws + c.wts), tiles, n_tiles, g.top, M, g.Hp, g.Fp);
+  hipLaunchKernelGGL(dn, dim3((unsigned)most * ((g.Hp + Down::kCols - 1) / Down::kCols)), dim3(64 * Down::kWM * Down::kWN),
+                     Down::kLds, s, act, down, parts, order, reinterpret_cast<const float*>(ws + c.wts), tiles, n_tiles, g.top,
+                     rows_all, g.Hp, g.Fp);
   return hipGetLastError();
 }
 
+template <typename T, int BM, int BN, int WM, int WN, int D>
+struct TileOf {
+  static constexpr int kRows = BM, kCols = BN, kWM = WM, kWN = WN, kDepth = D;
+  static constexpr size_t kLds = MfmaTile<T, BM, BN, WM, WN, D>::kLds;
+};
+
 template <typename T>
-hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, int ldl, const T* gate_up,
-                     const T* down, int M, float* parts, uint8_t* ws, hipStream_t s) {
-  if (logit_parts < 1 || logit_parts > kMaxParts) return hipErrorInvalidValue;
+hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, size_t part_stride, int ldl,
+                     const T* gate_up, const T* down, int M, int rows_all, float* parts, uint8_t* ws, hipStream_t s) {
   const Scratch c = scratch_of(dtype, M, g.experts, g.top, g.Fp);
-  const int bm = tile_rows(M, g.experts, g.top);
+  const int bm = tile_rows(dtype, M, g.experts, g.top);
   int* ids = reinterpret_cast<int*>(ws + c.ids);
-  hipLaunchKernelGGL(moe_choose_kernel, dim3((M + 3) / 4), dim3(256), 0, s, logits, logit_parts, (size_t)M * ldl, ldl, M,
+  hipLaunchKernelGGL(moe_choose_kernel, dim3((M + 3) / 4), dim3(256), 0, s, logits, logit_parts, part_stride, ldl, M,
                      g.experts, g.top, ids, reinterpret_cast<float*>(ws + c.wts));
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   hipLaunchKernelGGL(moe_plan_kernel, dim3(g.experts), dim3(kPlanThreads), 0, s, ids, M * g.top, g.experts, bm,
                      reinterpret_cast<int*>(ws + c.order), reinterpret_cast<MoeTile*>(ws + c.tiles),
                      reinterpret_cast<int*>(ws + c.n_tiles));
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  return bm == 128 ? grouped<T, 128>(g, h, gate_up, down, M, parts, ws, c, s)
-                   : grouped<T, 64>(g, h, gate_up, down, M, parts, ws, c, s);
+  // (Us for gate and up, then down, of 16 experts, 4 per token. 1501 tokens, [2 x 2240][1536]: 128 x 128 124, 72, 128 x 256 128, 78;
+  // 2048 tokens, [2 x 4736][3584]: 673, 352 against 629, 312, 256 x 256 599, 340; 100 tokens, [2 x 2240][1536]: 64 x 128 49, 23 =
+  // 4.5 and 4.9 TB/s of weights, 128 x 128 53, 26. Before these shapes: 145, 106 for the first.)
+  if constexpr (sizeof(T) == 2) {
+    const long tiles_up = ((long)M * g.top / 128 + g.experts / 2) * (2 * g.Fp / 256);
+    const long tiles_down = ((long)M * g.top / 128 + g.experts / 2) * (g.Hp / 256);
+    using Small = TileOf<T, 128, 128, 2, 4, 2>;  // two workgroups per CU
+    using SmallUp = TileOf<T, 128, 128, 2, 2, 2>;
+    using Wide = TileOf<T, 128, 256, 2, 4, 2>;
+    if (bm == 256)
+      return grouped<TileOf<T, 256, 256, 2, 4, 2>, TileOf<T, 256, 256, 2, 4, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    if (bm == 128 && tiles_down >= 1000) return grouped<Wide, Wide>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    if (bm == 128 && tiles_up >= 1000) return grouped<Wide, Small>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    if (bm == 128) return grouped<SmallUp, Small>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    return grouped<TileOf<T, 64, 128, 2, 2, 4>, TileOf<T, 64, 128, 2, 4, 4>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+  } else {
+    if (bm == 128)
+      return grouped<TileOf<T, 128, 128, 2, 2, 1>, TileOf<T, 128, 128, 2, 2, 1>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    return grouped<TileOf<T, 64, 128, 2, 2, 1>, TileOf<T, 64, 128, 2, 2, 1>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+  }
+}
+
+// The gathered rows' byte offsets have 32 bits: more rows than that go in several turns, one after the other on the same scratch.
+template <typename T>
+hipError_t prefill_turns(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, int ldl,
+                         const T* gate_up, const T* down, int M, float* parts, uint8_t* ws, hipStream_t s) {
+  if (logit_parts < 1 || logit_parts > kMaxParts) return hipErrorInvalidValue;
+  const int turn = (int)std::min<size_t>(M, 0xFFFFFFFFu / (sizeof(T) * g.Hp));
+  for (int m = 0; m < M; m += turn)
+    if (hipError_t e = prefill_t(dtype, g, h + (size_t)m * g.Hp, logits + (size_t)m * ldl, logit_parts, (size_t)M * ldl, ldl,
+                                 gate_up, down, std::min(turn, M - m), M, parts + (size_t)m * g.Hp, ws, s);
+        e != hipSuccess)
+      return e;
+  return hipSuccess;
 }
 
 template <typename WT>
@@ -445,9 +517,9 @@ hipError_t launch_moe_prefill(int dtype, const MoeGeom& g, const void* h, const 
                               const void* gate_up, const void* down, int M, float* parts, void* scratch, hipStream_t s) {
   uint8_t* ws = static_cast<uint8_t*>(scratch);
   if (dtype == W4A32_LAYERED_BF16)
-    return prefill_t(dtype, g, static_cast<const __bf16*>(h), logits, logit_parts, ldl, static_cast<const __bf16*>(gate_up),
+    return prefill_turns(dtype, g, static_cast<const __bf16*>(h), logits, logit_parts, ldl, static_cast<const __bf16*>(gate_up),
                      static_cast<const __bf16*>(down), M, parts, ws, s);
-  return prefill_t(dtype, g, static_cast<const float*>(h), logits, logit_parts, ldl, static_cast<const float*>(gate_up),
+  return prefill_turns(dtype, g, static_cast<const float*>(h), logits, logit_parts, ldl, static_cast<const float*>(gate_up),
                    static_cast<const float*>(down), M, parts, ws, s);
 }
 

@@ -56,3 +56,62 @@ def test_norm_conv_leaves_its_tail_when_nobody_reads_the_ring(pkg, H, taps, firs
             # f32 sums of up to 5100 terms of size 1: a few 1e-6 of the largest value
             assert np.abs(y.double().cpu().numpy()[:, :H] - ref[at:at + n]).max() < 5e-6 * np.abs(ref).max(), (at, n)
             at += n
+
+
+# sizes at which each tile shape is chosen, rows and columns just past a tile, one to ten tiles of k
+@pytest.mark.parametrize("M,N,K", [(1025, 8963, 64), (1100, 9001, 256), (1025, 4483, 320), (513, 8961, 128), (513, 4483, 192),
+                                   (257, 4481, 640), (600, 3001, 128), (300, 2049, 192), (129, 2001, 64), (70, 130, 448), (1, 1, 64)])
+def test_bf16_product_of_every_shape(pkg, M, N, K):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = torch.randn((M, K), generator=g, device="cuda").bfloat16()
+    b = torch.randn((N, K), generator=g, device="cuda").bfloat16()
+    ref = a.double() @ b.double().t()
+    scale = float(ref.abs().max())
+    ldc = N + 5
+    for parts, c_bf16 in [(p, False) for p in sorted({1, min(2, K // 64), K // 64})] + [(1, True)]:
+        c = torch.full((parts * M + 1, ldc), 7.0, dtype=torch.bfloat16 if c_bf16 else torch.float32, device="cuda")
+        rc = pkg.lib().w4a32_op_matmul_bf16_nt(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, ldc, int(c_bf16), parts,
+                                               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        got = c[:parts * M, :N].double().view(parts, M, N).sum(0)
+        # exact products, f32 sums of up to 640 terms: 640 x 2^-24 at most, a sixth of it seen; bf16 results: half a step
+        assert float((got - ref).abs().max()) / scale < (4e-3 if c_bf16 else 4e-6), (parts, c_bf16)
+        assert bool((c[:parts * M, N:] == 7).all()) and bool((c[parts * M:] == 7).all())
+
+
+@pytest.mark.parametrize("rows,hidden,experts,top,ff", [
+    (190, 64, 2, 1, 64),      # 95 rows per expert: tiles of 64 rows; one tile of columns, half full
+    (200, 130, 2, 1, 130),    # 100: 128 rows
+    (1540, 72, 4, 2, 100),    # 770: 256 rows in bf16
+])
+def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    rnd = lambda *s, std=1.0: (torch.randn(s, generator=g, device="cuda") * std).bfloat16()
+    pad = lambda n: (n + 63) // 64 * 64
+    h, gate, up = rnd(rows, hidden), rnd(experts, ff, hidden, std=hidden ** -0.5), rnd(experts, ff, hidden, std=hidden ** -0.5)
+    down = rnd(experts, hidden, ff, std=ff ** -0.5)
+    # experts of unequal use, no close calls
+    logits = torch.stack([torch.randperm(experts, generator=g, device="cuda") for _ in range(rows)]).float()
+    logits[:rows // 3, 0] += 100
+    _, chosen = logits.topk(top, 1)
+    share = torch.softmax(logits.gather(1, chosen).double(), 1)
+    ref = torch.zeros((top, rows, hidden), dtype=torch.float64, device="cuda")
+    for e in range(experts):
+        r, slot = (chosen == e).nonzero(as_tuple=True)
+        x = h[r].double()
+        gg = (x @ gate[e].double().t()).clamp(max=0.9)
+        uu = (x @ up[e].double().t()).clamp(-0.9, 0.9)
+        ref[slot, r] = share[r, slot, None] * ((gg * torch.sigmoid(1.702 * gg) * (uu + 1)) @ down[e].double().t())
+    # tolerances of tests/test_gpu_lesarax.py::test_experts_alone, whose operands these are
+    for dtype, tol in ((torch.float32, 3e-6), (torch.bfloat16, 1e-2)):
+        hp = torch.zeros((rows, pad(hidden)), dtype=dtype, device="cuda")
+        hp[:, :hidden] = h
+        dp = torch.zeros((experts, pad(hidden), pad(ff)), dtype=dtype, device="cuda")
+        dp[:, :hidden, :ff] = down
+        parts = pkg.op_experts(hp, logits, pkg.pack_gate_up(gate.to(dtype), up.to(dtype)), dp, hidden, top, ff, 0.9).double()
+        assert bool((parts[:, :, hidden:] == 0).all())
+        assert float((parts[:, :, :hidden] - ref).abs().max()) < tol * float(ref.abs().max())
