@@ -83,6 +83,7 @@ struct Geom {
   size_t state_bytes;
   // workspace
   size_t x[2], y, raw, cx, q, mix, parts, ff, z, o, ml, amax_v, amax_i, logits, last, rec, ws_bytes;
+  size_t stats;                                       // per row: mean, 1 / deviation
   size_t cq, ke, ve, qa, head_out, router, moe, sel;  // latent attention, mixture of experts
   std::vector<int> expand_blk;                        // per run: blocks of keys the expansion has room for
 };
@@ -314,6 +315,7 @@ Geom geometry(const w4a32_layered_config* c) {
   g.router = take(sizeof(float) * w4::kMoeLogitParts * Mb * pad64(experts));
   g.moe = take(moe);
   g.sel = take(sizeof(int) * W4A32_LAYERED_MAX_TOP);
+  g.stats = take(sizeof(float2) * Mb);
   g.ws_bytes = o;
   return g;
 }
@@ -434,7 +436,7 @@ int prefill_layers(const Run& r, const int64_t* tokens, int M, int pos0, int n_l
   auto norm = [&](const float* w, const float* conv, size_t ring) {
     const int rc = from_hip(w4::launch_norm_conv(r.f32(g.x[cur]), r.f32(g.parts), pending, r.f32(g.x[cur ^ 1]), w,
                                                  spec, conv, r.stf(ring), c->canon_taps, M, H, Hp, pos0,
-                                                 r.ws + g.y, r.bf16(), r.s));
+                                                 r.ws + g.y, r.bf16(), reinterpret_cast<float2*>(r.ws + g.stats), r.s));
     if (pending) cur ^= 1;
     pending = 0;
     return rc;
@@ -795,7 +797,7 @@ int w4a32_op_layernorm_conv(const float* d_x, const float* d_parts, int n_parts,
   if (taps > W4A32_LAYERED_MAX_TAPS || !w4::norm_conv_fits(pad64(H), taps)) return W4A32_ENOTSUP;
   w4::NormSpec spec{eps};
   return from_hip(w4::launch_norm_conv(d_x, d_parts, n_parts, d_x_out, d_norm, spec, d_conv, d_ring, taps, M, H, pad64(H),
-                                       pos0, d_y, y_bf16 != 0, S(stream)));
+                                       pos0, d_y, y_bf16 != 0, nullptr, S(stream)));
 }
 
 int w4a32_op_short_conv(const float* d_x, int ldx, float* d_y, int ldy, const float* d_w, float* d_ring, int ldw,

@@ -125,9 +125,10 @@ struct NormSpec {
   float eps, part_scale = 1.0f;
   bool rms = false;
 };
+// stats: room for M pairs, or null (many rows then take longer)
 hipError_t launch_norm_conv(const float* x, const float* parts, int n_parts, float* x_out, const float* norm_w,
                             const NormSpec& spec, const float* conv, float* ring, int taps, int M, int H, int ld, int pos0,
-                            void* y, bool y_bf16, hipStream_t s);
+                            void* y, bool y_bf16, float2* stats, hipStream_t s);
 // layer norm of the wanted rows (x + parts), no convolution: y [n_want][ld]
 hipError_t launch_norm_want(const float* x, const float* parts, int n_parts, const float* norm_w,
                             const NormSpec& spec, const int* want, int n_want, int M, int H, int ld, void* y, bool y_bf16, hipStream_t s);

@@ -27,6 +27,25 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const int64_t* __restri
   for (int c = 4 * threadIdx.x; c < ld; c += 1024) store4(dst + c, load4(src + c));
 }
 
+// Sums over a workgroup of kWaves wavefronts, in every thread.
+template <int kWaves, int N>
+__device__ __forceinline__ void workgroup_sums(float (&v)[N], float (*s_part)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = wave_sum64(v[i]);
+  __syncthreads();  // s_part of an earlier call
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) s_part[threadIdx.x >> 6][i] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) v[i] += s_part[w][i];
+  }
+}
+
 // Layer norm (or the norm that takes no mean off) of one row by one wavefront: x + scale * parts -> LDS row s_h (h, zeros past H). The completed residual row goes to
 // x_out when that is given. Rows of up to 2048 channels stay in registers on the way.
 __device__ __forceinline__ void wave_layer_norm(const float* __restrict__ x, const float* __restrict__ parts,
@@ -184,6 +203,110 @@ __global__ __launch_bounds__(64 * kNcWaves) void norm_conv_kernel(
 }
 static_assert(kNcWaves >= W4A32_LAYERED_MAX_TAPS - 1, "a wavefront per row of the tail");
 
+// The same for many rows in two launches: statistics (and the completed residual row), then the convolution, whose threads walk
+// down the rows with the window in registers. norm_conv_kernel normalises taps - 1 rows for every block of a few again: at
+// [2048][3584], four taps and two partial rows it read 220 MB for 88 and took 88 us, these two take 29.
+template <int P>
+__global__ __launch_bounds__(256) void norm_stats_kernel(const float* __restrict__ x, const float* __restrict__ parts,
+                                                         int n_parts, size_t part_stride, float* __restrict__ x_out,
+                                                         NormSpec spec, int H, int ld, float2* __restrict__ stats) {
+  __shared__ float s_part[4][1];
+  const size_t row = (size_t)blockIdx.x * ld;
+  float4 v[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) v[p] = load4(x + row + min(4 * ((int)threadIdx.x + 256 * p), ld - 4));
+#pragma unroll 2
+  for (int i = 0; i < n_parts; ++i) {
+    float4 d[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) d[p] = load4(parts + i * part_stride + row + min(4 * ((int)threadIdx.x + 256 * p), ld - 4));
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      v[p].x += spec.part_scale * d[p].x; v[p].y += spec.part_scale * d[p].y;
+      v[p].z += spec.part_scale * d[p].z; v[p].w += spec.part_scale * d[p].w;
+    }
+  }
+  float t[1] = {0.0f};
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int c = 4 * ((int)threadIdx.x + 256 * p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e >= H) at4(v[p], e) = 0.0f;
+    if (x_out && c < ld) store4(x_out + row + c, v[p]);
+    t[0] += (v[p].x + v[p].y) + (v[p].z + v[p].w);
+  }
+  const float inv = 1.0f / (float)H;
+  float mean = 0.0f;
+  if (!spec.rms) {
+    workgroup_sums<4>(t, s_part);
+    mean = t[0] * inv;
+  }
+  t[0] = 0.0f;
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int c = 4 * ((int)threadIdx.x + 256 * p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = c + e < H ? at4(v[p], e) - mean : 0.0f;
+      t[0] = __fmaf_rn(d, d, t[0]);
+    }
+  }
+  workgroup_sums<4>(t, s_part);
+  if (threadIdx.x == 0) stats[blockIdx.x] = make_float2(mean, 1.0f / sqrtf(t[0] * inv + spec.eps));
+}
+
+constexpr int kStripRows = 16;
+// x: the completed rows (zeros past H). Columns belong to threads: the one that reads a column of the ring writes it.
+template <int TAPS, typename YT>
+__global__ __launch_bounds__(256) void strip_conv_kernel(const float* __restrict__ x, const float2* __restrict__ stats,
+                                                         const float* __restrict__ norm_w, const float* __restrict__ conv,
+                                                         float* __restrict__ ring, int M, int H, int ld, int pos0,
+                                                         YT* __restrict__ y) {
+  const int c = 4 * ((int)blockIdx.x * 256 + (int)threadIdx.x), t0 = blockIdx.y * kStripRows;
+  if (c >= ld) return;
+  const float4 nw = load4(norm_w + c);
+  float4 w[TAPS], win[TAPS];  // win[j]: h of the position j before the current one
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) w[j] = load4(conv + (size_t)j * ld + c);
+  auto normed = [&](float4 v, float2 st) {
+    float4 h, g = nw;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) at4(h, e) = c + e < H ? (at4(v, e) - st.x) * st.y * at4(g, e) : 0.0f;
+    return h;
+  };
+#pragma unroll
+  for (int j = 1; j < TAPS; ++j) {
+    const int t = t0 - j, q = pos0 + t;
+    if (t >= 0) win[j] = normed(load4(x + (size_t)t * ld + c), stats[t]);
+    else win[j] = q >= 0 ? load4(ring + (size_t)(q % TAPS) * ld + c) : make_float4(0, 0, 0, 0);
+  }
+  constexpr int kAhead = 8;
+#pragma unroll
+  for (int g = 0; g < kStripRows; g += kAhead) {
+    float4 v[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) v[i] = load4(x + (size_t)min(t0 + g + i, M - 1) * ld + c);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int t = t0 + g + i;
+      if (t >= M) break;
+      win[0] = normed(v[i], stats[t]);
+      float4 o = win[0];
+#pragma unroll
+      for (int j = TAPS - 1; j >= 0; --j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) at4(o, e) = __fmaf_rn(at4(w[TAPS - 1 - j], e), at4(win[j], e), at4(o, e));
+#pragma unroll
+      for (int j = TAPS - 1; j >= 1; --j) win[j] = win[j - 1];
+      store4(y + (size_t)t * ld + c, o);
+    }
+  }
+  if (blockIdx.y != 0) return;
+  for (int t = max(0, M - TAPS + 1); t < M; ++t)
+    store4(ring + (size_t)((pos0 + t) % TAPS) * ld + c, normed(load4(x + (size_t)t * ld + c), stats[t]));
+}
+
 template <typename YT>
 __global__ __launch_bounds__(64) void norm_want_kernel(const float* __restrict__ x, const float* __restrict__ parts,
                                                        int n_parts, const float* __restrict__ norm_w,
@@ -227,49 +350,56 @@ __global__ __launch_bounds__(256) void loop_rows_kernel(const float* __restrict_
   }
 }
 
-template <typename ZT>
-__global__ __launch_bounds__(256) void polynorm_kernel(ZT* __restrict__ z, int F, int ld, const float* __restrict__ act,
-                                                       float eps) {
-  extern __shared__ __align__(16) float s_z[];  // [ld]
-  __shared__ float s_part[4][3];
+// A row per workgroup, held in registers as it came, P pieces of 16 bytes per thread: the row is read once and the loads are all
+// on their way before the first is used. [2048][18944] in bf16, 155 MB: with the row in LDS as f32 (two workgroups per CU, a
+// load at a time) 55 us, so 26 us
+// (5.9 TB/s); [200][8960]: 7.4 -> 3.6.
+template <typename ZT, int kThreads, int P>
+__global__ __launch_bounds__(kThreads) void polynorm_kernel(ZT* __restrict__ z, int F, int ld, const float* __restrict__ act,
+                                                            float eps) {
+  constexpr int kE = 16 / (int)sizeof(ZT), kWaves = kThreads / 64;
+  __shared__ float s_part[kWaves][3];
   ZT* row = z + (size_t)blockIdx.x * ld;
-  float s2 = 0.0f, s4 = 0.0f, s6 = 0.0f;
-  for (int c = 4 * threadIdx.x; c < ld; c += 1024) {
-    float4 v = load4(row + c);
+  u32x4 raw[P];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (c + e >= F) at4(v, e) = 0.0f;
-      const float q = at4(v, e) * at4(v, e);
-      s2 += q;
-      s4 = __fmaf_rn(q, q, s4);
-      s6 = __fmaf_rn(q * q, q, s6);
+  for (int p = 0; p < P; ++p) {
+    const int c = kE * ((int)threadIdx.x + kThreads * p);
+    raw[p] = *reinterpret_cast<const u32x4*>(row + (c < ld ? c : 0));
+  }
+  auto get = [](const u32x4& v, int e) __attribute__((always_inline)) {
+    if constexpr (sizeof(ZT) == 2) return __uint_as_float(e & 1 ? v[e / 2] & 0xFFFF0000u : v[e / 2] << 16);
+    else return __uint_as_float(v[e]);
+  };
+  float t[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int c = kE * ((int)threadIdx.x + kThreads * p);
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+      const float x = c + e < F ? get(raw[p], e) : 0.0f, q = x * x;
+      t[0] += q;
+      t[1] = __fmaf_rn(q, q, t[1]);
+      t[2] = __fmaf_rn(q * q, q, t[2]);
     }
-    store4(s_z + c, v);
   }
-  s2 = wave_sum64(s2);
-  s4 = wave_sum64(s4);
-  s6 = wave_sum64(s6);
-  if ((threadIdx.x & 63) == 0) {
-    float* d = s_part[threadIdx.x >> 6];
-    d[0] = s2;
-    d[1] = s4;
-    d[2] = s6;
-  }
-  __syncthreads();
-  float t[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) t[i] = (s_part[0][i] + s_part[1][i]) + (s_part[2][i] + s_part[3][i]);
+  workgroup_sums<kWaves>(t, s_part);
   const float inv = 1.0f / (float)F;
   const float r1 = act[0] / sqrtf(t[0] * inv + eps), r2 = act[1] / sqrtf(t[1] * inv + eps);
   const float r3 = act[2] / sqrtf(t[2] * inv + eps), e0 = act[3];
-  for (int c = 4 * threadIdx.x; c < ld; c += 1024) {  // the elements this thread wrote
-    float4 v = load4(s_z + c);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float q = at4(v, e);
-      at4(v, e) = c + e < F ? q * (r1 + q * (r2 + q * r3)) + e0 : 0.0f;
+  for (int p = 0; p < P; ++p) {
+    const int c = kE * ((int)threadIdx.x + kThreads * p);
+    if (c >= ld) continue;
+#pragma unroll
+    for (int h = 0; h < kE; h += 4) {
+      float4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float q = get(raw[p], h + e);
+        at4(v, e) = c + h + e < F ? q * (r1 + q * (r2 + q * r3)) + e0 : 0.0f;
+      }
+      store4(row + c + h, v);
     }
-    store4(row + c, v);
   }
 }
 
@@ -386,13 +516,39 @@ static hipError_t norm_conv_t(const float* x, const float* parts, int n_parts, f
   return hipGetLastError();
 }
 
+template <int TAPS, typename YT>
+static hipError_t two_launches_t(const float* x, const float* parts, int n_parts, float* x_out, const float* norm_w,
+                                 const NormSpec& spec, const float* conv, float* ring, int M, int H, int ld, int pos0, YT* y,
+                                 float2* stats, hipStream_t s) {
+  const size_t stride = (size_t)M * ld;
+  if (ld <= 4 * 1024)
+    hipLaunchKernelGGL(norm_stats_kernel<4>, dim3(M), dim3(256), 0, s, x, parts, n_parts, stride, x_out, spec, H, ld, stats);
+  else
+    hipLaunchKernelGGL(norm_stats_kernel<8>, dim3(M), dim3(256), 0, s, x, parts, n_parts, stride, x_out, spec, H, ld, stats);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  hipLaunchKernelGGL((strip_conv_kernel<TAPS, YT>), dim3((ld / 4 + 255) / 256, (M + kStripRows - 1) / kStripRows), dim3(256), 0,
+                     s, n_parts > 0 ? x_out : x, stats, norm_w, conv, ring, M, H, ld, pos0, y);
+  return hipGetLastError();
+}
+
+// Two launches where a row does not fit a wavefront's registers: then norm_conv_kernel reads it from memory several times and few
+// rows fit the LDS. us with one and two launches, two partial rows: 2304 channels, 64 / 512 / 2048 rows: 14.4, 11.2 / 17.5, 13.9 /
+// 29.7, 22.4; 3584 channels: 20.5, 11.4 / 32.0, 15.5 / 88.2, 28.9; but 1536 channels: 6.9, 10.6 / 8.7, 12.3 / 17.6, 18.1.
+static bool two_launches(int ld, int taps) { return taps >= 2 && ld > 2 * 1024 && ld <= 8 * 1024; }
+
 hipError_t launch_norm_conv(const float* x, const float* parts, int n_parts, float* x_out, const float* norm_w,
                             const NormSpec& spec, const float* conv, float* ring, int taps, int M, int H, int ld, int pos0,
-                            void* y, bool y_bf16, hipStream_t s) {
+                            void* y, bool y_bf16, float2* stats, hipStream_t s) {
   if (!norm_conv_fits(ld, taps)) return hipErrorInvalidValue;
   if (n_parts == 0) x_out = nullptr;  // the residual rows stay where they are
 #define W4_NORM_CONV(T)                                                                                            \
   case T:                                                                                                          \
+    if constexpr (T >= 2)                                                                                          \
+      if (stats && two_launches(ld, T))                                                                         \
+        return y_bf16 ? two_launches_t<T>(x, parts, n_parts, x_out, norm_w, spec, conv, ring, M, H, ld, pos0,       \
+                                          static_cast<__bf16*>(y), stats, s)                                        \
+                      : two_launches_t<T>(x, parts, n_parts, x_out, norm_w, spec, conv, ring, M, H, ld, pos0,       \
+                                          static_cast<float*>(y), stats, s);                                        \
     return y_bf16 ? norm_conv_t<T>(x, parts, n_parts, x_out, norm_w, spec, conv, ring, M, H, ld, pos0,              \
                                    static_cast<__bf16*>(y), s)                                                     \
                   : norm_conv_t<T>(x, parts, n_parts, x_out, norm_w, spec, conv, ring, M, H, ld, pos0,              \
@@ -452,25 +608,28 @@ hipError_t launch_add_parts(const float* x, const float* parts, int n_parts, flo
 
 bool polynorm_fits(int ld) { return sizeof(float) * (size_t)ld <= 156 * 1024; }
 
+template <typename ZT>
+static hipError_t polynorm_t(ZT* z, int M, int F, int ld, const float* act, float eps, hipStream_t s) {
+  constexpr int kE = 16 / (int)sizeof(ZT);
+  const int pieces = (ld + 512 * kE - 1) / (512 * kE);  // of 512 threads
+#define W4_POLY(THREADS, P)                                                                                              \
+  do {                                                                                                                  \
+    hipLaunchKernelGGL((polynorm_kernel<ZT, THREADS, P>), dim3(M), dim3(THREADS), 0, s, z, F, ld, act, eps);             \
+    return hipGetLastError();                                                                                           \
+  } while (0)
+  if (pieces <= 1) W4_POLY(256, 2);
+  if (pieces <= 2) W4_POLY(512, 2);
+  if (pieces <= 3) W4_POLY(512, 3);
+  if (pieces <= 5) W4_POLY(512, 5);
+  if (pieces <= 10) W4_POLY(512, 10);
+  W4_POLY(512, 20);  // f32 rows of more than 20480; the longest one allowed has 39936
+#undef W4_POLY
+}
+
 hipError_t launch_polynorm(void* z, bool z_bf16, int M, int F, int ld, const float* act, float eps, hipStream_t s) {
   if (!polynorm_fits(ld)) return hipErrorInvalidValue;
-  const size_t lds = sizeof(float) * ld;
-  if (z_bf16) {
-    static LdsLimitOnce raised;
-    if (lds > 60 * 1024)
-      if (hipError_t e = raised.raise(reinterpret_cast<const void*>(polynorm_kernel<__bf16>), 156 * 1024);
-          e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(polynorm_kernel<__bf16>, dim3(M), dim3(256), lds, s, static_cast<__bf16*>(z), F, ld, act, eps);
-  } else {
-    static LdsLimitOnce raised;
-    if (lds > 60 * 1024)
-      if (hipError_t e = raised.raise(reinterpret_cast<const void*>(polynorm_kernel<float>), 156 * 1024);
-          e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(polynorm_kernel<float>, dim3(M), dim3(256), lds, s, static_cast<float*>(z), F, ld, act, eps);
-  }
-  return hipGetLastError();
+  return z_bf16 ? polynorm_t(static_cast<__bf16*>(z), M, F, ld, act, eps, s)
+                : polynorm_t(static_cast<float*>(z), M, F, ld, act, eps, s);
 }
 
 hipError_t launch_short_conv(const float* x, int ldx, float* y, int ldy, const float* w, float* ring, int ldw, int taps,

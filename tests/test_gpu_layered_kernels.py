@@ -115,3 +115,38 @@ def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
         parts = pkg.op_experts(hp, logits, pkg.pack_gate_up(gate.to(dtype), up.to(dtype)), dp, hidden, top, ff, 0.9).double()
         assert bool((parts[:, :, hidden:] == 0).all())
         assert float((parts[:, :, :hidden] - ref).abs().max()) < tol * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,taps", [(2050, 4), (2500, 8), (4200, 3)])
+def test_norm_of_wide_rows_in_two_launches(width, taps, dtype):
+    """Portions of one to 40 rows (strips of 16), behind each other and in front of position 0."""
+    cfg = lm.config([lm.retention(1, 16, 16, 8, ff=70), lm.attention(2, 1, 16, 16, 64, 8)], width=width, taps=taps)
+    w = lm.random_weights(cfg, seed=width)
+    tokens = np.random.default_rng(width).integers(0, cfg["vocab"], 40)
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, w, dtype, max_seq=41)
+    state = dec.new_state()
+    for portions in ([40], [2] * 20, [17, 3, 1, 16, 3], [33, 7]):
+        at = 0
+        for n in portions:
+            got = dec.forward(state, tokens[at:at + n], at)
+            assert lm.errors(got, ref[at:at + n]).max() < TOL[dtype], (portions, at)
+            at += n
+
+
+@pytest.mark.parametrize("F,ld", [(2049, 2112), (4097, 4160), (6200, 6208), (10241, 10304), (20481, 20544), (39930, 39936)])
+def test_polynorm_of_every_row_length(pkg, F, ld):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(F)
+    act = torch.tensor([0.7, -0.4, 0.3, 0.05], device="cuda")
+    for dtype, tol in ((torch.float32, 3e-6), (torch.bfloat16, 4e-3)):
+        z = torch.randn((3, ld), generator=g, device="cuda").to(dtype)
+        x = z[:, :F].double()
+        rms = lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-5)
+        ref = 0.7 * rms(x) - 0.4 * rms(x ** 2) + 0.3 * rms(x ** 3) + 0.05
+        y = pkg.op_polynorm(z, F, act, 1e-5).double()
+        # f32 sums of up to 39930 positive terms by 512 threads: far below 1e-6; bf16: half a step of the largest result
+        assert float((y[:, :F] - ref).abs().max() / ref.abs().max()) < tol
+        assert bool((y[:, F:] == 0).all())
