@@ -9,6 +9,7 @@
 //   MatMul      mllm/Backends/Arm/Ops/MatMulOp.cpp:131-167     C = A B^T (transpose_b), f32
 #include "w4a32_decoder.h"
 #include "w4a32_internal.h"
+#include "w4a32_layered_kernels.h"
 
 namespace w4 {
 
@@ -198,7 +199,7 @@ hipError_t launch_matmul_nt(const float* a, const void* b, int b_dtype, float* c
 
 hipError_t launch_matmul_f32_nt(const float* a, const float* b, float* c, int M, int N, int K, hipStream_t s) {
   if (dense_rows_applies(M, K)) return launch_dense_rows(a, K, b, W4A32_DENSE_F32, c, M, N, K, s);
-  if (M <= 8) {
+  if (M <= kDenseRows) {
     const dim3 grid((N + 4 * kGemvRows - 1) / (4 * kGemvRows));
 #define W4_DENSE_GEMV(MM) \
   case MM: hipLaunchKernelGGL(dense_gemv_kernel<MM>, grid, dim3(256), 0, s, a, b, c, N, K); break
@@ -209,6 +210,7 @@ hipError_t launch_matmul_f32_nt(const float* a, const float* b, float* c, int M,
 #undef W4_DENSE_GEMV
     return hipGetLastError();
   }
+  if (K % 32 == 0) return launch_matmul_f32(a, b, c, M, N, K, 1, s);  // [300][1024] x [1024][4096]: 48 -> 35 us
   hipLaunchKernelGGL(dense_gemm_kernel<float>, dim3((N + kMmTile - 1) / kMmTile, (M + kMmTile - 1) / kMmTile),
                      dim3(256), 0, s, a, b, c, M, N, K);
   return hipGetLastError();

@@ -132,6 +132,7 @@ hipError_t launch_silu(const float* x, float* out, size_t n, hipStream_t s);
 hipError_t launch_mul(const float* a, const float* b, float* out, size_t n, hipStream_t s);
 hipError_t launch_rope_rows(const float* x, float* y, const float* sin_t, const float* cos_t, int M, int H,
                             int D, int pos0, hipStream_t s);
+constexpr int kDenseRows = 8;  // up to so many rows stream the [N][K] operand
 hipError_t launch_matmul_f32_nt(const float* a, const float* b, float* c, int M, int N, int K, hipStream_t s);
 // dense [N][K] operands held as f16 or f32 (b_dtype: W4A32_DENSE_*), w4a32_dense.hip
 hipError_t launch_matmul_nt(const float* a, const void* b, int b_dtype, float* c, int M, int N, int K, hipStream_t s);

@@ -415,14 +415,13 @@ struct Run {
 
 // C f32 or T [M][ldc] = A B^T; *parts: in the partial products the caller can take, out what was written
 int product(const Run& r, const void* a, const void* b, void* cc, int M, int N, int K, bool out_t, int* parts) {
-  if (r.bf16()) {
-    const int p = parts ? w4::matmul_bf16_parts(M, N, K) : 1;
-    if (parts) *parts = p;
-    return from_hip(w4::launch_matmul_bf16(a, b, cc, M, N, K, N, out_t, p, r.s));
-  }
-  if (parts) *parts = 1;
-  return from_hip(w4::launch_matmul_f32_nt(static_cast<const float*>(a), static_cast<const float*>(b),
-                                           static_cast<float*>(cc), M, N, K, r.s));
+  const bool few = !r.bf16() && M <= w4::kDenseRows;  // f32: streams the weights
+  const int p = parts && !few ? w4::matmul_parts(r.c->dtype, M, N, K) : 1;
+  if (parts) *parts = p;
+  if (r.bf16()) return from_hip(w4::launch_matmul_bf16(a, b, cc, M, N, K, N, out_t, p, r.s));
+  const float *fa = static_cast<const float*>(a), *fb = static_cast<const float*>(b);
+  float* fc = static_cast<float*>(cc);
+  return from_hip(few ? w4::launch_matmul_f32_nt(fa, fb, fc, M, N, K, r.s) : w4::launch_matmul_f32(fa, fb, fc, M, N, K, p, r.s));
 }
 
 // Rows of a portion. Leaves the residual rows in x[*cur] plus *pending partial rows in `parts`.
@@ -484,13 +483,14 @@ int prefill_layers(const Run& r, const int64_t* tokens, int M, int pos0, int n_l
     if (l.ff > 0 && l.experts > 0) {
       const int Ep = pad64(l.experts);
       W4_TRY(norm(lw.norm2, lw.canon2, g.st[i].canon2));
-      int rp = 1;  // few tiles: dealt over k as far as that goes
-      if (r.bf16()) {
-        rp = std::max(1, std::min(w4::kMoeLogitParts, Hp / 128));
+      // few tiles: dealt over k as far as that goes
+      const bool stream = !r.bf16() && M <= w4::kDenseRows;
+      const int rp = stream ? 1 : std::max(1, std::min(w4::kMoeLogitParts, Hp / 128));
+      if (stream) W4_TRY(product(r, r.ws + g.y, lw.router, r.f32(g.router), M, Ep, Hp, false, nullptr));
+      else if (r.bf16())
         W4_LAUNCH(w4::launch_matmul_bf16(r.ws + g.y, lw.router, r.f32(g.router), M, Ep, Hp, Ep, false, rp, r.s));
-      } else {
-        W4_TRY(product(r, r.ws + g.y, lw.router, r.f32(g.router), M, Ep, Hp, false, nullptr));
-      }
+      else
+        W4_LAUNCH(w4::launch_matmul_f32(r.f32(g.y), static_cast<const float*>(lw.router), r.f32(g.router), M, Ep, Hp, rp, r.s));
       W4_LAUNCH(w4::launch_moe_prefill(dt, moe_geom(c, l), r.ws + g.y, r.f32(g.router), rp, Ep, lw.gate_up, lw.experts_down, M,
                                        r.f32(g.parts), r.ws + g.moe, r.s));
       pending = l.top;

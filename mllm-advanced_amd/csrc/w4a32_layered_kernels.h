@@ -112,8 +112,10 @@ bool row_linear_fits(int Kp);
 // bf16 product; parts > 1: C [parts][M][ldc] f32 partial products
 hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int N, int K, int ldc, bool c_bf16,
                               int parts, hipStream_t s);
+// f32 product of [M][K] and [N][K], K % 32 == 0, likewise
+hipError_t launch_matmul_f32(const float* a, const float* b, float* c, int M, int N, int K, int parts, hipStream_t s);
 // Parts worth using: 1, or as many as fit max(kSplitFloats, 2 M N) floats.
-int matmul_bf16_parts(int M, int N, int K);
+int matmul_parts(int dtype, int M, int N, int K);
 constexpr size_t kSplitFloats = (size_t)768 * 128 * 128;
 
 // ---- rows of a prefill ----

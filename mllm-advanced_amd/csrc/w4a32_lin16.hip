@@ -1,7 +1,7 @@
 // Linears with bf16 (or f32) weights for the layered decoder.
 //
-//   matmul_bf16_kernel   C = A B^T, bf16 operands, f32 accumulation (v_mfma_f32_32x32x16_bf16), for prefill rows: tiles from
-//                        64 x 64 to 256 x 256, the k range dealt to several workgroups where the caller adds the parts up.
+//   matmul_kernel        C = A B^T, bf16 or f32 operands, f32 accumulation, for prefill rows: tiles from 64 x 64 to 256 x 256
+//                        (f32: 64 x 128), the k range dealt to several workgroups where the caller adds the parts up.
 //   row_linear_kernel    one decode row through [N][K] weights, read once, with the operator that produces the row
 //                        in front (residual add + norm + input convolution, merge of the attention's key slices,
 //                        per-head norm and gate, PolyNorm, none): HBM-bound, N * K * sizeof(weight) bytes.
@@ -19,11 +19,11 @@ namespace w4 {
 
 namespace {
 
-template <int BM, int BN, int WM, int WN, int D, typename CT>
-__global__ __launch_bounds__(64 * WM * WN) void matmul_bf16_kernel(const __bf16* __restrict__ a,
-                                                                   const __bf16* __restrict__ b, CT* __restrict__ c,
-                                                                   int M, int N, int K, int ldc, int mt, int nt) {
-  using Tile = MfmaTile<__bf16, BM, BN, WM, WN, D>;
+template <typename T, int BM, int BN, int WM, int WN, int D, typename CT>
+__global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restrict__ a, const T* __restrict__ b,
+                                                              CT* __restrict__ c, int M, int N, int K, int ldc, int mt,
+                                                              int nt) {
+  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
   constexpr int FM = Tile::FM, FN = Tile::FN, kBK = Tile::kBK;
   extern __shared__ __align__(16) uint8_t smem[];
 
@@ -39,13 +39,13 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_bf16_kernel(const __bf16*
 
   unsigned oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
-  for (int i = 0; i < Tile::LA; ++i) oa[i] = 2u * Tile::row(i) * K + Tile::column();
+  for (int i = 0; i < Tile::LA; ++i) oa[i] = (unsigned)sizeof(T) * Tile::row(i) * K + Tile::column();
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) ob[i] = 2u * Tile::row(i) * K + Tile::column();
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * K + Tile::column();
   const int ma = min(M - m0, BM), nb = min(N - n0, BN);
   f32x16 acc[FM][FN];
-  Tile::run(smem, rows_buffer(a + (size_t)m0 * K, (size_t)2 * ma * K), oa,
-            rows_buffer(b + (size_t)n0 * K, (size_t)2 * nb * K), ob, kb, ke, acc);
+  Tile::run(smem, rows_buffer(a + (size_t)m0 * K, sizeof(T) * ma * K), oa,
+            rows_buffer(b + (size_t)n0 * K, sizeof(T) * nb * K), ob, kb, ke, acc);
 
   // rows past the last one lie past the buffer's end, columns are sent there: what is stored there is dropped
   c += (size_t)blockIdx.y * M * ldc + (size_t)m0 * ldc;
@@ -68,11 +68,11 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_bf16_kernel(const __bf16*
     }
 }
 
-template <int BM, int BN, int WM, int WN, int D, typename CT>
-hipError_t launch_tile_t(const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
+template <typename T, int BM, int BN, int WM, int WN, int D, typename CT>
+hipError_t launch_tile_t(const T* a, const T* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
   const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
-  constexpr size_t lds = MfmaTile<__bf16, BM, BN, WM, WN, D>::kLds;
-  auto kern = matmul_bf16_kernel<BM, BN, WM, WN, D, CT>;
+  constexpr size_t lds = MfmaTile<T, BM, BN, WM, WN, D>::kLds;
+  auto kern = matmul_kernel<T, BM, BN, WM, WN, D, CT>;
   static LdsLimitOnce raised;
   if (lds > 64 * 1024)
     if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
@@ -82,20 +82,24 @@ hipError_t launch_tile_t(const __bf16* a, const __bf16* b, void* c, int M, int N
 }
 
 // The shapes, and what they cost. A CU that is alone takes tile_us per 64 k of a tile; with all of them busy the chip's clock
-// drops and it delivers `tflops`. (Fitted to 16 sizes from [40][1536] x [8960][1536] to [2048][3584] x [14336][3584], within
-// 15 %.)
+// drops and it delivers `tflops`. (Fitted to 16 sizes from [40][1536] x [8960][1536] to [2048][3584] x [14336][3584]; over 59
+// other sizes of up to 2048 rows the choice was 0.9 % slower than the best one, 10 % at most.)
 struct Shape {
   int bm, bn;
   double tile_us, tflops;
 };
 constexpr Shape kShapes[] = {
     {256, 256, 1.13, 1270}, {256, 128, 0.70, 1060}, {128, 128, 0.46, 950}, {64, 128, 0.36, 660}, {64, 64, 0.25, 490}};
-constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
+// The same in f32, per 32 k: bound by the matrix cores (157 TFLOP/s) whatever the shape, so the small one, which fills the CUs
+// first, unless there are many ([2000][2048] x [3000][2048]: 224 us, 64 x 128 190 = 130 TFLOP/s, 128 x 128 242). [300][4096] x
+// [1024][4096] took 100 us in one part of 64 x 64 without anything requested ahead; in one part of these 64, in four 34.
+constexpr Shape kShapesF32[] = {{64, 128, 0.91, 130}, {64, 64, 0.50, 118}};
 
 // us: rounds of the CUs, and the results' way to memory (and, as partial products, back)
-double shape_us(const Shape& t, int M, int N, int K, int parts, int c_bytes) {
+double shape_us(const Shape& t, int M, int N, double k_tiles, double tile_flops, int parts, int c_bytes) {
   const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
-  const double k_tiles = (double)K / 64 / parts, flops = 2.0 * t.bm * t.bn * 64 * k_tiles;
+  k_tiles /= parts;
+  const double flops = tile_flops * t.bm * t.bn * k_tiles;
   auto round_us = [&](long n) { return std::max(t.tile_us * k_tiles, n * flops / (t.tflops * 1e6)); };
   const double out = (double)M * N * c_bytes * (2 * parts - 1) / 5e6;
   return 2.5 + tiles / 256 * round_us(256) + (tiles % 256 ? round_us(tiles % 256) : 0.0) + out;
@@ -105,14 +109,16 @@ struct Plan {
   int shape, parts;
 };
 
-// The cheapest shape; with most_parts > 1 also the number of partial products (1, 2, 4, 8) that go with it.
-Plan best_plan(int M, int N, int K, int parts, int most_parts, int c_bytes) {
+// The cheapest shape; with most_parts > parts also the number of partial products (parts, twice that, ..) that go with it.
+Plan best_plan(bool f32, int M, int N, int K, int parts, int most_parts, int c_bytes) {
+  const Shape* shapes = f32 ? kShapesF32 : kShapes;
+  const int count = f32 ? sizeof(kShapesF32) / sizeof(Shape) : sizeof(kShapes) / sizeof(Shape), bk = f32 ? 32 : 64;
   Plan best{0, parts};
   double least = INFINITY;
   for (int p = parts; p <= most_parts; p *= 2) {
-    if (p > parts && K / p < 512) break;
-    for (int i = 0; i < kShapeCount; ++i) {
-      const double us = shape_us(kShapes[i], M, N, K, p, c_bytes);
+    if (p > parts && K / p < (f32 ? 128 : 512)) break;
+    for (int i = 0; i < count; ++i) {
+      const double us = shape_us(shapes[i], M, N, (double)K / bk, 2.0 * bk, p, c_bytes);
       if (us < least) {
         least = us;
         best = {i, p};
@@ -126,11 +132,11 @@ template <typename CT>
 hipError_t launch_shape(int shape, const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, int parts,
                         hipStream_t s) {
   switch (shape) {
-    case 0: return launch_tile_t<256, 256, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
-    case 1: return launch_tile_t<256, 128, 4, 2, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
-    case 2: return launch_tile_t<128, 128, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
-    case 3: return launch_tile_t<64, 128, 2, 4, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
-    default: return launch_tile_t<64, 64, 2, 2, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 0: return launch_tile_t<__bf16, 256, 256, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 1: return launch_tile_t<__bf16, 256, 128, 4, 2, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 2: return launch_tile_t<__bf16, 128, 128, 2, 4, 2, CT>(a, b, c, M, N, K, ldc, parts, s);
+    case 3: return launch_tile_t<__bf16, 64, 128, 2, 4, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
+    default: return launch_tile_t<__bf16, 64, 64, 2, 2, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
   }
 }
 
@@ -237,10 +243,10 @@ hipError_t launch_row_t(int kind, const RowPrologue& p, const void* w, int N, in
 
 }  // namespace
 
-int matmul_bf16_parts(int M, int N, int K) {
+int matmul_parts(int dtype, int M, int N, int K) {
   int most = 8;  // two always fit what the caller has for them
   while (most > 2 && (size_t)most * M * N > kSplitFloats) most /= 2;
-  return best_plan(M, N, K, 1, most, 4).parts;
+  return best_plan(dtype == W4A32_LAYERED_F32, M, N, K, 1, most, 4).parts;
 }
 
 hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int N, int K, int ldc, bool c_bf16,
@@ -248,9 +254,17 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
   if (K % kPad != 0 || parts < 1 || parts > K / kPad || (parts > 1 && c_bf16)) return hipErrorInvalidValue;
   const __bf16* pa = static_cast<const __bf16*>(a);
   const __bf16* pb = static_cast<const __bf16*>(b);
-  const int shape = best_plan(M, N, K, parts, parts, c_bf16 ? 2 : 4).shape;
+  const int shape = best_plan(false, M, N, K, parts, parts, c_bf16 ? 2 : 4).shape;
   return c_bf16 ? launch_shape<__bf16>(shape, pa, pb, c, M, N, K, ldc, parts, s)
                 : launch_shape<float>(shape, pa, pb, c, M, N, K, ldc, parts, s);
+}
+
+hipError_t launch_matmul_f32(const float* a, const float* b, float* c, int M, int N, int K, int parts, hipStream_t s) {
+  if (K % 32 != 0 || parts < 1 || parts > K / 32) return hipErrorInvalidValue;
+  switch (best_plan(true, M, N, K, parts, parts, 4).shape) {
+    case 0: return launch_tile_t<float, 64, 128, 2, 4, 2, float>(a, b, c, M, N, K, N, parts, s);
+    default: return launch_tile_t<float, 64, 64, 2, 2, 4, float>(a, b, c, M, N, K, N, parts, s);
+  }
 }
 
 int row_linear_partials(int N) { return row_grid(N) * kRowWaves; }

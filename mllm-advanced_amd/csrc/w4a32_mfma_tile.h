@@ -4,9 +4,9 @@
 // accumulators: lane l of a 32 x 32 block holds column l % 32 and, in register v, row 8 (v / 4) + 4 (l / 32) + v % 4. Every shape
 // adds the products of an output in the same order.
 //
-// bf16: tiles of 64 k, brought in through registers (D tiles requested ahead) and double-buffered in LDS as rows of 64 + 8
-// elements: the 144-byte stride puts 16 consecutive rows' 16-byte operands on all 64 banks once. What bounds a shape: a
-// wavefront reads FM + FN kilobytes of LDS for FM x FN products of 32 clocks on its SIMD, all four SIMDs share 128 bytes a
+// Tiles of 128 bytes of k (64 in bf16, 32 in f32), brought in through registers (D tiles requested ahead) and double-buffered in
+// LDS as rows of 128 + 16 bytes: that stride puts 16 consecutive rows' 16-byte operands on all 64 banks once. What bounds a shape
+// in bf16: a wavefront reads FM + FN kilobytes of LDS for FM x FN products of 32 clocks on its SIMD, all four SIMDs share 128 bytes a
 // clock, and the tile's own writes come on top. 128 x 128 on four wavefronts needs 768 LDS clocks for 512 clocks of products,
 // 256 x 128 on eight 1152 for 1024, 256 x 256 on eight 2048 for 2048 with two wavefronts to a SIMD that fill each other's gaps.
 // The order inside a tile is written out and fenced, as the compiler otherwise moves all LDS reads in front of the products:
@@ -15,7 +15,7 @@
 // fragments are in registers by then, so that the next tile's first fragments are on their way under them.
 // [2048][3584] x [14336][3584]: 128 x 128 on four wavefronts without this order 272 us (775 TFLOP/s), with it 235; 256 x 128
 // 213, 256 x 256 185 us (1140 TFLOP/s, and at 1.3 GHz the clock is what the chip sustains under it).
-// f32 (the exact format, not tuned): tiles of 16 k, rows of 16 + 1 floats.
+// f32 products take eight times as long for the same bytes: a SIMD with one wavefront is busy once its operands are there.
 #pragma once
 
 #include "w4a32_layered_kernels.h"
@@ -37,16 +37,35 @@ __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned lane_
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int D>
-struct MfmaTile;
+// A wavefront's operand of a step, and what a pair of them adds to a block of C: k 8 h .. 8 h + 7 of the step's 16 (bf16) from the
+// lanes of half h; of the step's 8 (f32) 4 h .. 4 h + 3, of which one product takes one k from each half.
+template <typename T>
+struct Frag;
+template <>
+struct Frag<__bf16> {
+  bf16x8 v;
+  static __device__ __forceinline__ void product(const Frag& a, const Frag& b, f32x16& c) {
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, c, 0, 0, 0);
+  }
+};
+template <>
+struct Frag<float> {
+  f32x4 v;
+  static __device__ __forceinline__ void product(const Frag& a, const Frag& b, f32x16& c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[e], b.v[e], c, 0, 0, 0);
+  }
+};
 
-template <int BM, int BN, int WM, int WN, int D>
-struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
+template <typename T, int BM, int BN, int WM, int WN, int D>
+struct MfmaTile {
   static constexpr int kThreads = 64 * WM * WN;
   static constexpr int FM = BM / WM / 32, FN = BN / WN / 32;            // 32 x 32 blocks of a wavefront
   static constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads;  // 16-byte pieces a thread brings per tile
-  static constexpr int kBK = 64, kLd = kBK + 8, kSteps = kBK / 16;      // k per LDS tile; LDS row, elements
-  static constexpr size_t kLds = 2 * (BM + BN) * kLd * sizeof(__bf16);
+  static constexpr int kBK = 128 / (int)sizeof(T), kSteps = 4;          // k per LDS tile and steps of its products
+  static constexpr int kLd = kBK + 16 / (int)sizeof(T);                 // LDS row, elements
+  static constexpr int kE = 16 / (int)sizeof(T);                        // of a piece
+  static constexpr size_t kLds = 2 * (BM + BN) * kLd * sizeof(T);
   // the row of A (B) that this thread's piece i is from, and the piece's first byte in it
   static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x + kThreads * i) >> 3; }
   static __device__ __forceinline__ unsigned column() { return 16 * (threadIdx.x & 7); }
@@ -56,20 +75,20 @@ struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
   static __device__ __forceinline__ void run(uint8_t* smem, __amdgpu_buffer_rsrc_t a, const unsigned (&oa)[LA],
                                              __amdgpu_buffer_rsrc_t b, const unsigned (&ob)[LB], int kb, int ke,
                                              f32x16 (&acc)[FM][FN]) {
-    __bf16* s_a = reinterpret_cast<__bf16*>(smem);  // [2][BM][kLd]
-    __bf16* s_b = s_a + 2 * BM * kLd;               // [2][BN][kLd]
+    T* s_a = reinterpret_cast<T*>(smem);  // [2][BM][kLd]
+    T* s_b = s_a + 2 * BM * kLd;          // [2][BN][kLd]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
     constexpr int kPieces = LA + LB, kFrags = FM + FN, kProducts = FM * FN;
     u32x4 ra[D][LA], rb[D][LB];
-    bf16x8 fa[2][FM], fb[2][FN];
-    __bf16* const sa_w = s_a + (tid >> 3) * kLd + 8 * (tid & 7);
-    __bf16* const sb_w = s_b + (tid >> 3) * kLd + 8 * (tid & 7);
-    const __bf16* const sa_r = s_a + (wm + (lane & 31)) * kLd + 8 * (lane >> 5);
-    const __bf16* const sb_r = s_b + (wn + (lane & 31)) * kLd + 8 * (lane >> 5);
+    Frag<T> fa[2][FM], fb[2][FN];
+    T* const sa_w = s_a + (tid >> 3) * kLd + kE * (tid & 7);
+    T* const sb_w = s_b + (tid >> 3) * kLd + kE * (tid & 7);
+    const T* const sa_r = s_a + (wm + (lane & 31)) * kLd + kE * (lane >> 5);
+    const T* const sb_r = s_b + (wn + (lane & 31)) * kLd + kE * (lane >> 5);
     auto fetch = [&](int set, int p, int k) __attribute__((always_inline)) {
-      if (p < LA) ra[set][p < LA ? p : 0] = load16(a, oa[p < LA ? p : 0], 2 * k);
-      else rb[set][p < LA ? 0 : p - LA] = load16(b, ob[p < LA ? 0 : p - LA], 2 * k);
+      if (p < LA) ra[set][p < LA ? p : 0] = load16(a, oa[p < LA ? p : 0], (int)sizeof(T) * k);
+      else rb[set][p < LA ? 0 : p - LA] = load16(b, ob[p < LA ? 0 : p - LA], (int)sizeof(T) * k);
     };
     auto stash = [&](int set, int p, int buf) __attribute__((always_inline)) {
       if (p < LA) *reinterpret_cast<u32x4*>(sa_w + (buf * BM + kThreads / 8 * p) * kLd) = ra[set][p < LA ? p : 0];
@@ -80,8 +99,8 @@ struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
       constexpr int kPairs = 2 * (FM < FN ? FM : FN);
       const bool of_b = r < kPairs ? (r & 1) == 0 : FN > FM;
       const int i = r < kPairs ? r / 2 : r - kPairs / 2;
-      if (of_b) fb[set][i] = *reinterpret_cast<const bf16x8*>(sb_r + (buf * BN + 32 * i) * kLd + 16 * ks);
-      else fa[set][i] = *reinterpret_cast<const bf16x8*>(sa_r + (buf * BM + 32 * i) * kLd + 16 * ks);
+      if (of_b) fb[set][i] = *reinterpret_cast<const Frag<T>*>(sb_r + (buf * BN + 32 * i) * kLd + 2 * kE * ks);
+      else fa[set][i] = *reinterpret_cast<const Frag<T>*>(sa_r + (buf * BM + 32 * i) * kLd + 2 * kE * ks);
     };
     // every wavefront's LDS traffic so far is done (loads from memory stay on their way)
     auto barrier = [] __attribute__((always_inline)) {
@@ -119,7 +138,7 @@ struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
 #pragma unroll
         for (int m = 0; m < kProducts; ++m) {
           const int i = m / FN, j = m % FN;
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks & 1][i], fb[ks & 1][j], acc[i][j], 0, 0, 0);
+          Frag<T>::product(fa[ks & 1][i], fb[ks & 1][j], acc[i][j]);
           // the fragments are spread over three quarters of the products
           constexpr int kSlots = kProducts < 4 ? 1 : kProducts * 3 / 4;
 #pragma unroll
@@ -148,61 +167,6 @@ struct MfmaTile<__bf16, BM, BN, WM, WN, D> {
 #pragma unroll
     for (int u = 0; u < kTurn - 1; ++u)  // (not by leaving the loop: its accumulators would be copied)
       if (k + u * kBK < ke) tile(u, last);
-  }
-};
-
-template <int BM, int BN, int WM, int WN, int D>
-struct MfmaTile<float, BM, BN, WM, WN, D> {
-  static constexpr int kThreads = 64 * WM * WN;
-  static constexpr int FM = BM / WM / 32, FN = BN / WN / 32;
-  static constexpr int LA = BM * 4 / kThreads, LB = BN * 4 / kThreads;
-  static constexpr int kBK = 16, kLd = kBK + 1;
-  static constexpr size_t kLds = (BM + BN) * kLd * sizeof(float);
-  static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x + kThreads * i) >> 2; }
-  static __device__ __forceinline__ unsigned column() { return 16 * (threadIdx.x & 3); }
-
-  static __device__ __forceinline__ void run(uint8_t* smem, __amdgpu_buffer_rsrc_t a, const unsigned (&oa)[LA],
-                                             __amdgpu_buffer_rsrc_t b, const unsigned (&ob)[LB], int kb, int ke,
-                                             f32x16 (&acc)[FM][FN]) {
-    float* s_a = reinterpret_cast<float*>(smem);
-    float* s_b = s_a + BM * kLd;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-    for (int k0 = kb; k0 < ke; k0 += kBK) {
-      f32x4 ra[LA], rb[LB];
-#pragma unroll
-      for (int i = 0; i < LA; ++i) ra[i] = __builtin_bit_cast(f32x4, load16(a, oa[i], 4 * k0));
-#pragma unroll
-      for (int i = 0; i < LB; ++i) rb[i] = __builtin_bit_cast(f32x4, load16(b, ob[i], 4 * k0));
-      __syncthreads();  // the previous tile's reads are done
-#pragma unroll
-      for (int i = 0; i < LA; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s_a[row(i) * kLd + 4 * (threadIdx.x & 3) + e] = ra[i][e];
-#pragma unroll
-      for (int i = 0; i < LB; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s_b[row(i) * kLd + 4 * (threadIdx.x & 3) + e] = rb[i][e];
-      __syncthreads();
-#pragma unroll
-      for (int kk = 0; kk < kBK; kk += 2) {
-        float fa[FM], fb[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) fa[i] = s_a[(wm + 32 * i + (lane & 31)) * kLd + kk + (lane >> 5)];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) fb[j] = s_b[(wn + 32 * j + (lane & 31)) * kLd + kk + (lane >> 5)];
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      }
-    }
   }
 };
 

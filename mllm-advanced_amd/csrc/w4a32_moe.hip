@@ -458,8 +458,8 @@ hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logit
     return grouped<TileOf<T, 64, 128, 2, 2, 4>, TileOf<T, 64, 128, 2, 4, 4>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
   } else {
     if (bm == 128)
-      return grouped<TileOf<T, 128, 128, 2, 2, 1>, TileOf<T, 128, 128, 2, 2, 1>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    return grouped<TileOf<T, 64, 128, 2, 2, 1>, TileOf<T, 64, 128, 2, 2, 1>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+      return grouped<TileOf<T, 128, 128, 2, 2, 2>, TileOf<T, 128, 128, 2, 2, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    return grouped<TileOf<T, 64, 128, 2, 2, 2>, TileOf<T, 64, 128, 2, 2, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
   }
 }
 

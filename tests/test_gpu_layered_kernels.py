@@ -150,3 +150,14 @@ def test_polynorm_of_every_row_length(pkg, F, ld):
         # f32 sums of up to 39930 positive terms by 512 threads: far below 1e-6; bf16: half a step of the largest result
         assert float((y[:, :F] - ref).abs().max() / ref.abs().max()) < tol
         assert bool((y[:, F:] == 0).all())
+
+
+@pytest.mark.parametrize("rows", [9, 63, 65, 130])
+@pytest.mark.parametrize("width,ff,vocab", [(70, 100, 130), (1030, 2100, 65)])
+def test_f32_products_of_a_prompt(width, ff, vocab, rows):
+    """The f32 product's tiles (64 x 64 and 64 x 128, in parts and not) through a model of one layer; every token's logits."""
+    cfg = lm.config([lm.retention(2, 24, 24, 8, ff=ff)], width=width, vocab=vocab)
+    w = lm.random_weights(cfg, seed=rows)
+    tokens = np.random.default_rng(rows).integers(0, vocab, rows)
+    dec = lm.runner(cfg, w, "float32", max_seq=rows)
+    assert lm.errors(dec.forward(dec.new_state(), tokens, 0), lo.forward(cfg, w, tokens)).max() < TOL["float32"]
