@@ -219,13 +219,23 @@ def _check(code, what):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = None
 
 
 def _stream():
-    import torch
+    """The current device's current stream, as the C ABI takes it. (torch.cuda.current_stream() makes an object of it, which
+    takes 3 us: as long as the kernel of a one-row Linear.)"""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
 
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.current_stream()  # initialises the device
+        device, stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+        _raw_stream = lambda: stream(device())
+    return _raw_stream()
 
 
 def packed_bytes(N, K):
@@ -435,15 +445,15 @@ def matmul(x, packed, N, ws=None, out=None):
 def matmul_ws(x, packed, N, ws=None, out=None):
     """The whole op with a workspace of stated size (w4a32_workspace_bytes_n by default: the library may then
     deal a long k range to several workgroups, as for down_proj at prefill sizes)."""
-    import torch
-
     M, K = x.shape
     if ws is None:
         ws = _dev_empty(int(lib().w4a32_workspace_bytes_n(M, K, N)))
     if out is None:
+        import torch
+
         out = torch.empty((M, N), dtype=torch.float32, device="cuda")
-    _check(lib().w4a32_matmul_ws(_ptr(out), _ptr(x), _ptr(packed), _ptr(ws), ws.numel() * ws.element_size(), M, K, N,
-                                 _stream()), "w4a32_matmul_ws")
+    _check(lib().w4a32_matmul_ws(out.data_ptr(), x.data_ptr(), packed.data_ptr(), ws.data_ptr(), ws.nbytes, M, K, N, _stream()),
+           "w4a32_matmul_ws")
     return out
 
 
