@@ -948,6 +948,15 @@ static hipError_t launch_f16_tile(int tile, float* y, const uint8_t* ws, const u
 }
 
 // tiles: 128 x 128 tiles of the problem; tiles160: 128 x 160 tiles; tiles256: 256 x 128 tiles; tiles96: 256 x 96.
+// Choice of tile shape, measured on MI355X at M = 128..8192 over the decoder and ViT shapes, by
+// the number of tiles the problem has. Up to half a 128 x 128 tile per CU the 128 x 64 tile doubles the
+// workgroups; up to one tile per CU the workgroup is alone on its CU and the eight-wavefront
+// arrangement hides some of its latencies; a problem whose 128 x 160 tiles come to (nearly) one or two per
+// CU takes those. The 256 x 128 tile reads each B fragment for two products, where LDS bandwidth bounds
+// the 128-row tiles, and wins wherever its coarser tiles still fill the chip: gate_proj from M = 1536 on
+// (M = 1792: 60 -> 50 us, 990 TFLOP/s; M = 8192: 253 -> 208 us, 1.08 PFLOP/s), q/o from M = 4096 on,
+// down_proj from M = 3456 on; in between 128 x 128 with three resident workgroups per CU. The 64 x 64 tile
+// no longer wins anywhere; it stays selectable by number.
 static int choose_f16_tile(long tiles, long tiles160, long tiles256, long tiles96, int K) {
   if (tiles <= 128) return 4;
   if (tiles <= 256) return 6;
@@ -965,15 +974,60 @@ static int choose_f16_tile(long tiles, long tiles160, long tiles256, long tiles9
   return 2;
 }
 
-// Choice of tile shape, measured on MI355X at M = 128..8192 over the decoder and ViT shapes, by
-// the number of tiles the problem has. Up to half a 128 x 128 tile per CU the 128 x 64 tile doubles the
-// workgroups; up to one tile per CU the workgroup is alone on its CU and the eight-wavefront
-// arrangement hides some of its latencies; a problem whose 128 x 160 tiles come to (nearly) one or two per
-// CU takes those. The 256 x 128 tile reads each B fragment for two products, where LDS bandwidth bounds
-// the 128-row tiles, and wins wherever its coarser tiles still fill the chip: gate_proj from M = 1536 on
-// (M = 1792: 60 -> 50 us, 990 TFLOP/s; M = 8192: 253 -> 208 us, 1.08 PFLOP/s), q/o from M = 4096 on,
-// down_proj from M = 3456 on; in between 128 x 128 with three resident workgroups per CU. The 64 x 64 tile
-// no longer wins anywhere; it stays selectable by number.
+// What a problem costs in a tile shape, us: `base` (launch, first loads, last tile's stores), then rounds of the 256 CUs, each as
+// long as a workgroup alone on its CU needs (stage_us per 64 k) or as the chip delivers `tflops`, then the results' way to memory;
+// for a split problem the second kernel and the partial sums' way there and back. Fitted to 60 problems (M = 9..8192, K =
+// 64..18944, N = 64..11303) in every shape and up to 16 parts.
+struct F16Cost {
+  int bm, bn;
+  double stage_us, base, tflops;
+};
+static constexpr F16Cost kF16Cost[10] = {
+    {64, 64, 0, 0, 0},  // never taken
+    {128, 64, 0.259, 3.7, 879},
+    {128, 128, 0.427, 4.7, 1479},
+    {256, 128, 0.616, 6.3, 1325},
+    {128, 64, 0.232, 4.2, 882},
+    {128, 160, 0.553, 5.6, 1235},
+    {128, 128, 0.342, 5.6, 1102},
+    {256, 96, 0.513, 6.1, 1230},
+    {256, 96, 0.487, 7.1, 1060},
+    {256, 128, 0.530, 8.6, 1280},
+};
+
+static double f16_us(int tile, int parts, int M, int K, int N) {
+  const F16Cost& t = kF16Cost[tile];
+  const int stages = (K + kF16BK - 1) / kF16BK, st = (stages + parts - 1) / parts;
+  const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
+  const double flops = 2.0 * t.bm * t.bn * kF16BK * st, out = (double)M * N * 4;
+  auto round_us = [&](long n) { return std::max(t.stage_us * st, n * flops / (t.tflops * 1e6)); };
+  return t.base + tiles / 256 * round_us(256) + (tiles % 256 ? round_us(tiles % 256) : 0.0) + out / 2.36e6 +
+         (parts > 1 ? 3.5 + 2.0 * parts * out / 6.44e6 : 0.0);
+}
+
+// The rules by tile counts (choose_f16_tile, splitk_plan) come from the decoder's and the vision encoder's shapes and are kept
+// where they are within 5 % of the cheapest of the 128-row shapes 1, 4 and 6; elsewhere that one is taken, in up to
+// most_parts parts of eight stages or more. What the rules split stays split, into no more parts than they say: the caller's
+// room is sized for those. Over the 60 problems the choice is 4 % slower than the best shape and number of parts, the rules
+// alone 13 %: M = 256, K = 5120, N = 1536: 23.9 -> 15.1 us in five parts; 190, 4768, 83: 22.8 -> 9.9 in eight.
+static SplitPlan cheaper_f16(SplitPlan rule, int M, int K, int N, int most_parts) {
+  const int stages = (K + kF16BK - 1) / kF16BK;
+  SplitPlan best = rule;
+  double least = 0.95 * f16_us(rule.tile, rule.parts, M, K, N);
+  for (int parts : {1, 2, 3, 4, 5, 6, 8, 10}) {
+    if (parts > most_parts || (parts > 1 && stages < 8 * parts)) break;
+    if (parts == 1 && rule.parts > 1) continue;
+    for (int tile : {1, 4, 6}) {
+      const double us = f16_us(tile, parts, M, K, N);
+      if (us < least) {
+        least = us;
+        best = {tile, parts};
+      }
+    }
+  }
+  return best;
+}
+
 hipError_t launch_gemm(float* y, const uint8_t* ws, const uint8_t* packed, int M, int K, int N,
                        int kernel, hipStream_t s) {
   if (kernel == kKernelGemmI8) {
@@ -987,8 +1041,8 @@ hipError_t launch_gemm(float* y, const uint8_t* ws, const uint8_t* packed, int M
   const long tiles160 = (long)((M + 127) / 128) * ((N + 159) / 160);
   const long tiles256 = (long)((M + 255) / 256) * ((N + 127) / 128);
   const long tiles96 = (long)((M + 255) / 256) * ((N + 95) / 96);
-  return launch_f16_tile(choose_f16_tile(tiles, tiles160, tiles256, tiles96, K), y, ws, packed, M, K, N, nullptr,
-                         nullptr, 0, 1, nullptr, s);
+  const SplitPlan p = cheaper_f16({choose_f16_tile(tiles, tiles160, tiles256, tiles96, K), 1}, M, K, N, 1);
+  return launch_f16_tile(p.tile, y, ws, packed, M, K, N, nullptr, nullptr, 0, 1, nullptr, s);
 }
 
 hipError_t launch_gemm_group(float* const* y, const uint8_t* ws, const uint8_t* const* packed,
@@ -1028,22 +1082,25 @@ hipError_t launch_gemm_pair(float* act, const uint8_t* ws, const uint8_t* gate, 
 
 // Split-K: tile shape and number of parts for a problem (parts == 1: not worth splitting).
 // Measured on MI355X (down_proj, K = 8960, N = 1536): M = 128: 44 -> 16 us, 256: 44 -> 21,
-// 512: 47 -> 29, 1024: 50 -> 45, 2048: 85 -> 82; at K = 1536 and K = 5120 the second kernel and the
-// partial sums' traffic cost what the shorter loops gain, so only long K qualifies. Parts: about one or
-// two workgroups per CU in all (10 parts up to 24 tiles, 5 up to 96, then 4); more parts only add
-// partial sums for the second kernel to read.
+// 512: 47 -> 29, 1024: 50 -> 45, 2048: 85 -> 82. By rule a long K alone is split, into about one or two workgroups
+// per CU in all (10 parts up to 24 tiles, 5 up to 96, then 4); other shapes are where their cost says so.
 SplitPlan splitk_plan(int M, int K, int N) {
-  SplitPlan p{2, 1};
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   const int nstages = (K + kF16BK - 1) / kF16BK;
-  if (M <= kGemvMaxM || nstages < 96 || tiles > 256) return p;
-  p.parts = tiles <= 24 ? 10 : tiles <= 96 ? 5 : 4;
-  if (tiles <= 16) {
-    p.tile = 1;  // 128 x 64: twice the workgroups (M = 128: 19 -> 16 us)
-  } else if (tiles * p.parts <= 256) {
-    p.tile = 6;  // every workgroup alone on its CU: the eight-wavefront shape (M = 512: 30.1 -> 29.1 us)
+  if (M <= kGemvMaxM) return {2, 1};
+  SplitPlan p{2, 1};
+  if (nstages >= 96 && tiles <= 256) {
+    p.parts = tiles <= 24 ? 10 : tiles <= 96 ? 5 : 4;
+    if (tiles <= 16) {
+      p.tile = 1;  // 128 x 64: twice the workgroups (M = 128: 19 -> 16 us)
+    } else if (tiles * p.parts <= 256) {
+      p.tile = 6;  // every workgroup alone on its CU: the eight-wavefront shape (M = 512: 30.1 -> 29.1 us)
+    }
+  } else {
+    p.tile = choose_f16_tile(tiles, (long)((M + 127) / 128) * ((N + 159) / 160),
+                             (long)((M + 255) / 256) * ((N + 127) / 128), (long)((M + 255) / 256) * ((N + 95) / 96), K);
   }
-  return p;
+  return cheaper_f16(p, M, K, N, p.parts > 1 ? p.parts : 10);
 }
 
 // y == nullptr: no reduction; part[i][M][N], i < parts, then holds sums that already carry the row and column
