@@ -9,7 +9,7 @@
 // A decode layer:   [add + norm + input convolution + in_proj] [mixer step] [merge or head norm + gate + out_proj]
 //                   [add + norm + input convolution + up] [PolyNorm + down]
 //                   latent mixer: [norm + q_up] [cache append, query folded] [attention] [merge + values + gate] [out_proj]
-//                   mixture of experts: [add + norm + router] [norm + choice + gate, up] [down]
+//                   mixture of experts: [add + norm + router + choice + gate, up] [down]; large routers alone in front
 // In front of a pass through looped layers: [add + loop_in].
 #include "w4a32_layered.h"
 
@@ -603,13 +603,15 @@ int decode_layers(const Run& r, const int64_t* token, int n_layers, int* cur_out
       p.ring = r.stf(g.st[i].canon2);
     }
     if (l.ff > 0 && l.experts > 0) {
-      W4_LAUNCH(w4::launch_row_linear(w4::kRowNorm, dt, p, lw.router, l.experts, Hp, r.f32(g.router), nullptr, nullptr, r.s));
+      if (!w4::moe_routes_itself(dt == W4A32_LAYERED_BF16 ? 2 : 4, moe_geom(c, l))) {
+        W4_LAUNCH(w4::launch_row_linear(w4::kRowNorm, dt, p, lw.router, l.experts, Hp, r.f32(g.router), nullptr, nullptr, r.s));
+        // the completed residual row is there now (an input convolution's ring is written with the same row again)
+        p.x = r.f32(g.x[cur ^ 1]);
+        p.n_parts = 0;
+        p.x_out = nullptr;
+      }
       cur ^= 1;
-      // the completed residual row is there now (an input convolution's ring is written with the same row again)
-      p.x = r.f32(g.x[cur]);
-      p.n_parts = 0;
-      p.x_out = nullptr;
-      W4_LAUNCH(w4::launch_moe_decode(dt, moe_geom(c, l), p, r.f32(g.router), lw.gate_up, lw.experts_down, r.f32(g.z),
+      W4_LAUNCH(w4::launch_moe_decode(dt, moe_geom(c, l), p, r.f32(g.router), lw.router, lw.gate_up, lw.experts_down, r.f32(g.z),
                                       reinterpret_cast<int*>(r.ws + g.sel), part, r.s));
     } else if (l.ff > 0) {
       W4_LAUNCH(w4::launch_row_linear(w4::kRowNorm, dt, p, lw.up, pad64(l.ff), Hp, r.f32(g.z), nullptr, nullptr, r.s));

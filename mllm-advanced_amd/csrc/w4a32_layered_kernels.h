@@ -232,10 +232,12 @@ size_t moe_scratch_bytes(int dtype, int M, int experts, int top, int Fp);
 // rows: h T [M][Hp], router logits f32 [logit_parts][M][ldl] -> parts f32 [top][M][Hp]
 hipError_t launch_moe_prefill(int dtype, const MoeGeom& g, const void* h, const float* logits, int logit_parts, int ldl,
                               const void* gate_up, const void* down, int M, float* parts, void* scratch, hipStream_t s);
-// one token: pro is the norm in front (its x_out must be null), z f32 [top * Fp], sel int [top]; out f32 [Hp]
+// one token: pro is the norm in front, z f32 [top * Fp], sel int [top]; out f32 [Hp]. Where the experts' launch multiplies a
+// router of elem_bytes elements itself, pro is the router's norm; else logits holds the router's products and pro.x_out is null.
 bool moe_decode_fits(const MoeGeom& g);
-hipError_t launch_moe_decode(int dtype, const MoeGeom& g, const RowPrologue& pro, const float* logits, const void* gate_up,
-                             const void* down, float* z, int* sel, float* out, hipStream_t s);
+bool moe_routes_itself(size_t elem_bytes, const MoeGeom& g);
+hipError_t launch_moe_decode(int dtype, const MoeGeom& g, const RowPrologue& pro, const float* logits, const void* router,
+                             const void* gate_up, const void* down, float* z, int* sel, float* out, hipStream_t s);
 
 // ---- recurrences with a matrix state ----
 // State of a layer: f32 [heads][dv16][D], transposed (a value row's D key dimensions are contiguous); dv16 = vdim

@@ -39,6 +39,29 @@ __device__ __forceinline__ void top_experts(float (&v)[kLogitRegs], int experts,
   const int lane = threadIdx.x & 63;
   int pick = 0;
   float mine = 0.0f, first = 0.0f, sum = 0.0f;
+  // A value per lane, all of them comparable: each lane counts what comes in front of it, four operations per expert. The rounds
+  // below are six exchanges between lanes each (the choice of 100 tokens, 4 of 16 experts: 6.2 -> 4.4 us).
+  if (experts <= 64 && __popcll(__ballot(v[0] > -INFINITY)) == experts) {
+    int rank = 0;
+    for (int j = 0; j < experts; ++j) {
+      const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v[0]), j));
+      rank += x > v[0] || (x == v[0] && j < lane) ? 1 : 0;
+    }
+    for (int t = 0; t < top; ++t) {
+      const int at = __ffsll((unsigned long long)__ballot(rank == t && lane < experts)) - 1;
+      const float best = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v[0]), at));
+      if (t == 0) first = best;
+      const float w = expf(best - first);
+      sum += w;
+      if (lane == t) {
+        pick = at;
+        mine = w;
+      }
+    }
+    *expert = pick;
+    *weight = mine / sum;
+    return;
+  }
   for (int t = 0; t < top; ++t) {
     float best = -INFINITY;
     int at = 0x7fffffff;
@@ -294,14 +317,16 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restr
 
 // ---------------------------------------------------------------------------------------------
 // z [slot][Fp] = weight * glu of the chosen experts; a group is P columns of one expert, gate and up row of each. The first
-// workgroup leaves the choice for the launch behind.
-template <typename WT, int P, int U>
+// workgroup leaves the choice for the launch behind. kRouter: every workgroup multiplies the router's rows [experts][Hp] itself,
+// else `logits` holds the products.
+template <typename WT, int P, int U, bool kRouter>
 __global__ __launch_bounds__(kRowThreads) void moe_row_gate_up_kernel(const RowPrologue p, const float* __restrict__ logits,
+                                                                      const WT* __restrict__ router,
                                                                       const WT* __restrict__ w, int experts, int top,
                                                                       int Hp, int Fp, float limit, float* __restrict__ z,
                                                                       int* __restrict__ sel) {
   extern __shared__ __align__(16) float s_x[];  // [Hp]
-  __shared__ float s_red[3 * kRowWaves];
+  __shared__ float s_red[3 * kRowWaves], s_logit[64];
   constexpr int R = 2 * P;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int gw = (int)blockIdx.x * kRowWaves + wave, nw = (int)gridDim.x * kRowWaves;
@@ -313,18 +338,37 @@ __global__ __launch_bounds__(kRowThreads) void moe_row_gate_up_kernel(const RowP
     const int row = (c >> 5) * 64 + (r & 1) * 32 + (c & 31);
     return w + ((size_t)__builtin_amdgcn_readlane(expert, slot) * 2 * Fp + row) * Hp + k;
   };
-  float v[kLogitRegs];
-#pragma unroll
-  for (int i = 0; i < kLogitRegs; ++i) v[i] = 64 * i + lane < experts ? logits[64 * i + lane] : -INFINITY;
   Raw<WT> cur[R][U];
-  row_prologue<WT, kRowNorm>(p, Hp, s_x, s_red, [&] {
+  float v[kLogitRegs];
+  if constexpr (kRouter) {
+    auto router_ptr = [&](int g, int, int k) { return router + (size_t)g * Hp + k; };
+    Raw<WT> rows[1][U];
+    row_prologue<WT, kRowNorm>(p, Hp, s_x, s_red, [&] {
+      __builtin_amdgcn_sched_barrier(0);
+      if (wave < experts) fetch_rows<WT, 1, U>(rows, wave, 0, Hp, router_ptr);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    __syncthreads();
+    stream_rows<WT, 1, U>(rows, wave, kRowWaves, experts, Hp, s_x, router_ptr, [&](int g, const float (&t)[1]) {
+      if (lane == 0) s_logit[g] = t[0];
+    });
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kLogitRegs; ++i) v[i] = i == 0 && lane < experts ? s_logit[lane] : -INFINITY;
     top_experts(v, experts, top, &expert, &weight);
-    __builtin_amdgcn_sched_barrier(0);
     if (gw < groups) fetch_rows<WT, R, U>(cur, gw, 0, Hp, ptr);
-    __builtin_amdgcn_sched_barrier(0);
-  });
+  } else {
+#pragma unroll
+    for (int i = 0; i < kLogitRegs; ++i) v[i] = 64 * i + lane < experts ? logits[64 * i + lane] : -INFINITY;
+    row_prologue<WT, kRowNorm>(p, Hp, s_x, s_red, [&] {
+      top_experts(v, experts, top, &expert, &weight);
+      __builtin_amdgcn_sched_barrier(0);
+      if (gw < groups) fetch_rows<WT, R, U>(cur, gw, 0, Hp, ptr);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    __syncthreads();
+  }
   if (blockIdx.x == 0 && wave == 0 && lane < top) sel[lane] = expert;
-  __syncthreads();
   stream_rows<WT, R, U>(cur, gw, nw, groups, Hp, s_x, ptr, [&](int g, const float (&t)[R]) {
     const int slot = g / per;
     const float a = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), slot));
@@ -478,21 +522,26 @@ hipError_t prefill_turns(int dtype, const MoeGeom& g, const T* h, const float* l
 }
 
 template <typename WT>
-hipError_t decode_t(const MoeGeom& g, const RowPrologue& pro, const float* logits, const WT* gate_up, const WT* down, float* z,
-                    int* sel, float* out, hipStream_t s) {
+hipError_t decode_t(const MoeGeom& g, const RowPrologue& pro, const float* logits, const WT* router, const WT* gate_up,
+                    const WT* down, float* z, int* sel, float* out, hipStream_t s) {
   {
-    // One column at a time, as the rows of w4a32_lin16.hip: bf16, four experts of [2 x 2240][1536]: 15.5 us = 3.6 TB/s, two
-    // columns 18.1 (4480 groups on 4096 wavefronts); [2 x 576][832]: 5.8 against 6.9; [2 x 4736][3584]: 46.5 against 46.2.
+    // One column at a time, as the rows of w4a32_lin16.hip: bf16, four experts of [2 x 2240][1536]: 15.5 us = 3.6 TB/s (17.0 with
+    // the router's products inside, 4.3 of a launch less), two columns 18.1 (4480 groups on 4096 wavefronts); [2 x 576][832]: 5.8 against 6.9; [2 x 4736][3584]: 46.5 against 46.2.
     constexpr int P = 1, U = 3;
-    auto kern = moe_row_gate_up_kernel<WT, P, U>;
-    const size_t lds = sizeof(float) * g.Hp;
-    static LdsLimitOnce raised;
-    if (lds > 60 * 1024)
-      if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), 159 * 1024); e != hipSuccess) return e;
     const int groups = g.top * g.Fp / P;
-    hipLaunchKernelGGL(kern, dim3(std::min((groups + kRowWaves - 1) / kRowWaves, 512)), dim3(kRowThreads), lds, s, pro, logits,
-                       gate_up, g.experts, g.top, g.Hp, g.Fp, g.limit, z, sel);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    const dim3 grid(std::min((groups + kRowWaves - 1) / kRowWaves, 512));
+    const size_t lds = sizeof(float) * g.Hp;
+    auto run = [&](auto kern) -> hipError_t {
+      static LdsLimitOnce raised;
+      if (lds > 60 * 1024)
+        if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), 159 * 1024); e != hipSuccess) return e;
+      hipLaunchKernelGGL(kern, grid, dim3(kRowThreads), lds, s, pro, logits, router, gate_up, g.experts, g.top, g.Hp, g.Fp,
+                         g.limit, z, sel);
+      return hipGetLastError();
+    };
+    const hipError_t e =
+        moe_routes_itself(sizeof(WT), g) ? run(moe_row_gate_up_kernel<WT, P, U, true>) : run(moe_row_gate_up_kernel<WT, P, U, false>);
+    if (e != hipSuccess) return e;
   }
   RowPrologue p{};
   p.K = g.top * g.Fp;
@@ -523,14 +572,23 @@ hipError_t launch_moe_prefill(int dtype, const MoeGeom& g, const void* h, const 
                    static_cast<const float*>(down), M, parts, ws, s);
 }
 
+// Up to 96 KB of router a launch of its own costs more than every workgroup's pass over it: per layer of a decode step with four
+// experts of [128][width], bf16, [16][1536]: 28.2 -> 26.3 us, [32][1536]: 29.6 -> 28.5, [64][1024]: 30.4 -> 30.7, [64][1536]: 31.7 ->
+// 32.6; f32, [16][1536]: 32.0 -> 30.1, [32][1536]: 33.0 -> 32.8, [64][1024]: 32.7 -> 34.9.
+bool moe_routes_itself(size_t elem_bytes, const MoeGeom& g) {
+  return g.experts <= 64 && (size_t)g.experts * g.Hp * elem_bytes <= 96 * 1024;
+}
+
 bool moe_decode_fits(const MoeGeom& g) { return row_linear_fits(g.Hp) && (long)g.top * g.Fp <= 35840; }
 
-hipError_t launch_moe_decode(int dtype, const MoeGeom& g, const RowPrologue& pro, const float* logits, const void* gate_up,
-                             const void* down, float* z, int* sel, float* out, hipStream_t s) {
+hipError_t launch_moe_decode(int dtype, const MoeGeom& g, const RowPrologue& pro, const float* logits, const void* router,
+                             const void* gate_up, const void* down, float* z, int* sel, float* out, hipStream_t s) {
   if (!moe_decode_fits(g)) return hipErrorInvalidValue;
   if (dtype == W4A32_LAYERED_BF16)
-    return decode_t(g, pro, logits, static_cast<const __bf16*>(gate_up), static_cast<const __bf16*>(down), z, sel, out, s);
-  return decode_t(g, pro, logits, static_cast<const float*>(gate_up), static_cast<const float*>(down), z, sel, out, s);
+    return decode_t(g, pro, logits, static_cast<const __bf16*>(router), static_cast<const __bf16*>(gate_up),
+                    static_cast<const __bf16*>(down), z, sel, out, s);
+  return decode_t(g, pro, logits, static_cast<const float*>(router), static_cast<const float*>(gate_up),
+                  static_cast<const float*>(down), z, sel, out, s);
 }
 
 }  // namespace w4

@@ -161,3 +161,18 @@ def test_f32_products_of_a_prompt(width, ff, vocab, rows):
     tokens = np.random.default_rng(rows).integers(0, vocab, rows)
     dec = lm.runner(cfg, w, "float32", max_seq=rows)
     assert lm.errors(dec.forward(dec.new_state(), tokens, 0), lo.forward(cfg, w, tokens)).max() < TOL["float32"]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,experts,top", [(70, 1, 1), (250, 9, 2), (700, 33, 16), (700, 64, 64 // 8), (1600, 64, 4), (64, 65, 3)])
+def test_router_inside_and_in_front_of_the_experts(width, experts, top, dtype):
+    # up to 64 experts by counting, up to 96 KB of router in the experts' launch; rows that agree: the lower expert is chosen
+    cfg = lm.lesarax([lm.rotary(1, 1, 16, 8, mlp=lm.moe(24, experts, top))], width=width, vocab=50)
+    w = lm.lesarax_weights(cfg, seed=experts)
+    router = next(k for k in w if k.endswith("router"))
+    w[router][experts // 2:experts // 2 * 2] = w[router][:experts // 2]
+    tokens = [3, 41, 7, 22, 9]
+    dec = lm.runner(cfg, w, dtype, max_seq=8)
+    state, ref = dec.new_state(), lo.forward(cfg, w, tokens)
+    for i, t in enumerate(tokens):
+        assert lm.errors(dec.forward(state, [t], i), ref[i:i + 1]).max() < TOL[dtype], i
