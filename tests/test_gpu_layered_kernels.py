@@ -176,3 +176,17 @@ def test_router_inside_and_in_front_of_the_experts(width, experts, top, dtype):
     state, ref = dec.new_state(), lo.forward(cfg, w, tokens)
     for i, t in enumerate(tokens):
         assert lm.errors(dec.forward(state, [t], i), ref[i:i + 1]).max() < TOL[dtype], i
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(9, 24, 23), (17, 40, 64), (1, 70, 130)])
+def test_recurrences_of_any_number_of_heads(heads, dim, vdim):
+    # the scan deals eight heads at a time; 65, 128 and 7 tokens: chunks with a rest, whole ones, less than one
+    cfg = lm.config([lm.delta(heads, heads, dim, vdim), lm.retention(heads, dim, vdim, 8)], width=66, vocab=50)
+    w = lm.random_weights(cfg, seed=heads)
+    tokens = [int(t) for t in np.random.default_rng(vdim).integers(0, 50, 200)]
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, w, "float32", max_seq=256)
+    state, at = dec.new_state(), 0
+    for n in (65, 128, 7):
+        assert lm.errors(dec.forward(state, tokens[at:at + n], at), ref[at:at + n]).max() < TOL["float32"], (at, n)
+        at += n
