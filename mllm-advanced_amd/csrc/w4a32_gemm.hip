@@ -1007,17 +1007,25 @@ static double f16_us(int tile, int parts, int M, int K, int N) {
 
 // The rules by tile counts (choose_f16_tile, splitk_plan) come from the decoder's and the vision encoder's shapes and are kept
 // where they are within 5 % of the cheapest of the 128-row shapes 1, 4 and 6; elsewhere that one is taken, in up to
-// most_parts parts of eight stages or more. What the rules split stays split, into no more parts than they say: the caller's
-// room is sized for those. Over the 60 problems the choice is 4 % slower than the best shape and number of parts, the rules
-// alone 13 %: M = 256, K = 5120, N = 1536: 23.9 -> 15.1 us in five parts; 190, 4768, 83: 22.8 -> 9.9 in eight.
+// most_parts parts of eight stages or more. A rule's 256-row shape is left for 9 % only: it delivers more than the cost says when
+// its last round is short (K = 8960, N = 1536, M = 5400..7500: 209..224 us, shape 6 for 6..7 % less by cost 212..229; 1280,
+// 5120, 1300: 24.8, 26.5; but 5120, 1280, 6410: 122 -> 95, 1536, 151936, 128: 122 -> 84, both 28 % by cost). What
+// the rules split stays split, into no more parts than they say, as the caller's room is sized for those, and in shape 6 into no
+// fewer than half: two parts for five at K = 8960, N = 1536 took 44.2 us for 44.1 at 896 rows, and 36.8 for 35.2 where the next
+// layer adds them up; three take 40.8 and 33.6. Over the 60 problems the choice is 4 % slower than the best shape and number of parts,
+// the rules alone 13 %: M = 256, K = 5120, N = 1536: 23.2 -> 15.6 us in five parts; 190, 4768, 83: 22.8 -> 9.9 in eight. What it
+// changes for long k (weights from memory; and without the second kernel): K = 8960, N = 1536, 131 rows: 18.4 -> 17.3 (13.6 -> 13.3),
+// 256: 23.1 -> 18.8 (15.6 -> 14.3), 640: 38.0 -> 33.4 (31.4 -> 27.7), 1400: 69.1 -> 61.5 (58.5 -> 51.7), 2300: 96.4 -> 87.6 (80.8
+// -> 76.4); K = 18944, N = 3584, 200 rows: 61.8 -> 49.7 (56.6 -> 45.1).
 static SplitPlan cheaper_f16(SplitPlan rule, int M, int K, int N, int most_parts) {
   const int stages = (K + kF16BK - 1) / kF16BK;
   SplitPlan best = rule;
-  double least = 0.95 * f16_us(rule.tile, rule.parts, M, K, N);
+  double least = (kF16Cost[rule.tile].bm == 256 ? 0.91 : 0.95) * f16_us(rule.tile, rule.parts, M, K, N);
   for (int parts : {1, 2, 3, 4, 5, 6, 8, 10}) {
     if (parts > most_parts || (parts > 1 && stages < 8 * parts)) break;
     if (parts == 1 && rule.parts > 1) continue;
     for (int tile : {1, 4, 6}) {
+      if (tile == 6 && 2 * parts < rule.parts) continue;
       const double us = f16_us(tile, parts, M, K, N);
       if (us < least) {
         least = us;
@@ -1081,9 +1089,10 @@ hipError_t launch_gemm_pair(float* act, const uint8_t* ws, const uint8_t* gate, 
 }
 
 // Split-K: tile shape and number of parts for a problem (parts == 1: not worth splitting).
-// Measured on MI355X (down_proj, K = 8960, N = 1536): M = 128: 44 -> 16 us, 256: 44 -> 21,
+// Measured on MI355X (down_proj, K = 8960, N = 1536), unsplit and as the rule says: M = 128: 44 -> 16 us, 256: 44 -> 21,
 // 512: 47 -> 29, 1024: 50 -> 45, 2048: 85 -> 82. By rule a long K alone is split, into about one or two workgroups
-// per CU in all (10 parts up to 24 tiles, 5 up to 96, then 4); other shapes are where their cost says so.
+// per CU in all (10 parts up to 24 tiles, 5 up to 96, then 4); other shapes, and other plans of these, are where their cost
+// says so: cheaper_f16.
 SplitPlan splitk_plan(int M, int K, int N) {
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   const int nstages = (K + kF16BK - 1) / kF16BK;
