@@ -359,12 +359,25 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(ZT* __restrict__ z, 
                                                             float eps) {
   constexpr int kE = 16 / (int)sizeof(ZT), kWaves = kThreads / 64;
   __shared__ float s_part[kWaves][3];
+  // ld is a multiple of four elements: of bf16, rows (and the tensor) start on 8 bytes, and a row may end in half a piece
+  typedef u32x4 Piece __attribute__((aligned(8)));
+  typedef uint32_t Half __attribute__((ext_vector_type(2)));
   ZT* row = z + (size_t)blockIdx.x * ld;
   u32x4 raw[P];
+  if (kE == 4 || ld % kE == 0) {
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    const int c = kE * ((int)threadIdx.x + kThreads * p);
-    raw[p] = *reinterpret_cast<const u32x4*>(row + (c < ld ? c : 0));
+    for (int p = 0; p < P; ++p) {
+      const int c = kE * ((int)threadIdx.x + kThreads * p);
+      raw[p] = *reinterpret_cast<const Piece*>(row + (c < ld ? c : 0));
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int c = kE * ((int)threadIdx.x + kThreads * p);
+      const Half lo = *reinterpret_cast<const Half*>(row + (c < ld ? c : 0));
+      const Half hi = *reinterpret_cast<const Half*>(row + (c + 4 < ld ? c + 4 : 0));
+      raw[p] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
   }
   auto get = [](const u32x4& v, int e) __attribute__((always_inline)) {
     if constexpr (sizeof(ZT) == 2) return __uint_as_float(e & 1 ? v[e / 2] & 0xFFFF0000u : v[e / 2] << 16);
@@ -389,9 +402,9 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(ZT* __restrict__ z, 
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int c = kE * ((int)threadIdx.x + kThreads * p);
-    if (c >= ld) continue;
 #pragma unroll
     for (int h = 0; h < kE; h += 4) {
+      if (c + h >= ld) continue;
       float4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {

@@ -152,6 +152,26 @@ def test_polynorm_of_every_row_length(pkg, F, ld):
         assert bool((y[:, F:] == 0).all())
 
 
+@pytest.mark.parametrize("F,ld", [(3, 4), (9, 12), (33, 36), (97, 100), (2050, 2052), (4099, 4100), (6150, 6156), (20480, 20484)])
+def test_polynorm_of_rows_that_end_in_half_a_piece(pkg, F, ld):
+    """bf16 rows of an odd number of four elements, starting on eight bytes only: no row touches another, or what lies around all."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(ld)
+    act = torch.tensor([0.7, -0.4, 0.3, 0.05], device="cuda")
+    rms = lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-5)
+    for dtype, tol in ((torch.float32, 3e-6), (torch.bfloat16, 4e-3)):  # as above
+        for rows, front in ((1, 0), (300, 4)):
+            z = torch.randn(front + rows * ld + ld, generator=g, device="cuda").to(dtype)
+            before, body = z.clone(), slice(front, front + rows * ld)
+            x = before[body].view(rows, ld)[:, :F].double()
+            ref = 0.7 * rms(x) - 0.4 * rms(x ** 2) + 0.3 * rms(x ** 3) + 0.05
+            y = pkg.op_polynorm(z[body].view(rows, ld), F, act, 1e-5).double()
+            assert float((y[:, :F] - ref).abs().max() / ref.abs().max()) < tol, (rows, dtype)
+            assert bool((y[:, F:] == 0).all())
+            assert torch.equal(z[:front], before[:front]) and torch.equal(z[front + rows * ld:], before[front + rows * ld:])
+
+
 @pytest.mark.parametrize("rows", [9, 63, 65, 130])
 @pytest.mark.parametrize("width,ff,vocab", [(70, 100, 130), (1030, 2100, 65)])
 def test_f32_products_of_a_prompt(width, ff, vocab, rows):
