@@ -19,7 +19,8 @@ namespace w4 {
 
 namespace {
 
-template <typename T, int BM, int BN, int WM, int WN, int D, typename CT>
+// kFar: operands or results whose rows are too long for 32-bit offsets
+template <typename T, int BM, int BN, int WM, int WN, int D, typename CT, bool kFar>
 __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                               CT* __restrict__ c, int M, int N, int K, int ldc, int mt,
                                                               int nt) {
@@ -37,18 +38,34 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restric
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
 
-  unsigned oa[Tile::LA], ob[Tile::LB];
-#pragma unroll
-  for (int i = 0; i < Tile::LA; ++i) oa[i] = (unsigned)sizeof(T) * Tile::row(i) * K + Tile::column();
-#pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * K + Tile::column();
   const int ma = min(M - m0, BM), nb = min(N - n0, BN);
+  RowOffset<kFar> oa[Tile::LA], ob[Tile::LB];
+  auto at = [&](int i, int rows) __attribute__((always_inline)) {
+    const int r = kFar ? min(Tile::row(i), rows - 1) : Tile::row(i);
+    return (RowOffset<kFar>)sizeof(T) * r * K + Tile::column();
+  };
+#pragma unroll
+  for (int i = 0; i < Tile::LA; ++i) oa[i] = at(i, ma);
+#pragma unroll
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = at(i, nb);
   f32x16 acc[FM][FN];
-  Tile::run(smem, rows_buffer(a + (size_t)m0 * K, sizeof(T) * ma * K), oa,
-            rows_buffer(b + (size_t)n0 * K, sizeof(T) * nb * K), ob, kb, ke, acc);
+  Tile::run(smem, tile_rows_at<kFar>(a + (size_t)m0 * K, sizeof(T) * ma * K), oa,
+            tile_rows_at<kFar>(b + (size_t)n0 * K, sizeof(T) * nb * K), ob, kb, ke, acc);
 
-  // rows past the last one lie past the buffer's end, columns are sent there: what is stored there is dropped
   c += (size_t)blockIdx.y * M * ldc + (size_t)m0 * ldc;
+  if constexpr (kFar) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int row = wm + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), col = n0 + wn + 32 * j + (lane & 31);
+          if (row < ma && col < N) c[(size_t)row * ldc + col] = (CT)acc[i][j][v];
+        }
+    return;
+  }
+  // rows past the last one lie past the buffer's end, columns are sent there: what is stored there is dropped
   const __amdgpu_buffer_rsrc_t out = rows_buffer(c, sizeof(CT) * ma * ldc);
   const unsigned step = (unsigned)sizeof(CT) * ldc;
 #pragma unroll
@@ -56,7 +73,7 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restric
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int col = n0 + wn + 32 * j + (lane & 31);
-      unsigned off = col < N ? (unsigned)sizeof(CT) * ((wm + 32 * i + 4 * (lane >> 5)) * ldc + col) : 0xF0000000u;
+      unsigned off = col < N ? (unsigned)sizeof(CT) * ((wm + 32 * i + 4 * (lane >> 5)) * ldc + col) : kPastEnd;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         float x = acc[i][j][v];
@@ -68,11 +85,11 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restric
     }
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int D, typename CT>
+template <typename T, int BM, int BN, int WM, int WN, int D, typename CT, bool kFar = false>
 hipError_t launch_tile_t(const T* a, const T* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
   const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
   constexpr size_t lds = MfmaTile<T, BM, BN, WM, WN, D>::kLds;
-  auto kern = matmul_kernel<T, BM, BN, WM, WN, D, CT>;
+  auto kern = matmul_kernel<T, BM, BN, WM, WN, D, CT, kFar>;
   static LdsLimitOnce raised;
   if (lds > 64 * 1024)
     if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
@@ -139,6 +156,14 @@ hipError_t launch_shape(int shape, const __bf16* a, const __bf16* b, void* c, in
     default: return launch_tile_t<__bf16, 64, 64, 2, 2, 4, CT>(a, b, c, M, N, K, ldc, parts, s);
   }
 }
+
+// Rows of millions of elements: one shape, with 64-bit offsets
+template <typename T, typename CT>
+hipError_t launch_far(const T* a, const T* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
+  return launch_tile_t<T, 64, 64, 2, 2, 4, CT, true>(a, b, c, M, N, K, ldc, parts, s);
+}
+template <typename T, typename CT>
+bool product_near(int K, int ldc) { return rows_near(sizeof(T) * (size_t)K) && results_near(sizeof(CT) * (size_t)ldc); }
 
 // ---------------------------------------------------------------------------------------------
 template <typename WT, int kKind, int R, int U>
@@ -254,6 +279,8 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
   if (K % kPad != 0 || parts < 1 || parts > K / kPad || (parts > 1 && c_bf16)) return hipErrorInvalidValue;
   const __bf16* pa = static_cast<const __bf16*>(a);
   const __bf16* pb = static_cast<const __bf16*>(b);
+  if (c_bf16 && !product_near<__bf16, __bf16>(K, ldc)) return launch_far<__bf16, __bf16>(pa, pb, c, M, N, K, ldc, parts, s);
+  if (!c_bf16 && !product_near<__bf16, float>(K, ldc)) return launch_far<__bf16, float>(pa, pb, c, M, N, K, ldc, parts, s);
   const int shape = best_plan(false, M, N, K, parts, parts, c_bf16 ? 2 : 4).shape;
   return c_bf16 ? launch_shape<__bf16>(shape, pa, pb, c, M, N, K, ldc, parts, s)
                 : launch_shape<float>(shape, pa, pb, c, M, N, K, ldc, parts, s);
@@ -261,6 +288,7 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
 
 hipError_t launch_matmul_f32(const float* a, const float* b, float* c, int M, int N, int K, int parts, hipStream_t s) {
   if (K % 32 != 0 || parts < 1 || parts > K / 32) return hipErrorInvalidValue;
+  if (!product_near<float, float>(K, N)) return launch_far<float, float>(a, b, c, M, N, K, N, parts, s);
   switch (best_plan(true, M, N, K, parts, parts, 4).shape) {
     case 0: return launch_tile_t<float, 64, 128, 2, 4, 2, float>(a, b, c, M, N, K, N, parts, s);
     default: return launch_tile_t<float, 64, 64, 2, 2, 4, float>(a, b, c, M, N, K, N, parts, s);

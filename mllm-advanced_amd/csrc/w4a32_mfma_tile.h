@@ -18,6 +18,8 @@
 // f32 products take eight times as long for the same bytes: a SIMD with one wavefront is busy once its operands are there.
 #pragma once
 
+#include <type_traits>
+
 #include "w4a32_layered_kernels.h"
 
 namespace w4 {
@@ -36,6 +38,27 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* base, 
 __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned lane_off, unsigned off) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
 }
+
+// Rows that lie further apart than a buffer's 32-bit offsets reach within a tile: plain loads, for which every row must be there.
+struct FarRows {
+  const uint8_t* base;
+};
+__device__ __forceinline__ u32x4 load16(FarRows r, size_t lane_off, size_t off) {
+  return *reinterpret_cast<const u32x4*>(r.base + lane_off + off);
+}
+template <bool kFar>
+__device__ __forceinline__ auto tile_rows_at(const void* base, size_t bytes) {
+  if constexpr (kFar) return FarRows{static_cast<const uint8_t*>(base)};
+  else return rows_buffer(base, bytes);
+}
+template <bool kFar>
+using RowOffset = std::conditional_t<kFar, size_t, unsigned>;
+
+// Whether a tile of up to 256 rows of `row_bytes` has them within a buffer; of results also with room for what is sent past the
+// buffer's end: from kPastEnd, 27 rows further on at most, without coming round to its start.
+constexpr unsigned kPastEnd = 0xF0000000u;
+inline bool rows_near(size_t row_bytes) { return 256 * row_bytes <= 0xFFFFFFFFu; }
+inline bool results_near(size_t row_bytes) { return 28 * row_bytes <= 0xFFFFFFFFu - kPastEnd; }
 
 // A wavefront's operand of a step, and what a pair of them adds to a block of C: k 8 h .. 8 h + 7 of the step's 16 (bf16) from the
 // lanes of half h; of the step's 8 (f32) 4 h .. 4 h + 3, of which one product takes one k from each half.
@@ -70,11 +93,11 @@ struct MfmaTile {
   static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x + kThreads * i) >> 3; }
   static __device__ __forceinline__ unsigned column() { return 16 * (threadIdx.x & 7); }
 
-  // acc = rows of A times rows of B over k in [kb, ke), a range of whole tiles that is not empty; oa, ob: where the pieces'
-  // rows start, with column() added
-  static __device__ __forceinline__ void run(uint8_t* smem, __amdgpu_buffer_rsrc_t a, const unsigned (&oa)[LA],
-                                             __amdgpu_buffer_rsrc_t b, const unsigned (&ob)[LB], int kb, int ke,
-                                             f32x16 (&acc)[FM][FN]) {
+  // acc = rows of A times rows of B over k in [kb, ke), a range of whole tiles that is not empty; a, b: buffers or FarRows; oa, ob:
+  // where the pieces' rows start, with column() added
+  template <typename Rows, typename Off>
+  static __device__ __forceinline__ void run(uint8_t* smem, Rows a, const Off (&oa)[LA], Rows b, const Off (&ob)[LB], int kb,
+                                             int ke, f32x16 (&acc)[FM][FN]) {
     T* s_a = reinterpret_cast<T*>(smem);  // [2][BM][kLd]
     T* s_b = s_a + 2 * BM * kLd;          // [2][BN][kLd]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -87,8 +110,8 @@ struct MfmaTile {
     const T* const sa_r = s_a + (wm + (lane & 31)) * kLd + kE * (lane >> 5);
     const T* const sb_r = s_b + (wn + (lane & 31)) * kLd + kE * (lane >> 5);
     auto fetch = [&](int set, int p, int k) __attribute__((always_inline)) {
-      if (p < LA) ra[set][p < LA ? p : 0] = load16(a, oa[p < LA ? p : 0], (int)sizeof(T) * k);
-      else rb[set][p < LA ? 0 : p - LA] = load16(b, ob[p < LA ? 0 : p - LA], (int)sizeof(T) * k);
+      if (p < LA) ra[set][p < LA ? p : 0] = load16(a, oa[p < LA ? p : 0], (Off)sizeof(T) * k);
+      else rb[set][p < LA ? 0 : p - LA] = load16(b, ob[p < LA ? 0 : p - LA], (Off)sizeof(T) * k);
     };
     auto stash = [&](int set, int p, int buf) __attribute__((always_inline)) {
       if (p < LA) *reinterpret_cast<u32x4*>(sa_w + (buf * BM + kThreads / 8 * p) * kLd) = ra[set][p < LA ? p : 0];

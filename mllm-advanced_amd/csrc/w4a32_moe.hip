@@ -220,7 +220,8 @@ __device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, cons
 }
 
 // act [sorted pair][Fp] = glu(h gate^T, h up^T). A wavefront's column blocks are gate and up of the same 32 columns, in turn.
-template <typename T, int BM, int BN, int WM, int WN, int D>
+// kFar, here and below: rows too long for 32-bit offsets.
+template <typename T, int BM, int BN, int WM, int WN, int D, bool kFar>
 __global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __restrict__ h, const T* __restrict__ w,
                                                                    T* __restrict__ act, const int* __restrict__ order,
                                                                    const MoeTile* __restrict__ tiles,
@@ -233,16 +234,32 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __re
   int n;
   const int N = 2 * Fp;
   if (!moe_tile(tiles, n_tiles, BM, (N + BN - 1) / BN, &tile, &n)) return;
-  const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  unsigned oa[Tile::LA], ob[Tile::LB];
+  const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nb = min(BN, N - n0);
+  RowOffset<kFar> oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
   for (int i = 0; i < Tile::LA; ++i)
-    oa[i] = (unsigned)sizeof(T) * (order[tile.row0 + min(Tile::row(i), tile.rows - 1)] / top) * Hp + Tile::column();
+    oa[i] = (RowOffset<kFar>)sizeof(T) * (order[tile.row0 + min(Tile::row(i), tile.rows - 1)] / top) * Hp + Tile::column();
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * Hp + Tile::column();
+  for (int i = 0; i < Tile::LB; ++i)
+    ob[i] = (RowOffset<kFar>)sizeof(T) * (kFar ? min(Tile::row(i), nb - 1) : Tile::row(i)) * Hp + Tile::column();
   f32x16 acc[Tile::FM][Tile::FN];
-  Tile::run(smem, rows_buffer(h, sizeof(T) * M * Hp), oa,
-            rows_buffer(w + ((size_t)tile.expert * N + n0) * Hp, sizeof(T) * min(BN, N - n0) * Hp), ob, 0, Hp, acc);
+  Tile::run(smem, tile_rows_at<kFar>(h, sizeof(T) * M * Hp), oa,
+            tile_rows_at<kFar>(w + ((size_t)tile.expert * N + n0) * Hp, sizeof(T) * nb * Hp), ob, 0, Hp, acc);
+  if constexpr (kFar) {
+#pragma unroll
+    for (int j = 0; j < Tile::FN; j += 2) {
+      const int col = (n0 + BN / WN * (wave % WN) + 32 * j) / 2 + (lane & 31);
+#pragma unroll
+      for (int i = 0; i < Tile::FM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int r = BM / WM * (wave / WN) + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          if (r < tile.rows && col < Fp)
+            act[(size_t)(tile.row0 + r) * Fp + col] = (T)clamped_glu<T>(acc[i][j][v], acc[i][j + 1][v], limit);
+        }
+    }
+    return;
+  }
   const __amdgpu_buffer_rsrc_t out = rows_buffer(act + (size_t)tile.row0 * Fp, sizeof(T) * tile.rows * Fp);
 #pragma unroll
   for (int j = 0; j < Tile::FN; j += 2) {
@@ -250,7 +267,7 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __re
 #pragma unroll
     for (int i = 0; i < Tile::FM; ++i) {
       const int r = BM / WM * (wave / WN) + 32 * i + 4 * (lane >> 5);
-      unsigned off = col < Fp ? (unsigned)sizeof(T) * (r * Fp + col) : 0xF0000000u;  // past the end: not stored
+      unsigned off = col < Fp ? (unsigned)sizeof(T) * (r * Fp + col) : kPastEnd;  // past the end: not stored
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         float g = acc[i][j][v], u = acc[i][j + 1][v];
@@ -265,7 +282,7 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __re
 }
 
 // parts [slot][token][Hp] = weight * act down^T; a slot has rows_all tokens
-template <typename T, int BM, int BN, int WM, int WN, int D>
+template <typename T, int BM, int BN, int WM, int WN, int D, bool kFar>
 __global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restrict__ act, const T* __restrict__ w,
                                                                 float* __restrict__ parts, const int* __restrict__ order,
                                                                 const float* __restrict__ wts,
@@ -281,14 +298,19 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restr
   // a row's place and weight, asked for now and handed round through LDS behind the products
   static_assert(BM <= Tile::kThreads, "a thread per row");
   const int own = order[tile.row0 + min((int)threadIdx.x, tile.rows - 1)];
-  unsigned oa[Tile::LA], ob[Tile::LB];
+  const int nb = min(BN, Hp - n0);
+  RowOffset<kFar> oa[Tile::LA], ob[Tile::LB];
+  auto at = [&](int i, int rows) __attribute__((always_inline)) {
+    const int r = kFar ? min(Tile::row(i), rows - 1) : Tile::row(i);
+    return (RowOffset<kFar>)sizeof(T) * r * Fp + Tile::column();
+  };
 #pragma unroll
-  for (int i = 0; i < Tile::LA; ++i) oa[i] = (unsigned)sizeof(T) * Tile::row(i) * Fp + Tile::column();
+  for (int i = 0; i < Tile::LA; ++i) oa[i] = at(i, tile.rows);
 #pragma unroll
-  for (int i = 0; i < Tile::LB; ++i) ob[i] = (unsigned)sizeof(T) * Tile::row(i) * Fp + Tile::column();
+  for (int i = 0; i < Tile::LB; ++i) ob[i] = at(i, nb);
   f32x16 acc[Tile::FM][Tile::FN];
-  Tile::run(smem, rows_buffer(act + (size_t)tile.row0 * Fp, sizeof(T) * tile.rows * Fp), oa,
-            rows_buffer(w + ((size_t)tile.expert * Hp + n0) * Fp, sizeof(T) * min(BN, Hp - n0) * Fp), ob, 0, Fp, acc);
+  Tile::run(smem, tile_rows_at<kFar>(act + (size_t)tile.row0 * Fp, sizeof(T) * tile.rows * Fp), oa,
+            tile_rows_at<kFar>(w + ((size_t)tile.expert * Hp + n0) * Fp, sizeof(T) * nb * Fp), ob, 0, Fp, acc);
   const float weight = wts[own];
   __syncthreads();
   float* s_w = reinterpret_cast<float*>(smem);            // [BM]
@@ -441,7 +463,7 @@ Scratch scratch_of(int dtype, int M, int experts, int top, int Fp) {
 }
 
 // Up, Down: the two products' tiles, of equal height
-template <typename Up, typename Down, typename T>
+template <typename Up, typename Down, bool kFar = false, typename T>
 hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down, int M, int rows_all, float* parts,
                    uint8_t* ws, const Scratch& c, hipStream_t s) {
   static_assert(Up::kRows == Down::kRows, "one list of tiles");
@@ -450,8 +472,8 @@ hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down
   int* n_tiles = reinterpret_cast<int*>(ws + c.n_tiles);
   T* act = reinterpret_cast<T*>(ws + c.act);
   const int most = (int)(((size_t)M * g.top + Up::kRows - 1) / Up::kRows) + g.experts;  // workgroups past the last tile return
-  auto up = moe_gate_up_kernel<T, Up::kRows, Up::kCols, Up::kWM, Up::kWN, Up::kDepth>;
-  auto dn = moe_down_kernel<T, Down::kRows, Down::kCols, Down::kWM, Down::kWN, Down::kDepth>;
+  auto up = moe_gate_up_kernel<T, Up::kRows, Up::kCols, Up::kWM, Up::kWN, Up::kDepth, kFar>;
+  auto dn = moe_down_kernel<T, Down::kRows, Down::kCols, Down::kWM, Down::kWN, Down::kDepth, kFar>;
   static LdsLimitOnce raised_up, raised_dn;
   if (Up::kLds > 64 * 1024)
     if (hipError_t e = raised_up.raise(reinterpret_cast<const void*>(up), Up::kLds); e != hipSuccess) return e;
@@ -473,10 +495,16 @@ struct TileOf {
 };
 
 template <typename T>
+bool experts_far(const MoeGeom& g) {
+  return !rows_near(sizeof(T) * (size_t)std::max(g.Hp, g.Fp)) || !results_near(sizeof(T) * (size_t)g.Fp);
+}
+
+template <typename T>
 hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, size_t part_stride, int ldl,
                      const T* gate_up, const T* down, int M, int rows_all, float* parts, uint8_t* ws, hipStream_t s) {
   const Scratch c = scratch_of(dtype, M, g.experts, g.top, g.Fp);
-  const int bm = tile_rows(dtype, M, g.experts, g.top);
+  const bool far = experts_far<T>(g);
+  const int bm = far ? 64 : tile_rows(dtype, M, g.experts, g.top);
   int* ids = reinterpret_cast<int*>(ws + c.ids);
   hipLaunchKernelGGL(moe_choose_kernel, dim3((M + 3) / 4), dim3(256), 0, s, logits, logit_parts, part_stride, ldl, M,
                      g.experts, g.top, ids, reinterpret_cast<float*>(ws + c.wts));
@@ -485,6 +513,10 @@ hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logit
                      reinterpret_cast<int*>(ws + c.order), reinterpret_cast<MoeTile*>(ws + c.tiles),
                      reinterpret_cast<int*>(ws + c.n_tiles));
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  if (far) {
+    using Far = TileOf<T, 64, 128, 2, 2, 2>;
+    return grouped<Far, Far, true>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+  }
   // (Us for gate and up, then down, of 16 experts, 4 per token. 1501 tokens, [2 x 2240][1536]: 128 x 128 124, 72, 128 x 256 128, 78;
   // 2048 tokens, [2 x 4736][3584]: 673, 352 against 629, 312, 256 x 256 599, 340; 100 tokens, [2 x 2240][1536]: 64 x 128 49, 23 =
   // 4.5 and 4.9 TB/s of weights, 128 x 128 53, 26. Before these shapes: 145, 106 for the first.)
@@ -512,7 +544,7 @@ template <typename T>
 hipError_t prefill_turns(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, int ldl,
                          const T* gate_up, const T* down, int M, float* parts, uint8_t* ws, hipStream_t s) {
   if (logit_parts < 1 || logit_parts > kMaxParts) return hipErrorInvalidValue;
-  const int turn = (int)std::min<size_t>(M, 0xFFFFFFFFu / (sizeof(T) * g.Hp));
+  const int turn = experts_far<T>(g) ? M : (int)std::min<size_t>(M, 0xFFFFFFFFu / (sizeof(T) * g.Hp));
   for (int m = 0; m < M; m += turn)
     if (hipError_t e = prefill_t(dtype, g, h + (size_t)m * g.Hp, logits + (size_t)m * ldl, logit_parts, (size_t)M * ldl, ldl,
                                  gate_up, down, std::min(turn, M - m), M, parts + (size_t)m * g.Hp, ws, s);

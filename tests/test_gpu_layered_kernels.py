@@ -117,6 +117,61 @@ def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
         assert float((parts[:, :, :hidden] - ref).abs().max()) < tol * float(ref.abs().max())
 
 
+# rows of results of 2396745 f32, 4793490 bf16 values are the longest whose stores have 32-bit offsets; of operands 8388607 bf16,
+# 4194303 f32 (in whole steps of 64 and 32)
+@pytest.mark.parametrize("M,N,K,kinds", [(9, 2396745, 64, "bf16 f32"), (67, 2396746, 64, "bf16 f32"), (9, 4793491, 64, "bf16 bf16"),
+                                         (67, 2396746, 32, "f32 f32"), (67, 70, 8388544, "bf16 f32"), (67, 70, 8388608, "bf16 f32"),
+                                         (9, 70, 8388608, "bf16 bf16"), (67, 70, 4194304, "f32 f32")])
+def test_products_of_rows_of_millions(pkg, M, N, K, kinds):
+    import torch
+
+    types = {"bf16": torch.bfloat16, "f32": torch.float32}
+    dtype, out = (types[t] for t in kinds.split())
+    g = torch.Generator(device="cuda").manual_seed(N)
+    # 0 and +-1: sums below 2^24 in size, exact in f32 in any order
+    a, b = (torch.randint(-1, 2, (n, K), generator=g, device="cuda", dtype=torch.int8).to(dtype) for n in (M, N))
+    ref = torch.zeros((M, N), device="cuda")
+    for k in range(0, K, 1 << 18):
+        ref += a[:, k:k + (1 << 18)].float() @ b[:, k:k + (1 << 18)].float().t().contiguous()
+    c = torch.full((M + 1, N), 7.0, dtype=out, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    if dtype == torch.float32:
+        rc = pkg.lib().w4a32_op_matmul_f32_nt(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, stream)
+    else:
+        rc = pkg.lib().w4a32_op_matmul_bf16_nt(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, N, int(out == dtype), 1, stream)
+    assert rc == 0
+    assert torch.equal(c[:M], ref.to(out)) and bool((c[M] == 7).all())
+
+
+@pytest.mark.parametrize("rows,hidden,ff,kind", [(67, 40, 4793450, "bfloat16"), (67, 40, 2396740, "float32"),
+                                                 (67, 8388600, 40, "bfloat16")])
+def test_experts_of_rows_of_millions(pkg, rows, hidden, ff, kind):
+    import torch
+
+    dtype = getattr(torch, kind)
+    g = torch.Generator(device="cuda").manual_seed(ff)
+    rnd = lambda *s, std=1.0: (torch.randn(s, generator=g, device="cuda") * std).bfloat16().to(dtype)
+    pad = lambda n: (n + 63) // 64 * 64
+    h, gate, up, down = rnd(rows, hidden), rnd(1, ff, hidden, std=hidden ** -0.5), rnd(1, ff, hidden, std=hidden ** -0.5), \
+        rnd(1, hidden, ff, std=ff ** -0.5)
+    hp = torch.zeros((rows, pad(hidden)), dtype=dtype, device="cuda")
+    hp[:, :hidden] = h
+    dp = torch.zeros((1, pad(hidden), pad(ff)), dtype=dtype, device="cuda")
+    dp[:, :hidden, :ff] = down
+    logits = torch.zeros((rows, 1), device="cuda")
+    parts = pkg.op_experts(hp, logits, pkg.pack_gate_up(gate, up), dp, hidden, 1, ff, 0.9)
+    del hp, dp
+    gg = (h.double() @ gate[0].double().t().contiguous()).clamp(max=0.9)
+    uu = (h.double() @ up[0].double().t().contiguous()).clamp(-0.9, 0.9)
+    act = gg * torch.sigmoid(1.702 * gg) * (uu + 1)
+    del gg, uu, gate, up
+    assert bool((parts[:, :, hidden:] == 0).all())
+    ref = act @ down[0].double().t().contiguous()
+    # f32 sums of n = 2.4 to 8.4 million terms, one after the other: each addition rounds the sum so far, sqrt(n) 2^-24 of the result
+    # in all, 1.7e-4 at the most; bf16 as in test_grouped_products_of_every_height
+    assert float((parts[0, :, :hidden] - ref).abs().max()) < (2e-4 if kind == "float32" else 1e-2) * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,taps", [(2050, 4), (2500, 8), (4200, 3)])
 def test_norm_of_wide_rows_in_two_launches(width, taps, dtype):
