@@ -563,16 +563,16 @@ hipError_t decode_t(const MoeGeom& g, const RowPrologue& pro, const float* logit
     const int groups = g.top * g.Fp / P;
     const dim3 grid(std::min((groups + kRowWaves - 1) / kRowWaves, 512));
     const size_t lds = sizeof(float) * g.Hp;
-    auto run = [&](auto kern) -> hipError_t {
-      static LdsLimitOnce raised;
+    auto run = [&](auto kern, LdsLimitOnce* raised) -> hipError_t {  // (both kernels have one type: a limit raised here would be for either)
       if (lds > 60 * 1024)
-        if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), 159 * 1024); e != hipSuccess) return e;
+        if (hipError_t e = raised->raise(reinterpret_cast<const void*>(kern), 159 * 1024); e != hipSuccess) return e;
       hipLaunchKernelGGL(kern, grid, dim3(kRowThreads), lds, s, pro, logits, router, gate_up, g.experts, g.top, g.Hp, g.Fp,
                          g.limit, z, sel);
       return hipGetLastError();
     };
-    const hipError_t e =
-        moe_routes_itself(sizeof(WT), g) ? run(moe_row_gate_up_kernel<WT, P, U, true>) : run(moe_row_gate_up_kernel<WT, P, U, false>);
+    static LdsLimitOnce raised_router, raised_plain;
+    const hipError_t e = moe_routes_itself(sizeof(WT), g) ? run(moe_row_gate_up_kernel<WT, P, U, true>, &raised_router)
+                                                          : run(moe_row_gate_up_kernel<WT, P, U, false>, &raised_plain);
     if (e != hipSuccess) return e;
   }
   RowPrologue p{};
