@@ -1093,12 +1093,15 @@ hipError_t launch_gemm_pair(float* act, const uint8_t* ws, const uint8_t* gate, 
 // 512: 47 -> 29, 1024: 50 -> 45, 2048: 85 -> 82. By rule a long K alone is split, into about one or two workgroups
 // per CU in all (10 parts up to 24 tiles, 5 up to 96, then 4); other shapes, and other plans of these, are where their cost
 // says so: cheaper_f16.
+bool splitk_by_rule(int M, int K, int N) {
+  return M > kGemvMaxM && K > 95 * kF16BK && (long)((M + 127) / 128) * ((N + 127) / 128) <= 256;
+}
+
 SplitPlan splitk_plan(int M, int K, int N) {
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-  const int nstages = (K + kF16BK - 1) / kF16BK;
   if (M <= kGemvMaxM) return {2, 1};
   SplitPlan p{2, 1};
-  if (nstages >= 96 && tiles <= 256) {
+  if (splitk_by_rule(M, K, N)) {
     p.parts = tiles <= 24 ? 10 : tiles <= 96 ? 5 : 4;
     if (tiles <= 16) {
       p.tile = 1;  // 128 x 64: twice the workgroups (M = 128: 19 -> 16 us)

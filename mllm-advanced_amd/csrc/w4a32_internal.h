@@ -91,6 +91,7 @@ struct SplitPlan {
   int tile, parts;
 };
 SplitPlan splitk_plan(int M, int K, int N);
+bool splitk_by_rule(int M, int K, int N);  // split for its long K, whatever the cost
 hipError_t launch_gemm_pair(float* act, const uint8_t* ws, const uint8_t* gate, const uint8_t* up, int M,
                             int K, int N, hipStream_t s);
 const float* linear_bias(const uint8_t* packed, int N, int K);  // the bias row inside a packed blob
