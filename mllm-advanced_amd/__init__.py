@@ -225,16 +225,23 @@ def _ptr(t):
 _raw_stream = None
 
 
+def _stream_getter(torch):
+    """Where the current device's current stream comes from. torch.cuda.current_stream() makes an object of it, which takes 3 us,
+    as long as the kernel of a one-row Linear; the getters behind it, 0.25 us, are torch's own and may go away."""
+    device, stream = (getattr(torch._C, n, None) for n in ("_cuda_getDevice", "_cuda_getCurrentRawStream"))
+    if device is None or stream is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: stream(device())
+
+
 def _stream():
-    """The current device's current stream, as the C ABI takes it. (torch.cuda.current_stream() makes an object of it, which
-    takes 3 us: as long as the kernel of a one-row Linear.)"""
+    """The current device's current stream, as the C ABI takes it."""
     global _raw_stream
     if _raw_stream is None:
         import torch
 
         torch.cuda.current_stream()  # initialises the device
-        device, stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
-        _raw_stream = lambda: stream(device())
+        _raw_stream = _stream_getter(torch)
     return _raw_stream()
 
 
@@ -452,8 +459,8 @@ def matmul_ws(x, packed, N, ws=None, out=None):
         import torch
 
         out = torch.empty((M, N), dtype=torch.float32, device="cuda")
-    _check(lib().w4a32_matmul_ws(out.data_ptr(), x.data_ptr(), packed.data_ptr(), ws.data_ptr(), ws.nbytes, M, K, N, _stream()),
-           "w4a32_matmul_ws")
+    _check(lib().w4a32_matmul_ws(out.data_ptr(), x.data_ptr(), None if packed is None else packed.data_ptr(), ws.data_ptr(),
+                                 ws.nbytes, M, K, N, _stream()), "w4a32_matmul_ws")
     return out
 
 
