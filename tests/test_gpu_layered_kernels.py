@@ -172,6 +172,25 @@ def test_experts_of_rows_of_millions(pkg, rows, hidden, ff, kind):
     assert float((parts[0, :, :hidden] - ref).abs().max()) < (2e-4 if kind == "float32" else 1e-2) * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("kind", ["float32", "bfloat16"])
+def test_experts_gates_of_any_size(pkg, kind):
+    """Each result is one gate and one up value's, the other terms are 0: every value for itself, from where the sigmoid is 0 up."""
+    import torch
+
+    dtype, n = getattr(torch, kind), 192
+    g = torch.Generator(device="cuda").manual_seed(3)
+    eye = torch.eye(n, device="cuda", dtype=dtype)
+    gate = (torch.rand((n, n), generator=g, device="cuda") * 59.5 - 50.5).to(dtype)
+    gate[0, :8] = torch.tensor([-51.5, -52.5, -60.0, -100.0, -1000.0, -3e30, -0.0, 1e30], device="cuda")
+    up = (torch.randn((n, n), generator=g, device="cuda") * 3).to(dtype)
+    parts = pkg.op_experts(eye, torch.zeros((n, 1), device="cuda"), pkg.pack_gate_up(gate[None], up[None]), eye[None].contiguous(), n,
+                           1, n, 7.0)[0].double()
+    gg, uu = gate.double().clamp(max=7.0).t(), up.double().clamp(-7.0, 7.0).t()
+    ref = gg * torch.sigmoid(1.702 * gg) * (uu + 1)
+    # 1.702 g rounded, up to 86: 86 x 2^-24 = 5.1e-6 in the exponential; a rounding to bf16: 2^-9. Below 2^-126 sigmoids may be 0
+    assert bool((((parts - ref).abs() - 51.5 * 2.0 ** -126 * 22) <= ref.abs() * (1e-5 if kind == "float32" else 2.0 ** -8)).all())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,taps", [(2050, 4), (2500, 8), (4200, 3)])
 def test_norm_of_wide_rows_in_two_launches(width, taps, dtype):
