@@ -49,9 +49,11 @@ __device__ __forceinline__ void top_experts(float (&v)[kLogitRegs], int experts,
   const int lane = threadIdx.x & 63;
   int pick = 0;
   float mine = 0.0f, first = 0.0f, sum = 0.0f;
-  // A value per lane, all of them comparable: each lane counts what comes in front of it, four operations per expert. The rounds
-  // below are six exchanges between lanes each (the choice of 100 tokens, 4 of 16 experts: 6.2 -> 4.4 us).
-  if (experts <= 64 && __popcll(__ballot(v[0] > -INFINITY)) == experts) {
+  // A value per lane, all of them comparable: each lane counts what comes in front of it, four operations per expert and a few
+  // per choice. The rounds below are six exchanges between lanes each, whatever the number of experts. Us of a launch that
+  // chooses, counting / rounds, 100 tokens: 4 of 16 experts 2.8 / 4.8, 8 of 64 4.9 / 7.7, 4 of 64 4.6 / 4.7, 2 of 32 3.2 / 3.3; but 1 of 16
+  // 2.6 / 2.6, 1 of 64 4.4 / 2.5, 2 of 48 3.8 / 3.3 (one token: 4.0 / 2.2 and 3.5 / 2.9): a round is worth 18 experts.
+  if (experts <= min(64, 18 * top - 4) && __popcll(__ballot(v[0] > -INFINITY)) == experts) {
     int rank = 0;
     for (int j = 0; j < experts; ++j) {
       const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v[0]), j));

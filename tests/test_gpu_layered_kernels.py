@@ -258,9 +258,11 @@ def test_f32_products_of_a_prompt(width, ff, vocab, rows):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("width,experts,top", [(70, 1, 1), (250, 9, 2), (700, 33, 16), (700, 64, 64 // 8), (1600, 64, 4), (64, 65, 3)])
+@pytest.mark.parametrize("width,experts,top", [(70, 1, 1), (250, 9, 2), (700, 33, 16), (700, 64, 64 // 8), (1600, 64, 4), (64, 65, 3),
+                                               (70, 13, 1), (70, 16, 1), (130, 32, 2), (130, 33, 2), (200, 49, 3), (200, 56, 3)])
 def test_router_inside_and_in_front_of_the_experts(width, experts, top, dtype):
-    # up to 64 experts by counting, up to 96 KB of router in the experts' launch; rows that agree: the lower expert is chosen
+    # up to 64 experts, and 18 for each that is chosen less 4, by counting, else by rounds; up to 96 KB of router in the experts'
+    # launch; rows that agree: the lower expert is chosen
     cfg = lm.lesarax([lm.rotary(1, 1, 16, 8, mlp=lm.moe(24, experts, top))], width=width, vocab=50)
     w = lm.lesarax_weights(cfg, seed=experts)
     router = next(k for k in w if k.endswith("router"))
