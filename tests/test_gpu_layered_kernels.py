@@ -85,6 +85,8 @@ def test_bf16_product_of_every_shape(pkg, M, N, K):
     (190, 64, 2, 1, 64),      # 95 rows per expert: tiles of 64 rows; one tile of columns, half full
     (200, 130, 2, 1, 130),    # 100: 128 rows
     (1540, 72, 4, 2, 100),    # 770: 256 rows in bf16
+    (12400, 70, 128, 1, 900),   # 96, about 160 tiles of rows: bf16 gate and up in 128 x 256, down in 128 x 128
+    (12400, 1800, 128, 1, 60),  # ... both in 128 x 256; column counts that are no multiple of it
 ])
 def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
     import torch
@@ -246,10 +248,22 @@ def test_polynorm_of_rows_that_end_in_half_a_piece(pkg, F, ld):
             assert torch.equal(z[:front], before[:front]) and torch.equal(z[front + rows * ld:], before[front + rows * ld:])
 
 
+@pytest.mark.parametrize("M,N,K", [(2000, 3001, 256), (1985, 2945, 288), (65, 3003, 96), (9, 65, 32)])
+def test_f32_products_in_one_part(pkg, M, N, K):
+    """64 x 128 (the first two) and 64 x 64, from one to nine tiles of k."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = (torch.randn((n, K), generator=g, device="cuda") for n in (M, N))
+    ref = a.double() @ b.double().t().contiguous()
+    # f32 products and sums of K terms of size 1: sqrt(K) roundings of 2^-24 of a sum of up to 5 sqrt(K), K = 288
+    assert float((pkg.op_matmul_f32_nt(a, b).double() - ref).abs().max()) < 288 * 5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("rows", [9, 63, 65, 130])
 @pytest.mark.parametrize("width,ff,vocab", [(70, 100, 130), (1030, 2100, 65)])
 def test_f32_products_of_a_prompt(width, ff, vocab, rows):
-    """The f32 product's tiles (64 x 64 and 64 x 128, in parts and not) through a model of one layer; every token's logits."""
+    """The f32 product's tiles through a model of one layer, where the norm behind takes parts; every token's logits."""
     cfg = lm.config([lm.retention(2, 24, 24, 8, ff=ff)], width=width, vocab=vocab)
     w = lm.random_weights(cfg, seed=rows)
     tokens = np.random.default_rng(rows).integers(0, vocab, rows)
