@@ -141,10 +141,11 @@ int w4a32_matmul_quantized_ex(float* d_y, const void* d_ws, const void* d_packed
                               int N, int kernel, void* stream);
 
 /* The same product for callers that can lend scratch memory: when the problem has few output
- * tiles and a long K (down_proj at prefill sizes) each tile's k range is dealt to several
- * workgroups, which leave partial sums in d_scratch; a second kernel adds them in a fixed order.
- * w4a32_splitk_scratch_bytes() returns the bytes this needs, 0 when the library would not split the
- * shape; with less scratch than that the call is w4a32_matmul_quantized(). The reference has no
+ * tiles for its K (a long K by rule, as down_proj at prefill sizes; others where their estimated cost says
+ * so) each tile's k range is dealt to several workgroups, which leave partial sums in d_scratch; a second
+ * kernel adds them in a fixed order. w4a32_splitk_scratch_bytes() returns the bytes this needs, 0 when the
+ * library would not split the shape; with less scratch than that the call is w4a32_matmul_quantized(), and also,
+ * unless K > 6080, with d_y or d_scratch not on 16 bytes (W4A32_EINVAL then). The reference has no
  * counterpart: its matmul splits M over threads only (kai_linear.cpp:366-396). */
 size_t w4a32_splitk_scratch_bytes(int M, int K, int N);
 int w4a32_matmul_quantized_splitk(float* d_y, const void* d_ws, const void* d_packed, int M, int K,
@@ -157,7 +158,7 @@ int w4a32_matmul(float* d_y, const float* d_x, const void* d_packed, void* d_ws,
 
 /* The whole op for a caller that says how large its workspace is: with at least w4a32_workspace_bytes_n(M, K, N)
  * bytes at d_ws (the activation workspace plus, behind it, room for the partial sums of a product whose k range
- * the library deals to several workgroups: down_proj at prefill sizes) the call takes that faster form itself;
+ * the library deals to several workgroups) the call takes that faster form itself;
  * with at least w4a32_workspace_bytes(M, K) it is w4a32_matmul; with less, W4A32_EINVAL. One call per Linear,
  * as ...::matmul (kai_linear.cpp:350-398) is called from ArmLinearOp::forward
  * (mllm/Backends/Arm/Ops/LinearOp.cpp:67-83), whose workspace_size() this pair replaces. Results equal

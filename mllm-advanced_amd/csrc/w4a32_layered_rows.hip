@@ -135,7 +135,8 @@ constexpr int kNcWaves = 8;
 // A workgroup normalises the rows t0 - (TAPS - 1) .. t0 + TR - 1 into LDS, a wavefront per row (rows before the portion
 // come from the ring), and convolves its TR rows from there. The first one also leaves the portion's tail in the ring, which no
 // other may then read: a portion that has rows in front of it goes in blocks of at least TAPS - 1 rows (kRowsAndTail), or, where
-// so many do not fit the LDS, in two launches.
+// so many do not fit the LDS, in two launches. (Four taps, 8..100 rows of 1536 in front of position 0 and behind others: 5.8 and 6.4
+// us, of 3584 13.7 and 14.6; from 300 rows on blocks are that long anyway.)
 enum NormConvPhase { kRowsAndTail, kRowsOnly, kTailOnly };
 template <int TAPS, typename YT>
 __global__ __launch_bounds__(64 * kNcWaves) void norm_conv_kernel(
@@ -545,8 +546,10 @@ static hipError_t two_launches_t(const float* x, const float* parts, int n_parts
 }
 
 // Two launches where a row does not fit a wavefront's registers: then norm_conv_kernel reads it from memory several times and few
-// rows fit the LDS. us with one and two launches, two partial rows: 2304 channels, 64 / 512 / 2048 rows: 14.4, 11.2 / 17.5, 13.9 /
-// 29.7, 22.4; 3584 channels: 20.5, 11.4 / 32.0, 15.5 / 88.2, 28.9; but 1536 channels: 6.9, 10.6 / 8.7, 12.3 / 17.6, 18.1.
+// rows fit the LDS. us with one and two launches, two partial rows: 2304 channels, 2 / 16 / 64 / 512 / 2048 rows: 14.5, 5.3 / 14.5,
+// 10.4 / 14.4, 11.2 / 17.5, 13.9 / 29.7, 22.4; without partial rows 2 / 16 / 64: 9.9, 4.4 / 10.0, 8.3 / 9.9, 8.8; 3584 channels,
+// 2 / 64 / 512 / 2048: 20.6, 5.4 / 20.5, 11.4 / 32.0, 15.5 / 88.2, 28.9; 8192, 2 / 64: 42.8, 6.2 / 42.4, 12.5; but 1536 channels, 64 /
+// 512 / 2048: 6.9, 10.6 / 8.7, 12.3 / 17.6, 18.1.
 static bool two_launches(int ld, int taps) { return taps >= 2 && ld > 2 * 1024 && ld <= 8 * 1024; }
 
 hipError_t launch_norm_conv(const float* x, const float* parts, int n_parts, float* x_out, const float* norm_w,

@@ -14,7 +14,8 @@
 // last two the request for a tile D further on. The one barrier per tile stands in front of the last step's products, whose
 // fragments are in registers by then, so that the next tile's first fragments are on their way under them.
 // [2048][3584] x [14336][3584]: 128 x 128 on four wavefronts without this order 272 us (775 TFLOP/s), with it 235; 256 x 128
-// 213, 256 x 256 185 us (1140 TFLOP/s, and at 1.3 GHz the clock is what the chip sustains under it).
+// 213, 256 x 256 185 us (1140 TFLOP/s). Its matrix pipes are busy for 84 % of a wavefront's clocks, LDS has no bank conflicts, and
+// the rest is the chip's clock under it: a few launches in a row take 172 us (1.6 GHz), twenty or more 215..229 (1.2..1.3 GHz).
 // f32 products take eight times as long for the same bytes: a SIMD with one wavefront is busy once its operands are there.
 #pragma once
 
@@ -180,8 +181,8 @@ struct MfmaTile {
         }
       }
     };
-    constexpr int kTurn = D < 2 ? 2 : D;
-    static_assert(kTurn % 2 == 0, "buffers and register sets come round together");
+    constexpr int kTurn = D;
+    static_assert(D % 2 == 0, "buffers and register sets come round together");
     int k = kb;
     for (; k + (kTurn - 1) * kBK < ke; k += kTurn * kBK) {
 #pragma unroll
