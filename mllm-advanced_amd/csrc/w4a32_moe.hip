@@ -7,6 +7,7 @@
 // order in which workgroups run.
 // Decode: [norm + choice + gate, up + activation] [down of all chosen experts as one product over their joined columns].
 #include <algorithm>
+#include <cmath>
 
 #include "w4a32_layered.h"
 #include "w4a32_layered_kernels.h"
@@ -138,10 +139,10 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
   }
 }
 
-// A tile of an expert: all of them say the same, so that a workgroup needs one of them only, whichever of them it takes.
+// A tile of an expert: those of one height all say the same, so that a workgroup needs one of them only, whichever it takes.
 struct MoeTile {
-  int expert, row0, rows;  // the expert's rows of the sorted list
-  int first, tiles;        // its first tile and how many it has
+  int expert, row0, rows;  // the expert's rows of the sorted list that go in tiles of this height
+  int first, tiles;        // the first of these tiles and how many there are
   int pad[3];
 };
 
@@ -169,13 +170,25 @@ __device__ __forceinline__ int block_scan(int x, int* s_w, int* total) {
   return before + inc - x;
 }
 
+// Tiles of bm = 2^log_bm rows, of which an expert's last one has `rest` rows where its rows fit that (0: never).
+struct MoeHeights {
+  int log_bm, rest;
+  // tiles of bm rows that `count` rows go in
+  __host__ __device__ int whole(int count) const {
+    const int n = count >> log_bm;
+    return n + (count - (n << log_bm) > rest ? 1 : 0);
+  }
+};
+
 // A workgroup per expert: where its run of the sorted list starts (all of them count everything), its pairs in ascending order,
-// its tiles.
-__global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __restrict__ ids, int n, int experts, int bm,
-                                                                int* __restrict__ order, MoeTile* __restrict__ tiles,
-                                                                int* __restrict__ n_tiles) {
+// its tiles in the two products' lists. In a list the tiles of bm rows stand first (n_tiles[0] of them), then those of `rest` rows
+// (n_tiles[1]).
+__global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __restrict__ ids, int n, int experts,
+                                                                const MoeHeights up, const MoeHeights down,
+                                                                int* __restrict__ order, MoeTile* __restrict__ up_tiles,
+                                                                MoeTile* __restrict__ down_tiles, int* __restrict__ n_tiles) {
   __shared__ int s_count[W4A32_LAYERED_MAX_EXPERTS];
-  __shared__ int s_w[kPlanWaves];
+  __shared__ int s_w[kPlanWaves], s_sums[2][5];
   const int e = blockIdx.x, tid = threadIdx.x;
   for (int i = tid; i < experts; i += kPlanThreads) s_count[i] = 0;
   __syncthreads();
@@ -196,32 +209,60 @@ __global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __res
     mine += ids[i] == e;
   }
   __syncthreads();
-  int total;
-  const bool before = tid < experts && tid < e;
-  block_scan(before ? s_count[tid] : 0, s_w, &total);
-  const int offset = total;
-  block_scan(before ? (s_count[tid] + bm - 1) / bm : 0, s_w, &total);
-  const int first = total;
-  int at = offset + block_scan(mine, s_w, &total);
+  // what comes in front of this expert, and in all: a wavefront adds up each list's tiles
+  if (tid < 128) {
+    const MoeHeights g = tid < 64 ? up : down;
+    int sums[5] = {0, 0, 0, 0, 0};  // rows; whole tiles, rests; the same of all experts
+    for (int i = tid & 63; i < experts; i += 64) {
+      const int c = s_count[i], whole = g.whole(c), rest = c > whole << g.log_bm ? 1 : 0;
+      sums[0] += i < e ? c : 0;
+      sums[1] += i < e ? whole : 0;
+      sums[2] += i < e ? rest : 0;
+      sums[3] += whole;
+      sums[4] += rest;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+      for (int i = 0; i < 5; ++i) sums[i] += __shfl_xor(sums[i], off, 64);
+    if ((tid & 63) == 0)
+#pragma unroll
+      for (int i = 0; i < 5; ++i) s_sums[tid >> 6][i] = sums[i];
+  }
+  int count;
+  const int before_mine = block_scan(mine, s_w, &count), offset = s_sums[0][0];
+  int at = offset + before_mine;
 #pragma unroll
   for (int i = 0; i < kRegs; ++i)
     if (lo + i < hi && id[i] == e) order[at++] = lo + i;
   for (int i = lo + kRegs; i < hi; ++i)
     if (ids[i] == e) order[at++] = i;
-  const int count = total, mt = (count + bm - 1) / bm;
-  for (int t = tid; t < mt; t += kPlanThreads)
-    tiles[first + t] = MoeTile{e, offset, count, first, mt, {0, 0, 0}};
-  if (e == experts - 1 && tid == 0) *n_tiles = first + mt;
+  if (tid < 128) {  // a wavefront per list
+    const int list = tid >> 6, lane = tid & 63;
+    const MoeHeights g = list ? down : up;
+    MoeTile* tiles = list ? down_tiles : up_tiles;
+    const int whole = g.whole(count), in_whole = min(count, whole << g.log_bm), first = s_sums[list][1];
+    for (int t = lane; t < whole; t += 64) tiles[first + t] = MoeTile{e, offset, in_whole, first, whole, {0, 0, 0}};
+    if (lane == 0 && count > in_whole) {
+      const int t = s_sums[list][3] + s_sums[list][2];
+      tiles[t] = MoeTile{e, offset + in_whole, count - in_whole, t, 1, {0, 0, 0}};
+    }
+    if (e == 0 && lane < 2) n_tiles[2 * list + lane] = s_sums[list][3 + lane];
+  }
 }
 static_assert(kPlanThreads >= W4A32_LAYERED_MAX_EXPERTS, "a thread per expert");
 
-// The tile of a workgroup: an expert's tiles are numbered rows fastest, experts one after the other; consecutive numbers on one
-// XCD. `row0` and `rows` become the tile's. Returns false past the last one.
+// The tile of a workgroup: first those of bm rows, then those of fewer, which the CUs take that come free early. An expert's
+// tiles are numbered rows fastest, experts one after the other; consecutive numbers on one XCD. `row0` and `rows` become the tile's.
+// Returns false past the last one.
 __device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, const int* __restrict__ n_tiles, int bm, int nt,
-                                         MoeTile* tile, int* n) {
-  const int total = *n_tiles * nt;
-  if ((int)blockIdx.x >= total) return false;
-  const int t = xcd_tile(blockIdx.x, total);
+                                         MoeTile* tile, int* n, bool* rest) {
+  const int whole = n_tiles[0], all = whole + n_tiles[1];
+  int b = blockIdx.x;
+  if (b >= all * nt) return false;
+  *rest = b >= whole * nt;
+  if (*rest) b -= whole * nt;
+  const int t = xcd_tile(b, (*rest ? all - whole : whole) * nt) + (*rest ? whole * nt : 0);
   *tile = tiles[t / nt];
   if (tile->tiles <= 0) return false;
   const int local = t - tile->first * nt, at = local % tile->tiles * bm;
@@ -231,21 +272,23 @@ __device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, cons
   return true;
 }
 
+template <typename T, int BM, int BN, int WM, int WN, int D>
+struct TileOf {
+  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
+  static constexpr int kRows = BM, kCols = BN, kWM = WM, kWN = WN, kThreads = Tile::kThreads;
+  static constexpr size_t kLds = Tile::kLds;
+};
+
 // act [sorted pair][Fp] = glu(h gate^T, h up^T). A wavefront's column blocks are gate and up of the same 32 columns, in turn.
 // kFar, here and below: rows too long for 32-bit offsets.
-template <typename T, int BM, int BN, int WM, int WN, int D, bool kFar>
-__global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __restrict__ h, const T* __restrict__ w,
-                                                                   T* __restrict__ act, const int* __restrict__ order,
-                                                                   const MoeTile* __restrict__ tiles,
-                                                                   const int* __restrict__ n_tiles, int M, int top, int Hp,
-                                                                   int Fp, float limit) {
-  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
+template <typename T, typename Shape, bool kFar>
+__device__ __forceinline__ void gate_up_tile(uint8_t* smem, const MoeTile& tile, int n, const T* __restrict__ h,
+                                             const T* __restrict__ w, T* __restrict__ act, const int* __restrict__ order, int M,
+                                             int top, int Hp, int Fp, float limit) {
+  using Tile = typename Shape::Tile;
+  constexpr int BM = Shape::kRows, BN = Shape::kCols, WM = Shape::kWM, WN = Shape::kWN;
   static_assert(Tile::FN % 2 == 0, "gate and up in one wavefront");
-  extern __shared__ __align__(16) uint8_t smem[];
-  MoeTile tile;
-  int n;
   const int N = 2 * Fp;
-  if (!moe_tile(tiles, n_tiles, BM, (N + BN - 1) / BN, &tile, &n)) return;
   const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nb = min(BN, N - n0);
   RowOffset<kFar> oa[Tile::LA], ob[Tile::LB];
 #pragma unroll
@@ -293,19 +336,30 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_gate_up_kernel(const T* __re
   }
 }
 
-// parts [slot][token][Hp] = weight * act down^T; a slot has rows_all tokens
-template <typename T, int BM, int BN, int WM, int WN, int D, bool kFar>
-__global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restrict__ act, const T* __restrict__ w,
-                                                                float* __restrict__ parts, const int* __restrict__ order,
-                                                                const float* __restrict__ wts,
-                                                                const MoeTile* __restrict__ tiles,
-                                                                const int* __restrict__ n_tiles, int top, int rows_all, int Hp,
-                                                                int Fp) {
-  using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
+template <typename T, typename Big, typename Rest, bool kFar>
+__global__ __launch_bounds__(Big::kThreads) void moe_gate_up_kernel(const T* __restrict__ h, const T* __restrict__ w,
+                                                                    T* __restrict__ act, const int* __restrict__ order,
+                                                                    const MoeTile* __restrict__ tiles,
+                                                                    const int* __restrict__ n_tiles, int M, int top, int Hp,
+                                                                    int Fp, float limit) {
   extern __shared__ __align__(16) uint8_t smem[];
   MoeTile tile;
   int n;
-  if (!moe_tile(tiles, n_tiles, BM, (Hp + BN - 1) / BN, &tile, &n)) return;
+  bool rest;
+  if (!moe_tile(tiles, n_tiles, Big::kRows, (2 * Fp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
+  if (Rest::kRows < Big::kRows && rest)
+    gate_up_tile<T, Rest, kFar>(smem, tile, n, h, w, act, order, M, top, Hp, Fp, limit);
+  else
+    gate_up_tile<T, Big, kFar>(smem, tile, n, h, w, act, order, M, top, Hp, Fp, limit);
+}
+
+// parts [slot][token][Hp] = weight * act down^T; a slot has rows_all tokens
+template <typename T, typename Shape, bool kFar>
+__device__ __forceinline__ void down_tile(uint8_t* smem, const MoeTile& tile, int n, const T* __restrict__ act,
+                                          const T* __restrict__ w, float* __restrict__ parts, const int* __restrict__ order,
+                                          const float* __restrict__ wts, int top, int rows_all, int Hp, int Fp) {
+  using Tile = typename Shape::Tile;
+  constexpr int BM = Shape::kRows, BN = Shape::kCols, WM = Shape::kWM, WN = Shape::kWN;
   const int n0 = BN * n, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // a row's place and weight, asked for now and handed round through LDS behind the products
   static_assert(BM <= Tile::kThreads, "a thread per row");
@@ -347,6 +401,24 @@ __global__ __launch_bounds__(64 * WM * WN) void moe_down_kernel(const T* __restr
         if (col < Hp) dst[col] = a * acc[i][j][v];
       }
     }
+}
+
+template <typename T, typename Big, typename Rest, bool kFar>
+__global__ __launch_bounds__(Big::kThreads) void moe_down_kernel(const T* __restrict__ act, const T* __restrict__ w,
+                                                                 float* __restrict__ parts, const int* __restrict__ order,
+                                                                 const float* __restrict__ wts,
+                                                                 const MoeTile* __restrict__ tiles,
+                                                                 const int* __restrict__ n_tiles, int top, int rows_all, int Hp,
+                                                                 int Fp) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  MoeTile tile;
+  int n;
+  bool rest;
+  if (!moe_tile(tiles, n_tiles, Big::kRows, (Hp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
+  if (Rest::kRows < Big::kRows && rest)
+    down_tile<T, Rest, kFar>(smem, tile, n, act, w, parts, order, wts, top, rows_all, Hp, Fp);
+  else
+    down_tile<T, Big, kFar>(smem, tile, n, act, w, parts, order, wts, top, rows_all, Hp, Fp);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -447,13 +519,9 @@ inline size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 
 // what a portion's experts work in
 struct Scratch {
-  size_t ids, wts, order, tiles, n_tiles, act, bytes;
+  size_t ids, wts, order, up_tiles, down_tiles, n_tiles, act, bytes;
   int max_tiles;
 };
-int tile_rows(int dtype, int M, int experts, int top) {
-  const long per = (long)M * top / experts;  // rows an expert has on average
-  return per >= 768 && dtype == W4A32_LAYERED_BF16 ? 256 : per >= 96 ? 128 : 64;
-}
 Scratch scratch_of(int dtype, int M, int experts, int top, int Fp) {
   const size_t n = (size_t)M * top, elem = dtype == W4A32_LAYERED_BF16 ? 2 : 4;
   Scratch c;
@@ -467,87 +535,158 @@ Scratch scratch_of(int dtype, int M, int experts, int top, int Fp) {
   c.ids = take(4 * n);
   c.wts = take(4 * n);
   c.order = take(4 * n);
-  c.tiles = take(sizeof(MoeTile) * c.max_tiles);
-  c.n_tiles = take(4);
+  c.up_tiles = take(sizeof(MoeTile) * c.max_tiles);
+  c.down_tiles = take(sizeof(MoeTile) * c.max_tiles);
+  c.n_tiles = take(4 * 4);
   c.act = take(elem * n * Fp);
   c.bytes = o;
   return c;
 }
 
-// Up, Down: the two products' tiles, of equal height
-template <typename Up, typename Down, bool kFar = false, typename T>
-hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down, int M, int rows_all, float* parts,
-                   uint8_t* ws, const Scratch& c, hipStream_t s) {
-  static_assert(Up::kRows == Down::kRows, "one list of tiles");
-  int* order = reinterpret_cast<int*>(ws + c.order);
-  MoeTile* tiles = reinterpret_cast<MoeTile*>(ws + c.tiles);
-  int* n_tiles = reinterpret_cast<int*>(ws + c.n_tiles);
-  T* act = reinterpret_cast<T*>(ws + c.act);
-  const int most = (int)(((size_t)M * g.top + Up::kRows - 1) / Up::kRows) + g.experts;  // workgroups past the last tile return
-  auto up = moe_gate_up_kernel<T, Up::kRows, Up::kCols, Up::kWM, Up::kWN, Up::kDepth, kFar>;
-  auto dn = moe_down_kernel<T, Down::kRows, Down::kCols, Down::kWM, Down::kWN, Down::kDepth, kFar>;
-  static LdsLimitOnce raised_up, raised_dn;
-  if (Up::kLds > 64 * 1024)
-    if (hipError_t e = raised_up.raise(reinterpret_cast<const void*>(up), Up::kLds); e != hipSuccess) return e;
-  if (Down::kLds > 64 * 1024)
-    if (hipError_t e = raised_dn.raise(reinterpret_cast<const void*>(dn), Down::kLds); e != hipSuccess) return e;
-  hipLaunchKernelGGL(up, dim3((unsigned)most * ((2 * g.Fp + Up::kCols - 1) / Up::kCols)), dim3(64 * Up::kWM * Up::kWN), Up::kLds,
-                     s, h, gate_up, act, order, tiles, n_tiles, M, g.top, g.Hp, g.Fp, g.limit);
-  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  hipLaunchKernelGGL(dn, dim3((unsigned)most * ((g.Hp + Down::kCols - 1) / Down::kCols)), dim3(64 * Down::kWM * Down::kWN),
-                     Down::kLds, s, act, down, parts, order, reinterpret_cast<const float*>(ws + c.wts), tiles, n_tiles, g.top,
-                     rows_all, g.Hp, g.Fp);
+// The shapes of the grouped products. Rest: the tile of an expert's last rows where they fit it.
+template <typename T, int BM, int BN, int WM, int WN, int D, int RM = BM>
+struct ShapeOf {
+  using Big = TileOf<T, BM, BN, WM, WN, D>;
+  using Rest = TileOf<T, RM, BN, WM, WN, D>;
+  static_assert(Rest::kLds <= Big::kLds && Rest::kThreads == Big::kThreads);
+  static_assert((BM & (BM - 1)) == 0);
+  static constexpr MoeHeights heights() { return {BM == 256 ? 8 : BM == 128 ? 7 : 6, RM < BM ? RM : 0}; }
+  // workgroups; those past the last tile return
+  static unsigned grid(const MoeGeom& g, int M, int N) {
+    return (unsigned)((size_t)M * g.top / BM + g.experts) * (unsigned)((N + BN - 1) / BN);
+  }
+};
+
+template <typename Shape, bool kFar = false, typename T>
+hipError_t launch_gate_up(const MoeGeom& g, const T* h, const T* gate_up, int M, uint8_t* ws, const Scratch& c, hipStream_t s) {
+  using Big = typename Shape::Big;
+  auto kern = moe_gate_up_kernel<T, Big, typename Shape::Rest, kFar>;
+  static LdsLimitOnce raised;
+  if (Big::kLds > 64 * 1024)
+    if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), Big::kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(Shape::grid(g, M, 2 * g.Fp)), dim3(Big::kThreads), Big::kLds, s, h, gate_up,
+                     reinterpret_cast<T*>(ws + c.act), reinterpret_cast<const int*>(ws + c.order),
+                     reinterpret_cast<const MoeTile*>(ws + c.up_tiles), reinterpret_cast<const int*>(ws + c.n_tiles), M, g.top,
+                     g.Hp, g.Fp, g.limit);
   return hipGetLastError();
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int D>
-struct TileOf {
-  static constexpr int kRows = BM, kCols = BN, kWM = WM, kWN = WN, kDepth = D;
-  static constexpr size_t kLds = MfmaTile<T, BM, BN, WM, WN, D>::kLds;
+template <typename Shape, bool kFar = false, typename T>
+hipError_t launch_down(const MoeGeom& g, const T* down, int M, int rows_all, float* parts, uint8_t* ws, const Scratch& c,
+                       hipStream_t s) {
+  using Big = typename Shape::Big;
+  auto kern = moe_down_kernel<T, Big, typename Shape::Rest, kFar>;
+  static LdsLimitOnce raised;
+  if (Big::kLds > 64 * 1024)
+    if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), Big::kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(Shape::grid(g, M, g.Hp)), dim3(Big::kThreads), Big::kLds, s,
+                     reinterpret_cast<const T*>(ws + c.act), down, parts, reinterpret_cast<const int*>(ws + c.order),
+                     reinterpret_cast<const float*>(ws + c.wts), reinterpret_cast<const MoeTile*>(ws + c.down_tiles),
+                     reinterpret_cast<const int*>(ws + c.n_tiles) + 2, g.top, rows_all, g.Hp, g.Fp);
+  return hipGetLastError();
+}
+
+// Gate and up / down of 16 experts, 4 per token, in 128 x 128 throughout, 128 x 256 throughout, and 256 x 256 with last rows in
+// 128 x 256 (us): 1501 tokens, [2 x 2240][1536]: 109 / 69, 113 / 77, 106 / 57; 2048 tokens: 147 / 90, 157 / 78, 135 / 62; 900: 82 / 46,
+// 88 / 41, 90 / 53; 2048 tokens, [2 x 4736][3584]: 730 / 346, 688 / 310, 607 / 282. Whole tiles stand in front of the last rows':
+// mixed they took 116 / 57 for the first, as the large ones then end late. 100 tokens, [2 x 2240][1536], 64 x 128: 49 / 23 = 4.5
+// and 4.9 TB/s of weights, 128 x 128 53 / 26. A 256 x 256 tile takes 42 us of which its activation and stores are 5: with one
+// workgroup per CU nothing runs under them.
+//
+// What the bf16 shapes cost: us per 64 k of a tile and of the rest's tile with all CUs busy, and per tile for what stands in front of
+// and behind its products (gate and up / down), on `slots` tiles at once. Fitted to 19 problems of 200 to 1024 rows per expert
+// from [2 x 400][768] to [2 x 4736][3584] (7 % of error on average).
+struct MoeShape {
+  int bm, rest, bn, slots;
+  double tile_us, rest_us, up_us, down_us;
 };
+constexpr MoeShape kTall = {256, 128, 256, 256, 1.375, 1.37, 7.5, 9.0}, kWide = {128, 0, 256, 256, 0.967, 0, 2.9, 4.5},
+                   kSmall = {128, 0, 128, 512, 1.106, 0, 1.5, 4.8};  // kSmall: two tiles per CU, alone on it one takes half as long
+
+double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
+  const int N = up ? 2 * g.Fp : g.Hp, nt = (N + t.bn - 1) / t.bn;
+  const double k = (up ? g.Hp : g.Fp) / 64.0, over = up ? t.up_us : t.down_us;
+  const double per = (double)M * g.top / g.experts, spread = std::sqrt(per);
+  const MoeHeights heights{t.bm == 256 ? 8 : 7, t.rest};
+  double whole = 0.0, rest = 0.0;  // experts with about `per` rows, in three classes
+  for (int i = -1; i <= 1; ++i) {
+    const int count = (int)(per + i * spread), n = heights.whole(count);
+    whole += g.experts / 3.0 * nt * n;
+    rest += g.experts / 3.0 * nt * (count > n * t.bm ? 1 : 0);
+  }
+  const double tile_us = t.tile_us * k + over, rest_us = t.rest_us * k + over / 2;
+  const double rounds = std::floor(whole / t.slots), left = whole - rounds * t.slots;
+  double end = rounds * tile_us;
+  if (&t == &kSmall) return end + (left <= 0.0 ? 0.0 : left > 256 ? tile_us : 0.5 * tile_us);
+  // the slots with a tile of the last round and those without one, as the rests come to them
+  double free_at[2] = {left > 0.0 ? end + tile_us : end, end};
+  const double slots[2] = {left > 0.0 ? left : t.slots, left > 0.0 ? t.slots - left : 0.0};
+  end = free_at[0];
+  while (rest > 0.0) {
+    const int i = slots[1] > 0.0 && free_at[1] <= free_at[0] ? 1 : 0;
+    rest -= slots[i];
+    free_at[i] += rest_us;
+    end = std::max(end, free_at[i]);
+  }
+  return end;
+}
 
 template <typename T>
 bool experts_far(const MoeGeom& g) {
   return !rows_near(sizeof(T) * (size_t)std::max(g.Hp, g.Fp)) || !results_near(sizeof(T) * (size_t)g.Fp);
 }
 
+template <typename Up, typename Down, bool kFar = false, typename T>
+hipError_t grouped(const MoeGeom& g, const T* h, const T* gate_up, const T* down, int M, int rows_all, float* parts,
+                   uint8_t* ws, const Scratch& c, hipStream_t s) {
+  hipLaunchKernelGGL(moe_plan_kernel, dim3(g.experts), dim3(kPlanThreads), 0, s, reinterpret_cast<const int*>(ws + c.ids),
+                     M * g.top, g.experts, Up::heights(), Down::heights(), reinterpret_cast<int*>(ws + c.order),
+                     reinterpret_cast<MoeTile*>(ws + c.up_tiles), reinterpret_cast<MoeTile*>(ws + c.down_tiles),
+                     reinterpret_cast<int*>(ws + c.n_tiles));
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  if (hipError_t e = launch_gate_up<Up, kFar>(g, h, gate_up, M, ws, c, s); e != hipSuccess) return e;
+  return launch_down<Down, kFar>(g, down, M, rows_all, parts, ws, c, s);
+}
+
 template <typename T>
 hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logits, int logit_parts, size_t part_stride, int ldl,
                      const T* gate_up, const T* down, int M, int rows_all, float* parts, uint8_t* ws, hipStream_t s) {
   const Scratch c = scratch_of(dtype, M, g.experts, g.top, g.Fp);
-  const bool far = experts_far<T>(g);
-  const int bm = far ? 64 : tile_rows(dtype, M, g.experts, g.top);
-  int* ids = reinterpret_cast<int*>(ws + c.ids);
   hipLaunchKernelGGL(moe_choose_kernel, dim3((M + 3) / 4), dim3(256), 0, s, logits, logit_parts, part_stride, ldl, M,
-                     g.experts, g.top, ids, reinterpret_cast<float*>(ws + c.wts));
+                     g.experts, g.top, reinterpret_cast<int*>(ws + c.ids), reinterpret_cast<float*>(ws + c.wts));
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  hipLaunchKernelGGL(moe_plan_kernel, dim3(g.experts), dim3(kPlanThreads), 0, s, ids, M * g.top, g.experts, bm,
-                     reinterpret_cast<int*>(ws + c.order), reinterpret_cast<MoeTile*>(ws + c.tiles),
-                     reinterpret_cast<int*>(ws + c.n_tiles));
-  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (far) {
-    using Far = TileOf<T, 64, 128, 2, 2, 2>;
+  auto run = [&](auto up, auto down_shape) {
+    return grouped<decltype(up), decltype(down_shape)>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+  };
+  if (experts_far<T>(g)) {
+    using Far = ShapeOf<T, 64, 128, 2, 2, 2>;
     return grouped<Far, Far, true>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
   }
-  // (Us for gate and up, then down, of 16 experts, 4 per token. 1501 tokens, [2 x 2240][1536]: 128 x 128 124, 72, 128 x 256 128, 78;
-  // 2048 tokens, [2 x 4736][3584]: 673, 352 against 629, 312, 256 x 256 599, 340; 100 tokens, [2 x 2240][1536]: 64 x 128 49, 23 =
-  // 4.5 and 4.9 TB/s of weights, 128 x 128 53, 26. Before these shapes: 145, 106 for the first.)
+  const bool few = (long)M * g.top / g.experts < 96;  // rows an expert has on average
   if constexpr (sizeof(T) == 2) {
-    const long tiles_up = ((long)M * g.top / 128 + g.experts / 2) * (2 * g.Fp / 256);
-    const long tiles_down = ((long)M * g.top / 128 + g.experts / 2) * (g.Hp / 256);
-    using Small = TileOf<T, 128, 128, 2, 4, 2>;  // two workgroups per CU
-    using SmallUp = TileOf<T, 128, 128, 2, 2, 2>;
-    using Wide = TileOf<T, 128, 256, 2, 4, 2>;
-    if (bm == 256)
-      return grouped<TileOf<T, 256, 256, 2, 4, 2>, TileOf<T, 256, 256, 2, 4, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    if (bm == 128 && tiles_down >= 1000) return grouped<Wide, Wide>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    if (bm == 128 && tiles_up >= 1000) return grouped<Wide, Small>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    if (bm == 128) return grouped<SmallUp, Small>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    return grouped<TileOf<T, 64, 128, 2, 2, 4>, TileOf<T, 64, 128, 2, 4, 4>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    if (few) return run(ShapeOf<T, 64, 128, 2, 2, 4>{}, ShapeOf<T, 64, 128, 2, 4, 4>{});
+    // 128 x 256 is one workgroup per CU, 128 x 128 two that fill each other's gaps, which the costs do not know: it has to be clearly
+    // cheaper
+    auto choose = [&](bool up) {
+      const double tall = moe_shape_us(kTall, g, M, up), wide = moe_shape_us(kWide, g, M, up), small = moe_shape_us(kSmall, g, M, up);
+      const bool wider = wide < 0.93 * small;
+      return tall < (wider ? wide : small) ? 0 : wider ? 1 : 2;
+    };
+    auto with = [&](auto up) {
+      switch (choose(false)) {
+        case 0: return run(up, ShapeOf<T, 256, 256, 2, 4, 2, 128>{});
+        case 1: return run(up, ShapeOf<T, 128, 256, 2, 4, 2>{});
+        default: return run(up, ShapeOf<T, 128, 128, 2, 4, 2>{});
+      }
+    };
+    switch (choose(true)) {
+      case 0: return with(ShapeOf<T, 256, 256, 2, 4, 2, 128>{});
+      case 1: return with(ShapeOf<T, 128, 256, 2, 4, 2>{});
+      default: return with(ShapeOf<T, 128, 128, 2, 2, 2>{});
+    }
   } else {
-    if (bm == 128)
-      return grouped<TileOf<T, 128, 128, 2, 2, 2>, TileOf<T, 128, 128, 2, 2, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
-    return grouped<TileOf<T, 64, 128, 2, 2, 2>, TileOf<T, 64, 128, 2, 2, 2>>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
+    if (few) return run(ShapeOf<T, 64, 128, 2, 2, 2>{}, ShapeOf<T, 64, 128, 2, 2, 2>{});
+    return run(ShapeOf<T, 128, 128, 2, 2, 2>{}, ShapeOf<T, 128, 128, 2, 2, 2>{});
   }
 }
 

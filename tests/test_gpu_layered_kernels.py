@@ -84,9 +84,13 @@ def test_bf16_product_of_every_shape(pkg, M, N, K):
 @pytest.mark.parametrize("rows,hidden,experts,top,ff", [
     (190, 64, 2, 1, 64),      # 95 rows per expert: tiles of 64 rows; one tile of columns, half full
     (200, 130, 2, 1, 130),    # 100: 128 rows
-    (1540, 72, 4, 2, 100),    # 770: 256 rows in bf16
-    (12400, 70, 128, 1, 900),   # 96, about 160 tiles of rows: bf16 gate and up in 128 x 256, down in 128 x 128
-    (12400, 1800, 128, 1, 60),  # ... both in 128 x 256; column counts that are no multiple of it
+    (1540, 72, 4, 2, 100),    # 770
+    (12400, 70, 128, 1, 900),   # 96, about 160 tiles of rows
+    (12400, 1800, 128, 1, 60),  # ... column counts that are no multiple of a tile
+    (1900, 1530, 40, 3, 60),    # bf16: gate and up in 128 x 128, down in 256 x 256 and experts' last rows in 128 x 256
+    (1100, 1530, 8, 2, 1500),   # the other way round, down in 128 x 256
+    (2500, 1800, 40, 2, 310),   # both in 128 x 256
+    (2500, 1800, 4, 2, 900),    # both in 256 x 256 with last rows
 ])
 def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
     import torch
