@@ -16,6 +16,7 @@
 //                         query, the online softmax is per lane, scores go from accumulator to operand without a
 //                         cross-lane move). The softmax weights stay f32: they enter the second product as a sum of
 //                         two bf16 terms.
+//   attn_tile_kernel      the same for long prompts: keys and values through LDS, products and softmax under each other
 //   attn_rows_kernel      prefill, f32: one wavefront per (head, query)
 //   attn_decode_kernel    one token: convolution, cache append, block mean and attention over one slice of the visible
 //                         keys per workgroup; the slices are merged by the Linear that follows
@@ -161,6 +162,33 @@ struct PrefillExtra {
   int rot_part, rot_dims;
   const float *sin_t, *cos_t;
 };
+
+// A lane's share of a query's output: register v of o[c] is dimension 32 c + 8 (v / 4) + 4 hh + v % 4.
+template <int C>
+__device__ __forceinline__ void store_attention(const f32x16 (&o)[C], float inv, const PrefillExtra& x, __bf16* out, int ldo, int m,
+                                                int h, int heads, int vdim, int hh) {
+  if (x.gate) inv *= sigmoid_f(x.gate[(size_t)m * x.ldg + h]);
+  __bf16* row = out + (size_t)m * ldo;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const int d = 32 * c + 8 * g4 + 4 * hh;
+      const float4 v = make_float4(o[c][4 * g4] * inv, o[c][4 * g4 + 1] * inv, o[c][4 * g4 + 2] * inv,
+                                   o[c][4 * g4 + 3] * inv);
+      if ((vdim & 3) == 0) {
+        if (d < vdim) store4(row + h * vdim + d, v);
+      } else {
+        const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (d + e < vdim) row[h * vdim + d + e] = (__bf16)f[e];
+      }
+    }
+  if (h == heads - 1) {
+    for (int c = heads * vdim + hh; c < ldo; c += 2) row[c] = (__bf16)0.0f;
+  }
+}
 
 // Workgroup = (head, 32 queries); its wavefronts take the blocks of 32 pooled entries and of 32 tokens round-robin and
 // merge through LDS. S^T = K Q^T: A = keys (lane: key l % 32, dims 16 s + 8 (l / 32) ..), B = queries from LDS.
@@ -369,28 +397,350 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void attn_mfma_kernel(
       for (int v = 0; v < 16; ++v) o[c][v] += src[(16 * c + v) * 64] * wt;
   }
   if (32 * qb + j >= M) return;
-  float inv = 1.0f / total;  // every query sees its own key
-  if (x.gate) inv *= sigmoid_f(x.gate[(size_t)(32 * qb + j) * x.ldg + h]);
-  __bf16* row = out + (size_t)(32 * qb + j) * ldo;
+  store_attention<C>(o, 1.0f / total, x, out, ldo, 32 * qb + j, h, heads, vdim, hh);  // every query sees its own key
+}
+
+// ---------------------------------------------------------------------------------------------
+// Larger of x in lanes l and l ^ 32.
+__device__ __forceinline__ float max_of_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// The same attention for long prompts. Workgroup = (head, 64 queries): two sets of two wavefronts, a wavefront per 32 queries in each
+// set. A set takes every second block of 32 keys; its block comes through LDS once for both of its wavefronts, the one after it is
+// on its way through registers meanwhile. The sets' sums are merged through LDS at the end.
+//
+// In attn_mfma_kernel every wavefront reads its operands for 32 queries only, and what it does between the products takes longer
+// than they do. Here a block's D / 16 + KR + D / 8 products of 32 clocks run above the exponentials, sums and conversions: the
+// scores of the next block between the steps that make this block's weights, whose second half is made between the products of its
+// first. The order is written out and fenced. A maximum is taken over only where it has grown by more than 2^8 (weights of that size
+// keep their digits), so that the sums are rescaled a few times per prompt only; masks only in blocks that need them.
+// D = 128, us before / now: 28 heads of 2048 queries, window 1024 and pooled blocks behind it, 110 / 62; 16 heads, window 1024: 59 /
+// 39; 12 heads of 1501 queries without a window 38 / 36, with a second part of 64 dimensions and window 1024 50 / 40. What bounds it: a
+// wavefront issues about 370 instructions per block, of which 24 are products, and two wavefronts fit a SIMD. Workgroups of 128
+// queries (28 heads: 60 us, 12 heads: 54) and of four sets (87, 31) are better on some sizes only.
+constexpr int kTileSets = 2, kTileWaves = 2, kTileQueries = 32 * kTileWaves;
+
+template <int D, int KR>
+__global__ __launch_bounds__(64 * kTileSets * kTileWaves, 2) void attn_tile_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ kc, const __bf16* __restrict__ vt,
+    const __bf16* __restrict__ kp, const __bf16* __restrict__ vpt, __bf16* __restrict__ out, int ldo, int M, int heads,
+    int kv_heads, int dim, int vdim, int cap, int capp, int window, int pool, int pos0, float scale, const PrefillExtra x) {
+  constexpr int QW = kTileWaves, KW = kTileSets;
+  constexpr int KS = D / 16, C = D / 32, R = 16 * C + 2;
+  constexpr int kPerK = (KS + QW - 1) / QW, kPerR = (KR + QW - 1) / QW;  // kilobytes of a block's keys (values), second parts that a wavefront brings
+  constexpr int kBlk = 32 * D;                   // elements of a block of keys or values
+  extern __shared__ __align__(16) uint8_t smem[];
+  bf16x8* const s_k = reinterpret_cast<bf16x8*>(smem);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int set = wave / QW, wq = wave % QW, j = lane & 31, hh = lane >> 5;
+
+  const int h = (int)blockIdx.x % heads, g = h / (heads / kv_heads);
+  // the later query blocks see more keys (until the window is full): they start first
+  const int q0 = kTileQueries * ((M + kTileQueries - 1) / kTileQueries - 1 - (int)blockIdx.x / heads);
+
+  // what the workgroup's queries see: pooled blocks, then token blocks from tok_first on
+  const int wg_last = pos0 + min(q0 + kTileQueries - 1, M - 1);
+  const int pool_blocks = (pooled_visible(wg_last, window, pool) + 31) / 32;
+  const int tok_first = max(0, pos0 + q0 - window + 1) / 32;
+  const int blocks = pool_blocks + wg_last / 32 - tok_first + 1;
+  // ... this wavefront's queries, and this lane's
+  const int m0 = q0 + 32 * wq;
+  const bool any = m0 < M;
+  const int m_q = min(m0 + j, M - 1), p = pos0 + m_q;
+  const int p_first = pos0 + min(m0, M - 1), p_last = pos0 + min(m0 + 31, M - 1);
+  const int nb = pooled_visible(p, window, pool), nb_first = pooled_visible(p_first, window, pool);
+  const int nb_last = pooled_visible(p_last, window, pool);
+  const int own_first = max(0, p_first - window + 1) / 32, own_last = p_last / 32;
+
+  const __bf16* const kt = kc + (size_t)g * cap * D + (size_t)(tok_first - x.blk0) * kBlk;
+  const __bf16* const kpt = kp + (size_t)g * capp * D;
+  const __bf16* const vtt = vt + (size_t)g * cap * D + (size_t)(tok_first - x.blk0) * kBlk;
+  const __bf16* const vptt = vpt + (size_t)g * capp * D;
+  // a kilobyte of values is 16 dimensions of 32 entries: into LDS with a quarter of the entries of all 16 side by side
+  const unsigned k_off = 8 * lane, v_off = 32 * (lane & 15) + 8 * (lane >> 4);
+
+  // Keys are read a turn before the values of their block: two buffers for each, s_k [2][KW][KS + KR][64], s_v [2][KW][KS][64].
+  bf16x8* const s_v = s_k + 2 * KW * (KS + KR) * 64;
+  bf16x8 pk[kPerK], pr[kPerR > 0 ? kPerR : 1], pv[kPerK];
+  auto fetch = [&](int k_turn, int v_turn) __attribute__((always_inline)) {
+    const int kb = min(k_turn * KW + set, blocks - 1), vb = min(v_turn * KW + set, blocks - 1);
+    const __bf16* ks = kb < pool_blocks ? kpt + (size_t)kb * kBlk : kt + (size_t)(kb - pool_blocks) * kBlk;
+    const __bf16* vs = vb < pool_blocks ? vptt + (size_t)vb * kBlk : vtt + (size_t)(vb - pool_blocks) * kBlk;
+    const __bf16* rs = ks;
+    if constexpr (KR > 0) rs = static_cast<const __bf16*>(x.kr) + (size_t)(tok_first + kb - pool_blocks) * x.kr_block;
+#pragma unroll
+    for (int i = 0; i < kPerK; ++i) pk[i] = *reinterpret_cast<const bf16x8*>(ks + 512 * min(wq + QW * i, KS - 1) + k_off);
+#pragma unroll
+    for (int i = 0; i < kPerR; ++i) pr[i] = *reinterpret_cast<const bf16x8*>(rs + 512 * min(wq + QW * i, KR - 1) + k_off);
+#pragma unroll
+    for (int i = 0; i < kPerK; ++i) pv[i] = *reinterpret_cast<const bf16x8*>(vs + 512 * min(wq + QW * i, KS - 1) + v_off);
+  };
+  auto stash = [&](int k_buf, int v_buf) __attribute__((always_inline)) {
+    bf16x8* const dk = s_k + (k_buf * KW + set) * (KS + KR) * 64 + lane;
+    bf16x8* const dv = s_v + (v_buf * KW + set) * KS * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < kPerK; ++i)
+      if (KS % QW == 0 || wq + QW * i < KS) dk[(wq + QW * i) * 64] = pk[i];
+#pragma unroll
+    for (int i = 0; i < kPerR; ++i)
+      if (KR % QW == 0 || wq + QW * i < KR) dk[(KS + wq + QW * i) * 64] = pr[i];
+#pragma unroll
+    for (int i = 0; i < kPerK; ++i)
+      if (KS % QW == 0 || wq + QW * i < KS) dv[(wq + QW * i) * 64] = pv[i];
+  };
+
+  fetch(0, 0);
+  // this lane's query: dimensions 16 s + 8 hh .. of it
+  bf16x8 qop[KS + KR];
+  {
+    const __bf16* src = q + (size_t)m_q * x.qld + (size_t)h * x.qstride;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int d0 = 16 * s + 8 * hh;
+      if (KR == 0 || ((x.qstride & 7) == 0 && d0 + 8 <= dim)) {
+        qop[s] = *reinterpret_cast<const bf16x8*>(src + d0);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (d0 + e >= dim) qop[s][e] = (__bf16)0.0f;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qop[s][e] = d0 + e < dim ? src[d0 + e] : (__bf16)0.0f;
+      }
+    }
+    if constexpr (KR > 0) {
+      const int half = x.rot_dims / 2;
+      if (((x.qstride | dim | half | x.rot_part) & 7) == 0) {  // eight dimensions are rotated alike, or none
+#pragma unroll
+        for (int s = 0; s < KR; ++s) {
+          const int d = 16 * s + 8 * hh, i = d < half ? d : d - half;
+          bf16x8 y = bf16x8{};
+          if (d < x.rot_part) y = *reinterpret_cast<const bf16x8*>(src + dim + d);
+          if (d < x.rot_dims) {
+            const bf16x8 z = *reinterpret_cast<const bf16x8*>(src + dim + (d < half ? d + half : d - half));
+#pragma unroll
+            for (int e4 = 0; e4 < 8; e4 += 4) {
+              const f32x4 cs = *reinterpret_cast<const f32x4*>(x.cos_t + (size_t)p * half + i + e4);
+              const f32x4 sn = *reinterpret_cast<const f32x4*>(x.sin_t + (size_t)p * half + i + e4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float a = (float)y[e4 + e], b = (float)z[e4 + e];
+                y[e4 + e] = (__bf16)(d < half ? a * cs[e] - b * sn[e] : a * cs[e] + b * sn[e]);
+              }
+            }
+          }
+          qop[KS + s] = y;
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < KR; ++s)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int d = 16 * s + 8 * hh + e;
+            float y = d < x.rot_part ? (float)src[dim + d] : 0.0f;
+            if (d < x.rot_dims)
+              y = rotated(y, (float)src[dim + rot_partner(d, x.rot_dims)], d, x.rot_dims, (size_t)p, x.sin_t, x.cos_t);
+            qop[KS + s][e] = (__bf16)y;
+          }
+      }
+    }
+  }
+  stash(0, 0);
+  fetch(1, 0);
+
+  // exponents are powers of two; the scale is positive, so that the largest product is the largest score
+  const float unit = scale * 1.44269504f;
+  f32x16 o[C];
 #pragma unroll
   for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d = 32 * c + 8 * g4 + 4 * hh;
-      const float4 v = make_float4(o[c][4 * g4] * inv, o[c][4 * g4 + 1] * inv, o[c][4 * g4 + 2] * inv,
-                                   o[c][4 * g4 + 3] * inv);
-      if ((vdim & 3) == 0) {
-        if (d < vdim) store4(row + h * vdim + d, v);
-      } else {
-        const float f[4] = {v.x, v.y, v.z, v.w};
+    for (int v = 0; v < 16; ++v) o[c][v] = 0.0f;
+  float run_max = -INFINITY, run_sum = 0.0f;  // the sum: of the keys in this lane's registers
+  if (x.sinks && set == 0) {                  // a term of the denominator without a value
+    run_max = x.sinks[h] * 1.44269504f;
+    run_sum = hh == 0 ? 1.0f : 0.0f;
+  }
+  // every wavefront's LDS traffic so far is done (loads from memory stay on their way)
+  auto barrier = [] __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  stash(1, 0);
+  fetch(2, 1);
+  barrier();
+
+  const bf16x8 *k_ops, *v_ops;  // of the turn
+  auto k_of = [&](int turn) { return s_k + ((turn & 1) * KW + set) * (KS + KR) * 64 + lane; };
+  f32x16 st;  // the scores of the turn's block
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (d + e < vdim) row[h * vdim + d + e] = (__bf16)f[e];
+  for (int v = 0; v < 16; ++v) st[v] = 0.0f;
+  k_ops = k_of(0);
+#pragma unroll
+  for (int s = 0; s < KS + KR; ++s) st = mfma_bf16(k_ops[64 * s], qop[s], st);
+
+  // One block: its softmax weights and values, and the next block's scores. edge: some query does not see some key of it.
+  auto step = [&](bool edge, int key0, bool pooled, auto bring) __attribute__((always_inline)) {
+    constexpr int kQ = KS + KR, kAhead = 4, kFront = kQ / 2;  // products of scores in front of the exponentials
+    f32x16 next;
+    bf16x8 kop[kQ], vop[C];
+    u32x4 hi[2], lo[2];
+    auto score = [&](int s) __attribute__((always_inline)) {
+      if (s == 0)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) next[v] = 0.0f;
+      next = mfma_bf16(kop[s], qop[s], next);
+      if (s + kAhead < kQ) kop[s + kAhead] = k_ops[64 * (s + kAhead)];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto value = [&](int c, int ks) __attribute__((always_inline)) { vop[c] = v_ops[128 * c + 32 * ks]; };
+    // entries past the last one any query sees may hold anything: a zero weight must not meet them
+    const int last = (pooled ? nb_last - 1 : p_last) - key0;
+    auto clear = [&](int ks) __attribute__((always_inline)) {
+      if (31 > last)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (16 * ks + 8 * (e >> 2) + 4 * hh + (e & 3) > last) vop[c][e] = (__bf16)0.0f;
+    };
+#pragma unroll
+    for (int s = 0; s < kAhead && s < kQ; ++s) kop[s] = k_ops[64 * s];
+    if (edge) {
+      const int lo_key = (pooled ? 0 : p - window + 1) - key0 - 4 * hh, hi_key = (pooled ? nb - 1 : p) - key0 - 4 * hh;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int key = 8 * (v >> 2) + (v & 3);
+        st[v] = key >= lo_key && key <= hi_key ? st[v] : -INFINITY;
       }
     }
-  if (h == heads - 1) {
-    for (int c = heads * vdim + hh; c < ldo; c += 2) row[c] = (__bf16)0.0f;
+    __builtin_amdgcn_sched_barrier(0);
+    float blk_max = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kFront; ++i) {
+      score(i);
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (v * kFront / 16 == i) blk_max = fmaxf(blk_max, st[v]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const float new_max = fmaxf(run_max, max_of_halves(blk_max) * unit);
+    if (__any(new_max > run_max + 8.0f)) {
+      const float corr = new_max > run_max ? __builtin_amdgcn_exp2f(run_max - new_max) : 1.0f;
+      run_sum *= corr;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[c][v] *= corr;
+      run_max = new_max;
+    }
+    const float base = run_max == -INFINITY ? 0.0f : run_max;
+    auto pair = [&](int e) __attribute__((always_inline)) {  // the weights as a sum of two bf16 terms
+      const float w0 = __builtin_amdgcn_exp2f(__fmaf_rn(st[2 * e], unit, -base));
+      const float w1 = __builtin_amdgcn_exp2f(__fmaf_rn(st[2 * e + 1], unit, -base));
+      run_sum += w0;
+      run_sum += w1;
+      const unsigned top = bf16_pair(w0, w1);
+      hi[e >> 2][e & 3] = top;
+      lo[e >> 2][e & 3] = bf16_pair(w0 - __uint_as_float(top << 16), w1 - __uint_as_float(top & 0xFFFF0000u));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int c = 0; c < C; ++c) value(c, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      pair(e);
+#pragma unroll
+      for (int s = kFront; s < kQ; ++s)
+        if ((s - kFront) * 4 / (kQ - kFront) == e) score(s);
+    }
+    bring();  // (the LDS has nothing to read meanwhile)
+    if (edge) clear(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < 2 * C; ++m) {
+      o[m % C] = mfma_bf16(vop[m % C], __builtin_bit_cast(bf16x8, m < C ? lo[0] : hi[0]), o[m % C]);
+      if (m >= C) value(m % C, 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e * 2 * C / 4 == m) pair(4 + e);
+    }
+    if (edge) clear(1);
+#pragma unroll
+    for (int m = 0; m < 2 * C; ++m) o[m % C] = mfma_bf16(vop[m % C], __builtin_bit_cast(bf16x8, m < C ? lo[1] : hi[1]), o[m % C]);
+    st = next;
+  };
+
+  const int turns = (blocks + KW - 1) / KW;
+  for (int turn = 0; turn < turns; ++turn) {
+    auto bring = [&] __attribute__((always_inline)) {
+      stash(turn & 1, (turn + 1) & 1);
+      fetch(turn + 3, turn + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    barrier();
+    k_ops = k_of(turn + 1);
+    v_ops = s_v + ((turn & 1) * KW + set) * KS * 64 + 64 * (j >> 4) + 16 * hh + (j & 15);
+    const int b = turn * KW + set;
+    const bool pooled = b < pool_blocks;
+    const int block = pooled ? b : tok_first + b - pool_blocks, key0 = 32 * block;
+    if (!any || b >= blocks || !(pooled ? key0 < nb_last : block >= own_first && block <= own_last)) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) st[v] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS + KR; ++s) st = mfma_bf16(k_ops[64 * s], qop[s], st);
+      bring();
+    } else {
+      step(!(pooled ? key0 + 32 <= nb_first : key0 > p_last - window && key0 + 31 <= p_first), key0, pooled, bring);
+    }
   }
+  barrier();
+
+  if constexpr (KW > 1) {
+    float* const s_merge = reinterpret_cast<float*>(smem);  // [KW - 1][QW][R][64]
+    if (set > 0) {
+      float* dst = s_merge + (size_t)((set - 1) * QW + wq) * R * 64 + lane;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) dst[(16 * c + v) * 64] = o[c][v];
+      dst[(R - 2) * 64] = run_max;
+      dst[(R - 1) * 64] = run_sum;
+    }
+    __syncthreads();
+    if (set > 0) return;
+    float total_max = run_max;
+#pragma unroll
+    for (int w = 0; w < KW - 1; ++w) total_max = fmaxf(total_max, s_merge[((size_t)(w * QW + wq) * R + R - 2) * 64 + lane]);
+    const float base = total_max == -INFINITY ? 0.0f : total_max, own = __builtin_amdgcn_exp2f(run_max - base);
+    run_sum *= own;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[c][v] *= own;
+#pragma unroll
+    for (int w = 0; w < KW - 1; ++w) {
+      const float* src = s_merge + (size_t)(w * QW + wq) * R * 64 + lane;
+      const float wt = __builtin_amdgcn_exp2f(src[(R - 2) * 64] - base);
+      run_sum += src[(R - 1) * 64] * wt;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[c][v] += src[(16 * c + v) * 64] * wt;
+    }
+  }
+  run_sum += __shfl_xor(run_sum, 32, 64);
+  if (m0 + j >= M) return;
+  store_attention<C>(o, 1.0f / run_sum, x, out, ldo, m0 + j, h, heads, vdim, hh);  // every query sees its own key
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -791,9 +1141,46 @@ hipError_t qkv_t(const AttnGeom& g, const AttnMem& m, const float* raw, int ldr,
   return hipGetLastError();
 }
 
+// Whether attn_tile_kernel is the quicker one. Its longest workgroup has to be hidden behind the others: `longest` blocks of keys
+// against what 512 workgroups, as many as fit at once, have to do on average. Measured on 30 sizes of D = 128 (60 to 1024
+// workgroups) and 21 of D = 64, all of which the rule decides right; on its two sides, for instance, 12 heads without a window: 1280
+// queries 26.8 us here 31.5, 1501 queries 37.9 / 35.6; 28 heads: 200 queries 9.0 / 10.9, 512 queries 17.8 / 16.9.
+bool tile_is_quicker(const AttnGeom& g, int M, int pos0) {
+  const int tiles = (M + kTileQueries - 1) / kTileQueries;
+  if ((g.D != 64 && g.D != 128) || !(g.scale > 0.0f) || (long)g.heads * tiles < 128) return false;
+  long longest = 0, all = 0;
+  for (int t = 0; t < tiles; ++t) {
+    const long first = (long)pos0 + (long)kTileQueries * t, last = (long)pos0 + std::min((long)kTileQueries * (t + 1), (long)M) - 1;
+    const long behind = g.pool > 0 ? std::max(0l, last - g.window + 1) / g.pool : 0;
+    const long blocks = last / 32 - std::max(0l, first - g.window + 1) / 32 + 1 + (behind + 31) / 32;
+    longest = std::max(longest, blocks);
+    all += blocks;
+  }
+  const double average = (double)all * g.heads / 512;
+  return g.D == 128 ? longest <= 3.0 * average + 5.0 : longest <= 1.5 * average + 1.0;
+}
+
+template <int D, int KR>
+hipError_t tile_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M, int pos0,
+                  hipStream_t s) {
+  auto kern = attn_tile_kernel<D, KR>;
+  constexpr size_t lds = std::max<size_t>((size_t)2 * kTileSets * (D / 8 + KR) * 1024,
+                                          sizeof(float) * (kTileSets - 1) * kTileWaves * (D / 2 + 2) * 64);
+  static LdsLimitOnce raised;
+  if (lds > 64 * 1024)
+    if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)g.heads * ((M + kTileQueries - 1) / kTileQueries)), dim3(64 * kTileSets * kTileWaves), lds, s,
+                     static_cast<const __bf16*>(q), static_cast<const __bf16*>(m.k), static_cast<const __bf16*>(m.vt),
+                     static_cast<const __bf16*>(m.kp), static_cast<const __bf16*>(m.vpt), static_cast<__bf16*>(out), ldo, M,
+                     g.heads, g.kv_heads, g.dim, g.vdim, g.cap, g.capp, g.window, g.pool, pos0, g.scale, x);
+  return hipGetLastError();
+}
+
 template <int D, int KR>
 hipError_t mfma_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M,
                   int pos0, hipStream_t s) {
+  if constexpr ((D == 64 || D == 128) && KR <= 4)
+    if (tile_is_quicker(g, M, pos0)) return tile_d<D, KR>(g, m, x, q, out, ldo, M, pos0, s);
   auto kern = attn_mfma_kernel<D, KR>;
   constexpr size_t lds = (D / 16 + KR) * 64 * 16 + sizeof(float) * (kMfmaWaves - 1) * (D / 2 + 2) * 64;
   static LdsLimitOnce raised;

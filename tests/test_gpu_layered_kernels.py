@@ -304,3 +304,35 @@ def test_recurrences_of_any_number_of_heads(heads, dim, vdim):
     for n in (65, 128, 7):
         assert lm.errors(dec.forward(state, tokens[at:at + n], at), ref[at:at + n]).max() < TOL["float32"], (at, n)
         at += n
+
+
+# ---------------------------------------------------------------------------------------------- attention of long prompts
+# (head, 64 queries) tiles in numbers that take the kernel with keys and values in LDS: two sets of blocks, 64 queries of which the
+# last are missing, windows inside of a block and across pooled ones, positions off the blocks' borders in the second portion
+@pytest.mark.parametrize("arch,layer,T", [
+    ("suripel", lm.attention(32, 4, 100, 124, 70, 8), 300),
+    ("suripel", lm.attention(96, 16, 50, 64, 33, 4), 390),
+    ("lesarax", lm.rotary(48, 2, 128, 40), 200),
+    ("lesarax", lm.latent(60, 64, 64, 48, 40, 64, 40), 450),
+    ("lesarax", lm.latent(44, 120, 16, 128, 40, 100, 50), 230),  # rotated eight dimensions at a time ...
+    ("lesarax", lm.latent(36, 100, 28, 90, 40, 64, 10**6), 260),   # ... and one by one
+])
+def test_attention_of_long_prompts(arch, layer, T):
+    import torch
+
+    cfg = lm.config([layer], width=72) if arch == "suripel" else lm.lesarax([layer], width=72)
+    w = (lm.random_weights if arch == "suripel" else lm.lesarax_weights)(cfg, seed=T)
+    tokens = np.random.default_rng(T).integers(0, cfg["vocab"], T)
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, w, "bfloat16", T + 70)
+    state = dec.new_state()
+    whole = dec.forward(state, tokens, 0)
+    assert lm.errors(whole, ref).max() < TOL["bfloat16"]
+    parts = torch.cat([dec.forward(state, tokens[:37], 0), dec.forward(state, tokens[37:], 37)])
+    assert lm.errors(parts, ref).max() < TOL["bfloat16"]
+    # what the cache holds past the sequence does not matter: a longer one of values that are not finite lay there
+    bad = lm.runner(cfg, w, "bfloat16", T + 70)
+    bad._keep[-3][:, :] = float("inf")
+    state = bad.new_state()
+    bad.forward(state, np.zeros(T + 64, dtype=np.int64), 0, want=[])
+    assert torch.equal(dec.forward(state, tokens, 0), whole)
