@@ -19,22 +19,12 @@ namespace w4 {
 
 namespace {
 
-// kFar: operands or results whose rows are too long for 32-bit offsets
+// The tile of C from row m0 and column n0 on, over k in [kb, ke). kFar: operands or results whose rows are too long for 32-bit offsets
 template <typename T, int BM, int BN, int WM, int WN, int D, typename CT, bool kFar>
-__global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restrict__ a, const T* __restrict__ b,
-                                                              CT* __restrict__ c, int M, int N, int K, int ldc, int mt,
-                                                              int nt) {
+__device__ __forceinline__ void matmul_tile(uint8_t* smem, const T* __restrict__ a, const T* __restrict__ b, CT* __restrict__ c,
+                                            int M, int N, int K, int ldc, int m0, int n0, int kb, int ke) {
   using Tile = MfmaTile<T, BM, BN, WM, WN, D>;
-  constexpr int FM = Tile::FM, FN = Tile::FN, kBK = Tile::kBK;
-  extern __shared__ __align__(16) uint8_t smem[];
-
-  // tile number: consecutive ones on one XCD
-  const int t = xcd_tile(blockIdx.x, mt * nt);
-  const int m0 = (t % mt) * BM, n0 = (t / mt) * BN;
-  // this workgroup's share of the k range, in whole LDS tiles
-  const int k_steps = K / kBK;
-  const int kb = (int)((long)k_steps * blockIdx.y / gridDim.y) * kBK;
-  const int ke = (int)((long)k_steps * (blockIdx.y + 1) / gridDim.y) * kBK;
+  constexpr int FM = Tile::FM, FN = Tile::FN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
 
@@ -52,7 +42,7 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restric
   Tile::run(smem, tile_rows_at<kFar>(a + (size_t)m0 * K, sizeof(T) * ma * K), oa,
             tile_rows_at<kFar>(b + (size_t)n0 * K, sizeof(T) * nb * K), ob, kb, ke, acc);
 
-  c += (size_t)blockIdx.y * M * ldc + (size_t)m0 * ldc;
+  c += (size_t)m0 * ldc;
   if constexpr (kFar) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -85,6 +75,39 @@ __global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restric
     }
 }
 
+template <typename T, int BM, int BN, int WM, int WN, int D, typename CT, bool kFar>
+__global__ __launch_bounds__(64 * WM * WN) void matmul_kernel(const T* __restrict__ a, const T* __restrict__ b,
+                                                              CT* __restrict__ c, int M, int N, int K, int ldc, int mt,
+                                                              int nt) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  // tile number: consecutive ones on one XCD
+  const int t = xcd_tile(blockIdx.x, mt * nt);
+  // this workgroup's share of the k range, in whole LDS tiles
+  constexpr int kBK = MfmaTile<T, BM, BN, WM, WN, D>::kBK;
+  const int k_steps = K / kBK;
+  const int kb = (int)((long)k_steps * blockIdx.y / gridDim.y) * kBK;
+  const int ke = (int)((long)k_steps * (blockIdx.y + 1) / gridDim.y) * kBK;
+  matmul_tile<T, BM, BN, WM, WN, D, CT, kFar>(smem, a, b, c + (size_t)blockIdx.y * M * ldc, M, N, K, ldc, (t % mt) * BM, (t / mt) * BN,
+                                              kb, ke);
+}
+
+// The first `whole` bands of columns in tiles of 256 x 256, the others, behind them, in tiles of 128 x 256: whole rounds of the CUs
+// in the large tile, what is left of C in one that takes half as long. [2048][3584] x [18944][3584], 592 large tiles: 259 us, as 512
+// and 160 small ones 243; [2048][3584] x [10752][3584]: 164 (256 x 128) and 150; [2048][1536] x [8960][1536]: 68 (128 x 128) and 61.
+template <typename CT>
+__global__ __launch_bounds__(512) void matmul_two_heights_kernel(const __bf16* __restrict__ a, const __bf16* __restrict__ b,
+                                                                 CT* __restrict__ c, int M, int N, int K, int ldc, int nt, int whole) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int mt = (M + 255) / 256, rt = (M + 127) / 128;
+  if ((int)blockIdx.x < whole * mt) {
+    const int t = xcd_tile(blockIdx.x, whole * mt);
+    matmul_tile<__bf16, 256, 256, 2, 4, 2, CT, false>(smem, a, b, c, M, N, K, ldc, t % mt * 256, t / mt * 256, 0, K);
+  } else {
+    const int t = xcd_tile((int)blockIdx.x - whole * mt, (nt - whole) * rt);
+    matmul_tile<__bf16, 128, 256, 2, 4, 2, CT, false>(smem, a, b, c, M, N, K, ldc, t % rt * 128, (whole + t / rt) * 256, 0, K);
+  }
+}
+
 template <typename T, int BM, int BN, int WM, int WN, int D, typename CT, bool kFar = false>
 hipError_t launch_tile_t(const T* a, const T* b, void* c, int M, int N, int K, int ldc, int parts, hipStream_t s) {
   const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
@@ -95,6 +118,17 @@ hipError_t launch_tile_t(const T* a, const T* b, void* c, int M, int N, int K, i
     if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
   // parts <= K / kBK: no share is empty
   hipLaunchKernelGGL(kern, dim3(mt * nt, parts), dim3(64 * WM * WN), lds, s, a, b, static_cast<CT*>(c), M, N, K, ldc, mt, nt);
+  return hipGetLastError();
+}
+
+template <typename CT>
+hipError_t launch_two_heights(const __bf16* a, const __bf16* b, void* c, int M, int N, int K, int ldc, int whole, hipStream_t s) {
+  const int mt = (M + 255) / 256, rt = (M + 127) / 128, nt = (N + 255) / 256;
+  constexpr size_t lds = MfmaTile<__bf16, 256, 256, 2, 4, 2>::kLds;
+  auto kern = matmul_two_heights_kernel<CT>;
+  static LdsLimitOnce raised;
+  if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(whole * mt + (nt - whole) * rt), dim3(512), lds, s, a, b, static_cast<CT*>(c), M, N, K, ldc, nt, whole);
   return hipGetLastError();
 }
 
@@ -112,6 +146,8 @@ constexpr Shape kShapes[] = {
 // [1024][4096] took 100 us in one part of 64 x 64 without anything requested ahead; in one part of these 64, in four 34.
 constexpr Shape kShapesF32[] = {{64, 128, 0.91, 130}, {64, 64, 0.50, 118}};
 
+constexpr Shape kHalf = {128, 256, 0.70, 1060};  // half of the first one
+
 // us: rounds of the CUs, and the results' way to memory (and, as partial products, back)
 double shape_us(const Shape& t, int M, int N, double k_tiles, double tile_flops, int parts, int c_bytes) {
   const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
@@ -124,13 +160,28 @@ double shape_us(const Shape& t, int M, int N, double k_tiles, double tile_flops,
 
 struct Plan {
   int shape, parts;
+  int whole;  // bands of 256 columns in tiles of 256 rows, the others in tiles of 128; 0: one shape throughout
 };
+
+// us of 256 x 256 tiles whose last, incomplete round is cut into tiles of half the height, and how many bands are left whole
+double two_heights_us(int M, int N, double k_tiles, double tile_flops, int c_bytes, int* whole) {
+  const Shape& t = kShapes[0];
+  const int mt = (M + t.bm - 1) / t.bm, nt = (N + t.bn - 1) / t.bn;
+  *whole = (int)((long)mt * nt / 256 * 256 / mt);
+  if (*whole < 1 || *whole >= nt) return INFINITY;
+  auto round_us = [&](const Shape& s, long n) {
+    return std::max(s.tile_us * k_tiles, n * tile_flops * s.bm * s.bn * k_tiles / (s.tflops * 1e6));
+  };
+  const long rests = (long)(nt - *whole) * ((M + kHalf.bm - 1) / kHalf.bm);
+  return 2.5 + (double)*whole * mt / 256 * round_us(t, 256) + rests / 256 * round_us(kHalf, 256) +
+         (rests % 256 ? round_us(kHalf, rests % 256) : 0.0) + (double)M * N * c_bytes / 5e6;
+}
 
 // The cheapest shape; with most_parts > parts also the number of partial products (parts, twice that, ..) that go with it.
 Plan best_plan(bool f32, int M, int N, int K, int parts, int most_parts, int c_bytes) {
   const Shape* shapes = f32 ? kShapesF32 : kShapes;
   const int count = f32 ? sizeof(kShapesF32) / sizeof(Shape) : sizeof(kShapes) / sizeof(Shape), bk = f32 ? 32 : 64;
-  Plan best{0, parts};
+  Plan best{0, parts, 0};
   double least = INFINITY;
   for (int p = parts; p <= most_parts; p *= 2) {
     if (p > parts && K / p < (f32 ? 128 : 512)) break;
@@ -138,10 +189,12 @@ Plan best_plan(bool f32, int M, int N, int K, int parts, int most_parts, int c_b
       const double us = shape_us(shapes[i], M, N, (double)K / bk, 2.0 * bk, p, c_bytes);
       if (us < least) {
         least = us;
-        best = {i, p};
+        best = {i, p, 0};
       }
     }
   }
+  // (3 % cheaper at least: that far the costs of products whose last round is nearly full were seen to be off)
+  if (int whole; !f32 && best.parts == 1 && two_heights_us(M, N, K / 64.0, 2.0 * 64, c_bytes, &whole) < 0.97 * least) best = {0, 1, whole};
   return best;
 }
 
@@ -281,7 +334,11 @@ hipError_t launch_matmul_bf16(const void* a, const void* b, void* c, int M, int 
   const __bf16* pb = static_cast<const __bf16*>(b);
   if (c_bf16 && !product_near<__bf16, __bf16>(K, ldc)) return launch_far<__bf16, __bf16>(pa, pb, c, M, N, K, ldc, parts, s);
   if (!c_bf16 && !product_near<__bf16, float>(K, ldc)) return launch_far<__bf16, float>(pa, pb, c, M, N, K, ldc, parts, s);
-  const int shape = best_plan(false, M, N, K, parts, parts, c_bf16 ? 2 : 4).shape;
+  const Plan plan = best_plan(false, M, N, K, parts, parts, c_bf16 ? 2 : 4);
+  if (plan.whole > 0)
+    return c_bf16 ? launch_two_heights<__bf16>(pa, pb, c, M, N, K, ldc, plan.whole, s)
+                  : launch_two_heights<float>(pa, pb, c, M, N, K, ldc, plan.whole, s);
+  const int shape = plan.shape;
   return c_bf16 ? launch_shape<__bf16>(shape, pa, pb, c, M, N, K, ldc, parts, s)
                 : launch_shape<float>(shape, pa, pb, c, M, N, K, ldc, parts, s);
 }

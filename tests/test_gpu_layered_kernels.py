@@ -59,7 +59,9 @@ def test_norm_conv_leaves_its_tail_when_nobody_reads_the_ring(pkg, H, taps, firs
 
 
 # sizes at which each tile shape is chosen, rows and columns just past a tile, one to ten tiles of k
-@pytest.mark.parametrize("M,N,K", [(1025, 8963, 64), (1100, 9001, 256), (1025, 4483, 320), (513, 8961, 128), (513, 4483, 192),
+# (the first two: 256 x 256 with the last bands of columns in 128 x 256)
+@pytest.mark.parametrize("M,N,K", [(1025, 18001, 128), (515, 33091, 192),
+                                   (1025, 8963, 64), (1100, 9001, 256), (1025, 4483, 320), (513, 8961, 128), (513, 4483, 192),
                                    (257, 4481, 640), (600, 3001, 128), (300, 2049, 192), (129, 2001, 64), (70, 130, 448), (1, 1, 64)])
 def test_bf16_product_of_every_shape(pkg, M, N, K):
     import torch
