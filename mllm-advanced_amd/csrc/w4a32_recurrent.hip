@@ -442,71 +442,72 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(float* __restrict__ state
   }
 }
 
-// grid (chunks, heads), 256 threads; wavefront w: tokens 16 w ..
+// grid (chunks, heads), 256 threads; wavefront w: tokens 16 w .. The operands of 16 value dimensions, D / 16 + 4 kilobytes of state and U, come
+// through LDS once for all four wavefronts, the next ones meanwhile through registers.
 template <int D, typename T>
-__global__ __launch_bounds__(256) void rec_out_kernel(const RecGeom g, const float* __restrict__ raw,
-                                                      const float* __restrict__ scratch, T* __restrict__ out, int ldo,
-                                                      int M) {
-  constexpr int KQ = D / 4, NT = D / 16;
-  const int chunk = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+__global__ __launch_bounds__(256, D <= 128 ? 4 : 2) void rec_out_kernel(const RecGeom g, const float* __restrict__ raw,
+                                                                        const float* __restrict__ scratch, T* __restrict__ out,
+                                                                        int ldo, int M) {
+  constexpr int KQ = D / 4, NT = D / 16, kPieces = KQ / 4 + 4, kPer = (kPieces + 3) / 4;
+  __shared__ f32x4 s_op[2][kPieces][64];
+  const int chunk = blockIdx.x, h = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
   const int dv16 = (g.vdim + 15) & ~15;
   const ChunkOff off = chunk_off(D, dv16);
   const float* p = scratch + ((size_t)h * gridDim.x + chunk) * off.total;
+  auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
 
-  float4 q[KQ / 4], a[4];
-#pragma unroll
-  for (int i = 0; i < KQ / 4; ++i) q[i] = load4(p + off.q + ((wave * (KQ / 4) + i) * 64 + lane) * 4);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) a[i] = load4(p + off.a + ((wave * 4 + i) * 64 + lane) * 4);
-
-  struct Ops {
-    float4 s[KQ / 4], u[4];
-  };
-  auto fetch = [&](int nt, Ops& b) __attribute__((always_inline)) {
+  f32x4 piece[kPer];
+  auto fetch = [&](int nt) __attribute__((always_inline)) {
     const int t = min(nt, dv16 / 16 - 1);
 #pragma unroll
-    for (int i = 0; i < KQ / 4; ++i) b.s[i] = load4(p + off.s + ((t * (KQ / 4) + i) * 64 + lane) * 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b.u[i] = load4(p + off.u + ((t * 4 + i) * 64 + lane) * 4);
+    for (int i = 0; i < kPer; ++i) {
+      const int n = min(wave + 4 * i, kPieces - 1);
+      const float* src = n < KQ / 4 ? p + off.s + (size_t)(t * (KQ / 4) + n) * 256 : p + off.u + (size_t)(t * 4 + n - KQ / 4) * 256;
+      piece[i] = ld(src + 4 * lane);
+    }
   };
+  auto stash = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      if (kPieces % 4 == 0 || wave + 4 * i < kPieces) s_op[buf][wave + 4 * i][lane] = piece[i];
+  };
+  fetch(0);
+  f32x4 q[KQ / 4], a[4];
+#pragma unroll
+  for (int i = 0; i < KQ / 4; ++i) q[i] = ld(p + off.q + ((wave * (KQ / 4) + i) * 64 + lane) * 4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a[i] = ld(p + off.a + ((wave * 4 + i) * 64 + lane) * 4);
+  stash(0);
+  fetch(1);
+
   f32x4 o[NT];
   float ss[4] = {0, 0, 0, 0};
-  auto multiply = [&](int nt, const Ops& b) __attribute__((always_inline)) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    if (16 * nt >= dv16) break;
+    // what every wavefront has written and read in LDS so far is done; loads from memory stay on their way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     f32x4 o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < KQ / 4; ++i) {
-      o0 = mfma4(q[i].x, b.s[i].x, o0);
-      o1 = mfma4(q[i].y, b.s[i].y, o1);
-      o0 = mfma4(q[i].z, b.s[i].z, o0);
-      o1 = mfma4(q[i].w, b.s[i].w, o1);
+    for (int i = 0; i < kPieces; ++i) {
+      const f32x4 x = i < KQ / 4 ? q[i < KQ / 4 ? i : 0] : a[i < KQ / 4 ? 0 : i - KQ / 4], y = s_op[nt & 1][i][lane];
+      o0 = mfma4(x[0], y[0], o0);
+      o1 = mfma4(x[1], y[1], o1);
+      o0 = mfma4(x[2], y[2], o0);
+      o1 = mfma4(x[3], y[3], o1);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o0 = mfma4(a[i].x, b.u[i].x, o0);
-      o1 = mfma4(a[i].y, b.u[i].y, o1);
-      o0 = mfma4(a[i].z, b.u[i].z, o0);
-      o1 = mfma4(a[i].w, b.u[i].w, o1);
+    if (nt + 1 < NT) {
+      stash((nt + 1) & 1);
+      if (nt + 2 < NT) fetch(nt + 2);
     }
     o0 = o0 + o1;
     const float keep = 16 * nt + col < g.vdim ? 1.0f : 0.0f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) ss[r] = __fmaf_rn(o0[r] * keep, o0[r], ss[r]);
     o[nt] = o0;
-  };
-  // two register sets: a block's operands are requested while the one before it is multiplied
-  Ops b0, b1;
-  fetch(0, b0);
-#pragma unroll
-  for (int nt = 0; nt < NT; nt += 2) {
-    if (16 * nt < dv16) {
-      fetch(nt + 1, b1);
-      multiply(nt, b0);
-    }
-    if (nt + 1 < NT && 16 * (nt + 1) < dv16) {
-      fetch(nt + 2, b0);
-      multiply(nt + 1, b1);
-    }
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
