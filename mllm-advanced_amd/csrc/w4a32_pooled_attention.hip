@@ -17,7 +17,8 @@
 //                         cross-lane move). The softmax weights stay f32: they enter the second product as a sum of
 //                         two bf16 terms.
 //   attn_tile_kernel      the same for long prompts: keys and values through LDS, products and softmax under each other
-//   attn_rows_kernel      prefill, f32: one wavefront per (head, query)
+//   attn_f32_kernel       prefill, f32: as attn_mfma_kernel, on the f32 matrix instruction
+//   attn_rows_kernel      a few tokens, f32: one wavefront per (head, query)
 //   attn_decode_kernel    one token: convolution, cache append, block mean and attention over one slice of the visible
 //                         keys per workgroup; the slices are merged by the Linear that follows
 #include <algorithm>
@@ -744,6 +745,212 @@ __global__ __launch_bounds__(64 * kTileSets * kTileWaves, 2) void attn_tile_kern
 }
 
 // ---------------------------------------------------------------------------------------------
+// f32: workgroup = (head, 32 queries) as in attn_mfma_kernel, the products on v_mfma_f32_32x32x2_f32. An operand of that instruction is
+// one number per lane, so a lane's eight of a piece (16 dimensions of the keys, 16 entries of the values) serve eight products; pieces
+// are requested three ahead, straight from the caches' layout. A block of D = 128 is 128 products of 64 clocks and little else:
+// bound by the matrix cores. 18 heads of 1538 queries, window 269, D = 128: 1762 us in one wavefront per query, here 87; 8 heads of
+// 300 queries 107, here 29.
+template <int D, int KR>
+__global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_kernel(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vt, const float* __restrict__ kp,
+    const float* __restrict__ vpt, float* __restrict__ out, int ldo, int M, int heads, int kv_heads, int dim, int vdim, int cap,
+    int capp, int window, int pool, int pos0, float scale, const PrefillExtra x) {
+  constexpr int KS = D / 16, C = D / 32, R = 16 * C + 2;
+  constexpr int kKeys = KS + KR, kPieces = kKeys + 2 * C, kRing = 4, kSteps = (kPieces + kRing - 1) / kRing * kRing;
+  extern __shared__ __align__(16) uint8_t smem[];
+  f32x4* const s_q = reinterpret_cast<f32x4*>(smem);                                      // [kKeys][2][64]
+  float* const s_merge = reinterpret_cast<float*>(smem + (size_t)kKeys * 2 * 64 * 16);     // [waves - 1][R][64]
+  const int h = blockIdx.x, g = h / (heads / kv_heads);
+  const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // the later query blocks see more keys: they start first
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int j = lane & 31, hh = lane >> 5;
+
+  const int m_q = min(32 * qb + j, M - 1), p = pos0 + m_q;
+  const int p_first = pos0 + 32 * qb, p_last = pos0 + min(32 * qb + 31, M - 1);
+  const int nb = pooled_visible(p, window, pool), nb_first = pooled_visible(p_first, window, pool);
+  const int nb_last = pooled_visible(p_last, window, pool);
+  const int pool_blocks = (nb_last + 31) / 32;
+  const int tok_first = max(0, p_first - window + 1) / 32;
+  const int blocks = pool_blocks + p_last / 32 - tok_first + 1;
+
+  for (int it = threadIdx.x; it < kKeys * 64; it += 64 * kMfmaWaves) {
+    const int s = it >> 6, l = it & 63, d0 = 16 * (s < KS ? s : s - KS) + 8 * (l >> 5), m = min(32 * qb + (l & 31), M - 1);
+    const float* src = q + (size_t)m * x.qld + (size_t)h * x.qstride;
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int d = d0 + e;
+      if (s < KS) {
+        y[e] = d < dim ? src[d] : 0.0f;
+      } else {
+        y[e] = d < x.rot_part ? src[dim + d] : 0.0f;
+        if (d < x.rot_dims) y[e] = rotated(y[e], src[dim + rot_partner(d, x.rot_dims)], d, x.rot_dims, (size_t)(pos0 + m), x.sin_t, x.cos_t);
+      }
+    }
+    s_q[(2 * s) * 64 + l] = f32x4{y[0], y[1], y[2], y[3]};
+    s_q[(2 * s + 1) * 64 + l] = f32x4{y[4], y[5], y[6], y[7]};
+  }
+  __syncthreads();
+
+  constexpr int kBlk = 32 * D;  // elements of a block
+  const float* const kt = kc + (size_t)g * cap * D + (size_t)(tok_first - x.blk0) * kBlk;
+  const float* const kpt = kp + (size_t)g * capp * D;
+  const float* const vtt = vt + (size_t)g * cap * D + (size_t)(tok_first - x.blk0) * kBlk;
+  const float* const vptt = vpt + (size_t)g * capp * D;
+  const unsigned k_off = 8 * lane, v_off = 32 * j + 8 * hh;
+
+  struct Block {
+    const float *k, *r, *v;
+  };
+  auto block_of = [&](int b) __attribute__((always_inline)) {
+    const bool pooled = b < pool_blocks;
+    Block at;
+    at.k = pooled ? kpt + (size_t)b * kBlk : kt + (size_t)(b - pool_blocks) * kBlk;
+    at.v = pooled ? vptt + (size_t)b * kBlk : vtt + (size_t)(b - pool_blocks) * kBlk;
+    at.r = KR > 0 ? static_cast<const float*>(x.kr) + (size_t)(tok_first + b - pool_blocks) * x.kr_block : nullptr;
+    return at;
+  };
+  f32x4 ring[kRing][2];
+  auto request = [&](const Block& at, int n) __attribute__((always_inline)) {
+    typedef const f32x4 __attribute__((address_space(1))) * Global;  // (or the loads are flat ones, which the LDS' counter waits for too)
+    const float* src = n < KS      ? at.k + 512 * n + k_off
+                       : n < kKeys ? at.r + 512 * (n - KS) + k_off
+                                   : at.v + 1024 * ((n - kKeys) / 2) + 16 * ((n - kKeys) % 2) + v_off;
+    ring[n % kRing][0] = *(Global)src;
+    ring[n % kRing][1] = *(Global)(src + 4);
+  };
+
+  f32x16 o[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[c][v] = 0.0f;
+  float run_max = -INFINITY, run_sum = 0.0f;  // the sum: of the keys in this lane's registers
+  if (x.sinks && wave == 0) {                 // a term of the denominator without a value
+    run_max = x.sinks[h];
+    run_sum = hh == 0 ? 1.0f : 0.0f;
+  }
+
+  if (wave < blocks)
+#pragma unroll
+    for (int n = 0; n < kRing - 1; ++n) request(block_of(wave), n);
+  for (int b = wave; b < blocks; b += kMfmaWaves) {
+    const bool pooled = b < pool_blocks;
+    const int key0 = 32 * (pooled ? b : tok_first + b - pool_blocks);
+    const bool edge = !(pooled ? key0 + 32 <= nb_first : key0 > p_last - window && key0 + 31 <= p_first);
+    const Block here = block_of(b), next = block_of(min(b + kMfmaWaves, blocks - 1));
+    const int last = (pooled ? nb_last - 1 : p_last) - key0;  // the last entry any query sees
+    auto ahead = [&](int n) __attribute__((always_inline)) {
+      const int to = n + kRing - 1;
+      if (to < kPieces) request(here, to);
+      else if (to >= kSteps) request(next, to - kSteps);
+    };
+    f32x16 st, st1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) st[v] = st1[v] = 0.0f;
+#pragma unroll
+    for (int n = 0; n < kKeys; ++n) {
+      ahead(n);
+      const f32x4 q0 = s_q[2 * n * 64 + lane], q1 = s_q[(2 * n + 1) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // two accumulators take turns
+        st = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[n % kRing][0][e], q0[e], st, 0, 0, 0);
+        st1 = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[n % kRing][1][e], q1[e], st1, 0, 0, 0);
+      }
+    }
+    // the range of this block's keys that the lane's query sees
+    const int lo = (pooled ? 0 : p - window + 1) - key0 - 4 * hh, hi = (pooled ? nb - 1 : p) - key0 - 4 * hh;
+    float blk_max = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int key = 8 * (v >> 2) + (v & 3);
+      st[v] = (st[v] + st1[v]) * scale;
+      if (edge) st[v] = key >= lo && key <= hi ? st[v] : -INFINITY;
+      blk_max = fmaxf(blk_max, st[v]);
+    }
+    const float new_max = fmaxf(run_max, max_of_halves(blk_max));
+    if (__any(new_max != run_max)) {
+      const float corr = run_max == -INFINITY ? 0.0f : expf(run_max - new_max);
+      run_sum *= corr;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[c][v] *= corr;
+      run_max = new_max;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      st[v] = st[v] == -INFINITY ? 0.0f : expf(st[v] - run_max);
+      run_sum += st[v];
+    }
+#pragma unroll
+    for (int n = kKeys; n < kSteps; ++n) {
+      ahead(n);
+      if (n >= kPieces) continue;
+      const int c = (n - kKeys) / 2, ks = (n - kKeys) % 2;
+      f32x4 v0 = ring[n % kRing][0], v1 = ring[n % kRing][1];
+      // entries past the last one any query sees may hold anything: a zero weight must not meet them
+      if (31 > last) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (16 * ks + 4 * hh + e > last) v0[e] = 0.0f;
+          if (16 * ks + 8 + 4 * hh + e > last) v1[e] = 0.0f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v0[e], st[8 * ks + e], o[c], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v1[e], st[8 * ks + 4 + e], o[c], 0, 0, 0);
+    }
+  }
+
+  if (wave > 0) {
+    float* dst = s_merge + (size_t)(wave - 1) * R * 64 + lane;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) dst[(16 * c + v) * 64] = o[c][v];
+    dst[(R - 2) * 64] = run_max;
+    dst[(R - 1) * 64] = run_sum;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  float total_max = run_max;
+#pragma unroll
+  for (int w = 0; w < kMfmaWaves - 1; ++w) total_max = fmaxf(total_max, s_merge[((size_t)w * R + R - 2) * 64 + lane]);
+  const float own = run_max == -INFINITY ? 0.0f : expf(run_max - total_max);
+  run_sum *= own;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[c][v] *= own;
+#pragma unroll
+  for (int w = 0; w < kMfmaWaves - 1; ++w) {
+    const float* src = s_merge + (size_t)w * R * 64 + lane;
+    const float theirs = src[(R - 2) * 64], wt = theirs == -INFINITY ? 0.0f : expf(theirs - total_max);
+    run_sum += src[(R - 1) * 64] * wt;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[c][v] += src[(16 * c + v) * 64] * wt;
+  }
+  run_sum += __shfl_xor(run_sum, 32, 64);  // (every query sees its own key)
+  const int m = 32 * qb + j;
+  if (m >= M) return;
+  const float gate = x.gate ? sigmoid_f(x.gate[(size_t)m * x.ldg + h]) : 1.0f;
+  float* row = out + (size_t)m * ldo;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int d = 32 * c + 8 * (v >> 2) + 4 * hh + (v & 3);
+      if (d < vdim) row[h * vdim + d] = o[c][v] / run_sum * gate;
+    }
+  if (h == heads - 1)
+    for (int c = heads * vdim + hh; c < ldo; c += 2) row[c] = 0.0f;
+}
+
+// ---------------------------------------------------------------------------------------------
 // One wavefront per (head, query), everything f32: a lane per key for the scores, a lane per value dimension for
 // the sums.
 template <typename T>
@@ -1267,8 +1474,36 @@ static hipError_t prefill_bf16(const AttnGeom& g, const AttnMem& m, const Prefil
   }
 }
 
+// Whether attn_f32_kernel is the quicker one: a block of 32 keys costs it 4 us of matrix instructions and its start 15, so that few
+// tokens on few keys stay with one wavefront per query. Us here / in attn_rows_kernel, 8 heads, D = 128: 14 tokens 20 / 11, 45: 20 / 14,
+// 64: 19 / 16, 96: 19 / 26, 130: 23 / 38, 300 with a window of 64 19 / 44; 24 heads, D = 64: 45 tokens 10 / 9, 130: 12 / 34.
+static bool f32_tiles(const AttnGeom& g, int M, int pos0) { return M > 64 || std::min((long)g.window, (long)pos0 + M) > 128; }
+
+template <int D, int KR>
+static hipError_t f32_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M, int pos0,
+                        hipStream_t s) {
+  auto kern = attn_f32_kernel<D, KR>;
+  constexpr size_t lds = (size_t)(D / 16 + KR) * 2 * 64 * 16 + sizeof(float) * (kMfmaWaves - 1) * (D / 2 + 2) * 64;
+  static LdsLimitOnce raised;
+  if (lds > 64 * 1024)
+    if (hipError_t e = raised.raise(reinterpret_cast<const void*>(kern), lds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(g.heads, (M + 31) / 32), dim3(64 * kMfmaWaves), lds, s, static_cast<const float*>(q),
+                     static_cast<const float*>(m.k), static_cast<const float*>(m.vt), static_cast<const float*>(m.kp),
+                     static_cast<const float*>(m.vpt), static_cast<float*>(out), ldo, M, g.heads, g.kv_heads, g.dim, g.vdim, g.cap,
+                     g.capp, g.window, g.pool, pos0, g.scale, x);
+  return hipGetLastError();
+}
+
+template <int KR>
 static hipError_t prefill_f32(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo,
                               int M, int pos0, hipStream_t s) {
+  if (f32_tiles(g, M, pos0)) switch (g.D) {
+    case 32: return f32_d<32, KR>(g, m, x, q, out, ldo, M, pos0, s);
+    case 64: return f32_d<64, KR>(g, m, x, q, out, ldo, M, pos0, s);
+    case 128: return f32_d<128, KR>(g, m, x, q, out, ldo, M, pos0, s);
+    case 256: return f32_d<256, KR>(g, m, x, q, out, ldo, M, pos0, s);
+    default: return hipErrorInvalidValue;
+  }
   hipLaunchKernelGGL(attn_rows_kernel<float>, dim3(g.heads, M), dim3(64), 0, s, static_cast<const float*>(q),
                      static_cast<const float*>(m.k), static_cast<const float*>(m.vt), static_cast<const float*>(m.kp),
                      static_cast<const float*>(m.vpt), static_cast<float*>(out), ldo, g.heads, g.kv_heads, g.dim, g.vdim,
@@ -1283,7 +1518,7 @@ hipError_t launch_attn_prefill(int dtype, const AttnGeom& g, const AttnMem& m, c
   x.qld = g.heads * g.D;
   x.qstride = g.D;
   if (dtype == W4A32_LAYERED_BF16) return prefill_bf16<0>(g, m, x, q, out, ldo, M, pos0, s);
-  return prefill_f32(g, m, x, q, out, ldo, M, pos0, s);
+  return prefill_f32<0>(g, m, x, q, out, ldo, M, pos0, s);
 }
 
 int latent_rot_pad(int rot_part) { return rot_part <= 16 ? 16 : rot_part <= 32 ? 32 : rot_part <= 64 ? 64 : 128; }
@@ -1312,12 +1547,14 @@ hipError_t launch_latent_prefill(int dtype, const LatentGeom& g, const void* k, 
   x.rot_dims = g.rot_dims;
   x.sin_t = g.sin_t;
   x.cos_t = g.cos_t;
-  if (dtype != W4A32_LAYERED_BF16) return prefill_f32(a, m, x, q, out, ldo, M, pos0, s);
+  const bool f32 = dtype != W4A32_LAYERED_BF16;
+#define W4_REST(DR)                                                              \
+  case DR:                                                                       \
+    return f32 ? prefill_f32<DR / 16>(a, m, x, q, out, ldo, M, pos0, s)          \
+               : prefill_bf16<DR / 16>(a, m, x, q, out, ldo, M, pos0, s)
   switch (g.Dr) {
-    case 16: return prefill_bf16<1>(a, m, x, q, out, ldo, M, pos0, s);
-    case 32: return prefill_bf16<2>(a, m, x, q, out, ldo, M, pos0, s);
-    case 64: return prefill_bf16<4>(a, m, x, q, out, ldo, M, pos0, s);
-    case 128: return prefill_bf16<8>(a, m, x, q, out, ldo, M, pos0, s);
+    W4_REST(16); W4_REST(32); W4_REST(64); W4_REST(128);
+#undef W4_REST
     default: return hipErrorInvalidValue;
   }
 }

@@ -443,7 +443,8 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(float* __restrict__ state
 }
 
 // grid (chunks, heads), 256 threads; wavefront w: tokens 16 w .. The operands of 16 value dimensions, D / 16 + 4 kilobytes of state and U, come
-// through LDS once for all four wavefronts, the next ones meanwhile through registers.
+// through LDS once for all four wavefronts, the next ones meanwhile through registers: read by each wavefront for itself, from two sets of
+// registers, 28 heads of 128 x 128 in 32 chunks took 60 us, now 45 (129 MB of scratch: 26 us at the rate of a copy).
 template <int D, typename T>
 __global__ __launch_bounds__(256, D <= 128 ? 4 : 2) void rec_out_kernel(const RecGeom g, const float* __restrict__ raw,
                                                                         const float* __restrict__ scratch, T* __restrict__ out,

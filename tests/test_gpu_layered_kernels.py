@@ -310,7 +310,9 @@ def test_recurrences_of_any_number_of_heads(heads, dim, vdim):
 
 # ---------------------------------------------------------------------------------------------- attention of long prompts
 # (head, 64 queries) tiles in numbers that take the kernel with keys and values in LDS: two sets of blocks, 64 queries of which the
-# last are missing, windows inside of a block and across pooled ones, positions off the blocks' borders in the second portion
+# last are missing, windows inside of a block and across pooled ones, positions off the blocks' borders in the second portion; in f32
+# the kernel on matrix instructions in the whole prompt and the second portion, in the first one wavefront per query
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("arch,layer,T", [
     ("suripel", lm.attention(32, 4, 100, 124, 70, 8), 300),
     ("suripel", lm.attention(96, 16, 50, 64, 33, 4), 390),
@@ -319,21 +321,21 @@ def test_recurrences_of_any_number_of_heads(heads, dim, vdim):
     ("lesarax", lm.latent(44, 120, 16, 128, 40, 100, 50), 230),  # rotated eight dimensions at a time ...
     ("lesarax", lm.latent(36, 100, 28, 90, 40, 64, 10**6), 260),   # ... and one by one
 ])
-def test_attention_of_long_prompts(arch, layer, T):
+def test_attention_of_long_prompts(arch, layer, T, dtype):
     import torch
 
     cfg = lm.config([layer], width=72) if arch == "suripel" else lm.lesarax([layer], width=72)
     w = (lm.random_weights if arch == "suripel" else lm.lesarax_weights)(cfg, seed=T)
     tokens = np.random.default_rng(T).integers(0, cfg["vocab"], T)
     ref = lo.forward(cfg, w, tokens)
-    dec = lm.runner(cfg, w, "bfloat16", T + 70)
+    dec = lm.runner(cfg, w, dtype, T + 70)
     state = dec.new_state()
     whole = dec.forward(state, tokens, 0)
-    assert lm.errors(whole, ref).max() < TOL["bfloat16"]
+    assert lm.errors(whole, ref).max() < TOL[dtype]
     parts = torch.cat([dec.forward(state, tokens[:37], 0), dec.forward(state, tokens[37:], 37)])
-    assert lm.errors(parts, ref).max() < TOL["bfloat16"]
+    assert lm.errors(parts, ref).max() < TOL[dtype]
     # what the cache holds past the sequence does not matter: a longer one of values that are not finite lay there
-    bad = lm.runner(cfg, w, "bfloat16", T + 70)
+    bad = lm.runner(cfg, w, dtype, T + 70)
     bad._keep[-3][:, :] = float("inf")
     state = bad.new_state()
     bad.forward(state, np.zeros(T + 64, dtype=np.int64), 0, want=[])
