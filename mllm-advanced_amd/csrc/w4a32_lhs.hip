@@ -57,10 +57,12 @@ __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(f[e], p);
-    uint2 packed;
-    packed.x = pack4(q);
-    packed.y = pack4(q + 4);
-    *reinterpret_cast<uint2*>(dst + i) = packed;
+    if (aq) {
+      uint2 packed;
+      packed.x = pack4(q);
+      packed.y = pack4(q + 4);
+      *reinterpret_cast<uint2*>(dst + i) = packed;
+    }
     if (ah) {
       // a_q - zp lies in [-255, 255]: exact in f16. Stored in the order a weight dword unpacks.
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -233,10 +235,12 @@ __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(v[r][e], p);
-    uint2 packed;
-    packed.x = pack4(q);
-    packed.y = pack4(q + 4);
-    *reinterpret_cast<uint2*>(dst + i) = packed;
+    if (aq) {
+      uint2 packed;
+      packed.x = pack4(q);
+      packed.y = pack4(q + 4);
+      *reinterpret_cast<uint2*>(dst + i) = packed;
+    }
     if (ah) {
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
@@ -255,11 +259,11 @@ constexpr int kQuantRowsMaxK = 8 * 8 * kLhsThreads;
 template <int SRC>
 static hipError_t launch_quant_rows(const float* a, const float* b, const float* norm_w, float eps,
                                     float* h_out, int M, int K, int lda, uint8_t* ws, hipStream_t s,
-                                    int nparts = 0, const float* part_bias = nullptr) {
+                                    bool bytes, int nparts = 0, const float* part_bias = nullptr) {
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = reinterpret_cast<int8_t*>(ws + g.aq_off);
+  int8_t* aq = bytes || M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   const int groups = (K + 8 * kLhsThreads - 1) / (8 * kLhsThreads);
 #define W4_LAUNCH_ROWS(R)                                                                          \
@@ -277,31 +281,31 @@ static hipError_t launch_quant_rows(const float* a, const float* b, const float*
 bool quant_rows_fusable(int K) { return K <= kQuantRowsMaxK; }
 
 hipError_t launch_quant_lhs_norm(const float* h, const float* delta, const float* norm_w, float eps,
-                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s) {
-  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s);
+                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s, bool bytes) {
+  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s, bytes);
 }
 
 // The same with delta = the sum of a split-K product's `nparts` scaled parts ([nparts][M][K]) + bias.
 hipError_t launch_quant_lhs_norm_parts(const float* h, const float* parts, int nparts, const float* bias,
                                        const float* norm_w, float eps, float* h_out, int M, int K,
-                                       uint8_t* ws, hipStream_t s) {
+                                       uint8_t* ws, hipStream_t s, bool bytes) {
   if (nparts < 1 || !parts || !bias) return hipErrorInvalidValue;
-  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, nparts, bias);
+  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, bytes, nparts, bias);
 }
 
 hipError_t launch_quant_lhs_silu_mul(const float* gate, const float* up, int M, int K, uint8_t* ws,
                                      hipStream_t s) {
-  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s);
+  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s, true);
 }
 
-hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s) {
+hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s, bool bytes) {
   if (K <= kQuantRowsMaxK) {
-    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s);
+    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s, bytes);
   }
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = reinterpret_cast<int8_t*>(ws + g.aq_off);
+  int8_t* aq = bytes || M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   hipLaunchKernelGGL(quant_lhs_kernel, dim3(M), dim3(kLhsThreads), 0, s, x, K, ldx, recip, negzp,
                      aq, ah);
