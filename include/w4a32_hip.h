@@ -128,7 +128,7 @@ int w4a32_matmul_quantized(float* d_y, const void* d_ws, const void* d_packed, i
  * (KaiLinear_f32_qai8dxp_qsi4c32p_mxk_nxk::Tiles, kai_linear.hpp:76-118). */
 #define W4A32_KERNEL_AUTO 0       /* M <= 8: GEMV, else f16 MFMA */
 #define W4A32_KERNEL_GEMV 1       /* v_dot4 decode kernel, M <= 8 */
-#define W4A32_KERNEL_GEMM_I8 2    /* int8 MFMA, exact int32 block sums, any M */
+#define W4A32_KERNEL_GEMM_I8 2    /* int8 MFMA, exact int32 block sums, any M; M > 8: makes the int8 rows in d_ws first */
 #define W4A32_KERNEL_GEMM_F16 3   /* f16 MFMA on exact f16 operands, M > 8; tile shape by size */
 /* The f16 kernel with one named tile shape, W4A32_KERNEL_GEMM_F16_TILE0 + i:
  * i = 0: 64 x 64, 1: 128 x 64, 2: 128 x 128, 3: 256 x 128 (rows x columns per workgroup),

@@ -52,19 +52,6 @@ int static_ws_ptr(void** out, hipStream_t stream) {
 
 }  // namespace
 
-namespace {
-
-// bytes: the int8 rows are wanted as well as what the product of this size reads
-int quantise(const float* d_x, int M, int K, int ldx, void* d_ws, bool bytes, void* stream) {
-  if (M <= 0) return W4A32_EINVAL;
-  if (int e = shape_ok(1, K)) return e;
-  if (!d_x || !d_ws || ldx < K) return W4A32_EINVAL;
-  if (!aligned(d_x, 16) || (ldx % 4) != 0 || !aligned(d_ws, 256)) return W4A32_EINVAL;
-  return from_hip(w4::launch_quant_lhs(d_x, M, K, ldx, static_cast<uint8_t*>(d_ws), static_cast<hipStream_t>(stream), bytes));
-}
-
-}  // namespace
-
 extern "C" {
 
 int w4a32_abi_version(void) { return 1; }
@@ -152,7 +139,12 @@ int w4a32_dequant(const void* d_packed, int N, int K, float* d_out, void* stream
 }
 
 int w4a32_quant_lhs(const float* d_x, int M, int K, int ldx, void* d_ws, void* stream) {
-  return quantise(d_x, M, K, ldx, d_ws, true, stream);
+  if (M <= 0) return W4A32_EINVAL;
+  if (int e = shape_ok(1, K)) return e;
+  if (!d_x || !d_ws || ldx < K) return W4A32_EINVAL;
+  if (!aligned(d_x, 16) || (ldx % 4) != 0 || !aligned(d_ws, 256)) return W4A32_EINVAL;
+  return from_hip(w4::launch_quant_lhs(d_x, M, K, ldx, static_cast<uint8_t*>(d_ws),
+                                       static_cast<hipStream_t>(stream)));
 }
 
 int w4a32_export_lhs(const void* d_ws, int M, int K, int8_t* d_aq, float* d_recip_scale,
@@ -163,7 +155,8 @@ int w4a32_export_lhs(const void* d_ws, int M, int K, int8_t* d_aq, float* d_reci
   const w4::WsGeom g = w4::ws_geom(M, K);
   const uint8_t* ws = static_cast<const uint8_t*>(d_ws);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e = hipMemcpyAsync(d_aq, ws + g.aq_off, (size_t)M * K, hipMemcpyDeviceToDevice, s);
+  hipError_t e = M > w4::kGemvMaxM ? w4::launch_lhs_bytes(ws, M, K, d_aq, s)
+                                   : hipMemcpyAsync(d_aq, ws + g.aq_off, (size_t)M * K, hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_recip_scale, ws + g.scale_off, (size_t)M * 4, hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess)
@@ -240,7 +233,7 @@ int w4a32_matmul(float* d_y, const float* d_x, const void* d_packed, void* d_ws,
     return from_hip(w4::launch_gemv_fused(d_y, d_x, K, static_cast<const uint8_t*>(d_packed), M, K,
                                           N, static_cast<hipStream_t>(stream)));
   }
-  if (int e = quantise(d_x, M, K, K, d_ws, false, stream)) return e;
+  if (int e = w4a32_quant_lhs(d_x, M, K, K, d_ws, stream)) return e;
   return w4a32_matmul_quantized(d_y, d_ws, d_packed, M, K, N, stream);
 }
 
@@ -258,7 +251,7 @@ int w4a32_matmul_ws(float* d_y, const float* d_x, const void* d_packed, void* d_
   if (!d_ws || ws_bytes < ws) return W4A32_EINVAL;
   const size_t parts = w4a32_splitk_scratch_bytes(M, K, N), parts_off = w4::round_up_sz(ws, 256);
   if (parts != 0 && ws_bytes >= parts_off + parts && aligned(d_y, 16)) {
-    if (int e = quantise(d_x, M, K, K, d_ws, false, stream)) return e;
+    if (int e = w4a32_quant_lhs(d_x, M, K, K, d_ws, stream)) return e;
     return w4a32_matmul_quantized_splitk(d_y, d_ws, d_packed, M, K, N, static_cast<uint8_t*>(d_ws) + parts_off,
                                          parts, stream);
   }
@@ -294,7 +287,7 @@ int w4a32_matmul_grouped(float* const* d_y, const float* d_x, const void* const*
   }
   // other sizes: quantise the rows once, then one launch of the f16 kernel over all the Linears
   // (M > 8) or one product per Linear
-  if (int e = quantise(d_x, M, K, K, d_ws, false, stream)) return e;
+  if (int e = w4a32_quant_lhs(d_x, M, K, K, d_ws, stream)) return e;
   return w4a32_matmul_quantized_grouped(d_y, d_ws, d_packed, N, count, M, K, stream);
 }
 

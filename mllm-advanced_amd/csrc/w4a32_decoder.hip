@@ -150,7 +150,6 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
 
   for (int l = 0; l < c->n_layers; ++l) {
     const w4a32_layer_weights& lw = w->layers[l];
-    if (fuse_rows && (!lw.attn_norm || !lw.ffn_norm)) return W4A32_EINVAL;
     float* kc = reinterpret_cast<float*>(st + g.kcache_off) + (size_t)l * g.cache_layer;
     float* vc = reinterpret_cast<float*>(st + g.vcache_off) + (size_t)l * g.cache_layer;
     // h += mlp output of the previous layer; xn = norm(h)
@@ -163,10 +162,10 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
           const uint8_t* down_prev = static_cast<const uint8_t*>(w->layers[l - 1].down);
           W4_TRY(from_hip(w4::launch_quant_lhs_norm_parts(h, gate, down_parts, w4::linear_bias(down_prev, H, I),
                                                           lw.attn_norm, c->rms_eps, h, M, H,
-                                                          static_cast<uint8_t*>(ws), s, false)));
+                                                          static_cast<uint8_t*>(ws), s)));
         } else {
-          W4_TRY(from_hip(w4::launch_quant_lhs_norm(h, l == 0 ? nullptr : delta, lw.attn_norm, c->rms_eps, h, M, H,
-                                                    static_cast<uint8_t*>(ws), s, false)));
+          W4_TRY(w4a32_quant_lhs_norm(h, l == 0 ? nullptr : delta, lw.attn_norm, c->rms_eps, h, M, H, ws,
+                                      stream));
         }
         W4_TRY(w4a32_matmul_quantized_grouped(ys, ws, ps, ns, 3, M, H, stream));
       } else {
@@ -207,8 +206,7 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
       const int ns[2] = {I, I};
       if (fuse_rows) {
         // gate, up, SiLU and the multiply in one launch: only silu(gate) * up is stored
-        W4_TRY(from_hip(w4::launch_quant_lhs_norm(h, delta, lw.ffn_norm, c->rms_eps, h, M, H, static_cast<uint8_t*>(ws), s,
-                                                  false)));
+        W4_TRY(w4a32_quant_lhs_norm(h, delta, lw.ffn_norm, c->rms_eps, h, M, H, ws, stream));
         W4_TRY(w4a32_matmul_quantized_silu_pair(act, ws, lw.gate, lw.up, M, H, I, stream));
       } else {
         W4_TRY(from_hip(w4::launch_rmsnorm(h, delta, lw.ffn_norm, M, H, c->rms_eps, h, xn, s)));
@@ -216,8 +214,12 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
       }
     }
     if (M > w4::kGemvMaxM) {
-      if (!fuse_rows) W4_TRY(from_hip(w4::launch_silu_mul(gate, up, act, (size_t)M * I, s)));
-      W4_TRY(from_hip(w4::launch_quant_lhs(act, M, I, I, static_cast<uint8_t*>(ws), s, false)));
+      if (fuse_rows) {
+        W4_TRY(w4a32_quant_lhs(act, M, I, I, ws, stream));
+      } else {
+        W4_TRY(from_hip(w4::launch_silu_mul(gate, up, act, (size_t)M * I, s)));
+        W4_TRY(w4a32_quant_lhs(act, M, I, I, ws, stream));
+      }
       // few output tiles, long K: split-K, with the partial sums in the gate and up buffers,
       // which are dead once the quantised rows of silu(gate) * up exist
       delta_in_parts = defer_sum && l + 1 < c->n_layers;

@@ -884,6 +884,10 @@ static hipError_t launch_gemm_i8(float* y, const uint8_t* ws, const uint8_t* pac
                                  int N, hipStream_t s) {
   const WeightGeom g = weight_geom(N, K);
   const WsGeom w = ws_geom(M, K);
+  if (M > kGemvMaxM) {  // into the place that the workspace has for them
+    int8_t* aq = const_cast<int8_t*>(reinterpret_cast<const int8_t*>(ws + w.aq_off));
+    if (hipError_t e = launch_lhs_bytes(ws, M, K, aq, s); e != hipSuccess) return e;
+  }
   dim3 grid((g.NT + kGemmI8Waves - 1) / kGemmI8Waves,
             (M + 16 * kGemmI8MTiles - 1) / (16 * kGemmI8MTiles));
   hipLaunchKernelGGL(gemm_i8_kernel, grid, dim3(64 * kGemmI8Waves), 0, s, y,

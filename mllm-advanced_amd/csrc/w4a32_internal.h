@@ -23,19 +23,19 @@ hipError_t launch_unpack_kai(const uint8_t* blob, int N, int K, int nr, int kr, 
                              uint16_t* scales, float* bias, hipStream_t s);
 
 // activations (every forward)
-// bytes, here and below: the int8 rows are wanted too. The f16 product (M > kGemvMaxM) reads the f16 copy alone, so a call that
-// quantises for it leaves a third of the stores out (us before / now: [512][8960] 8.3 / 7.5, [1024][5120] 8.2 / 7.6, [1024][1280] 5.2 / 4.3).
-hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s, bool bytes = true);
+hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s);
+// int8 values of the rows of a workspace for more than kGemvMaxM of them, which holds them as f16
+hipError_t launch_lhs_bytes(const uint8_t* ws, int M, int K, int8_t* out, hipStream_t s);
 // the quantiser with the operator that produces its rows in front (prefill sizes): residual add +
 // RMSNorm, or silu(gate) * up; K must satisfy quant_rows_fusable()
 bool quant_rows_fusable(int K);
 hipError_t launch_quant_lhs_norm(const float* h, const float* delta, const float* norm_w, float eps,
-                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s, bool bytes = true);
+                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s);
 // ... with delta = ((parts[0] + parts[1]) + ...) + bias, parts = [nparts][M][K] as launch_gemm_splitk leaves
 // them when it is given no output
 hipError_t launch_quant_lhs_norm_parts(const float* h, const float* parts, int nparts, const float* bias,
                                        const float* norm_w, float eps, float* h_out, int M, int K,
-                                       uint8_t* ws, hipStream_t s, bool bytes = true);
+                                       uint8_t* ws, hipStream_t s);
 hipError_t launch_quant_lhs_silu_mul(const float* gate, const float* up, int M, int K, uint8_t* ws,
                                      hipStream_t s);
 

@@ -35,8 +35,8 @@
 //   [4*Mp, 8*Mp)         i32  neg_zp[m]        (the "lhs offset" = -zero_point)
 //   hdr = round_up(8*Mp, 256)
 //   [hdr, hdr + Mp*K)    i8   a_q[m][k] row-major
-//   then, 256-aligned    f16  a_h = (a_q + neg_zp) exactly (|.| <= 255), only written when M > 8,
-//                        stored as 2 KiB chunks so that the f16 MFMA kernel reads whole
+//   then, 256-aligned    f16  a_h = (a_q + neg_zp) exactly (|.| <= 255), written instead of a_q when M > 8
+//                        (a_q's place is filled from it when the int8 product is asked for), stored as 2 KiB chunks so that the f16 MFMA kernel reads whole
 //                        chunks instead of 32 rows lying K*2 bytes apart:
 //                          chunk (mt, kb) = rows 32*mt..+31, k 32*kb..+31, at
 //                          (mt * K/32 + kb) * 2048, row-major inside: row i at i*64, its four

@@ -13,8 +13,11 @@ namespace w4 {
 constexpr int kLhsThreads = 256;
 
 // One workgroup per row. Pass 1 reads the row for min/max, pass 2 re-reads it (it is L2/L1
-// resident: at most 35 KB) and writes 8 int8 per thread per step, plus the f16 copy of
-// (a_q - zp), tiled in MFMA operand order, that the f16 MFMA prefill kernel consumes.
+// resident: at most 35 KB) and writes 8 values per thread per step: up to kGemvMaxM rows as int8, which
+// the decode kernels read, more rows as f16 (a_q - zp), tiled in MFMA operand order, for the f16 MFMA
+// prefill kernel. Both forms of those rows would be a third more stores (us with both / as it is:
+// [512][8960] 8.3 / 7.5, [1024][5120] 8.2 / 7.6, [1024][1280] 5.2 / 4.3); who wants their int8 values
+// has them made from the f16 ones (lhs_bytes_kernel).
 __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     const float* __restrict__ x, int K, int ldx, float* __restrict__ recip_out,
     int32_t* __restrict__ negzp_out, int8_t* __restrict__ aq, _Float16* __restrict__ ah) {
@@ -57,13 +60,12 @@ __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(f[e], p);
-    if (aq) {
+    if (!ah) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
-    }
-    if (ah) {
+    } else {
       // a_q - zp lies in [-255, 255]: exact in f16. Stored in the order a weight dword unpacks.
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
@@ -235,13 +237,12 @@ __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(v[r][e], p);
-    if (aq) {
+    if (!ah) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
-    }
-    if (ah) {
+    } else {
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
 #pragma unroll
@@ -259,11 +260,11 @@ constexpr int kQuantRowsMaxK = 8 * 8 * kLhsThreads;
 template <int SRC>
 static hipError_t launch_quant_rows(const float* a, const float* b, const float* norm_w, float eps,
                                     float* h_out, int M, int K, int lda, uint8_t* ws, hipStream_t s,
-                                    bool bytes, int nparts = 0, const float* part_bias = nullptr) {
+                                    int nparts = 0, const float* part_bias = nullptr) {
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = bytes || M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
+  int8_t* aq = M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   const int groups = (K + 8 * kLhsThreads - 1) / (8 * kLhsThreads);
 #define W4_LAUNCH_ROWS(R)                                                                          \
@@ -281,34 +282,69 @@ static hipError_t launch_quant_rows(const float* a, const float* b, const float*
 bool quant_rows_fusable(int K) { return K <= kQuantRowsMaxK; }
 
 hipError_t launch_quant_lhs_norm(const float* h, const float* delta, const float* norm_w, float eps,
-                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s, bool bytes) {
-  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s, bytes);
+                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s) {
+  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s);
 }
 
 // The same with delta = the sum of a split-K product's `nparts` scaled parts ([nparts][M][K]) + bias.
 hipError_t launch_quant_lhs_norm_parts(const float* h, const float* parts, int nparts, const float* bias,
                                        const float* norm_w, float eps, float* h_out, int M, int K,
-                                       uint8_t* ws, hipStream_t s, bool bytes) {
+                                       uint8_t* ws, hipStream_t s) {
   if (nparts < 1 || !parts || !bias) return hipErrorInvalidValue;
-  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, bytes, nparts, bias);
+  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, nparts, bias);
 }
 
 hipError_t launch_quant_lhs_silu_mul(const float* gate, const float* up, int M, int K, uint8_t* ws,
                                      hipStream_t s) {
-  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s, true);
+  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s);
 }
 
-hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s, bool bytes) {
+hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s) {
   if (K <= kQuantRowsMaxK) {
-    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s, bytes);
+    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s);
   }
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = bytes || M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
+  int8_t* aq = M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   hipLaunchKernelGGL(quant_lhs_kernel, dim3(M), dim3(kLhsThreads), 0, s, x, K, ldx, recip, negzp,
                      aq, ah);
+  return hipGetLastError();
+}
+
+// The int8 values of rows that were stored as f16 (a_q - zp): exact, both are whole numbers within 255.
+// A thread per eight values. Runs for the inspection of a workspace and in front of the int8 product only.
+__global__ __launch_bounds__(kLhsThreads) void lhs_bytes_kernel(const _Float16* __restrict__ ah,
+                                                                const int32_t* __restrict__ negzp, int M, int K,
+                                                                int8_t* __restrict__ out) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  const size_t n = (size_t)blockIdx.x * kLhsThreads + threadIdx.x, per_row = K / 8;
+  if (n >= M * per_row) return;
+  const int m = (int)(n / per_row), i = 8 * (int)(n % per_row);
+  const size_t chunk = (size_t)(m >> 5) * (K >> 5) + (i >> 5);
+  const h8 hv = *reinterpret_cast<const h8*>(ah + chunk * 1024 + (m & 31) * 32 + ((i >> 3) & 3) * 8);
+  int q[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) q[kHalfOrder[e]] = (int)(float)hv[e] - negzp[m];
+  int8_t* dst = out + (size_t)m * K + i;
+  if ((reinterpret_cast<uintptr_t>(out) & 7) == 0) {
+    uint2 packed;
+    packed.x = pack4(q);
+    packed.y = pack4(q + 4);
+    *reinterpret_cast<uint2*>(dst) = packed;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dst[e] = (int8_t)q[e];
+  }
+}
+
+hipError_t launch_lhs_bytes(const uint8_t* ws, int M, int K, int8_t* out, hipStream_t s) {
+  const WsGeom g = ws_geom(M, K);
+  const size_t blocks = ((size_t)M * (K / 8) + kLhsThreads - 1) / kLhsThreads;
+  hipLaunchKernelGGL(lhs_bytes_kernel, dim3((unsigned)blocks), dim3(kLhsThreads), 0, s,
+                     reinterpret_cast<const _Float16*>(ws + g.ah_off), reinterpret_cast<const int32_t*>(ws + g.off_off), M, K,
+                     out);
   return hipGetLastError();
 }
 

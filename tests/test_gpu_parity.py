@@ -148,6 +148,29 @@ def test_quant_lhs_bit_exact(pkg, orc, m, k, seed):
     assert np.array_equal(host(aq), aq_ref)
 
 
+# a whole call of more than eight rows leaves them quantised in its workspace, for whatever is done with
+# them next (k = 16416: too long for the quantiser that holds a row in registers)
+@pytest.mark.parametrize("m,k", [(9, 32), (33, 1536), (300, 96), (10, 16416)])
+def test_rows_in_the_workspace_of_a_whole_call(pkg, orc, m, k):
+    n = 48
+    x = make_acts(m, k, seed=m, outlier_frac=0.05)
+    u4, sc = orc.quant_rhs(make_weights(n, k, seed=k))
+    packed = pkg.repack_native(dev(u4), dev(sc.view(np.int16)), None, n, k)
+    aq_ref, recip_ref, negzp_ref, _ = orc.quant_lhs(x)
+    ws = torch.zeros(pkg.workspace_bytes(m, k), dtype=torch.uint8, device="cuda")
+    y = pkg.matmul(dev(x), packed, n, ws=ws)
+    off_by_one = torch.zeros(m * k + 1, dtype=torch.int8, device="cuda")
+    recip, negzp = torch.empty(m, dtype=torch.float32, device="cuda"), torch.empty(m, dtype=torch.int32, device="cuda")
+    for aq in (off_by_one[:-1], off_by_one[1:]):
+        assert pkg.lib().w4a32_export_lhs(ws.data_ptr(), m, k, aq.data_ptr(), recip.data_ptr(), negzp.data_ptr(), 0) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(host(aq).reshape(m, k), aq_ref)
+    assert np.array_equal(host(negzp), negzp_ref)
+    assert np.array_equal(host(recip).view(np.uint32), recip_ref.view(np.uint32))
+    again = pkg.matmul_quantized(ws, packed, m, k, n, kernel=pkg.KERNEL_GEMM_I8)
+    assert max_abs_rel(host(again), host(y)) < TIGHT
+
+
 # ------------------------------------------------------------------------- products
 
 def run_linear(pkg, orc, m, k, n, has_bias, wseed=0, xseed=1, outliers=0.0, threads=8, rows=None):
