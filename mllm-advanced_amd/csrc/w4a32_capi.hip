@@ -155,8 +155,8 @@ int w4a32_export_lhs(const void* d_ws, int M, int K, int8_t* d_aq, float* d_reci
   const w4::WsGeom g = w4::ws_geom(M, K);
   const uint8_t* ws = static_cast<const uint8_t*>(d_ws);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e = M > w4::kGemvMaxM ? w4::launch_lhs_bytes(ws, M, K, d_aq, s)
-                                   : hipMemcpyAsync(d_aq, ws + g.aq_off, (size_t)M * K, hipMemcpyDeviceToDevice, s);
+  hipError_t e = w4::ws_has_bytes(M) ? hipMemcpyAsync(d_aq, ws + g.aq_off, (size_t)M * K, hipMemcpyDeviceToDevice, s)
+                                     : w4::launch_lhs_bytes(ws, M, K, d_aq, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_recip_scale, ws + g.scale_off, (size_t)M * 4, hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess)

@@ -884,7 +884,7 @@ static hipError_t launch_gemm_i8(float* y, const uint8_t* ws, const uint8_t* pac
                                  int N, hipStream_t s) {
   const WeightGeom g = weight_geom(N, K);
   const WsGeom w = ws_geom(M, K);
-  if (M > kGemvMaxM) {  // into the place that the workspace has for them
+  if (!ws_has_bytes(M)) {  // into the place that the workspace has for them
     int8_t* aq = const_cast<int8_t*>(reinterpret_cast<const int8_t*>(ws + w.aq_off));
     if (hipError_t e = launch_lhs_bytes(ws, M, K, aq, s); e != hipSuccess) return e;
   }

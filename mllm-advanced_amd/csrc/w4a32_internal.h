@@ -24,7 +24,7 @@ hipError_t launch_unpack_kai(const uint8_t* blob, int N, int K, int nr, int kr, 
 
 // activations (every forward)
 hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s);
-// int8 values of the rows of a workspace for more than kGemvMaxM of them, which holds them as f16
+// int8 values of the rows of a workspace that holds them as f16 alone (!ws_has_bytes(M))
 hipError_t launch_lhs_bytes(const uint8_t* ws, int M, int K, int8_t* out, hipStream_t s);
 // the quantiser with the operator that produces its rows in front (prefill sizes): residual add +
 // RMSNorm, or silu(gate) * up; K must satisfy quant_rows_fusable()

@@ -34,9 +34,9 @@
 //   [0, 4*Mp)            f32  recip_scale[m]   (the "lhs scale" applied to the output)
 //   [4*Mp, 8*Mp)         i32  neg_zp[m]        (the "lhs offset" = -zero_point)
 //   hdr = round_up(8*Mp, 256)
-//   [hdr, hdr + Mp*K)    i8   a_q[m][k] row-major
-//   then, 256-aligned    f16  a_h = (a_q + neg_zp) exactly (|.| <= 255), written instead of a_q when M > 8
-//                        (a_q's place is filled from it when the int8 product is asked for), stored as 2 KiB chunks so that the f16 MFMA kernel reads whole
+//   [hdr, hdr + Mp*K)    i8   a_q[m][k] row-major, only written when M <= 32
+//   then, 256-aligned    f16  a_h = (a_q + neg_zp) exactly (|.| <= 255), only written when M > 8,
+//                        stored as 2 KiB chunks so that the f16 MFMA kernel reads whole
 //                        chunks instead of 32 rows lying K*2 bytes apart:
 //                          chunk (mt, kb) = rows 32*mt..+31, k 32*kb..+31, at
 //                          (mt * K/32 + kb) * 2048, row-major inside: row i at i*64, its four
@@ -106,6 +106,10 @@ W4_HD WsGeom ws_geom(int M, int K) {
   g.total_bytes = g.ah_off + (M > kGemvMaxM ? (size_t)g.Mp * K * 2 : 0);
   return g;
 }
+
+// Whether the int8 values are among what M quantised rows leave: a workspace of up to 32 rows has one layout, and
+// its first rows are decode kernels' operands whatever M it was filled with.
+W4_HD bool ws_has_bytes(int M) { return M <= 32; }
 
 // Nibble position (0..7) inside a tile dword of the weight at k offset e (0..7) in its 8-group.
 W4_HD int nibble_pos(int e) { return e < 4 ? 2 * e : 2 * (e - 4) + 1; }

@@ -13,11 +13,11 @@ namespace w4 {
 constexpr int kLhsThreads = 256;
 
 // One workgroup per row. Pass 1 reads the row for min/max, pass 2 re-reads it (it is L2/L1
-// resident: at most 35 KB) and writes 8 values per thread per step: up to kGemvMaxM rows as int8, which
-// the decode kernels read, more rows as f16 (a_q - zp), tiled in MFMA operand order, for the f16 MFMA
-// prefill kernel. Both forms of those rows would be a third more stores (us with both / as it is:
-// [512][8960] 8.3 / 7.5, [1024][5120] 8.2 / 7.6, [1024][1280] 5.2 / 4.3); who wants their int8 values
-// has them made from the f16 ones (lhs_bytes_kernel).
+// resident: at most 35 KB) and writes 8 values per thread per step: as int8 (aq), which the decode
+// kernels read, where the workspace keeps int8 values (ws_has_bytes), and from kGemvMaxM + 1 rows on as
+// f16 (a_q - zp; ah), tiled in MFMA operand order, for the f16 MFMA prefill kernel. Both forms of many rows
+// would be a third more stores (us with both / with f16 alone: [512][8960] 8.3 / 7.5, [1024][5120] 8.2 /
+// 7.6, [1024][1280] 5.2 / 4.3); who wants their int8 values has them made from the f16 ones (lhs_bytes_kernel).
 __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     const float* __restrict__ x, int K, int ldx, float* __restrict__ recip_out,
     int32_t* __restrict__ negzp_out, int8_t* __restrict__ aq, _Float16* __restrict__ ah) {
@@ -60,12 +60,13 @@ __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(f[e], p);
-    if (!ah) {
+    if (aq) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
-    } else {
+    }
+    if (ah) {
       // a_q - zp lies in [-255, 255]: exact in f16. Stored in the order a weight dword unpacks.
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
@@ -237,12 +238,13 @@ __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(v[r][e], p);
-    if (!ah) {
+    if (aq) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
-    } else {
+    }
+    if (ah) {
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
 #pragma unroll
@@ -264,7 +266,7 @@ static hipError_t launch_quant_rows(const float* a, const float* b, const float*
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
+  int8_t* aq = ws_has_bytes(M) ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   const int groups = (K + 8 * kLhsThreads - 1) / (8 * kLhsThreads);
 #define W4_LAUNCH_ROWS(R)                                                                          \
@@ -306,7 +308,7 @@ hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, 
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = M <= kGemvMaxM ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
+  int8_t* aq = ws_has_bytes(M) ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
   _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
   hipLaunchKernelGGL(quant_lhs_kernel, dim3(M), dim3(kLhsThreads), 0, s, x, K, ldx, recip, negzp,
                      aq, ah);

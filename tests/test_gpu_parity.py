@@ -171,6 +171,30 @@ def test_rows_in_the_workspace_of_a_whole_call(pkg, orc, m, k):
     assert max_abs_rel(host(again), host(y)) < TIGHT
 
 
+# a workspace of up to 32 rows has one layout: a few of its rows are multiplied, and looked at, as if they alone
+# had been quantised into it
+@pytest.mark.parametrize("m,k", [(9, 64), (20, 1536), (32, 96), (10, 16416)])
+def test_first_rows_of_a_workspace(pkg, orc, m, k):
+    n = 48
+    x = make_acts(m, k, seed=m, outlier_frac=0.05)
+    u4, sc = orc.quant_rhs(make_weights(n, k, seed=k))
+    packed = pkg.repack_native(dev(u4), dev(sc.view(np.int16)), None, n, k)
+    aq_ref, recip_ref, negzp_ref, _ = orc.quant_lhs(x)
+    ref = orc.linear(x, u4, sc)
+    for fill in (lambda ws: pkg.lib().w4a32_quant_lhs(xd.data_ptr(), m, k, k, ws.data_ptr(), 0),
+                 lambda ws: pkg.matmul(xd, packed, n, ws=ws)):
+        xd, ws = dev(x), torch.full((pkg.workspace_bytes(m, k),), 0x55, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        fill(ws)
+        torch.cuda.synchronize()
+        for rows in (1, 5, 8):
+            y = host(pkg.matmul_quantized(ws, packed, rows, k, n))
+            assert max_abs_rel(y, ref[:rows]) < TIGHT, rows
+            aq, recip, negzp = pkg.export_lhs(ws, rows, k)
+            assert np.array_equal(host(aq), aq_ref[:rows]) and np.array_equal(host(negzp), negzp_ref[:rows])
+            assert np.array_equal(host(recip).view(np.uint32), recip_ref[:rows].view(np.uint32))
+
+
 # ------------------------------------------------------------------------- products
 
 def run_linear(pkg, orc, m, k, n, has_bias, wseed=0, xseed=1, outliers=0.0, threads=8, rows=None):
