@@ -109,7 +109,11 @@ int w4a32_unpack_kai(const void* d_kai_blob, int N, int K, int nr, int kr, int s
 /* Per-row asymmetric int8 quantisation of the activations into the workspace
  * (scale, offset, int8 values), bit-exact with the scalar model
  * tests/Arm/KaiLinearTest.hpp:163-230. Replaces the kai_run_lhs_quant_pack_qai8dxp_f32
- * call (kai_linear.cpp:358-362). ldx = row stride of d_x in elements. */
+ * call (kai_linear.cpp:358-362). ldx = row stride of d_x in elements. The values of more than 32 rows
+ * are kept as f16 (value - zero point), exactly; w4a32_export_lhs() returns them as int8 at any M.
+ * The products and w4a32_export_lhs() only read a workspace. They take the M that it was filled with: its layout
+ * depends on M rounded up to 32 (fewer rows of the same 32 are its first ones, but from one to
+ * W4A32_GEMV_MAX_M quantised rows only as many can be read). */
 int w4a32_quant_lhs(const float* d_x, int M, int K, int ldx, void* d_ws, void* stream);
 
 /* Copies the quantised rows out of a workspace for inspection: int8 [M][K], f32 [M]
@@ -128,7 +132,7 @@ int w4a32_matmul_quantized(float* d_y, const void* d_ws, const void* d_packed, i
  * (KaiLinear_f32_qai8dxp_qsi4c32p_mxk_nxk::Tiles, kai_linear.hpp:76-118). */
 #define W4A32_KERNEL_AUTO 0       /* M <= 8: GEMV, else f16 MFMA */
 #define W4A32_KERNEL_GEMV 1       /* v_dot4 decode kernel, M <= 8 */
-#define W4A32_KERNEL_GEMM_I8 2    /* int8 MFMA, exact int32 block sums, any M; M > 8: makes the int8 rows in d_ws first */
+#define W4A32_KERNEL_GEMM_I8 2    /* int8 MFMA, exact int32 block sums, any M */
 #define W4A32_KERNEL_GEMM_F16 3   /* f16 MFMA on exact f16 operands, M > 8; tile shape by size */
 /* The f16 kernel with one named tile shape, W4A32_KERNEL_GEMM_F16_TILE0 + i:
  * i = 0: 64 x 64, 1: 128 x 64, 2: 128 x 128, 3: 256 x 128 (rows x columns per workgroup),

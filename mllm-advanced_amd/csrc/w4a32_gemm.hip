@@ -18,7 +18,9 @@
 // (tests/Arm/KaiLinearTest.hpp:342-372); each is converted and scaled in f32 by the block's
 // scale. A wavefront owns one 16-row weight tile row and a 64-row slab of activations:
 // dword d of its 128-bit weight load is directly the B operand (two mask ops), the A operand
-// is 8 consecutive int8 of an activation row.
+// is 8 consecutive int8 of an activation row. A workspace of more than 32 rows holds a_q - zp in f16 alone,
+// from which the operand is made in registers: as a check of the other kernel this one is then independent in
+// the product, not in its rows (those have tests of their own).
 #include "w4a32_internal.h"
 
 #include <type_traits>
@@ -30,10 +32,25 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int kGemmI8MTiles = 4;   // 16-row activation tiles per wavefront
 constexpr int kGemmI8Waves = 4;    // weight tile rows per workgroup
 
+// Eight consecutive a_q from the f16 a_q - zp in the order of kHalfOrder: with zp + 128 + 1024 added they are
+// 1024 + (a_q + 128), whose low byte is a_q + 128 (all of it whole numbers below 2048, exact in f16).
+__device__ __forceinline__ long int8_of_halves(const uint4 h, uint32_t zp_bias) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  auto shifted = [&](uint32_t v) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, v) + __builtin_bit_cast(h2, zp_bias));
+  };
+  // h.x: k 0, 2; h.y: 4, 6; h.z: 1, 3; h.w: 5, 7
+  const uint32_t lo = __builtin_amdgcn_perm(shifted(h.z), shifted(h.x), 0x06020400u) ^ 0x80808080u;
+  const uint32_t hi = __builtin_amdgcn_perm(shifted(h.w), shifted(h.y), 0x06020400u) ^ 0x80808080u;
+  return (long)(((unsigned long)hi << 32) | lo);
+}
+
+// kHalves: the rows come from ah, else from aq
+template <bool kHalves>
 __global__ __launch_bounds__(64 * kGemmI8Waves) void gemm_i8_kernel(
-    float* __restrict__ y, const int8_t* __restrict__ aq, const float* __restrict__ recip,
-    const int32_t* __restrict__ negzp, const uint8_t* __restrict__ packed, int M, int Mp, int N,
-    int K, int NT, int KC, const float* __restrict__ rsum, const float* __restrict__ bias) {
+    float* __restrict__ y, const int8_t* __restrict__ aq, const _Float16* __restrict__ ah,
+    const float* __restrict__ recip, const int32_t* __restrict__ negzp, const uint8_t* __restrict__ packed, int M,
+    int Mp, int N, int K, int NT, int KC, const float* __restrict__ rsum, const float* __restrict__ bias) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int g = lane >> 4, j = lane & 15;
   const int nt = blockIdx.x * kGemmI8Waves + wave;
@@ -45,11 +62,16 @@ __global__ __launch_bounds__(64 * kGemmI8Waves) void gemm_i8_kernel(
   // A rows this lane feeds (row = lane % 16 of each 16-row tile); rows past Mp-1 are clamped,
   // their products land in output rows that are never stored.
   const int8_t* a_row[kGemmI8MTiles];
+  const _Float16* h_row[kGemmI8MTiles];
+  uint32_t zp_bias[kGemmI8MTiles];
 #pragma unroll
   for (int mt = 0; mt < kGemmI8MTiles; ++mt) {
     int r = m0 + 16 * mt + j;
     r = r < Mp ? r : Mp - 1;
     a_row[mt] = aq + (size_t)r * K + 8 * g;
+    h_row[mt] = ah + (size_t)(r >> 5) * (K >> 5) * 1024 + (r & 31) * 32 + 8 * g;  // chunks of 32 rows x 32 k
+    const _Float16 bias16 = (_Float16)(float)(kHalves ? 1024 + 128 - negzp[r] : 0);
+    zp_bias[mt] = __builtin_bit_cast(unsigned short, bias16) * 0x00010001u;
   }
 
   float acc[kGemmI8MTiles][4];
@@ -72,9 +94,16 @@ __global__ __launch_bounds__(64 * kGemmI8Waves) void gemm_i8_kernel(
       const uint32_t lo = (wv[d] << 4) & 0xF0F0F0F0u;
       const uint32_t hi = wv[d] & 0xF0F0F0F0u;
       const long b64 = (long)(((unsigned long)hi << 32) | lo);
+      uint4 halves[kGemmI8MTiles];
+      if constexpr (kHalves) {  // all requested before the first is used
+#pragma unroll
+        for (int mt = 0; mt < kGemmI8MTiles; ++mt) halves[mt] = *reinterpret_cast<const uint4*>(h_row[mt] + 32 * kk);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int mt = 0; mt < kGemmI8MTiles; ++mt) {
-        const long a64 = *reinterpret_cast<const long*>(a_row[mt] + kk);
+        const long a64 = kHalves ? int8_of_halves(halves[mt], zp_bias[mt])
+                                 : *reinterpret_cast<const long*>(a_row[mt] + kk);
         v4i c = {0, 0, 0, 0};
         c = __builtin_amdgcn_mfma_i32_16x16x32_i8(a64, b64, c, 0, 0, 0);
 #pragma unroll
@@ -884,14 +913,12 @@ static hipError_t launch_gemm_i8(float* y, const uint8_t* ws, const uint8_t* pac
                                  int N, hipStream_t s) {
   const WeightGeom g = weight_geom(N, K);
   const WsGeom w = ws_geom(M, K);
-  if (!ws_has_bytes(M)) {  // into the place that the workspace has for them
-    int8_t* aq = const_cast<int8_t*>(reinterpret_cast<const int8_t*>(ws + w.aq_off));
-    if (hipError_t e = launch_lhs_bytes(ws, M, K, aq, s); e != hipSuccess) return e;
-  }
   dim3 grid((g.NT + kGemmI8Waves - 1) / kGemmI8Waves,
             (M + 16 * kGemmI8MTiles - 1) / (16 * kGemmI8MTiles));
-  hipLaunchKernelGGL(gemm_i8_kernel, grid, dim3(64 * kGemmI8Waves), 0, s, y,
+  auto kern = ws_has_bytes(M) ? gemm_i8_kernel<false> : gemm_i8_kernel<true>;
+  hipLaunchKernelGGL(kern, grid, dim3(64 * kGemmI8Waves), 0, s, y,
                      reinterpret_cast<const int8_t*>(ws + w.aq_off),
+                     reinterpret_cast<const _Float16*>(ws + w.ah_off),
                      reinterpret_cast<const float*>(ws + w.scale_off),
                      reinterpret_cast<const int32_t*>(ws + w.off_off), packed, M, w.Mp, N, K, g.NT,
                      g.KC, reinterpret_cast<const float*>(packed + g.rsum_off),

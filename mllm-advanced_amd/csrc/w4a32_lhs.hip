@@ -316,7 +316,7 @@ hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, 
 }
 
 // The int8 values of rows that were stored as f16 (a_q - zp): exact, both are whole numbers within 255.
-// A thread per eight values. Runs for the inspection of a workspace and in front of the int8 product only.
+// A thread per eight values. Runs for the inspection of a workspace only.
 __global__ __launch_bounds__(kLhsThreads) void lhs_bytes_kernel(const _Float16* __restrict__ ah,
                                                                 const int32_t* __restrict__ negzp, int M, int K,
                                                                 int8_t* __restrict__ out) {

@@ -195,6 +195,26 @@ def test_first_rows_of_a_workspace(pkg, orc, m, k):
             assert np.array_equal(host(recip).view(np.uint32), recip_ref[:rows].view(np.uint32))
 
 
+# the int8 product takes a workspace as the others do: it leaves it as it is, so that products on several streams can share
+# it (rows of every kind of zero point; a k that ends inside of a weight tile; 32 rows are the last that are kept as int8)
+@pytest.mark.parametrize("m,k", [(32, 96), (33, 160), (70, 1536), (300, 32)])
+def test_int8_product_only_reads_its_workspace(pkg, orc, m, k):
+    n = 50
+    x = make_acts(m, k, seed=m, outlier_frac=0.05)
+    x[-12:] = special_acts(k)
+    u4, sc = orc.quant_rhs(make_weights(n, k, seed=k))
+    packed = pkg.repack_native(dev(u4), dev(sc.view(np.int16)), None, n, k)
+    ws = torch.full((pkg.workspace_bytes(m, k),), 0x55, dtype=torch.uint8, device="cuda")
+    f16 = pkg.matmul(dev(x), packed, n, ws=ws)
+    before = ws.clone()
+    y = pkg.matmul_quantized(ws, packed, m, k, n, kernel=pkg.KERNEL_GEMM_I8)
+    assert torch.equal(ws, before)
+    ref = orc.linear(x, u4, sc)
+    for got in (host(y), host(f16)):  # rows of very different size: each by itself
+        assert max(max_abs_rel(got[i], ref[i]) for i in range(m) if np.abs(ref[i]).max() > 0) < TIGHT
+        assert not got[np.abs(ref).max(1) == 0].any()
+
+
 # ------------------------------------------------------------------------- products
 
 def run_linear(pkg, orc, m, k, n, has_bias, wseed=0, xseed=1, outliers=0.0, threads=8, rows=None):
