@@ -17,6 +17,7 @@
 //
 // State layout in a sequence's state: transposed, [vdim rounded up to 16][D].
 #include <algorithm>
+#include <type_traits>
 
 #include "w4a32_layered.h"
 #include "w4a32_layered_kernels.h"
@@ -442,73 +443,111 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(float* __restrict__ state
   }
 }
 
-// grid (chunks, heads), 256 threads; wavefront w: tokens 16 w .. The operands of 16 value dimensions, D / 16 + 4 kilobytes of state and U, come
-// through LDS once for all four wavefronts, the next ones meanwhile through registers: read by each wavefront for itself, from two sets of
-// registers, 28 heads of 128 x 128 in 32 chunks took 60 us, now 45 (129 MB of scratch: 26 us at the rate of a copy).
-template <int D, typename T>
-__global__ __launch_bounds__(256, D <= 128 ? 4 : 2) void rec_out_kernel(const RecGeom g, const float* __restrict__ raw,
-                                                                        const float* __restrict__ scratch, T* __restrict__ out,
-                                                                        int ldo, int M) {
-  constexpr int KQ = D / 4, NT = D / 16, kPieces = KQ / 4 + 4, kPer = (kPieces + 3) / 4;
-  __shared__ f32x4 s_op[2][kPieces][64];
+// grid (chunks, heads), 256 threads; wavefront w: tokens 16 w .. The operands of 16 value dimensions are D / 16 + 4 kilobytes of state and
+// U. With kShared they come through LDS once for all four wavefronts, the next ones meanwhile through registers; without it each wavefront
+// reads them for itself, into two sets of registers in turn: the same bits, without a barrier and an LDS round trip per step, which nothing
+// hides where a workgroup has its CU to itself. 28 heads of 128 x 128 in 32 chunks (129 MB of scratch: 26 us at the rate of a copy) take 45 us
+// with kShared, 61 without. (out_shared() says which is launched.)
+template <int D, typename T, bool kShared>
+__global__ __launch_bounds__(256, !kShared ? 1 : D <= 128 ? 4 : 2) void rec_out_kernel(const RecGeom g, const float* __restrict__ raw,
+                                                                                       const float* __restrict__ scratch,
+                                                                                       T* __restrict__ out, int ldo, int M) {
+  constexpr int KQ = D / 4, NT = D / 16, kPieces = KQ / 4 + 4;
   const int chunk = blockIdx.x, h = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
   const int dv16 = (g.vdim + 15) & ~15;
   const ChunkOff off = chunk_off(D, dv16);
   const float* p = scratch + ((size_t)h * gridDim.x + chunk) * off.total;
   auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
-
-  f32x4 piece[kPer];
-  auto fetch = [&](int nt) __attribute__((always_inline)) {
-    const int t = min(nt, dv16 / 16 - 1);
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int n = min(wave + 4 * i, kPieces - 1);
-      const float* src = n < KQ / 4 ? p + off.s + (size_t)(t * (KQ / 4) + n) * 256 : p + off.u + (size_t)(t * 4 + n - KQ / 4) * 256;
-      piece[i] = ld(src + 4 * lane);
-    }
-  };
-  auto stash = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if (kPieces % 4 == 0 || wave + 4 * i < kPieces) s_op[buf][wave + 4 * i][lane] = piece[i];
-  };
-  fetch(0);
   f32x4 q[KQ / 4], a[4];
+  auto fetch_rows = [&] __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < KQ / 4; ++i) q[i] = ld(p + off.q + ((wave * (KQ / 4) + i) * 64 + lane) * 4);
+    for (int i = 0; i < KQ / 4; ++i) q[i] = ld(p + off.q + ((wave * (KQ / 4) + i) * 64 + lane) * 4);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) a[i] = ld(p + off.a + ((wave * 4 + i) * 64 + lane) * 4);
-  stash(0);
-  fetch(1);
-
+    for (int i = 0; i < 4; ++i) a[i] = ld(p + off.a + ((wave * 4 + i) * 64 + lane) * 4);
+  };
   f32x4 o[NT];
   float ss[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    if (16 * nt >= dv16) break;
-    // what every wavefront has written and read in LDS so far is done; loads from memory stay on their way
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+  auto multiply = [&](auto piece) __attribute__((always_inline)) {
     f32x4 o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      const f32x4 x = i < KQ / 4 ? q[i < KQ / 4 ? i : 0] : a[i < KQ / 4 ? 0 : i - KQ / 4], y = s_op[nt & 1][i][lane];
+      const f32x4 x = i < KQ / 4 ? q[i < KQ / 4 ? i : 0] : a[i < KQ / 4 ? 0 : i - KQ / 4], y = piece(i);
       o0 = mfma4(x[0], y[0], o0);
       o1 = mfma4(x[1], y[1], o1);
       o0 = mfma4(x[2], y[2], o0);
       o1 = mfma4(x[3], y[3], o1);
     }
-    if (nt + 1 < NT) {
-      stash((nt + 1) & 1);
-      if (nt + 2 < NT) fetch(nt + 2);
-    }
-    o0 = o0 + o1;
+    return o0 + o1;
+  };
+  auto keep_sum = [&](int nt) __attribute__((always_inline)) {
     const float keep = 16 * nt + col < g.vdim ? 1.0f : 0.0f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ss[r] = __fmaf_rn(o0[r] * keep, o0[r], ss[r]);
-    o[nt] = o0;
+    for (int r = 0; r < 4; ++r) ss[r] = __fmaf_rn(o[nt][r] * keep, o[nt][r], ss[r]);
+  };
+
+  if constexpr (kShared) {
+    constexpr int kPer = (kPieces + 3) / 4;
+    __shared__ f32x4 s_op[2][kPieces][64];
+    f32x4 piece[kPer];
+    auto fetch = [&](int nt) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int t = min(nt, dv16 / 16 - 1), n = min(wave + 4 * i, kPieces - 1);
+        const float* src = n < KQ / 4 ? p + off.s + (size_t)(t * (KQ / 4) + n) * 256 : p + off.u + (size_t)(t * 4 + n - KQ / 4) * 256;
+        piece[i] = ld(src + 4 * lane);
+      }
+    };
+    auto stash = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (kPieces % 4 == 0 || wave + 4 * i < kPieces) s_op[buf][wave + 4 * i][lane] = piece[i];
+    };
+    fetch(0);
+    fetch_rows();
+    stash(0);
+    fetch(1);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      if (16 * nt >= dv16) break;
+      // what every wavefront has written and read in LDS so far is done; loads from memory stay on their way
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const f32x4 sum = multiply([&](int i) { return s_op[nt & 1][i][lane]; });
+      if (nt + 1 < NT) {
+        stash((nt + 1) & 1);
+        if (nt + 2 < NT) fetch(nt + 2);
+      }
+      o[nt] = sum;
+      keep_sum(nt);
+    }
+  } else {
+    f32x4 ops0[kPieces], ops1[kPieces];
+    auto fetch = [&](int nt, f32x4(&ops)[kPieces]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const int t = min(nt, dv16 / 16 - 1);
+        ops[i] = i < KQ / 4 ? ld(p + off.s + ((t * (KQ / 4) + i) * 64 + lane) * 4) : ld(p + off.u + ((t * 4 + i - KQ / 4) * 64 + lane) * 4);
+      }
+    };
+    auto step = [&](int nt, const f32x4(&ops)[kPieces]) __attribute__((always_inline)) {
+      o[nt] = multiply([&](int i) { return ops[i]; });
+      keep_sum(nt);
+    };
+    fetch_rows();
+    fetch(0, ops0);
+#pragma unroll
+    for (int nt = 0; nt < NT; nt += 2) {
+      if (16 * nt < dv16) {
+        fetch(nt + 1, ops1);
+        step(nt, ops0);
+      }
+      if (16 * (nt + 1) < dv16) {
+        fetch(nt + 2, ops0);
+        step(nt + 1, ops1);
+      }
+    }
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -636,6 +675,11 @@ __global__ __launch_bounds__(256) void rec_decode_kernel(const RecGeom g, const 
   }
 }
 
+// Whether the output's operands come through LDS: where a CU has more than one of its workgroups. Us through LDS / without, D = 128: 8 heads x 4
+// chunks 14.6 / 13.0, 16 x 16 17.4 / 16.1, 48 x 8 24.4 / 32.8, 16 x 32 26.4 / 34.0; D = 256: 16 x 16 41.2 / 37.2, 48 x 8 62.9 / 72.1; D = 64: 28 x
+// 2 7.6 / 7.3, 28 x 8 equal, 48 x 8 11.8 / 13.8. D = 32 (two steps): 0.3 to 0.6 us better through LDS throughout.
+bool out_shared(int workgroups) { return workgroups > 256; }
+
 template <int D, bool kDelta>
 hipError_t prefill_d(int dtype, const RecGeom& g, const float* raw, const float* cx, int ldcx, float* state,
                      float* scratch, void* out, int ldo, int M, int pos0, hipStream_t s) {
@@ -651,13 +695,15 @@ hipError_t prefill_d(int dtype, const RecGeom& g, const float* raw, const float*
   hipLaunchKernelGGL((rec_scan_kernel<D, kDelta>), dim3(8, dv16 / 16, (g.heads + 7) / 8), dim3(256), 0, s, state,
                      scratch, g.heads, dv16, chunks, pos0 == 0 ? 1 : 0);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (dtype == W4A32_LAYERED_BF16) {
-    hipLaunchKernelGGL((rec_out_kernel<D, __bf16>), dim3(chunks, g.heads), dim3(256), 0, s, g, raw, scratch,
-                       static_cast<__bf16*>(out), ldo, M);
-  } else {
-    hipLaunchKernelGGL((rec_out_kernel<D, float>), dim3(chunks, g.heads), dim3(256), 0, s, g, raw, scratch,
-                       static_cast<float*>(out), ldo, M);
-  }
+  auto output = [&](auto* to) {
+    using T = std::remove_pointer_t<decltype(to)>;
+    auto kern = rec_out_kernel<D, T, true>;
+    if constexpr (D >= 64)
+      if (!out_shared(chunks * g.heads)) kern = rec_out_kernel<D, T, false>;
+    hipLaunchKernelGGL(kern, dim3(chunks, g.heads), dim3(256), 0, s, g, raw, scratch, to, ldo, M);
+  };
+  if (dtype == W4A32_LAYERED_BF16) output(static_cast<__bf16*>(out));
+  else output(static_cast<float*>(out));
   return hipGetLastError();
 }
 
