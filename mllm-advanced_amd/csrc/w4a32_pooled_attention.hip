@@ -745,13 +745,106 @@ __global__ __launch_bounds__(64 * kTileSets * kTileWaves, 2) void attn_tile_kern
 }
 
 // ---------------------------------------------------------------------------------------------
+// One query of a head by a wavefront, everything f32: a lane per key for the scores, a lane per value dimension for
+// the sums. Only the keys that the query sees are read.
+constexpr int kRowQuery = W4A32_LAYERED_MAX_DIM + W4A32_LAYERED_MAX_ROT_PART, kRowLds = kRowQuery + 64;  // floats
+
+// what the wavefront has written to LDS so far is what its lanes read from here on
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename T>
+__device__ __forceinline__ void attn_row(float* s_q, int h, int m, int lane, const T* __restrict__ q, const T* __restrict__ kc,
+                                         const T* __restrict__ vt, const T* __restrict__ kp, const T* __restrict__ vpt,
+                                         T* __restrict__ out, int ldo, int heads, int kv_heads, int dim, int vdim, int D, int cap,
+                                         int capp, int window, int pool, int pos0, float scale, const PrefillExtra& x) {
+  float* const s_p = s_q + kRowQuery;
+  const int p = pos0 + m, g = h / (heads / kv_heads);
+  const T* qrow = q + (size_t)m * x.qld + (size_t)h * x.qstride;
+  for (int d = lane; d < dim; d += 64) s_q[d] = (float)qrow[d];
+  for (int d = lane; d < x.rot_part; d += 64) {
+    const T* src = qrow + dim;
+    float y = (float)src[d];
+    if (d < x.rot_dims) y = rotated(y, (float)src[rot_partner(d, x.rot_dims)], d, x.rot_dims, (size_t)p, x.sin_t, x.cos_t);
+    s_q[dim + d] = y;
+  }
+  constexpr int kPer = W4A32_LAYERED_MAX_DIM / 64;
+  float acc[kPer] = {0};
+  float run_max = -INFINITY, run_sum = 0.0f;
+  if (x.sinks) {
+    run_max = x.sinks[h];
+    run_sum = 1.0f;
+  }
+  wave_lds_order();
+  // entries lo .. hi - 1; the buffers start at block blk0
+  auto segment = [&](const T* keys, const T* vals, int lo, int hi, int blk0) {
+    const int off = 32 * blk0;
+    for (int b = lo; b < hi; b += 64) {
+      const int n = min(64, hi - b);
+      float s = -INFINITY;
+      if (lane < n) {
+        s = 0.0f;
+        for (int d = 0; d < dim; ++d) s = __fmaf_rn(s_q[d], (float)keys[k_at(b + lane - off, d, D)], s);
+        const T* kr = static_cast<const T*>(x.kr) + (size_t)((b + lane) >> 5) * x.kr_block;
+        for (int d = 0; d < x.rot_part; ++d) s = __fmaf_rn(s_q[dim + d], (float)kr[k_at((b + lane) & 31, d, 0)], s);
+        s *= scale;
+      }
+      float mx = s;
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      const float new_max = fmaxf(run_max, mx);
+      const float corr = run_max == -INFINITY ? 0.0f : expf(run_max - new_max);
+      const float w = s == -INFINITY ? 0.0f : expf(s - new_max);
+      run_sum = run_sum * corr + wave_sum64(w);
+      run_max = new_max;
+      wave_lds_order();
+      s_p[lane] = w;
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int d = lane + 64 * i;
+        if (d >= vdim) break;
+        float a = acc[i] * corr;
+        for (int k = 0; k < n; ++k) a = __fmaf_rn(s_p[k], (float)vals[v_at(b + k - off, d, D)], a);
+        acc[i] = a;
+      }
+    }
+  };
+  segment(kp + (size_t)g * capp * D, vpt + (size_t)g * capp * D, 0, pooled_visible(p, window, pool), 0);
+  segment(kc + (size_t)g * cap * D, vt + (size_t)g * cap * D, max(0, p - window + 1), p + 1, x.blk0);
+  const float gate = x.gate ? sigmoid_f(x.gate[(size_t)m * x.ldg + h]) : 1.0f;
+  T* row = out + (size_t)m * ldo;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int d = lane + 64 * i;
+    if (d < vdim) row[h * vdim + d] = (T)(acc[i] / run_sum * gate);
+  }
+  if (h == heads - 1)
+    for (int c = heads * vdim + lane; c < ldo; c += 64) row[c] = (T)0.0f;
+}
+
+template <typename T>
+__global__ __launch_bounds__(64) void attn_rows_kernel(const T* __restrict__ q, const T* __restrict__ kc,
+                                                       const T* __restrict__ vt, const T* __restrict__ kp,
+                                                       const T* __restrict__ vpt, T* __restrict__ out, int ldo,
+                                                       int heads, int kv_heads, int dim, int vdim, int D, int cap,
+                                                       int capp, int window, int pool, int pos0, float scale,
+                                                       const PrefillExtra x) {
+  __shared__ float s_row[kRowLds];
+  attn_row(s_row, blockIdx.x, blockIdx.y, threadIdx.x, q, kc, vt, kp, vpt, out, ldo, heads, kv_heads, dim, vdim, D, cap, capp, window,
+           pool, pos0, scale, x);
+}
+
+// ---------------------------------------------------------------------------------------------
 // f32: workgroup = (head, 32 queries) as in attn_mfma_kernel, the products on v_mfma_f32_32x32x2_f32. An operand of that instruction is
 // one number per lane, so a lane's eight of a piece (16 dimensions of the keys, 16 entries of the values) serve eight products; pieces
 // are requested three ahead, straight from the caches' layout. A block of D = 128 is 128 products of 64 clocks and little else:
 // bound by the matrix cores. 18 heads of 1538 queries, window 269, D = 128: 1762 us in one wavefront per query, here 87; 8 heads of
 // 300 queries 107, here 29.
 template <int D, int KR>
-__global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_kernel(
+__global__ __launch_bounds__(64 * kMfmaWaves, D == 32 && KR == 0 ? 4 : D <= 128 ? 2 : 1) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vt, const float* __restrict__ kp,
     const float* __restrict__ vpt, float* __restrict__ out, int ldo, int M, int heads, int kv_heads, int dim, int vdim, int cap,
     int capp, int window, int pool, int pos0, float scale, const PrefillExtra x) {
@@ -760,6 +853,9 @@ __global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_ke
   extern __shared__ __align__(16) uint8_t smem[];
   f32x4* const s_q = reinterpret_cast<f32x4*>(smem);                                      // [kKeys][2][64]
   float* const s_merge = reinterpret_cast<float*>(smem + (size_t)kKeys * 2 * 64 * 16);     // [waves - 1][R][64]
+  static_assert((kMfmaWaves - 1) * R * 64 >= kMfmaWaves * kRowLds, "the merge's LDS serves attn_row of every wavefront");
+  __shared__ int s_odd;  // some sum is not finite
+  if (threadIdx.x == 0) s_odd = 0;
   const int h = blockIdx.x, g = h / (heads / kv_heads);
   const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // the later query blocks see more keys: they start first
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -903,6 +999,15 @@ __global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_ke
       for (int e = 0; e < 4; ++e) o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v1[e], st[8 * ks + 4 + e], o[c], 0, 0, 0);
     }
   }
+  // A weight of zero does not take an infinity or NaN out of a product: once one was met, it is in every query's sums.
+  float zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) zero[v & 7] = __fmaf_rn(o[c][v], 0.0f, zero[v & 7]);
+#pragma unroll
+  for (int i = 1; i < 8; ++i) zero[0] += zero[i];
+  if (__builtin_expect(zero[0] != zero[0], 0)) s_odd = 1;
 
   if (wave > 0) {
     float* dst = s_merge + (size_t)(wave - 1) * R * 64 + lane;
@@ -914,6 +1019,12 @@ __global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_ke
     dst[(R - 1) * 64] = run_sum;
   }
   __syncthreads();
+  if (__builtin_expect(s_odd, 0)) {  // query by query, over what each one sees
+    for (int m = 32 * qb + wave; m < min(32 * qb + 32, M); m += kMfmaWaves)
+      attn_row(s_merge + wave * kRowLds, h, m, lane, q, kc, vt, kp, vpt, out, ldo, heads, kv_heads, dim, vdim, D, cap, capp, window, pool,
+               pos0, scale, x);
+    return;
+  }
   if (wave > 0) return;
   float total_max = run_max;
 #pragma unroll
@@ -948,82 +1059,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, D <= 128 ? 2 : 1) void attn_f32_ke
     }
   if (h == heads - 1)
     for (int c = heads * vdim + hh; c < ldo; c += 2) row[c] = 0.0f;
-}
-
-// ---------------------------------------------------------------------------------------------
-// One wavefront per (head, query), everything f32: a lane per key for the scores, a lane per value dimension for
-// the sums.
-template <typename T>
-__global__ __launch_bounds__(64) void attn_rows_kernel(const T* __restrict__ q, const T* __restrict__ kc,
-                                                       const T* __restrict__ vt, const T* __restrict__ kp,
-                                                       const T* __restrict__ vpt, T* __restrict__ out, int ldo,
-                                                       int heads, int kv_heads, int dim, int vdim, int D, int cap,
-                                                       int capp, int window, int pool, int pos0, float scale,
-                                                       const PrefillExtra x) {
-  __shared__ float s_q[W4A32_LAYERED_MAX_DIM + W4A32_LAYERED_MAX_ROT_PART], s_p[64];
-  const int h = blockIdx.x, m = blockIdx.y, lane = threadIdx.x, g = h / (heads / kv_heads);
-  const int p = pos0 + m;
-  const T* qrow = q + (size_t)m * x.qld + (size_t)h * x.qstride;
-  for (int d = lane; d < dim; d += 64) s_q[d] = (float)qrow[d];
-  for (int d = lane; d < x.rot_part; d += 64) {
-    const T* src = qrow + dim;
-    float y = (float)src[d];
-    if (d < x.rot_dims) y = rotated(y, (float)src[rot_partner(d, x.rot_dims)], d, x.rot_dims, (size_t)p, x.sin_t, x.cos_t);
-    s_q[dim + d] = y;
-  }
-  constexpr int kPer = W4A32_LAYERED_MAX_DIM / 64;
-  float acc[kPer] = {0};
-  float run_max = -INFINITY, run_sum = 0.0f;
-  if (x.sinks) {
-    run_max = x.sinks[h];
-    run_sum = 1.0f;
-  }
-  __syncthreads();
-  // entries lo .. hi - 1; the buffers start at block blk0
-  auto segment = [&](const T* keys, const T* vals, int lo, int hi, int blk0) {
-    const int off = 32 * blk0;
-    for (int b = lo; b < hi; b += 64) {
-      const int n = min(64, hi - b);
-      float s = -INFINITY;
-      if (lane < n) {
-        s = 0.0f;
-        for (int d = 0; d < dim; ++d) s = __fmaf_rn(s_q[d], (float)keys[k_at(b + lane - off, d, D)], s);
-        const T* kr = static_cast<const T*>(x.kr) + (size_t)((b + lane) >> 5) * x.kr_block;
-        for (int d = 0; d < x.rot_part; ++d) s = __fmaf_rn(s_q[dim + d], (float)kr[k_at((b + lane) & 31, d, 0)], s);
-        s *= scale;
-      }
-      float mx = s;
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      const float new_max = fmaxf(run_max, mx);
-      const float corr = run_max == -INFINITY ? 0.0f : expf(run_max - new_max);
-      const float w = s == -INFINITY ? 0.0f : expf(s - new_max);
-      run_sum = run_sum * corr + wave_sum64(w);
-      run_max = new_max;
-      __syncthreads();
-      s_p[lane] = w;
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        const int d = lane + 64 * i;
-        if (d >= vdim) break;
-        float a = acc[i] * corr;
-        for (int k = 0; k < n; ++k) a = __fmaf_rn(s_p[k], (float)vals[v_at(b + k - off, d, D)], a);
-        acc[i] = a;
-      }
-    }
-  };
-  segment(kp + (size_t)g * capp * D, vpt + (size_t)g * capp * D, 0, pooled_visible(p, window, pool), 0);
-  segment(kc + (size_t)g * cap * D, vt + (size_t)g * cap * D, max(0, p - window + 1), p + 1, x.blk0);
-  const float gate = x.gate ? sigmoid_f(x.gate[(size_t)m * x.ldg + h]) : 1.0f;
-  T* row = out + (size_t)m * ldo;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int d = lane + 64 * i;
-    if (d < vdim) row[h * vdim + d] = (T)(acc[i] / run_sum * gate);
-  }
-  if (h == heads - 1)
-    for (int c = heads * vdim + lane; c < ldo; c += 64) row[c] = (T)0.0f;
 }
 
 // ---------------------------------------------------------------------------------------------

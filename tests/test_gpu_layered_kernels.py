@@ -360,3 +360,29 @@ def test_attention_of_long_prompts(arch, layer, T, dtype):
     state = bad.new_state()
     bad.forward(state, np.zeros(T + 64, dtype=np.int64), 0, want=[])
     assert torch.equal(dec.forward(state, tokens, 0), whole)
+
+
+# A token whose row of the embedding is not finite: its key and value are not, and nobody else's result may meet them but through attention to
+# it. In f32 every query in front of it, and behind it every one whose window has left it, keeps its value. (It stands inside of a block of 32
+# keys with both kinds; the last row has few tokens on few keys, one wavefront per query.)
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("arch,layer,T,at,left", [
+    ("lesarax", lm.rotary(4, 2, 64, 16), 110, 50, None),
+    ("lesarax", lm.rotary(3, 1, 24, 8), 100, 70, None),
+    ("lesarax", lm.latent(4, 100, 16, 90, 32, 48, 20), 150, 70, 90),
+    ("lesarax", lm.latent(2, 140, 40, 130, 32, 48, 33), 130, 40, 73),
+    ("suripel", lm.attention(4, 2, 40, 36, 10**6, 8), 90, 77, None),
+    ("suripel", lm.attention(4, 2, 40, 36, 24, 8), 130, 77, None),
+    ("lesarax", lm.rotary(4, 2, 64, 16), 40, 20, None),
+])
+def test_f32_attention_keeps_values_apart_that_are_not_finite(arch, layer, T, at, left, bad):
+    cfg = lm.config([layer], width=72) if arch == "suripel" else lm.lesarax([layer], width=72)
+    w = (lm.random_weights if arch == "suripel" else lm.lesarax_weights)(cfg, seed=T)
+    tokens = np.random.default_rng(T).integers(1, cfg["vocab"], T)
+    tokens[at] = 0
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, {**w, "embed": np.where(np.arange(cfg["vocab"])[:, None] == 0, bad, w["embed"])}, "float32", T)
+    got = dec.forward(dec.new_state(), tokens, 0)
+    kept = np.arange(T) < at if left is None else (np.arange(T) < at) | (np.arange(T) >= left)
+    # (the first logit of a model that shares its embedding with the head is that row's)
+    assert lm.errors(got[:, 1:], ref[:, 1:])[kept].max() < TOL["float32"]
