@@ -142,6 +142,13 @@ int w4a32_layered_head_rows(int dim, int vdim);
 /* Layer runs of a pass through the model (a looped layer counts once per pass). */
 int w4a32_layered_runs(const w4a32_layered_config* cfg);
 
+/* Which kernel attends in layer `layer` (attention, rotary, latent; else W4A32_EINVAL) of a portion of M > 1 tokens from
+ * position pos0 on: host arithmetic on the sizes, what w4a32_layered_forward() goes by. */
+#define W4A32_ATTENTION_QUERY 0 /* f32: a wavefront per query */
+#define W4A32_ATTENTION_32 1    /* 32 queries per workgroup, its wavefronts read keys and values for themselves */
+#define W4A32_ATTENTION_64 2    /* bf16: 64 queries per workgroup, keys and values through LDS */
+int w4a32_layered_attention_kernel(const w4a32_layered_config* cfg, int layer, int M, int pos0);
+
 /* What one sequence keeps (caches, convolution tails, recurrent states, position), and what a call works in
  * (activations, rotation tables; shared by all sequences of a model). 256-byte aligned bases. 0: see _check. */
 size_t w4a32_layered_state_bytes(const w4a32_layered_config* cfg);

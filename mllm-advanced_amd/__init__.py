@@ -95,6 +95,7 @@ ABI = {
     # include/w4a32_layered.h
     "w4a32_layered_check": (_ci, [_vp]),
     "w4a32_layered_head_rows": (_ci, [_ci, _ci]),
+    "w4a32_layered_attention_kernel": (_ci, [_vp, _ci, _ci, _ci]),
     "w4a32_layered_runs": (_ci, [_vp]),
     "w4a32_layered_state_bytes": (_sz, [_vp]),
     "w4a32_layered_workspace_bytes": (_sz, [_vp]),
@@ -147,6 +148,7 @@ class DecoderWeights(ctypes.Structure):
 LAYERED_BF16, LAYERED_F32 = 1, 2
 MIXERS = {"attention": 1, "delta": 2, "retention": 3, "rotary": 4, "latent": 5}
 NORM_LAYER, NORM_RMS = 0, 1
+ATTENTION_QUERY, ATTENTION_32, ATTENTION_64 = 0, 1, 2
 
 
 class LayerConfig(ctypes.Structure):

@@ -680,6 +680,20 @@ int w4a32_layered_check(const w4a32_layered_config* cfg) { return check_config(c
 
 int w4a32_layered_head_rows(int dim, int vdim) { return w4::head_bucket(std::max(dim, vdim)); }
 
+int w4a32_layered_attention_kernel(const w4a32_layered_config* cfg, int layer, int M, int pos0) {
+  if (int e = check_config(cfg); e != W4A32_OK) return e;
+  if (layer < 0 || layer >= cfg->n_layers || M < 2 || pos0 < 0 || M > cfg->max_seq - pos0) return W4A32_EINVAL;
+  const w4a32_layer_config& l = cfg->layers[layer];
+  if (l.mixer != W4A32_MIX_ATTENTION && l.mixer != W4A32_MIX_ROTARY && l.mixer != W4A32_MIX_LATENT) return W4A32_EINVAL;
+  w4::AttnGeom a{};
+  a.heads = l.heads;
+  a.D = w4::head_bucket(std::max(l.dim, l.vdim));
+  a.window = l.window > 0 ? l.window : w4::kNoWindow;
+  a.pool = l.mixer == W4A32_MIX_ATTENTION ? l.pool : 0;
+  a.scale = l.scale;
+  return w4::attn_prefill_kernel(cfg->dtype, a, l.mixer == W4A32_MIX_LATENT ? w4::latent_rot_pad(l.rot_part) : 0, M, pos0);
+}
+
 int w4a32_layered_runs(const w4a32_layered_config* cfg) {
   return check_config(cfg) == W4A32_OK ? (int)layer_runs(cfg).size() : 0;
 }

@@ -172,6 +172,8 @@ struct AttnMem {
   float* ring;
 };
 int head_bucket(int d);  // 32, 64, 128, 256
+// W4A32_ATTENTION_*: the kernel of a portion's attention (M > 1). rot_pad: dimensions of the keys' second part in memory, or 0
+int attn_prefill_kernel(int dtype, const AttnGeom& g, int rot_pad, int M, int pos0);
 // q, k, v rows of in_proj (f32 [M][ldr]) through the convolution: q -> T [M][heads][D], k and v -> caches
 hipError_t launch_attn_qkv(int dtype, const AttnGeom& g, const AttnMem& m, const float* raw, int ldr, const float* conv,
                            void* q, int M, int pos0, hipStream_t s);

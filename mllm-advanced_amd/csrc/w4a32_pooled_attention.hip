@@ -1383,13 +1383,16 @@ hipError_t qkv_t(const AttnGeom& g, const AttnMem& m, const float* raw, int ldr,
   return hipGetLastError();
 }
 
-// Whether attn_tile_kernel is the quicker one. Its longest workgroup has to be hidden behind the others: `longest` blocks of keys
-// against what 512 workgroups, as many as fit at once, have to do on average. Measured on 30 sizes of D = 128 (60 to 1024
-// workgroups) and 21 of D = 64, all of which the rule decides right; on its two sides, for instance, 12 heads without a window: 1280
-// queries 26.8 us here 31.5, 1501 queries 37.9 / 35.6; 28 heads: 200 queries 9.0 / 10.9, 512 queries 17.8 / 16.9.
+// Whether attn_tile_kernel is the quicker one. Not where attn_mfma_kernel's workgroups fit one per CU, so that nothing runs beside any
+// of them: us there / here, D = 128, 8 heads of 1024 queries with window 256 and pooled blocks (256 workgroups there) 12.4 / 16.2, 28
+// heads of 260 queries with a second part of 64 dimensions (252) 14.8 / 17.6; 28 of 300 from position 1500 on, window 300 (280) 28.4 / 20.1. And its
+// longest workgroup has to be hidden behind the others: `longest` blocks of keys against what 512 workgroups (as many as fit at once with D = 128)
+// have to do on average; on the two sides of that, for instance, 12 heads without a window: 1280 queries 26.8 / 31.5, 1501 queries 37.9 / 35.6; 28
+// heads of 512 queries 17.8 / 16.9. D = 64 has its own line. Of 1728 sizes (6 to 64 heads, 66 to 2048 queries from position 0 and later ones on, with
+// and without windows and second parts) none of the 464 that the rule brings here was slower than there.
 bool tile_is_quicker(const AttnGeom& g, int M, int pos0) {
   const int tiles = (M + kTileQueries - 1) / kTileQueries;
-  if ((g.D != 64 && g.D != 128) || !(g.scale > 0.0f) || (long)g.heads * tiles < 128) return false;
+  if ((g.D != 64 && g.D != 128) || !(g.scale > 0.0f) || (long)g.heads * ((M + 31) / 32) <= 256) return false;
   long longest = 0, all = 0;
   for (int t = 0; t < tiles; ++t) {
     const long first = (long)pos0 + (long)kTileQueries * t, last = (long)pos0 + std::min((long)kTileQueries * (t + 1), (long)M) - 1;
@@ -1401,6 +1404,11 @@ bool tile_is_quicker(const AttnGeom& g, int M, int pos0) {
   const double average = (double)all * g.heads / 512;
   return g.D == 128 ? longest <= 3.0 * average + 5.0 : longest <= 1.5 * average + 1.0;
 }
+
+// Whether attn_f32_kernel is the quicker one: a block of 32 keys costs it 4 us of matrix instructions and its start 15, so that few
+// tokens on few keys stay with one wavefront per query. Us here / in attn_rows_kernel, 8 heads, D = 128: 14 tokens 20 / 11, 45: 20 / 14,
+// 64: 19 / 16, 96: 19 / 26, 130: 23 / 38, 300 with a window of 64 19 / 44; 24 heads, D = 64: 45 tokens 10 / 9, 130: 12 / 34.
+bool f32_tiles(const AttnGeom& g, int M, int pos0) { return M > 64 || std::min((long)g.window, (long)pos0 + M) > 128; }
 
 template <int D, int KR>
 hipError_t tile_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M, int pos0,
@@ -1422,7 +1430,7 @@ template <int D, int KR>
 hipError_t mfma_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M,
                   int pos0, hipStream_t s) {
   if constexpr ((D == 64 || D == 128) && KR <= 4)
-    if (tile_is_quicker(g, M, pos0)) return tile_d<D, KR>(g, m, x, q, out, ldo, M, pos0, s);
+    if (attn_prefill_kernel(W4A32_LAYERED_BF16, g, 16 * KR, M, pos0) == W4A32_ATTENTION_64) return tile_d<D, KR>(g, m, x, q, out, ldo, M, pos0, s);
   auto kern = attn_mfma_kernel<D, KR>;
   constexpr size_t lds = (D / 16 + KR) * 64 * 16 + sizeof(float) * (kMfmaWaves - 1) * (D / 2 + 2) * 64;
   static LdsLimitOnce raised;
@@ -1473,6 +1481,11 @@ int attn_slices(const AttnGeom& g, int max_seq) {
   return std::min(std::max((blocks + 3) / 4, 4), kPoolAttnSlices);
 }
 
+int attn_prefill_kernel(int dtype, const AttnGeom& g, int rot_pad, int M, int pos0) {
+  if (dtype == W4A32_LAYERED_BF16) return rot_pad <= 64 && tile_is_quicker(g, M, pos0) ? W4A32_ATTENTION_64 : W4A32_ATTENTION_32;
+  return f32_tiles(g, M, pos0) ? W4A32_ATTENTION_32 : W4A32_ATTENTION_QUERY;
+}
+
 int head_bucket(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 256; }
 
 hipError_t launch_attn_qkv(int dtype, const AttnGeom& g, const AttnMem& m, const float* raw, int ldr, const float* conv,
@@ -1509,11 +1522,6 @@ static hipError_t prefill_bf16(const AttnGeom& g, const AttnMem& m, const Prefil
   }
 }
 
-// Whether attn_f32_kernel is the quicker one: a block of 32 keys costs it 4 us of matrix instructions and its start 15, so that few
-// tokens on few keys stay with one wavefront per query. Us here / in attn_rows_kernel, 8 heads, D = 128: 14 tokens 20 / 11, 45: 20 / 14,
-// 64: 19 / 16, 96: 19 / 26, 130: 23 / 38, 300 with a window of 64 19 / 44; 24 heads, D = 64: 45 tokens 10 / 9, 130: 12 / 34.
-static bool f32_tiles(const AttnGeom& g, int M, int pos0) { return M > 64 || std::min((long)g.window, (long)pos0 + M) > 128; }
-
 template <int D, int KR>
 static hipError_t f32_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M, int pos0,
                         hipStream_t s) {
@@ -1532,7 +1540,7 @@ static hipError_t f32_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra&
 template <int KR>
 static hipError_t prefill_f32(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo,
                               int M, int pos0, hipStream_t s) {
-  if (f32_tiles(g, M, pos0)) switch (g.D) {
+  if (attn_prefill_kernel(W4A32_LAYERED_F32, g, 16 * KR, M, pos0) == W4A32_ATTENTION_32) switch (g.D) {
     case 32: return f32_d<32, KR>(g, m, x, q, out, ldo, M, pos0, s);
     case 64: return f32_d<64, KR>(g, m, x, q, out, ldo, M, pos0, s);
     case 128: return f32_d<128, KR>(g, m, x, q, out, ldo, M, pos0, s);
