@@ -362,6 +362,31 @@ def test_attention_of_long_prompts(arch, layer, T, dtype):
     assert torch.equal(dec.forward(state, tokens, 0), whole)
 
 
+# the same kernel with each size of a head and of the keys' second part; the last 64 queries are 4, 10, 16 and 20; blocks with masks and, without
+# a window, ones in which every key is seen; positions off the blocks' borders in the second portion
+@pytest.mark.parametrize("layer,T", [
+    (lm.latent(40, 128, 64, 128, 40, 64, 100), 260),
+    (lm.latent(33, 120, 64, 128, 40, 64, 10**6), 330),
+    (lm.latent(64, 64, 16, 64, 40, 64, 100), 400),
+    (lm.latent(64, 60, 32, 50, 40, 64, 40), 404),
+])
+def test_latent_attention_of_long_prompts(pkg, layer, T):
+    import ctypes
+    import torch
+
+    cfg = lm.lesarax([layer], width=72)
+    w = lm.lesarax_weights(cfg, seed=T)
+    tokens = np.random.default_rng(T).integers(0, cfg["vocab"], T)
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, w, "bfloat16", T)
+    for M, pos0 in ((T, 0), (T - 37, 37)):
+        assert pkg.lib().w4a32_layered_attention_kernel(ctypes.byref(dec.cfg), 0, M, pos0) == pkg.ATTENTION_64
+    state = dec.new_state()
+    assert lm.errors(dec.forward(state, tokens, 0), ref).max() < TOL["bfloat16"]
+    parts = torch.cat([dec.forward(state, tokens[:37], 0), dec.forward(state, tokens[37:], 37)])
+    assert lm.errors(parts, ref).max() < TOL["bfloat16"]
+
+
 # A token whose row of the embedding is not finite: its key and value are not, and nobody else's result may meet them but through attention to
 # it. In f32 every query in front of it, and behind it every one whose window has left it, keeps its value. (It stands inside of a block of 32
 # keys with both kinds; the last row has few tokens on few keys, one wavefront per query.)

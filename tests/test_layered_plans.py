@@ -37,6 +37,15 @@ def test_bf16_prompts(pkg, mixer, heads, dim, window, pool, rot, M, pos0, which)
     assert kernel(pkg, "bf16", mixer, heads, dim, window, M, pos0, pool, rot) == which
 
 
+# what tests/test_gpu_layered_kernels.py runs as attention of long prompts is what it says
+@pytest.mark.parametrize("mixer,heads,dim,window,pool,rot,M", [("attention", 32, 124, 70, 8, 0, 300), ("attention", 96, 64, 33, 4, 0, 390),
+                                                               ("rotary", 48, 128, 0, 0, 40, 200), ("latent", 60, 64, 40, 0, 64, 450),
+                                                               ("latent", 44, 128, 50, 0, 16, 230), ("latent", 36, 100, 0, 0, 28, 260)])
+def test_long_prompts_of_the_gpu_tests(pkg, mixer, heads, dim, window, pool, rot, M):
+    assert kernel(pkg, "bf16", mixer, heads, dim, window, M, 0, pool, rot) == W64
+    assert kernel(pkg, "f32", mixer, heads, dim, window, M, 0, pool, rot) == W32
+
+
 @pytest.mark.parametrize("window,M,pos0,which", [(0, 64, 0, QUERY), (0, 65, 0, W32), (0, 2, 126, QUERY), (0, 2, 127, W32),
                                                  (128, 64, 4000, QUERY), (129, 64, 4000, W32)])
 def test_f32_prompts(pkg, window, M, pos0, which):
