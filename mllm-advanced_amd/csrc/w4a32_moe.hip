@@ -252,15 +252,16 @@ __global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __res
 }
 static_assert(kPlanThreads >= W4A32_LAYERED_MAX_EXPERTS, "a thread per expert");
 
-// The tile of a workgroup: first those of bm rows, then those of fewer, which the CUs take that come free early. An expert's
+// The tile of a workgroup: first those of bm rows, then (kRest) those of fewer, which the CUs take that come free early. An expert's
 // tiles are numbered rows fastest, experts one after the other; consecutive numbers on one XCD. `row0` and `rows` become the tile's.
 // Returns false past the last one.
+template <bool kRest>
 __device__ __forceinline__ bool moe_tile(const MoeTile* __restrict__ tiles, const int* __restrict__ n_tiles, int bm, int nt,
                                          MoeTile* tile, int* n, bool* rest) {
-  const int whole = n_tiles[0], all = whole + n_tiles[1];
+  const int whole = n_tiles[0], all = whole + (kRest ? n_tiles[1] : 0);
   int b = blockIdx.x;
   if (b >= all * nt) return false;
-  *rest = b >= whole * nt;
+  *rest = kRest && b >= whole * nt;
   if (*rest) b -= whole * nt;
   const int t = xcd_tile(b, (*rest ? all - whole : whole) * nt) + (*rest ? whole * nt : 0);
   *tile = tiles[t / nt];
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(Big::kThreads) void moe_gate_up_kernel(const T* __r
   MoeTile tile;
   int n;
   bool rest;
-  if (!moe_tile(tiles, n_tiles, Big::kRows, (2 * Fp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
+  if (!moe_tile<(Rest::kRows < Big::kRows)>(tiles, n_tiles, Big::kRows, (2 * Fp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
   if (Rest::kRows < Big::kRows && rest)
     gate_up_tile<T, Rest, kFar>(smem, tile, n, h, w, act, order, M, top, Hp, Fp, limit);
   else
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(Big::kThreads) void moe_down_kernel(const T* __rest
   MoeTile tile;
   int n;
   bool rest;
-  if (!moe_tile(tiles, n_tiles, Big::kRows, (Hp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
+  if (!moe_tile<(Rest::kRows < Big::kRows)>(tiles, n_tiles, Big::kRows, (Hp + Big::kCols - 1) / Big::kCols, &tile, &n, &rest)) return;
   if (Rest::kRows < Big::kRows && rest)
     down_tile<T, Rest, kFar>(smem, tile, n, act, w, parts, order, wts, top, rows_all, Hp, Fp);
   else
