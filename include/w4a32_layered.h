@@ -206,6 +206,9 @@ int w4a32_op_short_conv(const float* d_x, int ldx, float* d_y, int ldy, const fl
 /* The rows' mixture of experts: h T [M][pad(hidden)], router logits f32 [M][ld] -> d_parts f32 [top][M][pad(hidden)], one
  * row per chosen expert, weighted. d_scratch: w4a32_op_experts_scratch_bytes bytes, 256-byte aligned. */
 size_t w4a32_op_experts_scratch_bytes(int dtype, int M, int experts, int top, int ff);
+/* Rows << 16 | columns of the tiles that M > 1 rows' grouped products take (of gate and up, or with `down` of the product behind
+ * them); an expert's last rows may take lower ones. Host arithmetic on the sizes. */
+int w4a32_op_experts_tile(int dtype, int M, int hidden, int experts, int top, int ff, int down);
 int w4a32_op_experts(int dtype, const void* d_h, const float* d_logits, int ld, const void* d_gate_up, const void* d_down,
                      int M, int hidden, int experts, int top, int ff, float limit, float* d_parts, void* d_scratch,
                      void* stream);

@@ -110,6 +110,7 @@ ABI = {
     "w4a32_op_layernorm_conv": (_ci, [_vp, _vp, _ci, _vp, _vp, ctypes.c_float, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _ci,
                                       _vp]),
     "w4a32_op_short_conv": (_ci, [_vp, _ci, _vp, _ci, _vp, _vp] + [_ci] * 6 + [_vp]),
+    "w4a32_op_experts_tile": (_ci, [_ci] * 7),
     "w4a32_op_experts_scratch_bytes": (_sz, [_ci, _ci, _ci, _ci, _ci]),
     "w4a32_op_experts": (_ci, [_ci, _vp, _vp, _ci, _vp, _vp, _ci, _ci, _ci, _ci, _ci, ctypes.c_float, _vp, _vp, _vp]),
     "w4a32_op_polynorm": (_ci, [_vp, _ci, _ci, _ci, _ci, _vp, ctypes.c_float, _vp]),

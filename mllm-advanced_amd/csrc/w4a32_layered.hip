@@ -825,6 +825,14 @@ int w4a32_op_short_conv(const float* d_x, int ldx, float* d_y, int ldy, const fl
                                         S(stream)));
 }
 
+int w4a32_op_experts_tile(int dtype, int M, int hidden, int experts, int top, int ff, int down) {
+  if ((dtype != W4A32_LAYERED_BF16 && dtype != W4A32_LAYERED_F32) || M < 2 || hidden <= 0 || experts <= 0 || top <= 0 || top > experts ||
+      ff <= 0)
+    return W4A32_EINVAL;
+  const w4::MoeGeom g{hidden, pad64(hidden), ff, pad64(ff), experts, top, 0.0f};
+  return w4::moe_tile_size(dtype, g, M, !down);
+}
+
 size_t w4a32_op_experts_scratch_bytes(int dtype, int M, int experts, int top, int ff) {
   if (M <= 0 || experts <= 0 || top <= 0 || ff <= 0) return 0;
   return w4::moe_scratch_bytes(dtype, M, experts, top, pad64(ff));

@@ -250,7 +250,6 @@ __global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int* __res
     if (e == 0 && lane < 2) n_tiles[2 * list + lane] = s_sums[list][3 + lane];
   }
 }
-static_assert(kPlanThreads >= W4A32_LAYERED_MAX_EXPERTS, "a thread per expert");
 
 // The tile of a workgroup: first those of bm rows, then (kRest) those of fewer, which the CUs take that come free early. An expert's
 // tiles are numbered rows fastest, experts one after the other; consecutive numbers on one XCD. `row0` and `rows` become the tile's.
@@ -587,50 +586,87 @@ hipError_t launch_down(const MoeGeom& g, const T* down, int M, int rows_all, flo
   return hipGetLastError();
 }
 
-// Gate and up / down of 16 experts, 4 per token, in 128 x 128 throughout, 128 x 256 throughout, and 256 x 256 with last rows in
-// 128 x 256 (us): 1501 tokens, [2 x 2240][1536]: 109 / 69, 113 / 77, 106 / 57; 2048 tokens: 147 / 90, 157 / 78, 135 / 62; 900: 82 / 46,
-// 88 / 41, 90 / 53; 2048 tokens, [2 x 4736][3584]: 730 / 346, 688 / 310, 607 / 282. Whole tiles stand in front of the last rows':
-// mixed they took 116 / 57 for the first, as the large ones then end late. 100 tokens, [2 x 2240][1536], 64 x 128: 49 / 23 = 4.5
-// and 4.9 TB/s of weights, 128 x 128 53 / 26. A 256 x 256 tile takes 42 us of which its activation and stores are 5: with one
-// workgroup per CU nothing runs under them.
+// A 256 x 256 tile of [2 x 2240][1536] takes 42 us of which its activation and stores are 5: with one workgroup per CU nothing runs under
+// them. Whole tiles stand in front of the shorter last rows': mixed, 1501 tokens of 16 experts, 4 per token, took 116 / 57 us (gate and up /
+// down) against 106 / 57, as the large ones then end late. 100 tokens, [2 x 2240][1536], 64 x 128: 49 / 23 = 4.5 and 4.9 TB/s of weights, 128 x
+// 128 53 / 26.
 //
-// What the bf16 shapes cost: us per 64 k of a tile and of the rest's tile with all CUs busy, and per tile for what stands in front of
-// and behind its products (gate and up / down), on `slots` tiles at once. Fitted to 19 problems of 200 to 1024 rows per expert
-// from [2 x 400][768] to [2 x 4736][3584] (7 % of error on average).
+// What the bf16 shapes cost: us per 64 k of a tile with all CUs busy, and per tile for what stands in front of and behind its products, on
+// `slots` tiles at once. Fitted for the choice, not for the time (which is 10 to 20 % off: the weights' way from memory and what partly filled
+// CUs gain are not in it), to 300 problems of 96 to 2000 rows per expert, 4 to 128 experts, from [2 x 256][512] to [2 x 4736][3584].
 struct MoeShape {
   int bm, rest, bn, slots;
-  double tile_us, rest_us, up_us, down_us;
+  double up_tile_us, down_tile_us, up_us, down_us;
 };
-constexpr MoeShape kTall = {256, 128, 256, 256, 1.375, 1.37, 7.5, 9.0}, kWide = {128, 0, 256, 256, 0.967, 0, 2.9, 4.5},
-                   kSmall = {128, 0, 128, 512, 1.106, 0, 1.5, 4.8};  // kSmall: two tiles per CU, alone on it one takes half as long
+constexpr MoeShape kTall = {256, 128, 256, 256, 1.6, 1.6, 7.5, 9.0}, kWide = {128, 0, 256, 256, 0.967, 0.967, 2.9, 4.5},
+                   kSmall = {128, 0, 128, 512, 1.106, 1.2, 1.5, 4.8};
+
+struct MoeTiles {
+  double whole, rest;
+};
+// What an expert has on average where `per` rows come to it by independent choices (standard deviation sqrt(per)).
+MoeTiles expected_tiles(double per, int bm, int rest) {
+  const double sd = std::sqrt(per);
+  auto more_than = [&](double rows) { return 0.5 * std::erfc((rows + 0.5 - per) / (sd * std::sqrt(2.0))); };
+  int n = std::max(0, (int)((per - 5.0 * sd) / bm) - 1);  // so many are whole as good as always
+  MoeTiles t{(double)n, 0.0};
+  for (;; ++n) {
+    const double begun = n > 0 ? more_than((double)n * bm) : 1.0, full = n > 0 || rest > 0 ? more_than((double)n * bm + rest) : 1.0;
+    if (begun < 1e-4) return t;
+    t.whole += full;
+    t.rest += begun - full;
+  }
+}
 
 double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
   const int N = up ? 2 * g.Fp : g.Hp, nt = (N + t.bn - 1) / t.bn;
   const double k = (up ? g.Hp : g.Fp) / 64.0, over = up ? t.up_us : t.down_us;
-  const double per = (double)M * g.top / g.experts, spread = std::sqrt(per);
-  const MoeHeights heights{t.bm == 256 ? 8 : 7, t.rest};
-  double whole = 0.0, rest = 0.0;  // experts with about `per` rows, in three classes
-  for (int i = -1; i <= 1; ++i) {
-    const int count = (int)(per + i * spread), n = heights.whole(count);
-    whole += g.experts / 3.0 * nt * n;
-    rest += g.experts / 3.0 * nt * (count > n * t.bm ? 1 : 0);
-  }
-  const double tile_us = t.tile_us * k + over, rest_us = t.rest_us * k + over / 2;
-  const double rounds = std::floor(whole / t.slots), left = whole - rounds * t.slots;
+  const MoeTiles tiles = expected_tiles((double)M * g.top / g.experts, t.bm, t.rest);
+  const double whole = tiles.whole * g.experts * nt, tile_us = (up ? t.up_tile_us : t.down_tile_us) * k + over;
+  const double rounds = std::floor(whole / t.slots), left = whole - rounds * t.slots, begun = std::min(1.0, left);
   double end = rounds * tile_us;
-  if (&t == &kSmall) return end + (left <= 0.0 ? 0.0 : left > 256 ? tile_us : 0.5 * tile_us);
+  if (t.slots == 512) {  // two tiles per CU: alone on it one takes a little more than half as long
+    const double shared = std::min(1.0, std::max(0.0, left - 256.0) / 64.0);
+    return end + begun * tile_us * (0.55 + 0.45 * shared);
+  }
   // the slots with a tile of the last round and those without one, as the rests come to them
-  double free_at[2] = {left > 0.0 ? end + tile_us : end, end};
-  const double slots[2] = {left > 0.0 ? left : t.slots, left > 0.0 ? t.slots - left : 0.0};
-  end = free_at[0];
-  while (rest > 0.0) {
-    const int i = slots[1] > 0.0 && free_at[1] <= free_at[0] ? 1 : 0;
+  double free_at[2] = {left >= 1.0 ? end + tile_us : end, end};
+  const double slots[2] = {left >= 1.0 ? left : 0.0, left >= 1.0 ? t.slots - left : t.slots};
+  // a rest's tile beside whole ones takes as long as kWide's; the more of the time all CUs are at rests, the more they wait for memory
+  const double rest_us = (0.967 + 0.6 * std::min(1.0, tiles.rest / std::max(tiles.whole, 1e-9))) * k + over / 2;
+  end += tile_us * begun;
+  for (double rest = tiles.rest * g.experts * nt; rest > 0.5;) {
+    const int i = free_at[1] <= free_at[0] || slots[0] <= 0.0 ? 1 : 0;
     rest -= slots[i];
     free_at[i] += rest_us;
     end = std::max(end, free_at[i]);
   }
   return end;
 }
+
+// 0: kTall, 1: kWide, 2: kSmall. By rows per expert and tiles alone, unless another shape is estimated 7 % cheaper. (128 x 256 is one workgroup
+// per CU, 128 x 128 two that fill each other's gaps, which the costs do not know: it has to be clearly cheaper.) Over those problems and 300
+// products more, that is 4.6 % quicker than by rows and tiles alone, and slower by more than 3 % for 8 of the 600 (16 % at most); 1.8 % slower than the
+// best shape. Us in 256 x 256 with last rows in 128 x 256 / in 128 x 256 / in 128 x 128, and what is chosen, 16 experts, 4 per token:
+//   tokens, experts         gate and up                    down
+//   900, [2 x 2240][1536]   86.5 89.1 80.7 (128 x 128)     54.0 43.3 49.7 (128 x 256)
+//   1501                    103  115  112  (128 x 128)     57.4 77.7 69.3 (256 x 256)
+//   2048                    136  140  146  (256 x 256)     62.8 78.9 88.3 (256 x 256)
+//   512, [2 x 4736][3584]   257  282  293  (128 x 128)     110  170  165  (256 x 256)
+//   2048                    541  628  675  (256 x 256)     285  314  360  (256 x 256)
+// (1501 tokens, gate and up: in the whole model 256 x 256 is half a percent of it quicker.)
+int moe_shape(const MoeGeom& g, int M, bool up) {
+  const long bands = (long)M * g.top / 128 + g.experts / 2;
+  const int plain = (long)M * g.top / g.experts >= 768                                                  ? 0
+                    : bands * (g.Hp / 256) >= 1000 || (up && bands * (2 * g.Fp / 256) >= 1000) ? 1
+                                                                                                        : 2;
+  const double us[3] = {moe_shape_us(kTall, g, M, up), moe_shape_us(kWide, g, M, up) / 0.93, moe_shape_us(kSmall, g, M, up)};
+  const int least = (int)(std::min_element(us, us + 3) - us);
+  return us[least] < 0.93 * us[plain] ? least : plain;
+}
+
+// rows an expert has on average, too few of them for 128-row tiles
+bool moe_few(const MoeGeom& g, int M) { return (long)M * g.top / g.experts < 96; }
 
 template <typename T>
 bool experts_far(const MoeGeom& g) {
@@ -663,24 +699,17 @@ hipError_t prefill_t(int dtype, const MoeGeom& g, const T* h, const float* logit
     using Far = ShapeOf<T, 64, 128, 2, 2, 2>;
     return grouped<Far, Far, true>(g, h, gate_up, down, M, rows_all, parts, ws, c, s);
   }
-  const bool few = (long)M * g.top / g.experts < 96;  // rows an expert has on average
+  const bool few = moe_few(g, M);
   if constexpr (sizeof(T) == 2) {
     if (few) return run(ShapeOf<T, 64, 128, 2, 2, 4>{}, ShapeOf<T, 64, 128, 2, 4, 4>{});
-    // 128 x 256 is one workgroup per CU, 128 x 128 two that fill each other's gaps, which the costs do not know: it has to be clearly
-    // cheaper
-    auto choose = [&](bool up) {
-      const double tall = moe_shape_us(kTall, g, M, up), wide = moe_shape_us(kWide, g, M, up), small = moe_shape_us(kSmall, g, M, up);
-      const bool wider = wide < 0.93 * small;
-      return tall < (wider ? wide : small) ? 0 : wider ? 1 : 2;
-    };
     auto with = [&](auto up) {
-      switch (choose(false)) {
+      switch (moe_shape(g, M, false)) {
         case 0: return run(up, ShapeOf<T, 256, 256, 2, 4, 2, 128>{});
         case 1: return run(up, ShapeOf<T, 128, 256, 2, 4, 2>{});
         default: return run(up, ShapeOf<T, 128, 128, 2, 4, 2>{});
       }
     };
-    switch (choose(true)) {
+    switch (moe_shape(g, M, true)) {
       case 0: return with(ShapeOf<T, 256, 256, 2, 4, 2, 128>{});
       case 1: return with(ShapeOf<T, 128, 256, 2, 4, 2>{});
       default: return with(ShapeOf<T, 128, 128, 2, 2, 2>{});
@@ -743,6 +772,13 @@ hipError_t decode_t(const MoeGeom& g, const RowPrologue& pro, const float* logit
 }
 
 }  // namespace
+
+int moe_tile_size(int dtype, const MoeGeom& g, int M, bool up) {
+  const bool bf16 = dtype == W4A32_LAYERED_BF16;
+  if ((bf16 ? experts_far<__bf16>(g) : experts_far<float>(g)) || moe_few(g, M)) return 64 << 16 | 128;
+  const int shape = bf16 ? moe_shape(g, M, up) : 2;
+  return shape == 0 ? 256 << 16 | 256 : shape == 1 ? 128 << 16 | 256 : 128 << 16 | 128;
+}
 
 size_t moe_scratch_bytes(int dtype, int M, int experts, int top, int Fp) { return scratch_of(dtype, M, experts, top, Fp).bytes; }
 

@@ -89,12 +89,34 @@ def test_bf16_product_of_every_shape(pkg, M, N, K):
     (1540, 72, 4, 2, 100),    # 770
     (12400, 70, 128, 1, 900),   # 96, about 160 tiles of rows
     (12400, 1800, 128, 1, 60),  # ... column counts that are no multiple of a tile
-    (1900, 1530, 40, 3, 60),    # bf16: gate and up in 128 x 128, down in 256 x 256 and experts' last rows in 128 x 256
-    (1100, 1530, 8, 2, 1500),   # the other way round, down in 128 x 256
-    (2500, 1800, 40, 2, 310),   # both in 128 x 256
-    (2500, 1800, 4, 2, 900),    # both in 256 x 256 with last rows
+    (1900, 1530, 40, 3, 60),    # 142
+    (1100, 1530, 8, 2, 1500),   # 275
+    (2500, 1800, 40, 2, 310),   # 125
+    (2500, 1800, 4, 2, 900),    # 1250
 ])
 def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
+    grouped_products(pkg, rows, hidden, experts, top, ff)
+
+
+# bf16: every pair of tiles that two products take, by their costs; row and column counts that are no multiples of them
+@pytest.mark.parametrize("rows,hidden,experts,top,ff,up,down", [
+    (578, 123, 3, 1, 81, (128, 128), (128, 128)),
+    (1175, 1336, 3, 3, 63, (128, 128), (128, 256)),
+    (4767, 1170, 8, 2, 65, (128, 128), (256, 256)),    # an expert's last rows in 128 x 256, here and below
+    (5081, 1746, 2, 2, 211, (128, 256), (128, 128)),
+    (4367, 2438, 40, 4, 72, (128, 256), (128, 256)),
+    (4281, 2240, 40, 4, 76, (128, 256), (256, 256)),
+    (4336, 330, 16, 4, 333, (256, 256), (128, 128)),
+    (3228, 326, 8, 4, 490, (256, 256), (128, 256)),
+    (4486, 497, 8, 4, 334, (256, 256), (256, 256)),
+])
+def test_grouped_products_of_every_pair_of_tiles(pkg, rows, hidden, experts, top, ff, up, down):
+    for which, tile in ((0, up), (1, down)):
+        assert pkg.lib().w4a32_op_experts_tile(pkg.LAYERED_BF16, rows, hidden, experts, top, ff, which) == tile[0] << 16 | tile[1]
+    grouped_products(pkg, rows, hidden, experts, top, ff)
+
+
+def grouped_products(pkg, rows, hidden, experts, top, ff):
     import torch
 
     g = torch.Generator(device="cuda").manual_seed(rows)

@@ -1,4 +1,5 @@
-"""Which kernel a portion's attention takes in the layered decoder, at sizes where both were timed. No GPU: the choice is host code."""
+"""Which kernel a portion's attention takes in the layered decoder and which tiles its experts' products, at sizes where all of them
+were timed. No GPU: the choice is host code."""
 import ctypes
 
 import pytest
@@ -56,3 +57,34 @@ def test_what_has_no_attention_or_no_portion(pkg):
     assert kernel(pkg, "bf16", "rotary", 8, 128, 0, 1, 0, rot=64) < 0
     assert kernel(pkg, "bf16", "rotary", 8, 128, 0, 8192, 1, rot=64) < 0
     assert kernel(pkg, "bf16", "retention", 8, 128, 0, 64, 0, rot=64) < 0
+
+
+# us in tiles of 256 x 256 (an expert's last rows in 128 x 256), 128 x 256 and 128 x 128: the chosen one is at most a seventh slower than the best
+TILES = [256 << 16 | 256, 128 << 16 | 256, 128 << 16 | 128]
+
+
+@pytest.mark.parametrize("M,hidden,experts,top,ff,up,down", [
+    (900, 1536, 16, 4, 2240, [86.5, 89.1, 80.7], [54.0, 43.3, 49.7]),
+    (1501, 1536, 16, 4, 2240, [103.1, 114.5, 111.5], [57.4, 77.7, 69.3]),
+    (2048, 1536, 16, 4, 2240, [136.1, 139.7, 146.4], [62.8, 78.9, 88.3]),
+    (512, 3584, 16, 4, 4736, [256.7, 282.5, 293.4], [110.4, 170.3, 165.1]),
+    (2048, 3584, 16, 4, 4736, [541.1, 627.7, 674.9], [285.3, 313.6, 360.1]),
+    (3646, 512, 64, 4, 400, [33.4, 36.1, 24.7], [22.3, 27.0, 21.8]),
+    (3369, 2560, 64, 6, 1408, [434.9, 407.5, 404.1], [258.3, 230.6, 236.5]),
+    (1402, 1536, 24, 8, 256, [39.8, 28.4, 30.0], [35.2, 33.0, 27.1]),
+    (700, 1536, 16, 4, 2240, [90.1, 85.8, 75.7], [51.8, 41.3, 46.1]),
+    (1225, 1024, 64, 6, 1024, [63.6, 76.0, 68.6], [41.6, 53.2, 45.7]),
+    (3446, 2560, 8, 4, 1408, [201.1, 210.3, 228.1], [125.3, 130.7, 135.1]),
+])
+def test_tiles_of_the_experts(pkg, M, hidden, experts, top, ff, up, down):
+    for which, us in ((0, up), (1, down)):
+        tile = pkg.lib().w4a32_op_experts_tile(pkg.LAYERED_BF16, M, hidden, experts, top, ff, which)
+        assert us[TILES.index(tile)] <= 1.15 * min(us), which
+
+
+def test_tiles_of_few_rows_and_f32(pkg):
+    tile = lambda dtype, M: pkg.lib().w4a32_op_experts_tile(dtype, M, 1536, 16, 4, 2240, 0)
+    assert tile(pkg.LAYERED_BF16, 383) == tile(pkg.LAYERED_F32, 383) == 64 << 16 | 128
+    assert tile(pkg.LAYERED_BF16, 384) in TILES and tile(pkg.LAYERED_F32, 384) == TILES[2]
+    assert tile(pkg.LAYERED_F32, 4096) == TILES[2]
+    assert pkg.lib().w4a32_op_experts_tile(pkg.LAYERED_BF16, 100, 64, 4, 5, 64, 0) < 0
