@@ -1405,10 +1405,17 @@ bool tile_is_quicker(const AttnGeom& g, int M, int pos0) {
   return g.D == 128 ? longest <= 3.0 * average + 5.0 : longest <= 1.5 * average + 1.0;
 }
 
-// Whether attn_f32_kernel is the quicker one: a block of 32 keys costs it 4 us of matrix instructions and its start 15, so that few
-// tokens on few keys stay with one wavefront per query. Us here / in attn_rows_kernel, 8 heads, D = 128: 14 tokens 20 / 11, 45: 20 / 14,
-// 64: 19 / 16, 96: 19 / 26, 130: 23 / 38, 300 with a window of 64 19 / 44; 24 heads, D = 64: 45 tokens 10 / 9, 130: 12 / 34.
-bool f32_tiles(const AttnGeom& g, int M, int pos0) { return M > 64 || std::min((long)g.window, (long)pos0 + M) > 128; }
+// Whether attn_f32_kernel is the quicker one. A wavefront per query takes 64 of its entries (tokens and pooled blocks) at a time, 10 to 15 us each
+// at D = 128; here a block of 32 costs 4 us of matrix instructions, the blocks dealt to four wavefronts, and staging, merge and stores 15: few
+// tokens on few entries stay with a wavefront per query. Us there / here, 8 heads, D = 128: 14 tokens 11 / 20, 45: 14 / 20, 64: 16 / 19, 96: 26 / 19,
+// 130: 38 / 23, 300 with a window of 64 44 / 19; 2 tokens behind 1900, window 64, blocks of 4, 95 / 37; 24 heads, D = 64: 45 tokens 9 / 10,
+// 130: 34 / 12. The last line: 4 heads of 65 tokens, window 64, D = 128: 16.5 / 17.8, 16 heads 19.3 / 18.4.
+bool f32_tiles(const AttnGeom& g, int M, int pos0) {
+  const long last = (long)pos0 + M - 1, tokens = std::min((long)g.window, last + 1);
+  const long pooled = g.pool > 0 ? std::max(0l, last - g.window + 1) / g.pool : 0;
+  if (M > 80 || tokens + pooled > 128) return true;
+  return M > 64 && (tokens > 64 || g.D < 128 || g.heads > 8);
+}
 
 template <int D, int KR>
 hipError_t tile_d(const AttnGeom& g, const AttnMem& m, const PrefillExtra& x, const void* q, void* out, int ldo, int M, int pos0,

@@ -409,6 +409,27 @@ def test_latent_attention_of_long_prompts(pkg, layer, T):
     assert lm.errors(parts, ref).max() < TOL["bfloat16"]
 
 
+# f32, few tokens: a wavefront per query up to 80 of them on up to 64 tokens each; matrix instructions where a late portion sees many pooled blocks,
+# the last of 32 of them partly or by some queries only
+@pytest.mark.parametrize("dim,vdim,heads", [(100, 128, 4), (256, 200, 2), (30, 32, 6)])
+def test_f32_attention_of_short_portions(pkg, dim, vdim, heads):
+    import ctypes
+
+    cfg = lm.config([lm.attention(heads, 2, dim, vdim, 21, 3)], width=72)
+    w = lm.random_weights(cfg, seed=dim)
+    portions = [(80, pkg.ATTENTION_QUERY if dim > 64 else pkg.ATTENTION_32), (3, pkg.ATTENTION_QUERY), (250, pkg.ATTENTION_32),
+                (2, pkg.ATTENTION_QUERY), (64, pkg.ATTENTION_32), (7, pkg.ATTENTION_32)]
+    T = sum(n for n, _ in portions)
+    tokens = np.random.default_rng(dim).integers(0, cfg["vocab"], T)
+    ref = lo.forward(cfg, w, tokens)
+    dec = lm.runner(cfg, w, "float32", T)
+    state, at = dec.new_state(), 0
+    for n, which in portions:
+        assert pkg.lib().w4a32_layered_attention_kernel(ctypes.byref(dec.cfg), 0, n, at) == which, (n, at)
+        assert lm.errors(dec.forward(state, tokens[at:at + n], at), ref[at:at + n]).max() < TOL["float32"], (n, at)
+        at += n
+
+
 # A token whose row of the embedding is not finite: its key and value are not, and nobody else's result may meet them but through attention to
 # it. In f32 every query in front of it, and behind it every one whose window has left it, keeps its value. (It stands inside of a block of 32
 # keys with both kinds; the last row has few tokens on few keys, one wavefront per query.)

@@ -47,10 +47,19 @@ def test_long_prompts_of_the_gpu_tests(pkg, mixer, heads, dim, window, pool, rot
     assert kernel(pkg, "f32", mixer, heads, dim, window, M, 0, pool, rot) == W32
 
 
-@pytest.mark.parametrize("window,M,pos0,which", [(0, 64, 0, QUERY), (0, 65, 0, W32), (0, 2, 126, QUERY), (0, 2, 127, W32),
-                                                 (128, 64, 4000, QUERY), (129, 64, 4000, W32)])
-def test_f32_prompts(pkg, window, M, pos0, which):
-    assert kernel(pkg, "f32", "rotary", 8, 128, window, M, pos0, rot=64) == which
+# us of a wavefront per query / in the kernel of 32 queries
+@pytest.mark.parametrize("heads,dim,window,pool,M,pos0,which", [
+    (8, 128, 0, 0, 64, 0, QUERY), (8, 128, 0, 0, 65, 0, W32), (8, 128, 0, 0, 2, 126, QUERY), (8, 128, 0, 0, 2, 127, W32),
+    (8, 128, 128, 10**6, 64, 4000, QUERY), (8, 128, 129, 10**6, 64, 4000, W32),
+    (4, 128, 64, 4, 65, 0, QUERY), (4, 128, 64, 4, 80, 0, QUERY), (4, 128, 64, 4, 81, 0, W32),   # 16.5 / 17.8 (65)
+    (9, 128, 64, 4, 65, 0, W32), (16, 128, 64, 4, 65, 0, W32),                                   # 19.3 / 18.4 (16 heads)
+    (4, 64, 64, 4, 65, 0, W32),
+    (8, 128, 64, 4, 2, 318, QUERY), (8, 128, 64, 4, 2, 322, W32),   # 64 tokens and 64, 65 pooled blocks
+    (8, 128, 64, 4, 2, 1900, W32), (8, 128, 20, 4, 64, 1000, W32),  # 95 / 37, 61 / 29
+])
+def test_f32_prompts(pkg, heads, dim, window, pool, M, pos0, which):
+    mixer, rot = ("attention", 0) if pool else ("rotary", 64)
+    assert kernel(pkg, "f32", mixer, heads, dim, window, M, pos0, pool, rot) == which
 
 
 def test_what_has_no_attention_or_no_portion(pkg):
