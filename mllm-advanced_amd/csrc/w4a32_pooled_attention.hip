@@ -840,9 +840,11 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(const T* __restrict__ q, 
 // ---------------------------------------------------------------------------------------------
 // f32: workgroup = (head, 32 queries) as in attn_mfma_kernel, the products on v_mfma_f32_32x32x2_f32. An operand of that instruction is
 // one number per lane, so a lane's eight of a piece (16 dimensions of the keys, 16 entries of the values) serve eight products; pieces
-// are requested three ahead, straight from the caches' layout. A block of D = 128 is 128 products of 64 clocks and little else:
-// bound by the matrix cores. 18 heads of 1538 queries, window 269, D = 128: 1762 us in one wavefront per query, here 87; 8 heads of
-// 300 queries 107, here 29.
+// are requested three ahead, straight from the caches' layout. 18 heads of 1538 queries, window 269, D = 128: 1762 us in one wavefront per
+// query, here 87; 8 heads of 300 queries 107, here 29. A block of D = 128 is 128 products of 64 clocks: 32 of those 87 us are the matrix
+// cores'. The others are the start (15 us with one block: queries staged number by number, the first loads), the masks, exponentials and
+// sums between a block's two products, which nothing runs above, and the end, where one of four wavefronts merges and stores everything, with
+// 64 to 208 bytes per lane of its registers in scratch memory for D >= 128 (none in the loop). Sums that are not finite go a way of their own.
 template <int D, int KR>
 __global__ __launch_bounds__(64 * kMfmaWaves, D == 32 && KR == 0 ? 4 : D <= 128 ? 2 : 1) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vt, const float* __restrict__ kp,
