@@ -592,50 +592,45 @@ hipError_t launch_down(const MoeGeom& g, const T* down, int M, int rows_all, flo
 // 128 53 / 26.
 //
 // What the bf16 shapes cost: us per 64 k of a tile with all CUs busy, and per tile for what stands in front of and behind its products, on
-// `slots` tiles at once. Fitted for the choice, not for the time (which is 10 to 20 % off: the weights' way from memory and what partly filled
-// CUs gain are not in it), to 300 problems of 96 to 2000 rows per expert, 4 to 128 experts, from [2 x 256][512] to [2 x 4736][3584].
+// `slots` tiles at once. Fitted for the choice, not for the time (which is 10 to 20 % off: the weights' way from memory is not in it), to 1700
+// products of 96 to 2000 rows per expert, 4 to 128 experts, from [2 x 256][512] to [2 x 4736][3584].
 struct MoeShape {
   int bm, rest, bn, slots;
   double up_tile_us, down_tile_us, up_us, down_us;
 };
-constexpr MoeShape kTall = {256, 128, 256, 256, 1.6, 1.6, 7.5, 9.0}, kWide = {128, 0, 256, 256, 0.967, 0.967, 2.9, 4.5},
-                   kSmall = {128, 0, 128, 512, 1.106, 1.2, 1.5, 4.8};
+constexpr MoeShape kTall = {256, 128, 256, 256, 1.57, 1.57, 6.3, 10.8}, kWide = {128, 0, 256, 256, 0.967, 0.967, 2.2, 4.6},
+                   kSmall = {128, 0, 128, 512, 1.13, 1.36, 1.55, 3.0};
 
+// What an expert has where `per` rows come to it by independent choices (standard deviation sqrt(per)): on average, and the
+// variance of the whole tiles.
 struct MoeTiles {
-  double whole, rest;
+  double whole, rest, var;
 };
-// What an expert has on average where `per` rows come to it by independent choices (standard deviation sqrt(per)).
 MoeTiles expected_tiles(double per, int bm, int rest) {
   const double sd = std::sqrt(per);
   auto more_than = [&](double rows) { return 0.5 * std::erfc((rows + 0.5 - per) / (sd * std::sqrt(2.0))); };
   int n = std::max(0, (int)((per - 5.0 * sd) / bm) - 1);  // so many are whole as good as always
-  MoeTiles t{(double)n, 0.0};
+  MoeTiles t{(double)n, 0.0, 0.0};
   for (;; ++n) {
     const double begun = n > 0 ? more_than((double)n * bm) : 1.0, full = n > 0 || rest > 0 ? more_than((double)n * bm + rest) : 1.0;
     if (begun < 1e-4) return t;
     t.whole += full;
     t.rest += begun - full;
+    t.var += full * (1.0 - full);
   }
 }
 
-double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
-  const int N = up ? 2 * g.Fp : g.Hp, nt = (N + t.bn - 1) / t.bn;
-  const double k = (up ? g.Hp : g.Fp) / 64.0, over = up ? t.up_us : t.down_us;
-  const MoeTiles tiles = expected_tiles((double)M * g.top / g.experts, t.bm, t.rest);
-  const double whole = tiles.whole * g.experts * nt, tile_us = (up ? t.up_tile_us : t.down_tile_us) * k + over;
-  const double rounds = std::floor(whole / t.slots), left = whole - rounds * t.slots, begun = std::min(1.0, left);
-  double end = rounds * tile_us;
-  if (t.slots == 512) {  // two tiles per CU: alone on it one takes a little more than half as long
-    const double shared = std::min(1.0, std::max(0.0, left - 256.0) / 64.0);
-    return end + begun * tile_us * (0.55 + 0.45 * shared);
-  }
+// us of `whole` tiles, and with kTall of `rest` lower ones behind them
+double moe_rounds_us(const MoeShape& t, double whole, double rest, double tile_us, double rest_us) {
+  if (t.rest == 0) whole = std::max(1.0, whole - 0.5);
+  const double rounds = std::floor(whole / t.slots), left = whole - rounds * t.slots;
+  if (t.slots == 512)  // two tiles per CU: alone on it one takes half as long
+    return tile_us * (rounds + (left <= 0.0 ? 0.0 : left <= 256.0 ? 0.53 : 0.53 + 0.47 * std::min(1.0, (left - 256.0) / 14.0)));
+  if (t.rest == 0) return tile_us * (rounds + (left > 0.0 ? 1.0 : 0.0));
   // the slots with a tile of the last round and those without one, as the rests come to them
-  double free_at[2] = {left >= 1.0 ? end + tile_us : end, end};
+  double free_at[2] = {(rounds + (left >= 1.0 ? 1.0 : 0.0)) * tile_us, rounds * tile_us}, end = (rounds + std::min(1.0, left)) * tile_us;
   const double slots[2] = {left >= 1.0 ? left : 0.0, left >= 1.0 ? t.slots - left : t.slots};
-  // a rest's tile beside whole ones takes as long as kWide's; the more of the time all CUs are at rests, the more they wait for memory
-  const double rest_us = (0.967 + 0.6 * std::min(1.0, tiles.rest / std::max(tiles.whole, 1e-9))) * k + over / 2;
-  end += tile_us * begun;
-  for (double rest = tiles.rest * g.experts * nt; rest > 0.5;) {
+  while (rest > 0.5) {
     const int i = free_at[1] <= free_at[0] || slots[0] <= 0.0 ? 1 : 0;
     rest -= slots[i];
     free_at[i] += rest_us;
@@ -644,10 +639,22 @@ double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
   return end;
 }
 
-// 0: kTall, 1: kWide, 2: kSmall. By rows per expert and tiles alone, unless another shape is estimated 7 % cheaper. (128 x 256 is one workgroup
-// per CU, 128 x 128 two that fill each other's gaps, which the costs do not know: it has to be clearly cheaper.) Over those problems and 300
-// products more, that is 4.6 % quicker than by rows and tiles alone, and slower by more than 3 % for 8 of the 600 (16 % at most); 1.8 % slower than the
-// best shape. Us in 256 x 256 with last rows in 128 x 256 / in 128 x 256 / in 128 x 128, and what is chosen, 16 experts, 4 per token:
+double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
+  const int N = up ? 2 * g.Fp : g.Hp, nt = (N + t.bn - 1) / t.bn;
+  const double k = (up ? g.Hp : g.Fp) / 64.0, over = up ? t.up_us : t.down_us, tile_us = (up ? t.up_tile_us : t.down_tile_us) * k + over;
+  const MoeTiles tiles = expected_tiles((double)M * g.top / g.experts, t.bm, t.rest);
+  // a rest's tile beside whole ones takes about as long as kWide's; the more of the time all CUs are at rests, the more they wait for memory
+  const double rest_us = (1.03 + 0.49 * std::min(1.0, tiles.rest / std::max(tiles.whole, 1e-9))) * k + over / 2;
+  // the number of tiles is not known: a last round that a few of them begin counts as often as it comes
+  const double mean = tiles.whole * g.experts * nt, sd = nt * std::sqrt(g.experts * tiles.var), rest = tiles.rest * g.experts * nt;
+  auto at = [&](double z) { return moe_rounds_us(t, std::max(0.0, mean + z * sd), rest, tile_us, rest_us); };
+  return 0.25 * at(-1.22) + 0.5 * at(0.0) + 0.25 * at(1.22);
+}
+
+// The cheapest: 0 kTall, 1 kWide, 2 kSmall. (128 x 256 is one workgroup per CU, 128 x 128 two that fill each other's gaps, which the costs do not
+// know: it has to be clearly cheaper.) Over those products that is 1.0 % slower than the best shape; against a shape by rows per expert and
+// number of tiles alone 3.8 % quicker, and slower by more than 3 % for 27 of them (16 % at most). Us in 256 x 256 with last rows in 128 x 256 / in
+// 128 x 256 / in 128 x 128, and what is chosen, 16 experts, 4 per token:
 //   tokens, experts         gate and up                    down
 //   900, [2 x 2240][1536]   86.5 89.1 80.7 (128 x 128)     54.0 43.3 49.7 (128 x 256)
 //   1501                    103  115  112  (128 x 128)     57.4 77.7 69.3 (256 x 256)
@@ -656,13 +663,8 @@ double moe_shape_us(const MoeShape& t, const MoeGeom& g, int M, bool up) {
 //   2048                    541  628  675  (256 x 256)     285  314  360  (256 x 256)
 // (1501 tokens, gate and up: in the whole model 256 x 256 is half a percent of it quicker.)
 int moe_shape(const MoeGeom& g, int M, bool up) {
-  const long bands = (long)M * g.top / 128 + g.experts / 2;
-  const int plain = (long)M * g.top / g.experts >= 768                                                  ? 0
-                    : bands * (g.Hp / 256) >= 1000 || (up && bands * (2 * g.Fp / 256) >= 1000) ? 1
-                                                                                                        : 2;
-  const double us[3] = {moe_shape_us(kTall, g, M, up), moe_shape_us(kWide, g, M, up) / 0.93, moe_shape_us(kSmall, g, M, up)};
-  const int least = (int)(std::min_element(us, us + 3) - us);
-  return us[least] < 0.93 * us[plain] ? least : plain;
+  const double us[3] = {moe_shape_us(kTall, g, M, up), moe_shape_us(kWide, g, M, up) / 0.91, moe_shape_us(kSmall, g, M, up)};
+  return (int)(std::min_element(us, us + 3) - us);
 }
 
 // rows an expert has on average, too few of them for 128-row tiles

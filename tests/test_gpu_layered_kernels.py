@@ -101,14 +101,14 @@ def test_grouped_products_of_every_height(pkg, rows, hidden, experts, top, ff):
 # bf16: every pair of tiles that two products take, by their costs; row and column counts that are no multiples of them
 @pytest.mark.parametrize("rows,hidden,experts,top,ff,up,down", [
     (578, 123, 3, 1, 81, (128, 128), (128, 128)),
-    (1175, 1336, 3, 3, 63, (128, 128), (128, 256)),
-    (4767, 1170, 8, 2, 65, (128, 128), (256, 256)),    # an expert's last rows in 128 x 256, here and below
-    (5081, 1746, 2, 2, 211, (128, 256), (128, 128)),
-    (4367, 2438, 40, 4, 72, (128, 256), (128, 256)),
-    (4281, 2240, 40, 4, 76, (128, 256), (256, 256)),
-    (4336, 330, 16, 4, 333, (256, 256), (128, 128)),
-    (3228, 326, 8, 4, 490, (256, 256), (128, 256)),
-    (4486, 497, 8, 4, 334, (256, 256), (256, 256)),
+    (2517, 258, 40, 4, 432, (128, 128), (128, 256)),
+    (4459, 2725, 3, 1, 259, (128, 128), (256, 256)),   # an expert's last rows in 128 x 256, here and below
+    (3884, 826, 40, 4, 85, (128, 256), (128, 128)),
+    (5280, 880, 4, 1, 386, (128, 256), (128, 256)),
+    (3739, 1577, 4, 2, 260, (128, 256), (256, 256)),
+    (5819, 273, 40, 4, 210, (256, 256), (128, 128)),
+    (3596, 290, 8, 4, 448, (256, 256), (128, 256)),
+    (4132, 700, 40, 4, 257, (256, 256), (256, 256)),
 ])
 def test_grouped_products_of_every_pair_of_tiles(pkg, rows, hidden, experts, top, ff, up, down):
     for which, tile in ((0, up), (1, down)):
