@@ -109,6 +109,16 @@ StateGeom state_geom(const w4a32_decoder_config* c) {
     if (rc_ != W4A32_OK) return rc_; \
   } while (0)
 
+int quant_norm(const float* d_h, const float* d_delta, const float* d_weight, float eps, float* d_h_out, int M, int K,
+               void* d_ws, hipStream_t s, bool bytes) {
+  if (!d_h || !d_weight || !d_ws || M <= 0 || K <= 0) return W4A32_EINVAL;
+  if (d_delta && !d_h_out) return W4A32_EINVAL;
+  if (K % 32 != 0 || M <= w4::kGemvMaxM || !w4::quant_rows_fusable(K)) return W4A32_ESHAPE;
+  if ((reinterpret_cast<uintptr_t>(d_ws) & 255) != 0) return W4A32_EINVAL;
+  return from_hip(w4::launch_quant_lhs_norm(d_h, d_delta, d_weight, eps, d_h_out, M, K, static_cast<uint8_t*>(d_ws), s,
+                                            bytes));
+}
+
 // The model on M rows that are already embedded in the residual stream `h`. Leaves the last row's
 // logits in the state and the greedy token in *d_token_out. d_pos: device position of row 0.
 int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, uint8_t* st,
@@ -162,10 +172,9 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
           const uint8_t* down_prev = static_cast<const uint8_t*>(w->layers[l - 1].down);
           W4_TRY(from_hip(w4::launch_quant_lhs_norm_parts(h, gate, down_parts, w4::linear_bias(down_prev, H, I),
                                                           lw.attn_norm, c->rms_eps, h, M, H,
-                                                          static_cast<uint8_t*>(ws), s)));
+                                                          static_cast<uint8_t*>(ws), s, false)));
         } else {
-          W4_TRY(w4a32_quant_lhs_norm(h, l == 0 ? nullptr : delta, lw.attn_norm, c->rms_eps, h, M, H, ws,
-                                      stream));
+          W4_TRY(quant_norm(h, l == 0 ? nullptr : delta, lw.attn_norm, c->rms_eps, h, M, H, ws, s, false));
         }
         W4_TRY(w4a32_matmul_quantized_grouped(ys, ws, ps, ns, 3, M, H, stream));
       } else {
@@ -198,7 +207,12 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
                                                    lend, reinterpret_cast<unsigned int*>(st + g.pfcnt_off),
                                                    s)));
     }
-    W4_TRY(w4a32_matmul(delta, attn, lw.o, ws, M, qd, H, stream));
+    if (M > w4::kGemvMaxM) {
+      W4_TRY(from_hip(w4::launch_quant_lhs(attn, M, qd, qd, static_cast<uint8_t*>(ws), s, false)));
+      W4_TRY(w4a32_matmul_quantized(delta, ws, lw.o, M, qd, H, stream));
+    } else {
+      W4_TRY(w4a32_matmul(delta, attn, lw.o, ws, M, qd, H, stream));
+    }
     // h += attention output; xn = norm(h)
     {
       float* ys[2] = {gate, up};
@@ -206,7 +220,7 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
       const int ns[2] = {I, I};
       if (fuse_rows) {
         // gate, up, SiLU and the multiply in one launch: only silu(gate) * up is stored
-        W4_TRY(w4a32_quant_lhs_norm(h, delta, lw.ffn_norm, c->rms_eps, h, M, H, ws, stream));
+        W4_TRY(quant_norm(h, delta, lw.ffn_norm, c->rms_eps, h, M, H, ws, s, false));
         W4_TRY(w4a32_matmul_quantized_silu_pair(act, ws, lw.gate, lw.up, M, H, I, stream));
       } else {
         W4_TRY(from_hip(w4::launch_rmsnorm(h, delta, lw.ffn_norm, M, H, c->rms_eps, h, xn, s)));
@@ -214,12 +228,8 @@ int run_layers(const w4a32_decoder_config* c, const w4a32_decoder_weights* w, ui
       }
     }
     if (M > w4::kGemvMaxM) {
-      if (fuse_rows) {
-        W4_TRY(w4a32_quant_lhs(act, M, I, I, ws, stream));
-      } else {
-        W4_TRY(from_hip(w4::launch_silu_mul(gate, up, act, (size_t)M * I, s)));
-        W4_TRY(w4a32_quant_lhs(act, M, I, I, ws, stream));
-      }
+      if (!fuse_rows) W4_TRY(from_hip(w4::launch_silu_mul(gate, up, act, (size_t)M * I, s)));
+      W4_TRY(from_hip(w4::launch_quant_lhs(act, M, I, I, static_cast<uint8_t*>(ws), s, false)));
       // few output tiles, long K: split-K, with the partial sums in the gate and up buffers,
       // which are dead once the quantised rows of silu(gate) * up exist
       delta_in_parts = defer_sum && l + 1 < c->n_layers;
@@ -454,12 +464,7 @@ int w4a32_quant_lhs_norm_parts(const float* d_h, const void* d_parts, int parts,
 
 int w4a32_quant_lhs_norm(const float* d_h, const float* d_delta, const float* d_weight, float eps,
                          float* d_h_out, int M, int K, void* d_ws, void* stream) {
-  if (!d_h || !d_weight || !d_ws || M <= 0 || K <= 0) return W4A32_EINVAL;
-  if (d_delta && !d_h_out) return W4A32_EINVAL;
-  if (K % 32 != 0 || M <= w4::kGemvMaxM || !w4::quant_rows_fusable(K)) return W4A32_ESHAPE;
-  if ((reinterpret_cast<uintptr_t>(d_ws) & 255) != 0) return W4A32_EINVAL;
-  return from_hip(w4::launch_quant_lhs_norm(d_h, d_delta, d_weight, eps, d_h_out, M, K,
-                                            static_cast<uint8_t*>(d_ws), S(stream)));
+  return quant_norm(d_h, d_delta, d_weight, eps, d_h_out, M, K, d_ws, S(stream), true);
 }
 
 int w4a32_quant_lhs_silu_mul(const float* d_gate, const float* d_up, int M, int K, void* d_ws,

@@ -22,20 +22,21 @@ hipError_t launch_dequant(const uint8_t* packed, int N, int K, float* out, hipSt
 hipError_t launch_unpack_kai(const uint8_t* blob, int N, int K, int nr, int kr, int sr, uint8_t* u4,
                              uint16_t* scales, float* bias, hipStream_t s);
 
-// activations (every forward)
-hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s);
+// activations (every forward). `bytes`: whether a workspace that keeps int8 values (ws_has_bytes) gets them for more than
+// kGemvMaxM rows too; false only where no one reads its first rows by themselves: 0.2 us of a quantiser's 3 to 5
+hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s, bool bytes = true);
 // int8 values of the rows of a workspace that holds them as f16 alone (!ws_has_bytes(M))
 hipError_t launch_lhs_bytes(const uint8_t* ws, int M, int K, int8_t* out, hipStream_t s);
 // the quantiser with the operator that produces its rows in front (prefill sizes): residual add +
 // RMSNorm, or silu(gate) * up; K must satisfy quant_rows_fusable()
 bool quant_rows_fusable(int K);
 hipError_t launch_quant_lhs_norm(const float* h, const float* delta, const float* norm_w, float eps,
-                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s);
+                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s, bool bytes = true);
 // ... with delta = ((parts[0] + parts[1]) + ...) + bias, parts = [nparts][M][K] as launch_gemm_splitk leaves
 // them when it is given no output
 hipError_t launch_quant_lhs_norm_parts(const float* h, const float* parts, int nparts, const float* bias,
                                        const float* norm_w, float eps, float* h_out, int M, int K,
-                                       uint8_t* ws, hipStream_t s);
+                                       uint8_t* ws, hipStream_t s, bool bytes = true);
 hipError_t launch_quant_lhs_silu_mul(const float* gate, const float* up, int M, int K, uint8_t* ws,
                                      hipStream_t s);
 

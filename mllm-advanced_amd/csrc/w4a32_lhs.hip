@@ -5,6 +5,8 @@
 // the zero point is taken from the side with the smaller error, clamped, rounded to nearest
 // even; values are round_half_away(x * scale) + zero_point, clamped to int8. Every f32 product
 // and sum is an explicitly rounded intrinsic so no compiler flag can fuse them.
+#include <type_traits>
+
 #include "w4a32_internal.h"
 #include "w4a32_quant_math.h"
 
@@ -18,6 +20,10 @@ constexpr int kLhsThreads = 256;
 // f16 (a_q - zp; ah), tiled in MFMA operand order, for the f16 MFMA prefill kernel. Both forms of many rows
 // would be a third more stores (us with both / with f16 alone: [512][8960] 8.3 / 7.5, [1024][5120] 8.2 /
 // 7.6, [1024][1280] 5.2 / 4.3); who wants their int8 values has them made from the f16 ones (lhs_bytes_kernel).
+// kForm is known to the compiler: a test of the pointers cost 9 rows of [1536] .. [8960] 0.2 us of 3 to 5.
+constexpr int kFormBytes = 1, kFormHalves = 2;  // what is stored, or both
+
+template <int kForm>
 __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     const float* __restrict__ x, int K, int ldx, float* __restrict__ recip_out,
     int32_t* __restrict__ negzp_out, int8_t* __restrict__ aq, _Float16* __restrict__ ah) {
@@ -60,13 +66,13 @@ __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(f[e], p);
-    if (aq) {
+    if constexpr ((kForm & kFormBytes) != 0) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
     }
-    if (ah) {
+    if constexpr ((kForm & kFormHalves) != 0) {
       // a_q - zp lies in [-255, 255]: exact in f16. Stored in the order a weight dword unpacks.
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
@@ -91,7 +97,7 @@ __global__ __launch_bounds__(kLhsThreads) void quant_lhs_kernel(
 // the sum of squares is accumulated in another order than rmsnorm_kernel's.
 constexpr int kSrcPlain = 0, kSrcNorm = 1, kSrcSiluMul = 2;
 
-template <int SRC, int R>
+template <int SRC, int R, int kForm>
 __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
     const float* __restrict__ a, const float* __restrict__ b, const float* __restrict__ norm_w,
     const float* __restrict__ part_bias, float eps, int K, int lda, int nparts, size_t part_stride,
@@ -238,13 +244,13 @@ __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
     int q[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quant_one(v[r][e], p);
-    if (aq) {
+    if constexpr ((kForm & kFormBytes) != 0) {
       uint2 packed;
       packed.x = pack4(q);
       packed.y = pack4(q + 4);
       *reinterpret_cast<uint2*>(dst + i) = packed;
     }
-    if (ah) {
+    if constexpr ((kForm & kFormHalves) != 0) {
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
       h8 hv;
 #pragma unroll
@@ -259,60 +265,72 @@ __global__ __launch_bounds__(kLhsThreads) void quant_rows_kernel(
 // Largest K the register-resident kernel takes (8 values x 8 groups x 256 threads).
 constexpr int kQuantRowsMaxK = 8 * 8 * kLhsThreads;
 
+// f(the form that M rows are stored in)
+template <typename F>
+static hipError_t with_form(int M, bool bytes, F f) {
+  if (M <= kGemvMaxM) return f(std::integral_constant<int, kFormBytes>{});
+  if (bytes && ws_has_bytes(M)) return f(std::integral_constant<int, kFormBytes | kFormHalves>{});
+  return f(std::integral_constant<int, kFormHalves>{});
+}
+
 template <int SRC>
 static hipError_t launch_quant_rows(const float* a, const float* b, const float* norm_w, float eps,
                                     float* h_out, int M, int K, int lda, uint8_t* ws, hipStream_t s,
-                                    int nparts = 0, const float* part_bias = nullptr) {
+                                    bool bytes, int nparts = 0, const float* part_bias = nullptr) {
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = ws_has_bytes(M) ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
-  _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
+  int8_t* aq = reinterpret_cast<int8_t*>(ws + g.aq_off);
+  _Float16* ah = reinterpret_cast<_Float16*>(ws + g.ah_off);
   const int groups = (K + 8 * kLhsThreads - 1) / (8 * kLhsThreads);
-#define W4_LAUNCH_ROWS(R)                                                                          \
-  hipLaunchKernelGGL((quant_rows_kernel<SRC, R>), dim3(M), dim3(kLhsThreads), 0, s, a, b, norm_w,     \
+  return with_form(M, bytes, [&](auto form) {
+#define W4_LAUNCH_ROWS(R)                                                                                            \
+  hipLaunchKernelGGL((quant_rows_kernel<SRC, R, decltype(form)::value>), dim3(M), dim3(kLhsThreads), 0, s, a, b, norm_w, \
                      part_bias, eps, K, lda, nparts, (size_t)M * K, h_out, recip, negzp, aq, ah)
-  if (groups <= 1) W4_LAUNCH_ROWS(1);
-  else if (groups <= 2) W4_LAUNCH_ROWS(2);
-  else if (groups <= 5) W4_LAUNCH_ROWS(5);
-  else if (groups <= 8) W4_LAUNCH_ROWS(8);
-  else return hipErrorInvalidValue;
+    if (groups <= 1) W4_LAUNCH_ROWS(1);
+    else if (groups <= 2) W4_LAUNCH_ROWS(2);
+    else if (groups <= 5) W4_LAUNCH_ROWS(5);
+    else if (groups <= 8) W4_LAUNCH_ROWS(8);
+    else return hipErrorInvalidValue;
 #undef W4_LAUNCH_ROWS
-  return hipGetLastError();
+    return hipGetLastError();
+  });
 }
 
 bool quant_rows_fusable(int K) { return K <= kQuantRowsMaxK; }
 
 hipError_t launch_quant_lhs_norm(const float* h, const float* delta, const float* norm_w, float eps,
-                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s) {
-  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s);
+                                 float* h_out, int M, int K, uint8_t* ws, hipStream_t s, bool bytes) {
+  return launch_quant_rows<kSrcNorm>(h, delta, norm_w, eps, h_out, M, K, K, ws, s, bytes);
 }
 
 // The same with delta = the sum of a split-K product's `nparts` scaled parts ([nparts][M][K]) + bias.
 hipError_t launch_quant_lhs_norm_parts(const float* h, const float* parts, int nparts, const float* bias,
                                        const float* norm_w, float eps, float* h_out, int M, int K,
-                                       uint8_t* ws, hipStream_t s) {
+                                       uint8_t* ws, hipStream_t s, bool bytes) {
   if (nparts < 1 || !parts || !bias) return hipErrorInvalidValue;
-  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, nparts, bias);
+  return launch_quant_rows<kSrcNorm>(h, parts, norm_w, eps, h_out, M, K, K, ws, s, bytes, nparts, bias);
 }
 
 hipError_t launch_quant_lhs_silu_mul(const float* gate, const float* up, int M, int K, uint8_t* ws,
                                      hipStream_t s) {
-  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s);
+  return launch_quant_rows<kSrcSiluMul>(gate, up, nullptr, 0.0f, nullptr, M, K, K, ws, s, true);
 }
 
-hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s) {
+hipError_t launch_quant_lhs(const float* x, int M, int K, int ldx, uint8_t* ws, hipStream_t s, bool bytes) {
   if (K <= kQuantRowsMaxK) {
-    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s);
+    return launch_quant_rows<kSrcPlain>(x, nullptr, nullptr, 0.0f, nullptr, M, K, ldx, ws, s, bytes);
   }
   const WsGeom g = ws_geom(M, K);
   float* recip = reinterpret_cast<float*>(ws + g.scale_off);
   int32_t* negzp = reinterpret_cast<int32_t*>(ws + g.off_off);
-  int8_t* aq = ws_has_bytes(M) ? reinterpret_cast<int8_t*>(ws + g.aq_off) : nullptr;
-  _Float16* ah = (M > kGemvMaxM) ? reinterpret_cast<_Float16*>(ws + g.ah_off) : nullptr;
-  hipLaunchKernelGGL(quant_lhs_kernel, dim3(M), dim3(kLhsThreads), 0, s, x, K, ldx, recip, negzp,
-                     aq, ah);
-  return hipGetLastError();
+  int8_t* aq = reinterpret_cast<int8_t*>(ws + g.aq_off);
+  _Float16* ah = reinterpret_cast<_Float16*>(ws + g.ah_off);
+  return with_form(M, bytes, [&](auto form) {
+    hipLaunchKernelGGL(quant_lhs_kernel<decltype(form)::value>, dim3(M), dim3(kLhsThreads), 0, s, x, K, ldx, recip, negzp, aq,
+                       ah);
+    return hipGetLastError();
+  });
 }
 
 // The int8 values of rows that were stored as f16 (a_q - zp): exact, both are whole numbers within 255.
